@@ -16,8 +16,8 @@ the factor.
 The reference-mode path (fib_step) keeps the reference's factor 1.1: its
 list sets are part of the parity contract.
 
-The launch tiles (fib_set_tiles: legs per stage run of the vertex pass and
-neighbour loads in flight per lane, cells per wavefront of the list build)
+The launch tiles (fib_set_tiles: legs per write-out of the vertex pass and
+loads it keeps in flight, cells per wavefront of the list build)
 change no result, bit for bit, only the time; tune_tiles measures them on a
 live handle, one after the other.
 """
@@ -28,7 +28,7 @@ import time
 from .gpu import FibGPU, GPUError, default_params
 
 CANDIDATES = (1.10, 1.15, 1.20, 1.25, 1.30)
-# (legs per stage run, loads in flight per lane) of the vertex pass; cells
+# (legs per write-out, loads in flight) of the vertex pass; cells
 # per wavefront of the list build
 TRI_TILES = ((256, 4), (256, 2), (128, 4), (128, 2))
 NB_CELLS = (8, 4, 16)
@@ -84,7 +84,7 @@ def _ms_per_step(g, steps, warmup):
 
 def tune_tiles(g, steps=30, warmup=5, tri_tiles=TRI_TILES, nb_cells=NB_CELLS):
     """Launch tiles of a live handle in MD-step mode (ions fired, mid-run):
-    first the vertex pass's (stage size, loads in flight), then the list
+    first the vertex pass's (write-out size, loads in flight), then the list
     build's cells per wavefront with the best of those, each timed over
     `steps` MD steps after `warmup`.  Leaves the handle in the best tiles and
     returns (best (tri_ns, tri_batch, nb_cells), [(tiles, ms per step)])."""

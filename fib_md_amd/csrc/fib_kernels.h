@@ -62,9 +62,9 @@ struct DevBufs {
   int total_cells;           // total real cells
   int Wsw, Wion;             // ELL widths
   int cur;                   // current buffer of the double-buffered arrays
-  // launch tiles (0: the defaults): legs per k_tri stage run and legs per
-  // lane in flight; cells per k_nbuild wavefront.  Results do not depend on
-  // them, only the time.
+  // launch tiles (0: the defaults): legs per k_tri write-out (twice over)
+  // and its loads in flight; cells per k_nbuild wavefront.  Results do not
+  // depend on them, only the time.
   int tri_ns = 0, tri_tb = 0, nb_cells = 0;
   DInst *I;                  // [ninst]
   DCtl *ctl;                 // [ninst]
@@ -81,7 +81,6 @@ struct DevBufs {
   uint32_t *RA;              // per leg [NA * Wsw]: index into G of the partner's force
                              // on the atom (~0: none); needs NA * Wsw < 2^32
   uint64_t *amask;           // legs of the last evaluation, by list slot [NA]
-  int *cnt_leg;              // legs per atom of the last evaluation [NA]
   double *Fpart, *upart;     // own-term force and energy [3*NA], [NA]
   double4 *Xb;               // positions at the last list build [NA]
   float *disp;               // |X - Xb| after the last position update [NA]

@@ -32,6 +32,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "fib_device.h"
 #include "fib_kernels.h"
@@ -1034,41 +1035,42 @@ struct Leg {
   T rinv;        // 1/r (FP64: m^-1; mixed: sigma_Si^-1)
   T E;           // exp(gamma/(r/sigma - a))
   T g;           // d ln E / dr (same length unit as rinv)
-  uint32_t ks;   // neighbour index | (species == Ge) << 31
-  uint32_t slot; // list slot of the neighbour in the centre's row
-  uint32_t elo;  // mixed: low parts of e0, e1, e2 (see pack_lo); FP64: 0
+  T l0, l1, l2;  // mixed: low parts of e0, e1, e2 (see low_part); FP64: 0
 };
 
-// Low part of an FP32 unit-vector component h of the FP64 value x, in
-// units of ulp(h) / 1024 as a signed 10-bit field c of a word (|x - h| <=
-// ulp(h) / 2, so the field carries x - h to 2^-34 of |h|).  The three
-// fields ride in one word of the vertex pass's stage; with them the pass
-// forms cos + 1/3 from (nearly) the FP64 unit vectors, where it cancels
-// near the tetrahedral angle.
-__device__ __forceinline__ float ulp_of(float h) {
-  const uint32_t ex = __float_as_uint(h) & 0x7f800000u;
-  return ex > (23u << 23) ? __uint_as_float(ex - (23u << 23)) : 0.0f;
+// sqrt(a) and 1/sqrt(a) of a positive a (a squared distance, far from the
+// ends of the exponent range): the hardware's estimate (24 bits), one
+// Goldschmidt step and two residual corrections of the root, one Newton step
+// of its reciprocal -- 13 operations instead of the 28 of sqrt() and a
+// division, each within 1 ulp.
+__device__ __forceinline__ void sqrt_rsqrt(double a, double &s, double &si) {
+  const double y = __builtin_amdgcn_rsq(a);
+  double g = a * y, h = 0.5 * y;
+  const double e = __builtin_fma(-h, g, 0.5);
+  g = __builtin_fma(g, e, g);
+  h = __builtin_fma(h, e, h);
+  g = __builtin_fma(__builtin_fma(-g, g, a), h, g);
+  s = __builtin_fma(__builtin_fma(-g, g, a), h, g);
+  const double y1 = h + h;
+  si = __builtin_fma(y1, __builtin_fma(-s, y1, 1.0), y1);
 }
-__device__ __forceinline__ uint32_t pack_lo(double x, float h, int c) {
-  const float u = ulp_of(h);
-  if (!(u > 0.0f)) return 0u;
-  const int q = min(max((int)rint((x - (double)h) * (1024.0 / (double)u)), -511), 511);
-  return ((uint32_t)q & 0x3ffu) << (10 * c);
+// 1/x (x far from the ends of the exponent range): estimate and two Newton
+// steps, within 1 ulp
+__device__ __forceinline__ double fast_rcp(double x) {
+  double y = __builtin_amdgcn_rcp(x);
+  y = __builtin_fma(y, __builtin_fma(-x, y, 1.0), y);
+  return __builtin_fma(y, __builtin_fma(-x, y, 1.0), y);
 }
-__device__ __forceinline__ int lo_field(uint32_t w, int c) {
-  return (int)(w << (22 - 10 * c)) >> 22;
-}
-// the field times ulp(h) / 1024: for h = m 2^e with m in [0.5, 1), ulp(h)
-// = 2^(e - 24), so the field times 2^(e - 34) (h = 0 carries a zero field)
-__device__ __forceinline__ float lo_part(uint32_t w, float h, int c) {
-  return __builtin_amdgcn_ldexpf((float)lo_field(w, c), __builtin_amdgcn_frexp_expf(h) - 34);
-}
-// the low parts of the reversed vector
-__device__ __forceinline__ uint32_t neg_lo(uint32_t w) {
-  uint32_t r = 0;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) r |= ((uint32_t)(-lo_field(w, c)) & 0x3ffu) << (10 * c);
-  return r;
+
+// Low part of an FP32 unit-vector component h = fl(x) of the FP64 value x:
+// x - h rounded to a multiple of ulp(h)/1024 (a 10-bit number), as FP32.
+// With the low parts the vertex pass forms cos + 1/3 from (nearly) the FP64
+// unit vectors, where it cancels near the tetrahedral angle.  For h = m 2^e
+// with m in [0.5, 1), ulp(h) = 2^(e - 24); adding and taking away
+// 1.5 2^(e + 18) rounds to multiples of 2^(e - 34).
+__device__ __forceinline__ float low_part(double x, float h) {
+  const double big = __builtin_amdgcn_ldexp(1.5, __builtin_amdgcn_frexp_expf(h) + 18);
+  return (float)(((x - (double)h) + big) - big);
 }
 // a + b - s exactly, for s = fl(a + b) (TwoSum)
 __device__ __forceinline__ float two_sum_err(float a, float b, float s) {
@@ -1076,46 +1078,26 @@ __device__ __forceinline__ float two_sum_err(float a, float b, float s) {
   return (a - (s - bb)) + (b - bb);
 }
 
-__device__ __forceinline__ double ks_pack(double, uint32_t ks) {
-  return __longlong_as_double((long long)ks);
+// cos and D = cos + 1/3 of a vertex term with legs a and b, the same bits
+// for (a, b) and (b, a).
+__device__ __forceinline__ void cos_d(const Leg<double> &a, const Leg<double> &b, double &cs,
+                                      double &D) {
+  cs = a.e0 * b.e0 + a.e1 * b.e1 + a.e2 * b.e2;
+  D = cs + 1.0 / 3.0;
 }
-__device__ __forceinline__ float ks_pack(float, uint32_t ks) { return __uint_as_float(ks); }
-__device__ __forceinline__ uint32_t ks_unpack(double v) {
-  return (uint32_t)__double_as_longlong(v);
-}
-__device__ __forceinline__ uint32_t ks_unpack(float v) { return __float_as_uint(v); }
-__device__ __forceinline__ int ks_index(uint32_t ks) { return (int)(ks & 0x7fffffffu); }
-__device__ __forceinline__ int ks_ge(uint32_t ks) { return (int)(ks >> 31); }
-
-// Force on leg a of one vertex term (centre c, legs a and b), and h.
-// h = leps E(ra) E(rb) (cos+1/3)^2 with d cos/dx_a = -(e_b - cos e_a)/r_a and
-// d r_a/dx_a = -e_a, so F_a = -dh/dx_a = h g_a e_a + 2 leps Ea Eb D (e_b - cos e_a)/r_a.
-template <typename T>
-__device__ __forceinline__ void vterm(T leps, const Leg<T> &a, const Leg<T> &b, T *Fa, T &hh) {
-  const T cs = a.e0 * b.e0 + a.e1 * b.e1 + a.e2 * b.e2;
-  const T D = cs + T(1.0 / 3.0);
-  const T Eab = leps * a.E * b.E;
-  hh = Eab * D * D;
-  const T c1 = hh * a.g;
-  const T c2 = T(2) * Eab * D * a.rinv;
-  Fa[0] = c1 * a.e0 + c2 * (b.e0 - cs * a.e0);
-  Fa[1] = c1 * a.e1 + c2 * (b.e1 - cs * a.e1);
-  Fa[2] = c1 * a.e2 + c2 * (b.e2 - cs * a.e2);
-}
-// Mixed: cos and D = cos + 1/3 from the FP32 unit vectors and their low
-// parts, with the products' rounding errors (FMA) and the sums' (TwoSum)
-// carried along, each rounded to FP32 once; the rest of the term in FP32.
-// (The products and sums of cos_d stay unfused: an FMA formed from a
-// product and the following sum would break the TwoSum error terms.)
+// Mixed: from the FP32 unit vectors and their low parts, with the products'
+// rounding errors (FMA) and the sums' (TwoSum) carried along, each rounded
+// to FP32 once; the rest of the term is FP32.  (The products and sums stay
+// unfused: an FMA formed from a product and the following sum would break
+// the TwoSum error terms.)
 __device__ __forceinline__ void cos_d(const Leg<float> &a, const Leg<float> &b, float &cs,
                                       float &D) {
 #pragma clang fp contract(off)
   const float p0 = a.e0 * b.e0, p1 = a.e1 * b.e1, p2 = a.e2 * b.e2;
   const float rp = (__builtin_fmaf(a.e0, b.e0, -p0) + __builtin_fmaf(a.e1, b.e1, -p1)) +
                    __builtin_fmaf(a.e2, b.e2, -p2);
-  const float x = ((a.e0 * lo_part(b.elo, b.e0, 0) + lo_part(a.elo, a.e0, 0) * b.e0) +
-                   (a.e1 * lo_part(b.elo, b.e1, 1) + lo_part(a.elo, a.e1, 1) * b.e1)) +
-                  (a.e2 * lo_part(b.elo, b.e2, 2) + lo_part(a.elo, a.e2, 2) * b.e2);
+  const float x = ((a.e0 * b.l0 + a.l0 * b.e0) + (a.e1 * b.l1 + a.l1 * b.e1)) +
+                  (a.e2 * b.l2 + a.l2 * b.e2);
   const float s1 = p0 + p1, s2 = s1 + p2;
   const float lo = (two_sum_err(p0, p1, s1) + two_sum_err(s1, p2, s2)) + (rp + x);
   cs = s2 + lo;
@@ -1124,18 +1106,22 @@ __device__ __forceinline__ void cos_d(const Leg<float> &a, const Leg<float> &b, 
   const float s3 = s2 + THIRD_HI;
   D = s3 + (two_sum_err(s2, THIRD_HI, s3) + (lo + THIRD_LO));
 }
-template <>
-__device__ __forceinline__ void vterm<float>(float leps, const Leg<float> &a, const Leg<float> &b,
-                                             float *Fa, float &hh) {
-  float cs, D;
-  cos_d(a, b, cs, D);
-  const float Eab = leps * a.E * b.E;
+__device__ __forceinline__ double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ __forceinline__ float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+// Force on leg a of one vertex term (centre c, legs a and b), and h.
+// h = leps E(ra) E(rb) D^2, D = cos + 1/3, with d cos/dx_a = -(e_b - cos e_a)/r_a and
+// d r_a/dx_a = -e_a, so F_a = -dh/dx_a = h g_a e_a + 2 leps Ea Eb D (e_b - cos e_a)/r_a.
+template <typename T>
+__device__ __forceinline__ void vterm(T leps, const Leg<T> &a, const Leg<T> &b, T cs, T D, T *Fa,
+                                      T &hh) {
+  const T Eab = leps * a.E * b.E;
   hh = Eab * D * D;
-  const float c1 = hh * a.g;
-  const float c2 = 2.0f * Eab * D * a.rinv;
-  Fa[0] = c1 * a.e0 + c2 * (b.e0 - cs * a.e0);
-  Fa[1] = c1 * a.e1 + c2 * (b.e1 - cs * a.e1);
-  Fa[2] = c1 * a.e2 + c2 * (b.e2 - cs * a.e2);
+  const T c1 = hh * a.g;
+  const T c2 = T(2) * Eab * D * a.rinv;
+  // (fused by hand: the rounding does not depend on the compiler's choice)
+  Fa[0] = fma_t(fma_t(-cs, a.e0, b.e0), c2, c1 * a.e0);
+  Fa[1] = fma_t(fma_t(-cs, a.e1, b.e1), c2, c1 * a.e1);
+  Fa[2] = fma_t(fma_t(-cs, a.e2, b.e2), c2, c1 * a.e2);
 }
 
 // Minimum image with v_rndne (ties to even).  Neighbour pairs are far from
@@ -1156,27 +1142,21 @@ __device__ __forceinline__ T pick4(const T (&v)[4], int n) {
   return n == 0 ? v[0] : n == 1 ? v[1] : n == 2 ? v[2] : v[3];
 }
 
-// The leg from centre c to neighbour n (unit vector from n to c, 1/r, E, g),
-// with k_legs' arithmetic: FP64 as the reference (si.f90:491-509), or the
-// FP32 terms of the mixed mode.  Legs are not stored between passes: k_legs
-// decides which pairs are legs (its leg mask), and the passes that need the
-// values recompute them here from the positions.
+// The leg of difference d = x_centre - x_neighbour (unit vector from the
+// neighbour to the centre, 1/r, E, g), with k_legs' arithmetic: FP64 as the
+// reference (si.f90:491-509), or the FP32 terms of the mixed mode.  Legs are
+// not stored between passes: k_legs decides which pairs are legs (its leg
+// mask), and the passes that need the values recompute them here from the
+// positions.
 template <bool MIXED>
-__device__ __forceinline__ void make_leg(const double4 &xc, const double4 &xn, const DInst &in,
-                                         const FConst &fc, int tc, int tn, uint32_t jn,
-                                         uint32_t slot, Leg<typename Prec<MIXED>::T> &L) {
-  double d0, d1, d2;
-  min_image_fast(xc, xn, in, d0, d1, d2);
-  const double isg = fc.isig[tc == 2 ? 1 : 0][tn == 2 ? 1 : 0];
-  L.ks = jn | (tn == 2 ? 0x80000000u : 0u);
-  L.slot = slot;
-  L.elo = 0u;
-  if (!MIXED) {
-    const double rr = d0 * d0 + d1 * d1 + d2 * d2;
-    const double r = sqrt(rr);
-    const double rinv = 1.0 / r;
-    const double rs = r * isg;
-    const double inv_ra = 1.0 / (rs - fc.al);
+__device__ __forceinline__ void leg_values(double d0, double d1, double d2, double isg,
+                                           float rhof, const FConst &fc,
+                                           Leg<typename Prec<MIXED>::T> &L) {
+  L.l0 = L.l1 = L.l2 = 0;
+  if constexpr (!MIXED) {
+    double r, rinv;
+    sqrt_rsqrt(d0 * d0 + d1 * d1 + d2 * d2, r, rinv);
+    const double inv_ra = fast_rcp(r * isg - fc.al);
     L.e0 = d0 * rinv; L.e1 = d1 * rinv; L.e2 = d2 * rinv;
     L.rinv = rinv;
     L.E = exp(fc.gamma * inv_ra);
@@ -1185,17 +1165,26 @@ __device__ __forceinline__ void make_leg(const double4 &xc, const double4 &xn, c
     // every leg value from FP64 geometry, rounded to FP32 once: the FP32
     // vertex terms cannot recover accuracy their inputs do not carry
     const double s0 = d0 * isg, s1 = d1 * isg, s2 = d2 * isg;
-    const double rs = sqrt(s0 * s0 + s1 * s1 + s2 * s2);
-    const double rinv = 1.0 / rs;
-    const double inv_ra = 1.0 / (rs - fc.al);
-    const double rho = fc.rho[tc == 2 ? 1 : 0][tn == 2 ? 1 : 0];
+    double rs, rinv;
+    sqrt_rsqrt(s0 * s0 + s1 * s1 + s2 * s2, rs, rinv);
+    const double inv_ra = fast_rcp(rs - fc.al);
+    const double rho = rhof;
     const double x0 = s0 * rinv, x1 = s1 * rinv, x2 = s2 * rinv;
     L.e0 = (float)x0; L.e1 = (float)x1; L.e2 = (float)x2;
-    L.elo = pack_lo(x0, L.e0, 0) | pack_lo(x1, L.e1, 1) | pack_lo(x2, L.e2, 2);
+    L.l0 = low_part(x0, L.e0); L.l1 = low_part(x1, L.e1); L.l2 = low_part(x2, L.e2);
     L.rinv = (float)(rinv * rho);
     L.E = expf((float)(fc.gamma * inv_ra));
     L.g = (float)(-fc.gamma * inv_ra * inv_ra * rho);
   }
+}
+template <bool MIXED>
+__device__ __forceinline__ void make_leg(const double4 &xc, const double4 &xn, const DInst &in,
+                                         const FConst &fc, int tc, int tn,
+                                         Leg<typename Prec<MIXED>::T> &L) {
+  double d0, d1, d2;
+  min_image_fast(xc, xn, in, d0, d1, d2);
+  const int a = tc == 2 ? 1 : 0, b = tn == 2 ? 1 : 0;
+  leg_values<MIXED>(d0, d1, d2, fc.isig[a][b], fc.rho[a][b], fc, L);
 }
 
 // k_legs: list slots whose positions are loaded together (4 or 8).  Eight
@@ -1236,7 +1225,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
     const double4 *__restrict__ X, const DInst *__restrict__ I, const FConst fc,
     const TabEntry *__restrict__ tab, int NA, int Wsw, int Wion, const int *__restrict__ cnt_sw,
     const int *__restrict__ nbr_sw, const int *__restrict__ cnt_ion,
-    const int *__restrict__ nbr_ion, int *__restrict__ cnt_leg, uint64_t *__restrict__ amask,
+    const int *__restrict__ nbr_ion, uint64_t *__restrict__ amask,
     double *__restrict__ Fpart, double *__restrict__ upart, int pstride,
     double *__restrict__ partials, const int *__restrict__ halt) {
   HALT_OR_RETURN(halt);
@@ -1276,7 +1265,6 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
     W[6] += d2 * f0; W[7] += d2 * f1; W[8] += d2 * f2;
   };
 
-  int na = 0;
   uint64_t am = 0;
   // one buffered SW pair in list slot k: pair force, pair energy, leg
   auto pair = [&](int k, int jn, const double4 &xj) {
@@ -1315,7 +1303,6 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
           etot += ul;
         }
         am |= 1ull << k;
-        ++na;
       }
     } else {
       // Pair geometry in FP64 (pair units: sigma_ij), the pair force factor
@@ -1353,7 +1340,6 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
       // three-body sum: each of their terms is below 1e-9 eps/sigma
       if (rs < fc.mixed_xleg) {
         am |= 1ull << k;
-        ++na;
       }
     }
   };
@@ -1391,7 +1377,6 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
         if (k0 + v < cs) pair(k0 + v, jq[v], xq[v]);
     }
   }
-  st_nt<NTS>(cnt_leg + i, na);
   st_nt<NTS>(amask + i, am);
 
   // ---- Moliere pairs (si.f90:426-446): both atoms must be fired ----------
@@ -1467,48 +1452,70 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
 }
 
 
-// Lane-per-leg three-body pass.  Block = 4 wavefronts, each owning 64
-// consecutive atoms.  A wavefront computes the legs of a run of its atoms
-// (the pairs of their leg masks, from the positions) into LDS, so the vertex
-// terms, which read every leg of the centre once per leg, read LDS; no leg
-// record goes through HBM.  Runs end on atom boundaries and hold at most
-// TriStage::N legs.
+// Lane-per-leg three-body pass.  Block = 4 independent wavefronts, each
+// owning 64 consecutive atoms, whose legs (the pairs of their leg masks) it
+// takes in passes of whole atoms with at most 64 legs: one lane computes one
+// leg from the positions, and the legs of a pass share their values through
+// a small LDS stage; no leg record goes through HBM.  The pass is bound by
+// vector instructions (0.75 to 0.85 of a CU's issue cycles), so it is laid
+// out to need few of them:
+//  - every lane works on a leg, in the stage as in the terms;
+//  - mixed: the compensated cos + 1/3, two thirds of a vertex term's
+//    instructions and the same for both of its legs, is formed once per
+//    unordered pair.  Leg a of an atom's n takes the partners a + 1 ..
+//    a + n/2 around the ring of legs (of an even ring's opposite pairs, the
+//    first half takes them) and hands cos and D to both legs through LDS;
+//    then each leg sums its terms in leg order.  Atoms with more than
+//    TRI_QROWS legs have it formed per term instead.
+//  - the Ge selections are left out of passes without a Ge atom.
+// Results wait in LDS and leave plane by plane for up to NS/2 legs at once,
+// so that the stores coalesce.
+// 4 x 512 k thermal Si atoms, per step: mixed 4,903 vector instructions per
+// wavefront and 300 us with one term per (leg, partner), 3,090 and 213 us
+// so; FP64 245 -> 173 us (2 x 512 k).
 #ifndef TRI_BATCH
-#define TRI_BATCH 4  // legs per lane whose neighbour loads are in flight together
+#define TRI_BATCH 4  // 4: the next pass's positions load during this one; 2: only its row entries
 #endif
 #ifndef TRI_NS_MIXED
-#define TRI_NS_MIXED 256  // legs per stage run (mixed)
+#define TRI_NS_MIXED 256  // legs per write-out (mixed)
 #endif
 #ifndef TRI_NS_FP64
-#define TRI_NS_FP64 256  // legs per stage run (FP64); 128 measured 10 % slower on the dose batch
+#define TRI_NS_FP64 256  // legs per write-out (FP64)
 #endif
+#define TRI_QROWS 8   // most legs of an atom whose pairs share cos + 1/3 (mixed)
+#define TRI_TAB 384   // legs whose owner and list slot are tabled at once
 template <bool MIXED>
 struct TriStage {
-  static constexpr int N = MIXED ? TRI_NS_MIXED : TRI_NS_FP64;  // legs per run
+  static constexpr int N = MIXED ? TRI_NS_MIXED : TRI_NS_FP64;
 };
+// p[byte offset]: one 32-bit offset beside a scalar base, not a 64-bit
+// address per lane
+template <typename V>
+__device__ __forceinline__ V ld_off(const V *p, uint32_t byte) {
+  return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(p) + byte);
+}
 template <bool MIXED, bool EN, bool VIR, int NS, int TB>
 __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
     const double4 *__restrict__ X, const DInst *__restrict__ I, const FConst fc, int NA,
-    int Wsw, const int *__restrict__ cnt_leg, const int *__restrict__ nbr_sw,
-    uint16_t *__restrict__ rk_sw, const uint8_t *__restrict__ off_sw,
-    const uint64_t *__restrict__ amask, typename Prec<MIXED>::T4 *__restrict__ G,
-    uint32_t *__restrict__ RA, int pstride, double *__restrict__ partials,
-    const int *__restrict__ halt) {
+    int Wsw, const int *__restrict__ nbr_sw, uint16_t *__restrict__ rk_sw,
+    const uint8_t *__restrict__ off_sw, const uint64_t *__restrict__ amask,
+    typename Prec<MIXED>::T4 *__restrict__ G, uint32_t *__restrict__ RA, int pstride,
+    double *__restrict__ partials, const int *__restrict__ halt) {
   HALT_OR_RETURN(halt);
   typedef typename Prec<MIXED>::T T;
   typedef typename Prec<MIXED>::T4 T4;
-  constexpr int NW = FIB_BLOCK / FIB_WAVE;
+  constexpr int NW = FIB_BLOCK / FIB_WAVE, QR = TRI_QROWS, FL = NS / 2;
   constexpr bool NT = (FIB_NT_LD & 2) != 0, NTS = (FIB_NT_ST & 2) != 0;
-  // sA: e0, e1, e2 and E, negated when the leg's atom is Ge (E > 0);
-  // sB: g, 1/r, neighbour bits, list slot bits
-  __shared__ T4 sA[NW][NS];
-  __shared__ T4 sB[NW][NS];
-  __shared__ uint8_t owner[NW][NS];
-  __shared__ int soff[NW][FIB_WAVE + 1];
-  __shared__ uint8_t sge[NW][FIB_WAVE];
-  __shared__ uint32_t sR[NW][NS];
+  constexpr bool U = EN || VIR;  // the terms' energies are wanted
+  __shared__ T4 sE[NW][FIB_WAVE];  // e0, e1, e2 and E, negated when the leg's atom is Ge (E > 0)
+  __shared__ float4 sL[NW][MIXED ? FIB_WAVE : 1];       // l0, l1, l2
+  __shared__ float2 sQ[NW][MIXED ? QR * FIB_WAVE : 1];  // [partner][leg]: cos, D
+  __shared__ T4 sG[NW][FL];
+  __shared__ uint32_t sR[NW][FL];
+  __shared__ uint16_t tab[NW][TRI_TAB];  // owner lane | list slot << 6
   const int lb = xcd_remap(blockIdx.x, gridDim.x);
-  const int lane = threadIdx.x % FIB_WAVE, wid = threadIdx.x / FIB_WAVE;
+  const int lane = threadIdx.x % FIB_WAVE;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / FIB_WAVE);
   const int i0 = lb * FIB_BLOCK + wid * FIB_WAVE;
   const double escale = MIXED ? fc.eps[0][0] : 1.0;
   const double fscale = MIXED ? fc.eps[0][0] * fc.isig[0][0] : 1.0;
@@ -1519,194 +1526,221 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
   const T lp[4] = {(T)(fc.leps[0][0][0] * lu), (T)(fc.leps[0][0][1] * lu),
                    (T)(fc.leps[0][1][1] * lu), (T)(fc.leps[1][1][1] * lu)};
 
-  // legs of the wave's atoms: exclusive prefix sum in LDS
-  const int nl = ld_nt<NT>(cnt_leg + i0 + lane);
-  int inc = nl;
-  for (int o = 1; o < FIB_WAVE; o <<= 1) {
-    const int y = __shfl_up(inc, o);
-    if (lane >= o) inc += y;
-  }
-  soff[wid][lane] = inc - nl;
-  if (lane == FIB_WAVE - 1) soff[wid][FIB_WAVE] = inc;
   // this lane's atom as a centre; every block lies inside one instance
   const int ic = i0 + lane;
   const double4 xc = X[ic];
   const int tci = type_of(meta_of(xc));
   const uint64_t amc = amask[ic];
   const DInst &in = I[__builtin_amdgcn_readfirstlane(inst_of(meta_of(xc)))];
-  sge[wid][lane] = (tci == 2) ? 1 : 0;
+  // legs of the wave's atoms: this atom's are [exc, inc)
+  const int nl = __popcll(amc);
+  int inc = nl;
+  for (int o = 1; o < FIB_WAVE; o <<= 1) {
+    const int y = __shfl_up(inc, o);
+    if (lane >= o) inc += y;
+  }
+  const int exc = inc - nl;
 
-  T uc = 0;
+  double uc = 0;
   T W[9];
 #pragma unroll
   for (int w = 0; w < 9; ++w) W[w] = 0;
 
-  for (int o0 = 0; o0 < FIB_WAVE;) {
-    // run of atoms [o0, o1) whose legs [s0, s1) fit the stage (an atom has
-    // at most Wsw <= 64 legs, so every run takes at least one atom)
-    const int s0 = __shfl(inc - nl, o0);
-    const uint64_t fit = __ballot(lane >= o0 && inc - s0 <= NS);
-    const int o1 = o0 + __popcll(fit);
-    const int s1 = __shfl(inc, o1 - 1);
-    const bool mine = lane >= o0 && lane < o1;
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // owner of every leg of the run (LDS only), so that the stage below can
-    // give each lane legs rather than atoms
-    if (mine)
-      for (int a = 0; a < nl; ++a) owner[wid][inc - nl + a - s0] = (uint8_t)lane;
+  // results of the legs [fs, ...) of the atoms [f0, f1) wait in sG and sR
+  int f0 = 0, fs = 0;
+  auto write_out = [&](int f1) {
     wave_lds_sync();
-    // stage: one lane per leg, in list order within each atom, computed from
-    // the positions; TB legs per lane with their loads in flight together,
-    // every lane busy whatever the atoms' leg counts
-    {
-      const int nq = s1 - s0;
-      const int amlo = (int)(uint32_t)amc, amhi = (int)(uint32_t)(amc >> 32);
-      for (int q0 = 0; q0 < nq; q0 += FIB_WAVE * TB) {
-        int qv[TB], ov[TB], kq[TB], jq[TB], rq[TB];
-#pragma unroll
-        for (int u = 0; u < TB; ++u) {
-          qv[u] = q0 + u * FIB_WAVE + lane;
-          const bool ok = qv[u] < nq;
-          ov[u] = ok ? owner[wid][min(qv[u], NS - 1)] : 0;
-          // the owner's leg mask, from the owner's lane (every lane takes part)
-          const uint64_t am = ((uint64_t)(uint32_t)__shfl(amhi, ov[u]) << 32) |
-                              (uint64_t)(uint32_t)__shfl(amlo, ov[u]);
-          kq[u] = ok ? nth_bit(am, qv[u] + s0 - soff[wid][ov[u]]) : 0;
-          const size_t rw = (size_t)(i0 + ov[u]) * Wsw;
-          jq[u] = ok ? ld_nt<NT>(nbr_sw + rw + kq[u]) : i0 + ov[u];
-          rq[u] = ok ? (int)ld_nt<NT>(rk_sw + rw + kq[u]) : 0xffff;
-        }
-        // Where the partner j keeps the force of its own terms on the owner:
-        // G[n * NA + j], n = j's leg index of the owner.  The slot r of the
-        // owner in j's row follows from the stencil offsets (see k_nbuild), n
-        // from j's leg mask (legs are symmetric); 255 offsets (r >= Wsw)
-        // mark a j without a row.  The first time a pair is a leg after a
-        // build, r is worked out from j's offsets and kept in the row entry
-        // (RK_SLOT set); later steps read it there, without the gather of
-        // j's offsets.
-        double4 xq[TB];
-        uint64_t aq[TB];
-        int oq[TB];
-#pragma unroll
-        for (int u = 0; u < TB; ++u) {
-          xq[u] = X[jq[u]];
-          aq[u] = amask[jq[u]];
-          oq[u] = (rq[u] & RK_SLOT) ? 0 : off_sw[(size_t)jq[u] * OFF_W + 26 - (rq[u] >> 8)];
-        }
-#pragma unroll
-        for (int u = 0; u < TB; ++u) {
-          // the owner's position and species, from the owner's lane
-          double4 xo;
-          xo.x = __shfl(xc.x, ov[u]);
-          xo.y = __shfl(xc.y, ov[u]);
-          xo.z = __shfl(xc.z, ov[u]);
-          xo.w = 0.0;
-          const int to = __shfl(tci, ov[u]);
-          if (qv[u] < nq) {
-            Leg<T> L;
-            make_leg<MIXED>(xo, xq[u], in, fc, to, type_of(meta_of(xq[u])), (uint32_t)jq[u],
-                            (uint32_t)kq[u], L);
-            T4 x, y;
-            x.x = L.e0; x.y = L.e1; x.z = L.e2; x.w = ks_ge(L.ks) ? -L.E : L.E;
-            y.x = L.g; y.y = L.rinv; y.z = ks_pack(T(0), L.ks); y.w = ks_pack(T(0), L.elo);
-            const int q = qv[u];
-            sA[wid][q] = x;
-            sB[wid][q] = y;
-            const int r = (rq[u] & RK_SLOT) ? (rq[u] & ~RK_SLOT) : min(oq[u] + (rq[u] & 0xff), 127);
-            if (!(rq[u] & RK_SLOT))
-              rk_sw[(size_t)(i0 + ov[u]) * Wsw + kq[u]] = (uint16_t)(RK_SLOT | r);
-            sR[wid][q] = r < Wsw ? (uint32_t)__popcll(aq[u] & ((1ull << r) - 1ull)) *
-                                           (uint32_t)NA + (uint32_t)jq[u]
-                                 : ~0u;
-          }
-        }
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // mixed: each lane's legs' energy shares wait in registers until every
-    // lane is done reading the stage's fourth words (the low parts of the
-    // unit vectors)
-    T gus[MIXED ? NS / FIB_WAVE : 1];
-#pragma unroll
-    for (int k = 0; k < (MIXED ? NS / FIB_WAVE : 1); ++k) gus[k] = 0;
-    for (int g = s0 + lane, it = 0; g < s1; g += FIB_WAVE, ++it) {
-      const int q = g - s0;
-      const int o = owner[wid][q];
-      const int c0 = soff[wid][o] - s0;  // the centre's first leg in the stage
-      const int na = soff[wid][o + 1] - soff[wid][o];
-      const int a = g - soff[wid][o];
-      Leg<T> La;
-      {
-        const T4 x = sA[wid][q], y = sB[wid][q];
-        La.e0 = x.x; La.e1 = x.y; La.e2 = x.z; La.E = fabs(x.w);
-        La.g = y.x; La.rinv = y.y; La.ks = ks_unpack(y.z); La.elo = ks_unpack(y.w);
-      }
-      const int ga = sge[wid][o] + ks_ge(La.ks);
-      T Ga0 = 0, Ga1 = 0, Ga2 = 0, Gu = 0;
-      for (int b = 0; b < na; ++b) {
-        if (b == a) continue;
-        const T4 xb = sA[wid][c0 + b];
-        Leg<T> Lb;
-        Lb.e0 = xb.x; Lb.e1 = xb.y; Lb.e2 = xb.z; Lb.E = fabs(xb.w);
-        Lb.elo = MIXED ? ks_unpack(sB[wid][c0 + b].w) : 0u;
-        T Fa[3], hh;
-        vterm<T>(pick4(lp, ga + (xb.w < T(0) ? 1 : 0)), La, Lb, Fa, hh);
-        Ga0 += Fa[0]; Ga1 += Fa[1]; Ga2 += Fa[2];
-        Gu += hh;
-      }
-      // results go back through the stage and leave plane by plane below,
-      // with sR, so the stores coalesce: FP64, all four words at once (this
-      // lane alone reads sB[q]); mixed, the forces into the first three
-      // words now and the energy share after the loop
-      if constexpr (MIXED) {
-        sB[wid][q].x = Ga0; sB[wid][q].y = Ga1; sB[wid][q].z = Ga2;
-#pragma unroll
-        for (int k = 0; k < NS / FIB_WAVE; ++k)
-          if (k == it) gus[k] = Gu * T(1.0 / 3.0);
-      } else {
-        T4 gv;
-        gv.x = Ga0; gv.y = Ga1; gv.z = Ga2; gv.w = Gu * T(1.0 / 3.0);
-        sB[wid][q] = gv;
-      }
-      uc += Gu;
-      if (VIR) {
-        // r_a = x_a - x_i = -e_a / rinv_a
-        const T ra = -T(1) / La.rinv;
-        const T d0 = ra * La.e0, d1 = ra * La.e1, d2 = ra * La.e2;
-        W[0] += d0 * Ga0; W[1] += d0 * Ga1; W[2] += d0 * Ga2;
-        W[3] += d1 * Ga0; W[4] += d1 * Ga1; W[5] += d1 * Ga2;
-        W[6] += d2 * Ga0; W[7] += d2 * Ga1; W[8] += d2 * Ga2;
-      }
-    }
-    if constexpr (MIXED) {
-      // every lane is done with the fourth words: the energy shares go there
-      wave_lds_sync();
-#pragma unroll
-      for (int k = 0; k < NS / FIB_WAVE; ++k) {
-        const int g = s0 + lane + k * FIB_WAVE;
-        if (g < s1) sB[wid][g - s0].w = gus[k];
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const bool mine = lane >= f0 && lane < f1;
     for (int a = 0; __ballot(mine && a < nl) != 0ull; ++a) {
       if (mine && a < nl) {
-        const size_t at = (size_t)a * NA + i0 + lane;
-        const int q = inc - nl + a - s0;
-        st_nt<NTS>(G + at, sB[wid][q]);
+        const size_t at = (size_t)a * NA + ic;
+        const int q = exc + a - fs;
+        st_nt<NTS>(G + at, sG[wid][q]);
         st_nt<NTS>(RA + at, sR[wid][q]);
       }
     }
-    o0 = o1;
+    wave_lds_sync();
+  };
+
+  for (int r0 = 0; r0 < FIB_WAVE;) {
+    // atoms [r0, r1) whose legs fit the table (an atom has at most Wsw <= 64
+    // legs, so every run takes at least one atom, as does every pass)
+    const int rs = __builtin_amdgcn_readlane(exc, r0);
+    const int r1 = r0 + __popcll(__ballot(lane >= r0 && inc - rs <= TRI_TAB));
+    wave_lds_sync();
+    if (lane >= r0 && lane < r1) {
+      uint64_t m = amc;
+      for (int a = 0; a < nl; ++a) {
+        tab[wid][exc - rs + a] = (uint16_t)(lane | ((__ffsll((unsigned long long)m) - 1) << 6));
+        m &= m - 1;
+      }
+    }
+    wave_lds_sync();
+    // pass of the atoms [p0, p1), legs [ps, ps + n): this lane's leg, its row
+    // entry, and the partner's position, leg mask and row start
+    struct Pass {
+      int p0, p1, ps, n;
+      int o, k, j, rq;
+      double4 x;
+      uint64_t aq;
+      int oq;
+    };
+    auto entries = [&](Pass &P, int p0) {
+      P.p0 = p0;
+      P.ps = __builtin_amdgcn_readlane(exc, p0);
+      P.p1 = p0 + __popcll(__ballot(lane >= p0 && lane < r1 && inc - P.ps <= FIB_WAVE));
+      P.n = __builtin_amdgcn_readlane(inc, P.p1 - 1) - P.ps;
+      P.o = p0; P.k = 0; P.j = i0; P.rq = 0xffff;
+      if (lane < P.n) {
+        const int e = tab[wid][P.ps - rs + lane];
+        P.o = e & 63;
+        P.k = e >> 6;
+        const uint32_t at = (uint32_t)(i0 + P.o) * (uint32_t)Wsw + (uint32_t)P.k;
+        P.j = ld_nt<NT>(nbr_sw + at);
+        P.rq = (int)ld_nt<NT>(rk_sw + at);
+      }
+    };
+    // Where the partner j keeps the force of its own terms on the owner:
+    // G[n * NA + j], n = j's leg index of the owner.  The slot r of the
+    // owner in j's row follows from the stencil offsets (see k_nbuild), n
+    // from j's leg mask (legs are symmetric); 255 offsets (r >= Wsw) mark a
+    // j without a row.  The first time a pair is a leg after a build, r is
+    // worked out from j's offsets and kept in the row entry (RK_SLOT set);
+    // later steps read it there, without the gather of j's offsets.
+    auto partners = [&](Pass &P) {
+      P.x = ld_off(X, (uint32_t)P.j * 32u);
+      P.aq = ld_off(amask, (uint32_t)P.j * 8u);
+      P.oq = (P.rq & RK_SLOT) ? 0 : off_sw[(size_t)P.j * OFF_W + 26 - (P.rq >> 8)];
+    };
+    Pass P, Q;
+    entries(P, r0);
+    partners(P);
+    while (true) {
+      const bool more = P.p1 < r1;
+      if (more) entries(Q, P.p1);
+      const bool act = lane < P.n;
+      // the owner's position, species and legs, from the owner's lane
+      double4 xo;
+      xo.x = __shfl(xc.x, P.o);
+      xo.y = __shfl(xc.y, P.o);
+      xo.z = __shfl(xc.z, P.o);
+      xo.w = 0.0;
+      const int to = __shfl(tci, P.o);
+      const int c0 = __shfl(exc, P.o) - P.ps;  // the owner's first leg in the pass
+      const int no = __shfl(nl, P.o);          // (every lane takes part)
+      const int na = act ? no : 0;
+      const int a = lane - c0;
+      const int tn = type_of(meta_of(P.x));
+      Leg<T> La;
+      make_leg<MIXED>(xo, P.x, in, fc, to, tn, La);
+      {
+        T4 x;
+        x.x = La.e0; x.y = La.e1; x.z = La.e2; x.w = tn == 2 ? -La.E : La.E;
+        sE[wid][lane] = x;
+        if constexpr (MIXED) sL[wid][lane] = make_float4(La.l0, La.l1, La.l2, 0.0f);
+      }
+      uint32_t ra = ~0u;
+      {
+        const int r = (P.rq & RK_SLOT) ? (P.rq & ~RK_SLOT) : min(P.oq + (P.rq & 0xff), 127);
+        if (act && !(P.rq & RK_SLOT))
+          rk_sw[(size_t)(i0 + P.o) * Wsw + P.k] = (uint16_t)(RK_SLOT | r);
+        if (r < Wsw)
+          ra = (uint32_t)__popcll(P.aq & ((1ull << r) - 1ull)) * (uint32_t)NA + (uint32_t)P.j;
+      }
+      if (P.ps + P.n - fs > FL) {
+        write_out(P.p0);
+        f0 = P.p0;
+        fs = P.ps;
+      }
+      if (TB >= 4 && more) partners(Q);
+      wave_lds_sync();
+      auto low_of = [&](int q, Leg<T> &L) {
+        if constexpr (MIXED) {
+          const float4 l = sL[wid][q];
+          L.l0 = l.x; L.l1 = l.y; L.l2 = l.z;
+        }
+      };
+      // cos and D of every pair of the pass in sQ, or (not SHARED) per term;
+      // without a Ge atom in the pass (not GE) lambda eps is that of Si
+      const bool shared = MIXED && __ballot(na > QR) == 0ull;
+      const bool ge = __ballot(to == 2 || tn == 2) != 0ull;
+      T Ga0 = 0, Ga1 = 0, Ga2 = 0, Gu = 0;
+      if (shared) {
+        const int half = na >> 1, last = half - ((na & 1) == 0 && a >= half ? 1 : 0);
+        int b = a;
+        for (int t = 1; t <= last; ++t) {
+          b = b + 1 == na ? 0 : b + 1;
+          Leg<T> Lb;
+          const T4 x = sE[wid][c0 + b];
+          Lb.e0 = x.x; Lb.e1 = x.y; Lb.e2 = x.z;
+          low_of(c0 + b, Lb);
+          T cs, D;
+          cos_d(La, Lb, cs, D);
+          const float2 v = make_float2((float)cs, (float)D);
+          sQ[wid][b * FIB_WAVE + lane] = v;
+          sQ[wid][a * FIB_WAVE + c0 + b] = v;
+        }
+        wave_lds_sync();
+      }
+      auto terms = [&](auto GE_, auto SHARED_) {
+        constexpr bool GE = decltype(GE_)::value, SHARED = decltype(SHARED_)::value;
+        const int ga = GE ? (to == 2 ? 1 : 0) + (tn == 2 ? 1 : 0) : 0;
+        for (int b = a == 0 ? 1 : 0; b < na; b += b + 1 == a ? 2 : 1) {
+          Leg<T> Lb;
+          const T4 x = sE[wid][c0 + b];
+          Lb.e0 = x.x; Lb.e1 = x.y; Lb.e2 = x.z; Lb.E = GE ? fabs(x.w) : x.w;
+          T cs, D, Fa[3], hh;
+          if constexpr (SHARED) {
+            const float2 v = sQ[wid][b * FIB_WAVE + lane];
+            cs = (T)v.x;
+            D = (T)v.y;
+          } else {
+            low_of(c0 + b, Lb);
+            cos_d(La, Lb, cs, D);
+          }
+          vterm<T>(GE ? pick4(lp, ga + (x.w < T(0) ? 1 : 0)) : lp[0], La, Lb, cs, D, Fa, hh);
+          Ga0 += Fa[0]; Ga1 += Fa[1]; Ga2 += Fa[2];
+          if (U) Gu += hh;
+        }
+      };
+      using Yes = std::integral_constant<bool, true>;
+      using No = std::integral_constant<bool, false>;
+      if constexpr (MIXED) {
+        if (shared) {
+          if (ge) terms(Yes{}, Yes{}); else terms(No{}, Yes{});
+        } else {
+          terms(Yes{}, No{});
+        }
+      } else {
+        if (ge) terms(Yes{}, No{}); else terms(No{}, No{});
+      }
+      if (act) {
+        T4 gv;
+        gv.x = Ga0; gv.y = Ga1; gv.z = Ga2; gv.w = Gu * T(1.0 / 3.0);
+        sG[wid][P.ps - fs + lane] = gv;
+        sR[wid][P.ps - fs + lane] = ra;
+        if (U) uc += (double)Gu;
+        if (VIR) {
+          // r_a = x_a - x_i = -e_a / rinv_a
+          const T rl = -T(1) / La.rinv;
+          const T d0 = rl * La.e0, d1 = rl * La.e1, d2 = rl * La.e2;
+          W[0] += d0 * Ga0; W[1] += d0 * Ga1; W[2] += d0 * Ga2;
+          W[3] += d1 * Ga0; W[4] += d1 * Ga1; W[5] += d1 * Ga2;
+          W[6] += d2 * Ga0; W[7] += d2 * Ga1; W[8] += d2 * Ga2;
+        }
+      }
+      wave_lds_sync();
+      if (!more) break;
+      P = Q;
+      if (TB < 4) partners(P);
+    }
+    r0 = r1;
   }
+  write_out(FIB_WAVE);
   if (EN || VIR) {
     double v[10];
     // every unordered term was summed twice, as (a, b) and (b, a)
-    v[0] = (double)uc * 0.5 * escale;
+    v[0] = uc * 0.5 * escale;
     const double ws = MIXED ? fscale * lscale : 1.0;
 #pragma unroll
     for (int w = 0; w < 9; ++w) v[1 + w] = (double)W[w] * ws;
@@ -1734,7 +1768,7 @@ template <bool MIXED, bool EN, bool VIR>
 __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
     const double4 *__restrict__ X, const DInst *__restrict__ I, const FConst fc, int NA, int Wsw,
     const int *__restrict__ cnt_sw, const int *__restrict__ nbr_sw,
-    const int *__restrict__ cnt_leg, const uint64_t *__restrict__ amask,
+    const uint64_t *__restrict__ amask,
     const float *__restrict__ disp, DCtl *__restrict__ ctl, typename Prec<MIXED>::T4 *__restrict__ EX,
     typename Prec<MIXED>::T4 *__restrict__ EXself, uint64_t *__restrict__ exmask, int pstride,
     double *__restrict__ partials, const int *__restrict__ halt) {
@@ -1774,10 +1808,10 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
 #pragma unroll
   for (int w = 0; w < 9; ++w) W[w] = 0;
   if (live && tb < 3) {
-    const int na = cnt_leg[b];
     const int cs = min(cnt_sw[b], Wsw);
     const int *rowb = nbr_sw + (size_t)b * Wsw;
     const uint64_t amb = amask[b];
+    const int na = __popcll(amb);
     for (int n = 0; n < na; ++n) {
       const int kc = nth_bit(amb, n);  // b's list slot of c
       const int c = rowb[kc];
@@ -1785,7 +1819,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
       const double4 xc = X[c];
       const int tc = type_of(meta_of(xc));
       Leg<T> Lbc;  // b's leg to c: unit vector from c to b
-      make_leg<MIXED>(xb, xc, in, fc, tb, tc, (uint32_t)c, (uint32_t)kc, Lbc);
+      make_leg<MIXED>(xb, xc, in, fc, tb, tc, Lbc);
       const int *rowc = nbr_sw + (size_t)c * Wsw;
       const int cc = min(cnt_sw[c], Wsw);
       for (int k = 0; k < cs; ++k) {
@@ -1797,49 +1831,27 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
         double d0, d1, d2;
         min_image_fast(xc, xa, in, d0, d1, d2);
         const double isg = fc.isig[(tc == 2) ? 1 : 0][(ta == 2) ? 1 : 0];
+        const double s0 = MIXED ? d0 * isg : d0, s1 = MIXED ? d1 * isg : d1,
+                     s2 = MIXED ? d2 * isg : d2;
+        const double rr = s0 * s0 + s1 * s1 + s2 * s2;
+        if (MIXED && !(rr < fc.cut_sw2)) continue;
+        const double r = sqrt(rr);
+        if (!((MIXED ? r : r * isg) < (MIXED ? fc.mixed_xleg : fc.cut_sw))) continue;
+        bool listed = false;
+        for (int q = 0; q < cc; ++q) listed |= (rowc[q] == a);
+        if (listed) continue;
         Leg<T> Lca;
-        Lca.elo = 0u;
-        if (!MIXED) {
-          const double r = sqrt(d0 * d0 + d1 * d1 + d2 * d2);
-          const double rs = r * isg;
-          if (!(rs < fc.cut_sw)) continue;
-          bool listed = false;
-          for (int q = 0; q < cc; ++q) listed |= (rowc[q] == a);
-          if (listed) continue;
-          const double rinv = 1.0 / r, inv_ra = 1.0 / (rs - fc.al);
-          Lca.e0 = d0 * rinv; Lca.e1 = d1 * rinv; Lca.e2 = d2 * rinv;
-          Lca.rinv = rinv;
-          Lca.E = exp(fc.gamma * inv_ra);
-          Lca.g = -fc.gamma * inv_ra * inv_ra * isg;
-        } else {
-          // the leg values from FP64 geometry, as make_leg forms them
-          const double s0 = d0 * isg, s1 = d1 * isg, s2 = d2 * isg;
-          const double rr = s0 * s0 + s1 * s1 + s2 * s2;
-          if (!(rr < fc.cut_sw2)) continue;
-          const double rs = sqrt(rr);
-          if (!(rs < fc.mixed_xleg)) continue;
-          bool listed = false;
-          for (int q = 0; q < cc; ++q) listed |= (rowc[q] == a);
-          if (listed) continue;
-          const double rho = fc.rho[(tc == 2) ? 1 : 0][(ta == 2) ? 1 : 0];
-          const double rinv = 1.0 / rs;
-          const double inv_ra = 1.0 / (rs - fc.al);
-          const double x0 = s0 * rinv, x1 = s1 * rinv, x2 = s2 * rinv;
-          Lca.e0 = (float)x0; Lca.e1 = (float)x1; Lca.e2 = (float)x2;
-          Lca.elo = pack_lo(x0, Lca.e0, 0) | pack_lo(x1, Lca.e1, 1) | pack_lo(x2, Lca.e2, 2);
-          Lca.rinv = (float)(rinv * rho);
-          Lca.E = expf((float)(fc.gamma * inv_ra));
-          Lca.g = (float)(-fc.gamma * inv_ra * inv_ra * rho);
-        }
+        leg_values<MIXED>(d0, d1, d2, isg, fc.rho[(tc == 2) ? 1 : 0][(ta == 2) ? 1 : 0], fc, Lca);
         // leg c -> b is b's leg to c, reversed
         Leg<T> Lcb = Lbc;
         Lcb.e0 = -Lbc.e0; Lcb.e1 = -Lbc.e1; Lcb.e2 = -Lbc.e2;
-        Lcb.elo = neg_lo(Lbc.elo);
+        Lcb.l0 = -Lbc.l0; Lcb.l1 = -Lbc.l1; Lcb.l2 = -Lbc.l2;
         const int nge = (tc == 2) + (ta == 2) + (tb == 2);
-        T Fa[3], Fb[3], hh;
+        T Fa[3], Fb[3], hh, cosv, D;
+        cos_d(Lca, Lcb, cosv, D);
         // vterm gives the force on its first leg: once per end
-        vterm<T>(pick4(lp, nge), Lca, Lcb, Fa, hh);
-        vterm<T>(pick4(lp, nge), Lcb, Lca, Fb, hh);
+        vterm<T>(pick4(lp, nge), Lca, Lcb, cosv, D, Fa, hh);
+        vterm<T>(pick4(lp, nge), Lcb, Lca, cosv, D, Fb, hh);
         const T Fc0 = -(Fa[0] + Fb[0]), Fc1 = -(Fa[1] + Fb[1]), Fc2 = -(Fa[2] + Fb[2]);
         fb.add(Fb[0], Fb[1], Fb[2]);
         const T third = hh * T(1.0 / 3.0);
@@ -2342,7 +2354,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_force3(
     const int *__restrict__ nbr_sw, const uint16_t *__restrict__ rk_sw,
     const uint8_t *__restrict__ off_sw, const typename Prec<MIXED>::T4 *__restrict__ G,
     const uint32_t *__restrict__ RA,
-    const int *__restrict__ cnt_leg, const int *__restrict__ cnt_sw,
+    const uint64_t *__restrict__ amask, const int *__restrict__ cnt_sw,
     const double *__restrict__ Fpart, const double *__restrict__ upart, double fscale,
     double escale, double *__restrict__ Fout, double *__restrict__ uout, double *__restrict__ V,
     StepArgs sa, int pstride, double *__restrict__ partials, const DCtl *__restrict__ ctl,
@@ -2368,7 +2380,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_force3(
     const size_t row = (size_t)i * Wsw;
     double g0 = 0, g1 = 0, g2 = 0, gu = 0;
     // reaction on the centre: minus the forces its own terms put on its legs
-    const int na = ld_nt<NT>(cnt_leg + i);
+    const int na = __popcll(ld_nt<NT>(amask + i));
     for (int n = 0; n < na; ++n) {
       const T4 g = G[(size_t)n * NA + i];
       g0 -= (double)g.x; g1 -= (double)g.y; g2 -= (double)g.z;
@@ -2893,7 +2905,7 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
     KScope ks_(d, KT_LEGS);
     hipLaunchKernelGGL((k_legs<MIXED, EN, VIR>), dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), 0, s,
                        d.X[d.cur], d.I, fc, d.tab, d.NA, d.Wsw, d.Wion, d.cnt_sw, d.nbr_sw,
-                       d.cnt_ion, d.nbr_ion, d.cnt_leg, d.amask, d.Fpart, d.upart, d.pstride,
+                       d.cnt_ion, d.nbr_ion, d.amask, d.Fpart, d.upart, d.pstride,
                        d.partials, d.halt);
   }
   {
@@ -2904,7 +2916,7 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
     const int tb = (EN || VIR || !d.tri_tb) ? TRI_BATCH : d.tri_tb;
 #define TRI_LAUNCH(NS_, TB_)                                                                  \
   hipLaunchKernelGGL((k_tri<MIXED, EN, VIR, NS_, TB_>), dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), \
-                     0, s, d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.cnt_leg, d.nbr_sw, d.rk_sw,   \
+                     0, s, d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.nbr_sw, d.rk_sw,              \
                      d.off_sw, d.amask, (T4 *)d.G, d.RA, d.pstride,                          \
                      d.partials + (size_t)FIB_NRED * d.pstride, d.halt)
     if constexpr (EN || VIR) {
@@ -2923,7 +2935,7 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
   if (extra || EN || VIR) {
     KScope ks_(d, KT_EXTRA);
     hipLaunchKernelGGL((k_extra<MIXED, EN, VIR>), dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), 0, s,
-                       d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.cnt_sw, d.nbr_sw, d.cnt_leg, d.amask,
+                       d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.cnt_sw, d.nbr_sw, d.amask,
                        d.disp, d.ctl, (T4 *)d.EX,
                        (T4 *)d.EXself, d.exmask, d.pstride,
                        d.partials + (size_t)2 * FIB_NRED * d.pstride, d.halt);
@@ -2945,7 +2957,7 @@ static void force_c(const DevBufs &d, const FConst &fc, const StepArgs &sa, doub
     KScope ks_(d, KT_GATHER);
     hipLaunchKernelGGL((k_force3<MIXED, EN, MODE>), dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK),
                        0, s, d.X[d.cur], d.I, d.NA, d.Wsw, d.nbr_sw, d.rk_sw, d.off_sw,
-                       (const T4 *)d.G, d.RA, d.cnt_leg, d.cnt_sw, d.Fpart,
+                       (const T4 *)d.G, d.RA, d.amask, d.cnt_sw, d.Fpart,
                        d.upart, fscale, escale, Fo,
                        d.uout, d.V[d.cur], sa, d.pstride, d.partials, d.ctl, (const T4 *)d.EX,
                        (const T4 *)d.EXself, d.exmask, d.halt);

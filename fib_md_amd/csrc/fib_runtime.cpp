@@ -275,7 +275,7 @@ static int32_t free_bufs(fib_handle *h) {
   DevBufs &d = h->d;
   void *ptrs[] = {d.I, d.ctl, d.ibase, d.binst, d.X[0], d.X[1], d.V[0], d.V[1], d.F[0], d.F[1], d.Xi[0], d.Xi[1],
                   d.inv, d.bkey, d.brank, d.bcnt, d.cstart, d.perm, d.bsum, d.cnt_sw, d.nbr_sw,
-                  d.cnt_ion, d.nbr_ion, d.rk_sw, d.off_sw, d.G, d.RA, d.amask, d.cnt_leg, d.Xb, d.disp, d.EX, d.EXself, d.exmask, d.Fpart, d.upart, d.Fout, d.uout,
+                  d.cnt_ion, d.nbr_ion, d.rk_sw, d.off_sw, d.G, d.RA, d.amask, d.Xb, d.disp, d.EX, d.EXself, d.exmask, d.Fpart, d.upart, d.Fout, d.uout,
                   d.partials, d.fin_tmp, d.tab, d.xfer};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
@@ -451,7 +451,6 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
   ALLOC(d.cnt_sw, NA);
   ALLOC(d.cnt_ion, NA);
   ALLOC(d.amask, NA);
-  ALLOC(d.cnt_leg, NA);
   ALLOC(d.off_sw, (size_t)32 * NA);
   ALLOC(d.Xb, NA);
   ALLOC(d.disp, NA);
@@ -492,7 +491,6 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
   if (e == hipSuccess) e = hipMemset(d.cnt_sw, 0, sizeof(int) * NA);
   if (e == hipSuccess) e = hipMemset(d.cnt_ion, 0, sizeof(int) * NA);
   if (e == hipSuccess) e = hipMemset(d.amask, 0, sizeof(uint64_t) * NA);
-  if (e == hipSuccess) e = hipMemset(d.cnt_leg, 0, sizeof(int) * NA);
   if (e == hipSuccess) e = hipMemset(d.exmask, 0, sizeof(uint64_t) * NA);
   if (e == hipSuccess) e = hipMemset(d.off_sw, 0, (size_t)32 * NA);
   if (e == hipSuccess) e = hipMemset(d.disp, 0, sizeof(float) * NA);
@@ -1669,7 +1667,6 @@ int32_t fib_arena_force(const fib_params *p, int32_t precision, int32_t natm, in
   d.cnt_sw = A.take<int>(NA);
   d.cnt_ion = A.take<int>(NA);
   d.amask = A.take<uint64_t>(NA);
-  d.cnt_leg = A.take<int>(NA);
   d.off_sw = A.take<uint8_t>(32 * NA);
   d.Xb = A.take<double4>(NA);
   d.disp = A.take<float>(NA);
@@ -1700,7 +1697,6 @@ int32_t fib_arena_force(const fib_params *p, int32_t precision, int32_t natm, in
   fibk::launch_fill_zero(d.cnt_sw, NA * sizeof(int), s);
   fibk::launch_fill_zero(d.cnt_ion, NA * sizeof(int), s);
   fibk::launch_fill_zero(d.amask, NA * sizeof(uint64_t), s);
-  fibk::launch_fill_zero(d.cnt_leg, NA * sizeof(int), s);
   fibk::launch_fill_zero(d.exmask, NA * sizeof(uint64_t), s);
   fibk::launch_fill_zero(d.off_sw, 32 * NA, s);
   fibk::launch_fill_zero(d.disp, NA * sizeof(float), s);

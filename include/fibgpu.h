@@ -324,12 +324,14 @@ int32_t fib_md_energy(fib_handle *h, double *epot);
 int32_t fib_set_list_width(fib_handle *h, int32_t wsw, int32_t wion);
 int32_t fib_get_list_width(const fib_handle *h, int32_t *wsw, int32_t *wion);
 
-/* Launch tiles, for autotuning: tri_ns legs per stage run of the vertex pass
- * (128 or 256), tri_batch legs per lane whose neighbour loads are in flight
- * together (2 or 4), nb_cells cells per wavefront of the list build (4, 8 or
- * 16); 0 keeps a tile at its default (256, 4, 8).  Results are the same bit
- * for bit in every tile, only the time changes.  The reference's only
- * tuning knob of this kind is its cell count, rc and Nc (si.f90:55-56). */
+/* Launch tiles, for autotuning: tri_ns (128 or 256): the vertex pass holds
+ * the results of up to tri_ns / 2 legs of a wavefront back and writes them
+ * out together; tri_batch: 4 loads the next legs' positions during a pass
+ * over up to 64 legs, 2 only their row entries; nb_cells cells per wavefront
+ * of the list build (4, 8 or 16); 0 keeps a tile at its default (256, 4, 8).
+ * Results are the same bit for bit in every tile, only the time changes.
+ * The reference's only tuning knob of this kind is its cell count, rc and Nc
+ * (si.f90:55-56). */
 int32_t fib_set_tiles(fib_handle *h, int32_t tri_ns, int32_t tri_batch, int32_t nb_cells);
 int32_t fib_get_tiles(const fib_handle *h, int32_t tiles[3]);
 
