@@ -60,6 +60,7 @@ struct FConst {
   int32_t ntable;
   int32_t izero;      // first table index (1-based) whose T and successors are 0
   double mixed_r64;   // mixed precision: Moliere pairs below this use FP64
+  double near2;       // (cutoff + delta)^2 / sigma^2 of the near lists (k_legs)
   double skin;        // rc - (three-body range): pairs farther apart than rc at
                       // the build need a relative move above this to form a leg
   double mixed_xleg;  // mixed precision: three-body legs need r/sigma below
@@ -96,6 +97,7 @@ struct DCtl {
                         // a pair unlisted at the build can be within the cutoff
                         // only when maxdisp + maxdisp2 exceeds the skin
   double nmaxdisp;      // atoms at maxdisp (MD-step mode)
+  double movers;        // SW atoms farther than delta / 2 from the build (MD-step mode)
   double builds;        // list builds performed (count)
   // MD-step mode (per-instance adaptive dt)
   double cfg_dt;        // timestep of the next step (s)
@@ -119,6 +121,8 @@ struct DCtl {
   int32_t nonfinite;    // set by k_bin on a NaN/Inf position
   int32_t extra_any;    // k_extra found vertex terms outside a centre's list
   int32_t overflow;     // a neighbour list exceeded its width (sticky)
+  int32_t near_off;     // too many movers: no near lists until the next build
+  int32_t reserved;
   int32_t leave_overflow;  // more atoms left in one MD step than the removal
                            // list holds (sticky)
 };

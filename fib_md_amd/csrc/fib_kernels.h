@@ -25,6 +25,7 @@ struct StepArgs {
   double remove_dz;          // atoms higher than surf_z + remove_dz are removed
   double shell_w;            // Berendsen shells: x/y sides and the bottom (0 = off)
   double disp_r;             // displaced-atom threshold
+  float near_d;              // delta / 2: movement that takes an atom off its near list (m)
   double skin;               // rebuild when the two largest displacements exceed it
 };
 
@@ -77,6 +78,8 @@ struct DevBufs {
   int *cnt_sw, *nbr_sw, *cnt_ion, *nbr_ion;
   uint16_t *rk_sw;           // [NA * Wsw]: (stencil index << 8) | rank of each row entry
   uint8_t *off_sw;           // [NA * 32]: row start of each stencil cell, [27] = has a row
+  uint32_t *near;            // near lists [16 * NA] (null: none are kept)
+  uint8_t *nst;              // state of each atom's near list [NA], see k_legs
   void *G;                   // centre-term force on each leg, T4 [NA * Wsw]
   uint32_t *RA;              // per leg [NA * Wsw]: index into G of the partner's force
                              // on the atom (~0: none); needs NA * Wsw < 2^32

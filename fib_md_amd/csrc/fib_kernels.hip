@@ -97,6 +97,16 @@ __device__ __forceinline__ int xcd_remap(int w, int nb) {
   int x = w % nx, loc = w / nx;
   return (x < r) ? x * (q + 1) + loc : r * (q + 1) + (x - r) * q + loc;
 }
+// The same with every XCD taking a run of 2^xs blocks in turn, for passes
+// whose work differs from instance to instance (the pair pass does twice the
+// work where the lists are new): an instance is then spread over all XCDs.
+// One of four replicas rebuilt: k_legs 205 us with contiguous eighths of the
+// batch, where two XCDs had all of it; see xcd_shift for the run's length.
+__device__ __forceinline__ int xcd_remap(int w, int nb, int xs) {
+  const int full = nb >> (xs + 3) << (xs + 3);
+  if (w >= full) return full + xcd_remap(w - full, nb - full);
+  return (w >> (xs + 3) << (xs + 3)) + ((w & 7) << xs) + ((w >> 3) & ((1 << xs) - 1));
+}
 
 // LDS hand-off between the lanes of one wavefront (no workgroup barrier:
 // the wavefronts of a workgroup may work independently).
@@ -216,15 +226,12 @@ __device__ __forceinline__ void st_nt(V *p, const V &v) {
   }
 }
 
-// Compensated FP32 accumulation (TwoSum): s + c carries the exact sum of the
-// added terms up to O(u^2) relative error.
-__device__ __forceinline__ void kadd(float &s, float &c, float v) {
-  float t = s + v;
-  float bp = t - s;
-  c += (s - (t - bp)) + (v - bp);
-  s = t;
+// p[byte offset]: one 32-bit offset beside a scalar base, not a 64-bit
+// address per lane
+template <typename V>
+__device__ __forceinline__ V ld_off(const V *p, uint32_t byte) {
+  return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(p) + byte);
 }
-
 // ---------------------------------------------------------------------------
 // Reductions of NV doubles per slot.  Slot operations: RED_SUM, RED_MAX, and
 // the exact top two of a set of values over three slots (RED_TOP2 at slot k:
@@ -1063,14 +1070,16 @@ __device__ __forceinline__ double fast_rcp(double x) {
 }
 
 // Low part of an FP32 unit-vector component h = fl(x) of the FP64 value x:
-// x - h rounded to a multiple of ulp(h)/1024 (a 10-bit number), as FP32.
-// With the low parts the vertex pass forms cos + 1/3 from (nearly) the FP64
-// unit vectors, where it cancels near the tetrahedral angle.  For h = m 2^e
-// with m in [0.5, 1), ulp(h) = 2^(e - 24); adding and taking away
-// 1.5 2^(e + 18) rounds to multiples of 2^(e - 34).
+// x - h rounded to a multiple of ulp(h)/1024 and at most 511 of them (a
+// signed 10-bit number), as FP32.  With the low parts the vertex pass forms
+// cos + 1/3 from (nearly) the FP64 unit vectors, where it cancels near the
+// tetrahedral angle.  For h = m 2^e with m in [0.5, 1), ulp(h) = 2^(e - 24);
+// adding and taking away 1.5 2^(e + 18) rounds to multiples of 2^(e - 34).
 __device__ __forceinline__ float low_part(double x, float h) {
-  const double big = __builtin_amdgcn_ldexp(1.5, __builtin_amdgcn_frexp_expf(h) + 18);
-  return (float)(((x - (double)h) + big) - big);
+  const int e = __builtin_amdgcn_frexp_expf(h);
+  const double big = __builtin_amdgcn_ldexp(1.5, e + 18);
+  const float most = __builtin_amdgcn_ldexpf(511.0f, e - 34);
+  return __builtin_amdgcn_fmed3f((float)(((x - (double)h) + big) - big), -most, most);
 }
 // a + b - s exactly, for s = fl(a + b) (TwoSum)
 __device__ __forceinline__ float two_sum_err(float a, float b, float s) {
@@ -1169,7 +1178,11 @@ __device__ __forceinline__ void leg_values(double d0, double d1, double d2, doub
     sqrt_rsqrt(s0 * s0 + s1 * s1 + s2 * s2, rs, rinv);
     const double inv_ra = fast_rcp(rs - fc.al);
     const double rho = rhof;
-    const double x0 = s0 * rinv, x1 = s1 * rinv, x2 = s2 * rinv;
+    double x0, x1, x2;
+    {
+#pragma clang fp contract(off)
+      x0 = s0 * rinv; x1 = s1 * rinv; x2 = s2 * rinv;
+    }
     L.e0 = (float)x0; L.e1 = (float)x1; L.e2 = (float)x2;
     L.l0 = low_part(x0, L.e0); L.l1 = low_part(x1, L.e1); L.l2 = low_part(x2, L.e2);
     L.rinv = (float)(rinv * rho);
@@ -1187,24 +1200,16 @@ __device__ __forceinline__ void make_leg(const double4 &xc, const double4 &xn, c
   leg_values<MIXED>(d0, d1, d2, fc.isig[a][b], fc.rho[a][b], fc, L);
 }
 
-// k_legs: list slots whose positions are loaded together (4 or 8).  Eight
-// make the mixed pass 3.5 % faster on the 8.2 M-atom dose batch (110
-// VGPRs, four waves per SIMD); in FP64 (130 VGPRs) they gain nothing.
-#ifndef LEGS_BATCH_MIXED
-#define LEGS_BATCH_MIXED 8
-#endif
-#ifndef LEGS_BATCH_FP64
-#define LEGS_BATCH_FP64 4
-#endif
-
-// Register accumulator of one force vector: FP64, or FP32 with a TwoSum
-// compensation term (mixed).
+// Register sum of one force vector's terms a * (x, y, z): FP64, or FP32 with
+// a compensation term (mixed; TwoSum with the product in its place, unrounded).
 template <bool MIXED>
 struct FAcc;
 template <>
 struct FAcc<false> {
   double x = 0, y = 0, z = 0;
-  __device__ void add(double a, double b, double c) { x += a; y += b; z += c; }
+  __device__ void add(double a, double p, double q, double r) {
+    x = fma_t(a, p, x); y = fma_t(a, q, y); z = fma_t(a, r, z);
+  }
   __device__ void get(double s, double &a, double &b, double &c) const {
     a = x * s; b = y * s; c = z * s;
   }
@@ -1212,7 +1217,16 @@ struct FAcc<false> {
 template <>
 struct FAcc<true> {
   float x = 0, y = 0, z = 0, cx = 0, cy = 0, cz = 0;
-  __device__ void add(float a, float b, float c) { kadd(x, cx, a); kadd(y, cy, b); kadd(z, cz, c); }
+  __device__ __forceinline__ static void sum(float &s, float &c, float a, float p) {
+#pragma clang fp contract(off)
+    const float t = fma_t(a, p, s);
+    const float bp = t - s;
+    c += (s - (t - bp)) + fma_t(a, p, -bp);
+    s = t;
+  }
+  __device__ void add(float a, float p, float q, float r) {
+    sum(x, cx, a, p); sum(y, cy, a, q); sum(z, cz, a, r);
+  }
   __device__ void get(double s, double &a, double &b, double &c) const {
     a = ((double)x + (double)cx) * s;
     b = ((double)y + (double)cy) * s;
@@ -1220,18 +1234,81 @@ struct FAcc<true> {
   }
 };
 
+#define LEGS_BATCH 4  // k_legs: list slots whose positions are loaded together
+#define NEAR_BATCH 4  // and entries of a near list
+
+// Near lists.  Half of a row's entries lie so far beyond the cutoff that they
+// cannot come into range while no atom has moved much, and the pair pass is
+// bound by its gathers of the partners' positions (about 50 cycles for each
+// 16 bytes a lane).  The first pass after a build, at the positions of the
+// build, keeps the entries within cutoff + delta (FConst::near2, delta =
+// a tenth of the skin) in near[n * NA + i] = slot << 27 | partner, their
+// count in nst.  While neither the atom nor any partner of its row has moved
+// more than delta / 2 since the build, a pair left out is out of range, and
+// the pass runs over the near list alone.  An atom that moves farther
+// (k_md_pos, k_pos) takes itself and its partners off their near lists until
+// the next build.  Rows with more than NEAR_CAP near entries, or one past
+// slot 31, have no near list.  4 x 512 k thermal Si atoms under 2 keV ions,
+// mixed, per step: 181 us over whole rows before, 122 us over the near lists
+// and 207 us in the pass that makes them; 194 -> 144 us over 40 steps with 16
+// replica rebuilds (FP64, 2 x 512 k: 138 -> 111 us).
+#define NEAR_CAP 16
+#define NEAR_J 0x7ffffffu
+#define NEAR_MOVED 253  // moved more than delta / 2 and told its partners
+#define NEAR_FULL 254   // no near list
+#define NEAR_FRESH 255  // just built: the next pass makes the near list
+__device__ __forceinline__ void near_mark_moved(int i, int Wsw, const int *__restrict__ cnt_sw,
+                                                const int *__restrict__ nbr_sw,
+                                                uint8_t *__restrict__ nst) {
+  if (nst[i] == NEAR_MOVED) return;
+  const int n = min(cnt_sw[i], Wsw);
+  const int *row = nbr_sw + (size_t)i * Wsw;
+  for (int k = 0; k < n; ++k) {
+    const int j = row[k];
+    if (nst[j] != NEAR_MOVED) nst[j] = NEAR_FULL;
+  }
+  nst[i] = NEAR_MOVED;
+}
+
+// r^2 / sigma^2, rounded as the pair and leg values are
+template <bool MIXED>
+__device__ __forceinline__ double scaled_r2(double d0, double d1, double d2, double isg) {
+  if constexpr (MIXED) {
+    const double s0 = d0 * isg, s1 = d1 * isg, s2 = d2 * isg;
+    return s0 * s0 + s1 * s1 + s2 * s2;
+  } else {
+    return (d0 * d0 + d1 * d1 + d2 * d2) * (isg * isg);
+  }
+}
+
+// d <- d - rint(d / L) L (min_image_fast's form) for the lanes' values of one
+// axis, left out when every |d| is below half a box (by the upper words, so
+// up to 1e-6 less): rint is zero then.
+template <int N>
+__device__ __forceinline__ void wrap_axis(double (&d)[N], double ilb, double lb) {
+  const int half = __double2hiint(lb) - (1 << 20);
+  int far = 0;
+#pragma unroll
+  for (int v = 0; v < N; ++v) far = max(far, __double2hiint(d[v]) & 0x7fffffff);
+  if (__ballot(far >= half) != 0ull) {
+#pragma unroll
+    for (int v = 0; v < N; ++v) d[v] -= rint(d[v] * ilb) * lb;
+  }
+}
+
 template <bool MIXED, bool EN, bool VIR>
 __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
     const double4 *__restrict__ X, const DInst *__restrict__ I, const FConst fc,
     const TabEntry *__restrict__ tab, int NA, int Wsw, int Wion, const int *__restrict__ cnt_sw,
     const int *__restrict__ nbr_sw, const int *__restrict__ cnt_ion,
     const int *__restrict__ nbr_ion, uint64_t *__restrict__ amask,
-    double *__restrict__ Fpart, double *__restrict__ upart, int pstride,
-    double *__restrict__ partials, const int *__restrict__ halt) {
+    double *__restrict__ Fpart, double *__restrict__ upart, uint32_t *__restrict__ near,
+    uint8_t *__restrict__ nst, const DCtl *__restrict__ ctl, int pstride,
+    double *__restrict__ partials, const int *__restrict__ halt, int xs) {
   HALT_OR_RETURN(halt);
   typedef typename Prec<MIXED>::T T;
   constexpr bool NT = (FIB_NT_LD & 1) != 0, NTS = (FIB_NT_ST & 1) != 0;
-  const int lb = xcd_remap(blockIdx.x, gridDim.x);
+  const int lb = xcd_remap(blockIdx.x, gridDim.x, xs);
   const int i = lb * FIB_BLOCK + threadIdx.x;
   const double4 xi = X[i];
   const uint32_t mi = meta_of(xi);
@@ -1252,7 +1329,13 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
   // and the pair's length unit over sigma_Si, divided on the host
   const float fsA = fc.fsw[tr][0], fsB = fc.fsw[tr][1];
   const float rhoA = fc.rho[tr][0], rhoB = fc.rho[tr][1];
+  const double gate2 = MIXED ? fc.cut_sw2 : fc.r2gate;
+  const double leg2 = MIXED ? fc.mixed_xleg * fc.mixed_xleg : fc.cut_sw * fc.cut_sw;
+  const double iumax = MIXED ? 0.0 : 1.0 / fc.umax;
   const size_t row = (size_t)i * Wsw;
+  __shared__ uint32_t hold[FIB_BLOCK / FIB_WAVE][NEAR_CAP][FIB_WAVE];
+  const int lane = threadIdx.x % FIB_WAVE;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / FIB_WAVE);
 
   FAcc<MIXED> f;
   double ui = 0, etot = 0;
@@ -1265,44 +1348,34 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
     W[6] += d2 * f0; W[7] += d2 * f1; W[8] += d2 * f2;
   };
 
-  uint64_t am = 0;
-  // one buffered SW pair in list slot k: pair force, pair energy, leg
-  auto pair = [&](int k, int jn, const double4 &xj) {
-    const uint32_t mj = meta_of(xj);
-    // an atom removed since the build is out of the simulation (MD-step mode)
-    if (mj & META_DEAD) return;
-    const int tj = type_of(mj);
-    const bool jA = tj != 2;
+  // one SW pair in range: pair force and energy
+  auto pair = [&](double d0, double d1, double d2, bool jA) {
     const double isg = jA ? isgA : isgB;
-    double d0, d1, d2;
-    min_image_fast(xi, xj, in, d0, d1, d2);
-    if (!MIXED) {
-      const double rr = d0 * d0 + d1 * d1 + d2 * d2;
-      if (!(rr * (isg * isg) < fc.r2gate)) return;
-      const double r = sqrt(rr);
-      const double rinv = 1.0 / r;
+    if constexpr (!MIXED) {
+      double r, rinv;
+      sqrt_rsqrt(d0 * d0 + d1 * d1 + d2 * d2, r, rinv);
       const double rs = r * isg;
       // reference pair force: 3-point Lagrange on the derivative table
-      // (si.f90:416-424, 554-573)
-      const int t1 = (int)(rs / fc.umax * fc.tabn1) + 1;
+      // (si.f90:416-424, 554-573); rs / umax as its product with 1/umax,
+      // corrected by the remainder
+      const double q0 = rs * iumax;
+      const double q = __builtin_fma(__builtin_fma(-q0, fc.umax, rs), iumax, q0);
+      const int t1 = (int)(q * fc.tabn1) + 1;
       if (t1 < fc.izero) {
         const TabEntry te = tab[t1];
         const double e1 = rs - te.u0, e2 = rs - te.u1, e3 = rs - te.u2;
         const double df = 0.5 * e2 * e3 * te.t0 - e1 * e3 * te.t1 + 0.5 * e1 * e2 * te.t2;
         const double fs = -df * (jA ? esgA : esgB) * rinv;
-        f.add(fs * d0, fs * d1, fs * d2);
+        f.add(fs, d0, d1, d2);
         if (VIR) addW(d0, d1, d2, 0.5 * fs * d0, 0.5 * fs * d1, 0.5 * fs * d2);
       }
-      if (rs < fc.cut_sw) {
+      if (EN && rs < fc.cut_sw) {
         const double inv_ra = 1.0 / (rs - fc.al);
-        if (EN) {
-          const double rs2 = rs * rs;
-          const double ul =
-              0.5 * (jA ? epsA : epsB) * fc.A * (fc.B / (rs2 * rs2) - 1.0) * exp(inv_ra);
-          ui += ul;
-          etot += ul;
-        }
-        am |= 1ull << k;
+        const double rs2 = rs * rs;
+        const double ul =
+            0.5 * (jA ? epsA : epsB) * fc.A * (fc.B / (rs2 * rs2) - 1.0) * exp(inv_ra);
+        ui += ul;
+        etot += ul;
       }
     } else {
       // Pair geometry in FP64 (pair units: sigma_ij), the pair force factor
@@ -1311,12 +1384,10 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
       // the largest error of the mixed forces; the exponential and the
       // force vector stay FP32.
       const double s0 = d0 * isg, s1 = d1 * isg, s2 = d2 * isg;
-      const double rr = s0 * s0 + s1 * s1 + s2 * s2;
-      if (!(rr < fc.cut_sw2)) return;
-      const double rs = sqrt(rr);
+      double rs, rinv;
+      sqrt_rsqrt(s0 * s0 + s1 * s1 + s2 * s2, rs, rinv);
       if (!(rs < fc.cut_sw)) return;
-      const double rinv = 1.0 / rs;
-      const double inv_ra = 1.0 / (rs - fc.al);
+      const double inv_ra = fast_rcp(rs - fc.al);
       const double ex = (double)expf((float)inv_ra);
       const double ir2 = rinv * rinv;
       const double ir4 = ir2 * ir2;
@@ -1324,40 +1395,78 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
       const double br = -4.0 * fc.B * ir4 * rinv - (fc.B * ir4 - 1.0) * inv_ra * inv_ra;
       const float fs = (float)(-fc.A * ex * br * rinv * (double)(jA ? fsA : fsB));
       const float r0 = (float)s0, r1 = (float)s1, r2 = (float)s2;
-      const float f0 = fs * r0, f1 = fs * r1, f2 = fs * r2;
-      f.add(f0, f1, f2);
-      const float rho = jA ? rhoA : rhoB;  // 1 for Si-Si
+      f.add(fs, r0, r1, r2);
       if (VIR) {
-        const float q = 1.0f / rho;
-        addW(r0 * q, r1 * q, r2 * q, 0.5f * f0, 0.5f * f1, 0.5f * f2);
+        const float q = 1.0f / (jA ? rhoA : rhoB);  // 1 for Si-Si
+        const float h0 = fs * r0, h1 = fs * r1, h2 = fs * r2;
+        addW(r0 * q, r1 * q, r2 * q, 0.5f * h0, 0.5f * h1, 0.5f * h2);
       }
       if (EN) {
         const double ul = 0.5 * (jA ? epsA : epsB) * (fc.A * (fc.B * ir4 - 1.0) * ex);
         ui += ul;
         etot += ul;
       }
-      // legs with E = exp(gamma/(r-a)) < e^-30 are left out of the
-      // three-body sum: each of their terms is below 1e-9 eps/sigma
-      if (rs < fc.mixed_xleg) {
-        am |= 1ull << k;
-      }
     }
   };
 
-  if (sw_atom) {
-    const int cs = min(ld_nt<NT>(cnt_sw + i), Wsw);
+  uint64_t am = 0;
+  // A pair below gate2 is in range; one below leg2 is a leg (beyond, E =
+  // exp(gamma/(r-a)) is zero in FP64 and below e^-30 in the mixed mode: each
+  // of its terms is below 1e-9 eps/sigma).
+  const uint32_t st = near ? nst[i] : NEAR_FULL;
+  if (near && !ctl[kin].near_off && __ballot(st > NEAR_CAP) == 0ull) {
+    const int n = sw_atom ? (int)st : 0;
+    // NEAR_BATCH entries at a time: their positions load together, and the
+    // next entries while these arrive
+    uint32_t en[NEAR_BATCH];
+#pragma unroll
+    for (int v = 0; v < NEAR_BATCH; ++v)
+      en[v] = v < n ? ld_nt<NT>(near + (size_t)v * NA + i) : (uint32_t)i;
+    for (int q = 0; q < n; q += NEAR_BATCH) {
+      double4 xq[NEAR_BATCH];
+      uint32_t slot[NEAR_BATCH];
+#pragma unroll
+      for (int v = 0; v < NEAR_BATCH; ++v) {
+        xq[v] = ld_off(X, (en[v] & NEAR_J) * 32u);
+        slot[v] = en[v] >> 27;
+      }
+#pragma unroll
+      for (int v = 0; v < NEAR_BATCH; ++v)
+        en[v] = q + NEAR_BATCH + v < n ? ld_nt<NT>(near + (size_t)(q + NEAR_BATCH + v) * NA + i)
+                                       : (uint32_t)i;
+      double d[3][NEAR_BATCH];
+#pragma unroll
+      for (int v = 0; v < NEAR_BATCH; ++v) {
+        d[0][v] = xi.x - xq[v].x;
+        d[1][v] = xi.y - xq[v].y;
+        d[2][v] = xi.z - xq[v].z;
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c) wrap_axis<NEAR_BATCH>(d[c], in.ilb[c], in.lb[c]);
+#pragma unroll
+      for (int v = 0; v < NEAR_BATCH; ++v) {
+        const uint32_t mj = meta_of(xq[v]);
+        const bool jA = type_of(mj) != 2;
+        const double rr = scaled_r2<MIXED>(d[0][v], d[1][v], d[2][v], jA ? isgA : isgB);
+        if (q + v < n && !(mj & META_DEAD) && rr < gate2) {
+          pair(d[0][v], d[1][v], d[2][v], jA);
+          if (rr < leg2) am |= 1ull << slot[v];
+        }
+      }
+    }
+  } else {
+    const int cs = sw_atom ? min(ld_nt<NT>(cnt_sw + i), Wsw) : 0;
     const int4 *r4 = reinterpret_cast<const int4 *>(nbr_sw + row);
     // LEGS_BATCH slots at a time: their indices, then their positions; the
     // next indices are loaded while the positions arrive (every index read
     // lies below cs <= Wsw, inside the row)
-    constexpr int LEGS_BATCH = MIXED ? LEGS_BATCH_MIXED : LEGS_BATCH_FP64;
-    static_assert(LEGS_BATCH == 4 || LEGS_BATCH == 8, "LEGS_BATCH");
-    constexpr int NQ = LEGS_BATCH / 4;
+    constexpr int LB = LEGS_BATCH, NQ = LB / 4;
     int4 rn[NQ];
+    int nn = 0;  // near entries, also those past the list's end
 #pragma unroll
     for (int u = 0; u < NQ; ++u) rn[u] = (4 * u < cs) ? ld_nt<NT>(r4 + u) : make_int4(i, i, i, i);
-    for (int k0 = 0; k0 < cs; k0 += LEGS_BATCH) {
-      int jq[LEGS_BATCH];
+    for (int k0 = 0; __ballot(k0 < cs) != 0ull; k0 += LB) {
+      int jq[LB];
 #pragma unroll
       for (int u = 0; u < NQ; ++u) {
         const int b = k0 + 4 * u;
@@ -1366,15 +1475,41 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
         jq[4 * u + 2] = (b + 2 < cs) ? rn[u].z : i;
         jq[4 * u + 3] = (b + 3 < cs) ? rn[u].w : i;
       }
-      double4 xq[LEGS_BATCH];
+      double4 xq[LB];
 #pragma unroll
-      for (int v = 0; v < LEGS_BATCH; ++v) xq[v] = X[jq[v]];
+      for (int v = 0; v < LB; ++v) xq[v] = ld_off(X, (uint32_t)jq[v] * 32u);
 #pragma unroll
       for (int u = 0; u < NQ; ++u)
-        if (k0 + LEGS_BATCH + 4 * u < cs) rn[u] = ld_nt<NT>(r4 + ((k0 + LEGS_BATCH) >> 2) + u);
+        if (k0 + LB + 4 * u < cs) rn[u] = ld_nt<NT>(r4 + ((k0 + LB) >> 2) + u);
+      double d[3][LB];
 #pragma unroll
-      for (int v = 0; v < LEGS_BATCH; ++v)
-        if (k0 + v < cs) pair(k0 + v, jq[v], xq[v]);
+      for (int v = 0; v < LB; ++v) {
+        d[0][v] = xi.x - xq[v].x;
+        d[1][v] = xi.y - xq[v].y;
+        d[2][v] = xi.z - xq[v].z;
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c) wrap_axis<LB>(d[c], in.ilb[c], in.lb[c]);
+#pragma unroll
+      for (int v = 0; v < LB; ++v) {
+        const uint32_t mj = meta_of(xq[v]);
+        const bool jA = type_of(mj) != 2;
+        const double rr = scaled_r2<MIXED>(d[0][v], d[1][v], d[2][v], jA ? isgA : isgB);
+        // an atom removed since the build is out of the simulation (MD-step mode)
+        const bool ok = k0 + v < cs && !(mj & META_DEAD);
+        if (ok && rr < fc.near2) {
+          if (nn < NEAR_CAP) hold[wid][nn][lane] = (uint32_t)(k0 + v) << 27 | (uint32_t)jq[v];
+          nn += k0 + v < 32 ? 1 : NEAR_CAP + 1;
+          if (rr < gate2) pair(d[0][v], d[1][v], d[2][v], jA);
+          if (rr < leg2) am |= 1ull << (k0 + v);
+        }
+      }
+    }
+    // the near lists leave plane by plane, so that the stores coalesce
+    if (near && st == NEAR_FRESH) {
+      nst[i] = (uint8_t)(nn <= NEAR_CAP ? nn : NEAR_FULL);
+      for (int q = 0; q < min(nn, NEAR_CAP); ++q)
+        st_nt<NTS>(near + (size_t)q * NA + i, hold[wid][q][lane]);
     }
   }
   st_nt<NTS>(amask + i, am);
@@ -1407,10 +1542,10 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
                            fc.molc[2] * fc.molb[2] * e3) / aa;
         const double fcm = zz / r * (sa / r + sb);
         const double rinv = 1.0 / r;
-        const double f0 = fcm * d0 * rinv, f1 = fcm * d1 * rinv, f2 = fcm * d2 * rinv;
-        f.add((T)(f0 / fscale), (T)(f1 / fscale), (T)(f2 / fscale));
+        const double h0 = fcm * d0 * rinv, h1 = fcm * d1 * rinv, h2 = fcm * d2 * rinv;
+        f.add((T)1, (T)(h0 / fscale), (T)(h1 / fscale), (T)(h2 / fscale));
         if (VIR) addW((T)(d0 / lscale), (T)(d1 / lscale), (T)(d2 / lscale),
-                      (T)(0.5 * f0 / fscale), (T)(0.5 * f1 / fscale), (T)(0.5 * f2 / fscale));
+                      (T)(0.5 * h0 / fscale), (T)(0.5 * h1 / fscale), (T)(0.5 * h2 / fscale));
         if (EN) { const double ul = 0.5 * zz / r * sa; ui += ul; etot += ul; }
       } else {
         // FP32 with lengths in units of aa; F = (zz/aa^2) (1/x)(sa/x + sb) d/(aa x)
@@ -1424,11 +1559,12 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
         const float ix = __builtin_amdgcn_rcpf(x);
         const float fr = ix * (sa * ix + sb) * ix;
         const float scl = (float)(zz / (aa * aa) / fscale);
-        const float f0 = fr * (float)(d0 / aa) * scl, f1 = fr * (float)(d1 / aa) * scl,
-                    f2 = fr * (float)(d2 / aa) * scl;
-        f.add((T)f0, (T)f1, (T)f2);
-        if (VIR) addW((T)(d0 / lscale), (T)(d1 / lscale), (T)(d2 / lscale), (T)(0.5f * f0),
-                      (T)(0.5f * f1), (T)(0.5f * f2));
+        const float g0 = fr * (float)(d0 / aa), g1 = fr * (float)(d1 / aa),
+                    g2 = fr * (float)(d2 / aa);
+        const float h0 = g0 * scl, h1 = g1 * scl, h2 = g2 * scl;
+        f.add((T)scl, (T)g0, (T)g1, (T)g2);
+        if (VIR) addW((T)(d0 / lscale), (T)(d1 / lscale), (T)(d2 / lscale), (T)(0.5f * h0),
+                      (T)(0.5f * h1), (T)(0.5f * h2));
         if (EN) { const double ul = 0.5 * zz / aa * (double)(sa * ix); ui += ul; etot += ul; }
       }
     }
@@ -1484,23 +1620,18 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
 #endif
 #define TRI_QROWS 8   // most legs of an atom whose pairs share cos + 1/3 (mixed)
 #define TRI_TAB 384   // legs whose owner and list slot are tabled at once
+#define TRI_TAB_VIR 256
 template <bool MIXED>
 struct TriStage {
   static constexpr int N = MIXED ? TRI_NS_MIXED : TRI_NS_FP64;
 };
-// p[byte offset]: one 32-bit offset beside a scalar base, not a 64-bit
-// address per lane
-template <typename V>
-__device__ __forceinline__ V ld_off(const V *p, uint32_t byte) {
-  return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(p) + byte);
-}
 template <bool MIXED, bool EN, bool VIR, int NS, int TB>
 __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
     const double4 *__restrict__ X, const DInst *__restrict__ I, const FConst fc, int NA,
     int Wsw, const int *__restrict__ nbr_sw, uint16_t *__restrict__ rk_sw,
     const uint8_t *__restrict__ off_sw, const uint64_t *__restrict__ amask,
     typename Prec<MIXED>::T4 *__restrict__ G, uint32_t *__restrict__ RA, int pstride,
-    double *__restrict__ partials, const int *__restrict__ halt) {
+    double *__restrict__ partials, const int *__restrict__ halt, int xs) {
   HALT_OR_RETURN(halt);
   typedef typename Prec<MIXED>::T T;
   typedef typename Prec<MIXED>::T4 T4;
@@ -1512,8 +1643,12 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
   __shared__ float2 sQ[NW][MIXED ? QR * FIB_WAVE : 1];  // [partner][leg]: cos, D
   __shared__ T4 sG[NW][FL];
   __shared__ uint32_t sR[NW][FL];
-  __shared__ uint16_t tab[NW][TRI_TAB];  // owner lane | list slot << 6
-  const int lb = xcd_remap(blockIdx.x, gridDim.x);
+  constexpr int TAB = VIR ? TRI_TAB_VIR : TRI_TAB;
+  __shared__ uint16_t tab[NW][TAB];  // owner lane | list slot << 6
+  // the virial's terms of a run, which lane q % 64 sums for leg q (the FP32
+  // sums of the mixed mode then do not depend on how a run is cut into passes)
+  __shared__ T sW[NW][VIR ? 6 : 1][VIR ? TAB : 1];
+  const int lb = xcd_remap(blockIdx.x, gridDim.x, xs);
   const int lane = threadIdx.x % FIB_WAVE;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / FIB_WAVE);
   const int i0 = lb * FIB_BLOCK + wid * FIB_WAVE;
@@ -1566,7 +1701,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
     // atoms [r0, r1) whose legs fit the table (an atom has at most Wsw <= 64
     // legs, so every run takes at least one atom, as does every pass)
     const int rs = __builtin_amdgcn_readlane(exc, r0);
-    const int r1 = r0 + __popcll(__ballot(lane >= r0 && inc - rs <= TRI_TAB));
+    const int r1 = r0 + __popcll(__ballot(lane >= r0 && inc - rs <= TAB));
     wave_lds_sync();
     if (lane >= r0 && lane < r1) {
       uint64_t m = amc;
@@ -1723,16 +1858,25 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
         if (VIR) {
           // r_a = x_a - x_i = -e_a / rinv_a
           const T rl = -T(1) / La.rinv;
-          const T d0 = rl * La.e0, d1 = rl * La.e1, d2 = rl * La.e2;
-          W[0] += d0 * Ga0; W[1] += d0 * Ga1; W[2] += d0 * Ga2;
-          W[3] += d1 * Ga0; W[4] += d1 * Ga1; W[5] += d1 * Ga2;
-          W[6] += d2 * Ga0; W[7] += d2 * Ga1; W[8] += d2 * Ga2;
+          const T v[6] = {rl * La.e0, rl * La.e1, rl * La.e2, Ga0, Ga1, Ga2};
+#pragma unroll
+          for (int c = 0; c < 6; ++c) sW[wid][c][P.ps - rs + lane] = v[c];
         }
       }
       wave_lds_sync();
       if (!more) break;
       P = Q;
       if (TB < 4) partners(P);
+    }
+    if (VIR) {
+      const int nq = __builtin_amdgcn_readlane(inc, r1 - 1) - rs;
+      for (int q = lane; q < nq; q += FIB_WAVE) {
+        T v[6];
+#pragma unroll
+        for (int c = 0; c < 6; ++c) v[c] = sW[wid][c][q];
+#pragma unroll
+        for (int c = 0; c < 9; ++c) W[c] = fma_t(v[c / 3], v[3 + c % 3], W[c]);
+      }
     }
     r0 = r1;
   }
@@ -1802,7 +1946,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
                    (T)(fc.leps[0][1][1] * lu), (T)(fc.leps[1][1][1] * lu)};
   const float skin = (float)fc.skin;
   uint64_t em = 0;
-  FAcc<MIXED> fb;
+  double fb0 = 0, fb1 = 0, fb2 = 0;
   T ub = 0, et = 0;
   T W[9];
 #pragma unroll
@@ -1853,7 +1997,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
         vterm<T>(pick4(lp, nge), Lca, Lcb, cosv, D, Fa, hh);
         vterm<T>(pick4(lp, nge), Lcb, Lca, cosv, D, Fb, hh);
         const T Fc0 = -(Fa[0] + Fb[0]), Fc1 = -(Fa[1] + Fb[1]), Fc2 = -(Fa[2] + Fb[2]);
-        fb.add(Fb[0], Fb[1], Fb[2]);
+        fb0 += (double)Fb[0]; fb1 += (double)Fb[1]; fb2 += (double)Fb[2];
         const T third = hh * T(1.0 / 3.0);
         // forces on a (slot k) and c (slot kc) for them to gather
         const uint64_t bits[2] = {1ull << k, 1ull << kc};
@@ -1890,10 +2034,8 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
   }
   exmask[b] = em;
   {
-    double f0, f1, f2;
-    fb.get(1.0, f0, f1, f2);
     T4 g;
-    g.x = (T)f0; g.y = (T)f1; g.z = (T)f2; g.w = ub;
+    g.x = (T)fb0; g.y = (T)fb1; g.z = (T)fb2; g.w = ub;
     EXself[b] = g;
   }
   if (em) {
@@ -1912,7 +2054,8 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
 // After a list build: positions of the build, displacement bookkeeping reset.
 __global__ void k_mark_build(int NA, int ninst, int Wsw, int Wion, const double4 *__restrict__ X,
                              double4 *__restrict__ Xb, float *__restrict__ disp,
-                             DCtl *__restrict__ ctl, const int *__restrict__ binst,
+                             uint8_t *__restrict__ nst, DCtl *__restrict__ ctl,
+                             const int *__restrict__ binst,
                              const int *__restrict__ gate, int *__restrict__ halt, double inc) {
   GATE_OR_RETURN(gate);
   GRID_STRIDE(i, max(NA, ninst)) {
@@ -1920,8 +2063,10 @@ __global__ void k_mark_build(int NA, int ninst, int Wsw, int Wion, const double4
   if (i < NA && !block_gated_out(gate, binst, i)) {
     Xb[i] = X[i];
     disp[i] = 0.0f;
+    nst[i] = NEAR_FRESH;
   }
   if (i < ninst && !gated_out(gate, i)) {
+    ctl[i].near_off = 0;
     ctl[i].maxdisp = 0.0;
     ctl[i].maxdisp2 = 0.0;
     ctl[i].nmaxdisp = 0.0;
@@ -1966,11 +2111,14 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_md_pos(double4 *__restrict__ X,
                                                       const DCtl *__restrict__ ctl,
                                                       const double4 *__restrict__ Xb,
                                                       float *__restrict__ disp,
+                                                      int Wsw, const int *__restrict__ cnt_sw,
+                                                      const int *__restrict__ nbr_sw,
+                                                      uint8_t *__restrict__ nst,
                                                       int *__restrict__ leave,
-                                                      const int *__restrict__ halt) {
+                                                      const int *__restrict__ halt, int xs) {
   HALT_OR_RETURN(halt);
   constexpr bool NT = (FIB_NT_LD & 8) != 0, NTS = (FIB_NT_ST & 8) != 0;
-  const int lb = xcd_remap(blockIdx.x, gridDim.x);
+  const int lb = xcd_remap(blockIdx.x, gridDim.x, xs);
   const int i = lb * FIB_BLOCK + threadIdx.x;
   double4 x = X[i];
   uint32_t mi = meta_of(x);
@@ -1980,8 +2128,9 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_md_pos(double4 *__restrict__ X,
   const double dt = ctl[kin].cfg_dt, lam = ctl[kin].cfg_lambda;
   // the two largest displacements since the build (largest, how many share
   // it, largest below it), energy taken by the shells, energy of removed
-  // atoms; an atom out of the simulation counts as displaced by 0
-  double red[5] = {0.0, 1.0, -1.0e300, 0.0, 0.0};
+  // atoms, atoms off their near lists by their own movement; an atom out of
+  // the simulation counts as displaced by 0
+  double red[6] = {0.0, 1.0, -1.0e300, 0.0, 0.0, 0.0};
   if (live) {
     const int t = type_of(mi);
     const double m = sa.mass[t - 1];
@@ -2023,11 +2172,15 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_md_pos(double4 *__restrict__ X,
     const float dd = (float)sqrt(e0 * e0 + e1 * e1 + e2 * e2);
     st_nt<NTS>(disp + i, dd);
     red[0] = (double)dd;
+    if (dd > sa.near_d && t < 3) {
+      red[5] = 1.0;
+      if (!ctl[kin].near_off) near_mark_moved(i, Wsw, cnt_sw, nbr_sw, nst);
+    }
   } else {
     st_nt<NTS>(disp + i, 0.0f);
   }
-  const int op[5] = {RED_TOP2, RED_TOP2_CNT, RED_TOP2_SND, RED_SUM, RED_SUM};
-  block_partials<5, FIB_BLOCK>(red, op, lb, pstride, partials);
+  const int op[6] = {RED_TOP2, RED_TOP2_CNT, RED_TOP2_SND, RED_SUM, RED_SUM, RED_SUM};
+  block_partials<6, FIB_BLOCK>(red, op, lb, pstride, partials);
 }
 
 // Rebuild gates of the step: each instance whose two largest displacements
@@ -2225,6 +2378,9 @@ __global__ __launch_bounds__(DECIDE_T) void k_md_decide(
       const double m2 = c.nmaxdisp >= 2.0 ? c.maxdisp : fmax(c.maxdisp2, 0.0);
       g = (c.maxdisp + m2 > skin) ? 1 : 0;
       ctl[k].maxdisp2 = m2;  // the effective second maximum, for k_extra
+      // with many atoms off their near lists, telling their partners costs
+      // more than the lists that are left give
+      if (c.movers * 16.0 > (double)I[k].natm) ctl[k].near_off = 1;
       gate[1 + k] = g;
       if (g) w = I[k].nc[0] * I[k].nc[1] * I[k].nc[2];
     }
@@ -2360,11 +2516,11 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_force3(
     StepArgs sa, int pstride, double *__restrict__ partials, const DCtl *__restrict__ ctl,
     const typename Prec<MIXED>::T4 *__restrict__ EX,
     const typename Prec<MIXED>::T4 *__restrict__ EXself, const uint64_t *__restrict__ exmask,
-    const int *__restrict__ halt) {
+    const int *__restrict__ halt, int xs) {
   HALT_OR_RETURN(halt);
   typedef typename Prec<MIXED>::T4 T4;
   constexpr bool NT = (FIB_NT_LD & 4) != 0, NTS = (FIB_NT_ST & 4) != 0;
-  const int lb = xcd_remap(blockIdx.x, gridDim.x);
+  const int lb = xcd_remap(blockIdx.x, gridDim.x, xs);
   const int i = lb * FIB_BLOCK + threadIdx.x;
   const double4 xi = X[i];
   const uint32_t mi = meta_of(xi);
@@ -2513,7 +2669,10 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_pos(double4 *__restrict__ X,
                                                    int pstride, double *__restrict__ partials,
                                                    DCtl *__restrict__ ctl,
                                                    const double4 *__restrict__ Xb,
-                                                   float *__restrict__ disp) {
+                                                   float *__restrict__ disp, int Wsw,
+                                                   const int *__restrict__ cnt_sw,
+                                                   const int *__restrict__ nbr_sw,
+                                                   uint8_t *__restrict__ nst) {
 #pragma clang fp contract(off)
   const int nb = gridDim.x;
   const int lb = xcd_remap(blockIdx.x, nb);
@@ -2595,6 +2754,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_pos(double4 *__restrict__ X,
       disp[i] = (float)dd;
       red[2] = dd;
       red[3] = dd;
+      if ((float)dd > sa.near_d && t < 3) near_mark_moved(i, Wsw, cnt_sw, nbr_sw, nst);
     }
     for (int c = 0; c < 3; ++c) {
       V[(size_t)c * NA + i] = v[c];
@@ -2737,6 +2897,16 @@ static inline int nblk(long n, int b) { return (int)((n + b - 1) / b); }
 // grid of a GRID_STRIDE kernel over n elements
 static inline int gcap(long n) { return std::max(1, std::min(nblk(n, FIB_BLOCK), GRID_CAP)); }
 
+// Blocks (as a power of two) that an XCD takes in turn: an eighth of the
+// largest instance, so that each instance meets every XCD, and at least 32
+// (8 k atoms, about a layer of cells of a 512 k slab), so that most of a
+// block's neighbours are read by the same XCD.
+static int xcd_shift(const DevBufs &d) {
+  int s = 5;
+  while ((8 << s) < d.max_pad / FIB_BLOCK) ++s;
+  return s;
+}
+
 // Times the launches issued in its scope under one key.
 struct KScope {
   const KTimer *t;
@@ -2778,6 +2948,7 @@ static void finalize(const DevBufs &d, int nv, int bs, const int *op, const int 
     case 3: fin_launch<3>(d, rs, nch, gate, s); break;
     case 4: fin_launch<4>(d, rs, nch, gate, s); break;
     case 5: fin_launch<5>(d, rs, nch, gate, s); break;
+    case 6: fin_launch<6>(d, rs, nch, gate, s); break;
     default: fin_launch<10>(d, rs, nch, gate, s); break;
   }
 }
@@ -2905,8 +3076,8 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
     KScope ks_(d, KT_LEGS);
     hipLaunchKernelGGL((k_legs<MIXED, EN, VIR>), dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), 0, s,
                        d.X[d.cur], d.I, fc, d.tab, d.NA, d.Wsw, d.Wion, d.cnt_sw, d.nbr_sw,
-                       d.cnt_ion, d.nbr_ion, d.amask, d.Fpart, d.upart, d.pstride,
-                       d.partials, d.halt);
+                       d.cnt_ion, d.nbr_ion, d.amask, d.Fpart, d.upart, d.near,
+                       d.nst, d.ctl, d.pstride, d.partials, d.halt, xcd_shift(d));
   }
   {
     KScope ks_(d, KT_TRI);
@@ -2918,7 +3089,7 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
   hipLaunchKernelGGL((k_tri<MIXED, EN, VIR, NS_, TB_>), dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), \
                      0, s, d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.nbr_sw, d.rk_sw,              \
                      d.off_sw, d.amask, (T4 *)d.G, d.RA, d.pstride,                          \
-                     d.partials + (size_t)FIB_NRED * d.pstride, d.halt)
+                     d.partials + (size_t)FIB_NRED * d.pstride, d.halt, xcd_shift(d))
     if constexpr (EN || VIR) {
       TRI_LAUNCH(TriStage<MIXED>::N, TRI_BATCH);
     } else {
@@ -2960,7 +3131,7 @@ static void force_c(const DevBufs &d, const FConst &fc, const StepArgs &sa, doub
                        (const T4 *)d.G, d.RA, d.amask, d.cnt_sw, d.Fpart,
                        d.upart, fscale, escale, Fo,
                        d.uout, d.V[d.cur], sa, d.pstride, d.partials, d.ctl, (const T4 *)d.EX,
-                       (const T4 *)d.EXself, d.exmask, d.halt);
+                       (const T4 *)d.EXself, d.exmask, d.halt, xcd_shift(d));
   }
   if (MODE == 1) finalize_thermo(d, s);
   if (MODE == 2) {
@@ -3001,7 +3172,7 @@ void launch_pos(const DevBufs &d, const StepArgs &sa, hipStream_t s) {
     KScope ks_(d, KT_POS);
     hipLaunchKernelGGL(k_pos, dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), 0, s, d.X[d.cur], d.I, d.NA,
                        d.V[d.cur], d.F[d.cur], d.Xi[d.cur], sa, d.pstride, d.partials, d.ctl,
-                       d.Xb, d.disp);
+                       d.Xb, d.disp, d.Wsw, d.cnt_sw, d.nbr_sw, d.nst);
   }
   const int op[4] = {0, 1, 1, 1};
   const int dst[4] = {DCTL_IDX(eq_sum), DCTL_IDX(kemax), DCTL_IDX(maxdisp), DCTL_IDX(maxdisp2)};
@@ -3015,12 +3186,13 @@ void launch_md_pos(const DevBufs &d, const FConst &fc, const StepArgs &sa, int *
     KScope ks_(d, KT_POS);
     hipLaunchKernelGGL(k_md_pos, dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), 0, s, d.X[d.cur], d.I,
                        d.NA, d.V[d.cur], d.F[d.cur], d.Xi[d.cur], sa, d.pstride, d.partials,
-                       d.ctl, d.Xb, d.disp, leave, d.halt);
+                       d.ctl, d.Xb, d.disp, d.Wsw, d.cnt_sw, d.nbr_sw, d.nst, leave, d.halt,
+                       xcd_shift(d));
   }
-  const int op[5] = {RED_TOP2, RED_TOP2_CNT, RED_TOP2_SND, RED_SUM, RED_SUM};
-  const int dst[5] = {DCTL_IDX(maxdisp), DCTL_IDX(nmaxdisp), DCTL_IDX(maxdisp2),
-                      DCTL_IDX(e_bath_step), DCTL_IDX(e_out_step)};
-  finalize(d, 5, FIB_BLOCK, op, dst, s);
+  const int op[6] = {RED_TOP2, RED_TOP2_CNT, RED_TOP2_SND, RED_SUM, RED_SUM, RED_SUM};
+  const int dst[6] = {DCTL_IDX(maxdisp), DCTL_IDX(nmaxdisp), DCTL_IDX(maxdisp2),
+                      DCTL_IDX(e_bath_step), DCTL_IDX(e_out_step), DCTL_IDX(movers)};
+  finalize(d, 6, FIB_BLOCK, op, dst, s);
   hipLaunchKernelGGL(k_md_decide, dim3(1), dim3(DECIDE_T), 0, s, d.ninst, d.I, d.ctl, sa.skin,
                      gate, leave, d.X[d.cur], fc, d.Wsw, d.Wion, d.cnt_sw, d.nbr_sw, d.cnt_ion,
                      d.nbr_ion, d.halt);
@@ -3056,7 +3228,7 @@ void launch_md_report(const DevBufs &d, const StepArgs &sa, hipStream_t s) {
 void launch_mark_build(const DevBufs &d, hipStream_t s, bool count) {
   KScope ks_(d, KT_LISTAUX);
   hipLaunchKernelGGL(k_mark_build, dim3(gcap(std::max(d.NA, d.ninst))), dim3(FIB_BLOCK), 0,
-                     s, d.NA, d.ninst, d.Wsw, d.Wion, d.X[d.cur], d.Xb, d.disp, d.ctl, d.binst,
+                     s, d.NA, d.ninst, d.Wsw, d.Wion, d.X[d.cur], d.Xb, d.disp, d.nst, d.ctl, d.binst,
                      d.gate, d.halt, count ? 1.0 : 0.0);
 }
 

@@ -254,10 +254,17 @@ static void derive_constants(fib_handle *h) {
       c.fsw[a][b] = (float)(c.epssig[a][b] / (c.eps[0][0] * c.isig[0][0]));
     }
   c.skin = rc - c.cut_sw * std::max(p.sigma_si, p.sigma_ge);
+  double gate;  // the pair pass's cutoff in units of sigma
   {
     const double ug = std::max(c.umax * (double)(izero - 1) / (double)(nt - 1), c.cut_sw);
     c.r2gate = (1.001 * ug) * (1.001 * ug);
+    gate = h->prec == FIB_PREC_MIXED ? std::sqrt(c.cut_sw2) : 1.001 * ug;
   }
+  // near lists: delta is a tenth of the skin (the partners' movement counts
+  // in FP32, hence the margin)
+  const double delta = std::max(0.0, 0.1 * c.skin);
+  const double isgmax = std::max(c.isig[0][0], std::max(c.isig[0][1], c.isig[1][1]));
+  c.near2 = (gate + delta * isgmax * (1.0 + 1e-5)) * (gate + delta * isgmax * (1.0 + 1e-5));
   h->tab.assign(nt + 3, TabEntry{0, 0, 0, 0, 0, 0});
   for (int i = 1; i <= nt; ++i) {
     TabEntry &e = h->tab[i];
@@ -269,13 +276,14 @@ static void derive_constants(fib_handle *h) {
   b.mass[0] = p.mass_si; b.mass[1] = p.mass_ge; b.mass[2] = p.mass_ga;
   b.kB = p.kB;
   b.ec = p.ec;
+  b.near_d = (float)(0.5 * delta);
 }
 
 static int32_t free_bufs(fib_handle *h) {
   DevBufs &d = h->d;
   void *ptrs[] = {d.I, d.ctl, d.ibase, d.binst, d.X[0], d.X[1], d.V[0], d.V[1], d.F[0], d.F[1], d.Xi[0], d.Xi[1],
                   d.inv, d.bkey, d.brank, d.bcnt, d.cstart, d.perm, d.bsum, d.cnt_sw, d.nbr_sw,
-                  d.cnt_ion, d.nbr_ion, d.rk_sw, d.off_sw, d.G, d.RA, d.amask, d.Xb, d.disp, d.EX, d.EXself, d.exmask, d.Fpart, d.upart, d.Fout, d.uout,
+                  d.cnt_ion, d.nbr_ion, d.rk_sw, d.off_sw, d.near, d.nst, d.G, d.RA, d.amask, d.Xb, d.disp, d.EX, d.EXself, d.exmask, d.Fpart, d.upart, d.Fout, d.uout,
                   d.partials, d.fin_tmp, d.tab, d.xfer};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
@@ -451,6 +459,8 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
   ALLOC(d.cnt_sw, NA);
   ALLOC(d.cnt_ion, NA);
   ALLOC(d.amask, NA);
+  ALLOC(d.near, (size_t)16 * NA);
+  ALLOC(d.nst, NA);
   ALLOC(d.off_sw, (size_t)32 * NA);
   ALLOC(d.Xb, NA);
   ALLOC(d.disp, NA);
@@ -490,6 +500,7 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
   if (e == hipSuccess) e = hipMemset(d.ctl, 0, sizeof(DCtl) * ninst);
   if (e == hipSuccess) e = hipMemset(d.cnt_sw, 0, sizeof(int) * NA);
   if (e == hipSuccess) e = hipMemset(d.cnt_ion, 0, sizeof(int) * NA);
+  if (e == hipSuccess) e = hipMemset(d.nst, 254, NA);
   if (e == hipSuccess) e = hipMemset(d.amask, 0, sizeof(uint64_t) * NA);
   if (e == hipSuccess) e = hipMemset(d.exmask, 0, sizeof(uint64_t) * NA);
   if (e == hipSuccess) e = hipMemset(d.off_sw, 0, (size_t)32 * NA);
