@@ -653,9 +653,6 @@ __global__ void k_copyback(int NA, const double4 *__restrict__ X1, double4 *__re
 // neighbour build: one 64-lane block per real cell
 #define NB_CHUNK 128
 #define NB_ACC 384  // candidates whose acceptance masks are kept for the ranks
-#ifndef NB_CELLS
-#define NB_CELLS 8  // cells per k_nbuild wavefront
-#endif
 #ifndef NB_WAVES
 #define NB_WAVES 4  // independent wavefronts per k_nbuild workgroup
 #endif
@@ -690,6 +687,204 @@ __device__ __forceinline__ int stencil_axis(int c, int d, int n, bool &ok) {
     ok = false;
   }
   return v;
+}
+
+// v of another lane (uniform), through scalar registers
+__device__ __forceinline__ float bcast(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ double bcast(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+__device__ __forceinline__ int mbcnt(uint64_t m) {
+  return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// One cell whose halo fits two candidates per lane (all but very dense ones).
+// The build is bound by vector instructions, so the work that does not
+// depend on the atom is done once per cell:
+//  - the periodic shift k L of every candidate, from its difference to the
+//    cell's first atom (the reference's NINT gives the same k for every atom
+//    of the cell when no difference comes near half a box: checked);
+//  - candidates farther than the cutoff from the box around the cell's atoms
+//    are dropped (FP32 with a margin; of ~105 about 60 stay), the others
+//    compacted in order, so most cells test one candidate per lane.
+// The candidates then stay in registers, the atom's position comes through
+// scalar registers, and the reference's predicate is evaluated as ref_r2
+// does, without contraction.  False (nothing written) when a difference is
+// too close to half a box, as in boxes of few cells.
+// 2.1 M atoms (whole build): 720 -> 523 vector instructions a cell, 871 ->
+// 651 us (four waves per SIMD; asked for five or six it spills and takes
+// longer than before).
+__device__ __forceinline__ bool nbuild_cell_fast(
+    const double4 *__restrict__ X, const DInst &in, int i0, int ni, int rs, int rc, int my_lo,
+    int total, uint64_t lm0, uint64_t lm1, double rv2, double rv2lj, int Wsw, int Wion,
+    int *__restrict__ cnt_sw, int *__restrict__ nbr_sw, int *__restrict__ cnt_ion,
+    int *__restrict__ nbr_ion, uint16_t *__restrict__ rk_sw, uint8_t *__restrict__ off_sw,
+    double4 *s_x, int *s_j) {
+#pragma clang fp contract(off)
+  const int lane = threadIdx.x % FIB_WAVE;
+  constexpr bool NBNT = (FIB_NT_ST & 16) != 0;
+  constexpr uint32_t JM = (1u << NB_JBITS) - 1u;
+  // each stencil lane writes its own run of candidates, stencil cell above
+  for (int q = 0; __ballot(q < rc) != 0ull; ++q)
+    if (q < rc) s_j[my_lo + q] = (int)((uint32_t)lane << NB_JBITS | (uint32_t)(rs + q));
+  wave_lds_sync();
+  const double4 own = X[i0 + min(lane, ni - 1)];
+  const int town = type_of(meta_of(own));
+  const double c[3] = {bcast(own.x, 0), bcast(own.y, 0), bcast(own.z, 0)};
+  const float own0[3] = {(float)(own.x - c[0]), (float)(own.y - c[1]), (float)(own.z - c[2])};
+  float lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
+  for (int ii = 1; ii < ni; ++ii) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const float r = bcast(own0[a], ii);
+      lo[a] = fminf(lo[a], r);
+      hi[a] = fmaxf(hi[a], r);
+    }
+  }
+  // differences to the cell's first atom
+  const bool two = total > FIB_WAVE;
+  uint32_t up[2];
+  double4 x[2];
+  double e0[2][3];
+  bool have[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    have[t] = t * FIB_WAVE + lane < total;
+    up[t] = have[t] ? (uint32_t)s_j[t * FIB_WAVE + lane] : ~0u;
+    if (t == 0 || two) x[t] = X[have[t] ? (int)(up[t] & JM) : i0];
+  }
+  int far[3] = {0, 0, 0};
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    if (t == 1 && !two) x[1] = x[0];
+    e0[t][0] = c[0] - x[t].x;
+    e0[t][1] = c[1] - x[t].y;
+    e0[t][2] = c[2] - x[t].z;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) far[a] = max(far[a], __double2hiint(e0[t][a]) & 0x7fffffff);
+  }
+  // all of them below 0.12 of the box (by the upper words): then every
+  // difference from an atom of the cell is below 0.24 and no shift is wanted
+  bool any = false;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) any = any || far[a] >= __double2hiint(0.12 * in.lb[a]);
+  const bool wraps = __ballot(any) != 0ull;
+  uint32_t code[2] = {0x150u, 0x150u};
+  if (wraps) {
+    bool bad = false;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      const bool mine = (up[t] >> NB_JBITS) == 13u;
+      code[t] = 0;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const double k = rint(e0[t][a] * in.ilb[a]);
+        const double e = e0[t][a] - k * in.lb[a];
+        e0[t][a] = e;
+        // shifts 0 and +-1 are coded 1, 2, 0
+        code[t] |= (uint32_t)((int)k + 1) << (4 + 2 * a);
+        bad = bad || (have[t] && (fabs(k) > 1.0 || fabs(e) > 0.49 * in.lb[a] - 1.001 * in.h[a] ||
+                                  (mine && (k != 0.0 || fabs(e) > 1.001 * in.h[a]))));
+      }
+    }
+    if (__ballot(bad) != 0ull) return false;
+  }
+  float d2[2];
+  bool ion = town == 3;
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    float sum = 0.0f;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      const float r = (float)-e0[t][a];
+      const float d = fmaxf(fmaxf(lo[a] - r, r - hi[a]), 0.0f);
+      sum += d * d;
+    }
+    const uint32_t ty = meta_of(x[t]) & META_TYPE_MASK;
+    ion = ion || ty == 3u;
+    x[t].w = __longlong_as_double((long long)((uint64_t)up[t] << 32 | (uint64_t)(code[t] | ty)));
+    d2[t] = have[t] ? sum : 3.0e38f;
+  }
+  // without a Ga atom around, only pairs within the SW list radius are wanted
+  const bool ions = __ballot(ion) != 0ull;
+  const float r2max = (float)(ions ? fmax(rv2, rv2lj) : rv2) * 1.0001f;
+  const uint64_t k0 = __ballot(d2[0] <= r2max), k1 = __ballot(d2[1] <= r2max);
+  const int n0 = __popcll(k0), nk = n0 + __popcll(k1);
+  if (d2[0] <= r2max) s_x[mbcnt(k0)] = x[0];
+  if (d2[1] <= r2max) s_x[n0 + mbcnt(k1)] = x[1];
+  // kept candidates before stencil cell s (lane s)
+  const int klo = __popcll(k0 & lm0) + __popcll(k1 & lm1);
+  wave_lds_sync();
+  auto rows = [&](auto sets) {
+    constexpr int NS = decltype(sets)::value;
+    double y[NS][3];
+    uint32_t u[NS], low[NS];
+    uint64_t before_m[NS];
+    int acc[NS];  // atoms of the cell so far that the candidate accepted
+#pragma unroll
+    for (int t = 0; t < NS; ++t) {
+      const double4 v = s_x[t * FIB_WAVE + lane];  // (past nk: unused)
+      y[t][0] = v.x; y[t][1] = v.y; y[t][2] = v.z;
+      u[t] = (uint32_t)(wbits(v) >> 32);
+      low[t] = (uint32_t)wbits(v);
+      acc[t] = 0;
+      const int cut = min(max(klo - t * FIB_WAVE, 0), FIB_WAVE);
+      before_m[t] = cut >= FIB_WAVE ? ~0ull : ((1ull << cut) - 1ull);
+    }
+    for (int ii = 0; ii < ni; ++ii) {
+      const int i = i0 + ii;
+      int *const rowj = nbr_sw + (size_t)i * Wsw;
+      uint16_t *const rowk = rk_sw + (size_t)i * Wsw;
+      const double xi[3] = {bcast(own.x, ii), bcast(own.y, ii), bcast(own.z, ii)};
+      int nsw = 0, nion = 0, before = 0;
+#pragma unroll
+      for (int t = 0; t < NS; ++t) {
+        const int j = (int)(u[t] & JM);
+        double d[3];
+#pragma unroll
+        for (int a = 0; a < 3; ++a) d[a] = xi[a] - y[t][a];
+        if (wraps) {
+#pragma unroll
+          for (int a = 0; a < 3; ++a)
+            d[a] = d[a] - (double)((int)(low[t] >> (4 + 2 * a) & 3u) - 1) * in.lb[a];
+        }
+        const double r2 = ref_sq(d[0], d[1], d[2]);
+        const bool cand = t * FIB_WAVE + lane < nk && j != i;
+        bool sw = cand && r2 < rv2;
+        if (ions) {
+          const int ti = __builtin_amdgcn_readlane(town, ii);
+          const bool swp = max(ti, (int)(low[t] & META_TYPE_MASK)) < 3;
+          const bool io = cand && !swp && r2 < rv2lj;
+          sw = sw && swp;
+          const uint64_t mio = __ballot(io);
+          const int pos = nion + mbcnt(mio);
+          if (io && pos < Wion) st_nt<NBNT>(nbr_ion + (size_t)i * Wion + pos, j);
+          nion += __popcll(mio);
+        }
+        const uint64_t msw = __ballot(sw);
+        const int pos = nsw + mbcnt(msw);
+        if (sw && pos < Wsw) {
+          st_nt<NBNT>(rowj + pos, j);
+          st_nt<NBNT>(rowk + pos, (uint16_t)((u[t] >> NB_JBITS) << 8 | (uint32_t)acc[t]));
+        }
+        acc[t] += sw ? 1 : 0;
+        before += __popcll(msw & before_m[t]);
+        nsw += __popcll(msw);
+      }
+      if (lane < 27) st_nt<NBNT>(off_sw + (size_t)i * OFF_W + lane, (uint8_t)min(before, 254));
+      if (lane == 0) {
+        st_nt<NBNT>(cnt_sw + i, nsw);
+        st_nt<NBNT>(cnt_ion + i, nion);
+      }
+    }
+  };
+  if (nk <= FIB_WAVE) rows(std::integral_constant<int, 1>{});
+  else rows(std::integral_constant<int, 2>{});
+  return true;
 }
 
 // One cell (cx, cy, cz) of instance `in`, built by one wave.
@@ -736,6 +931,11 @@ __device__ __forceinline__ void nbuild_cell(
     const int cut = min(max(my_lo - b, 0), 64);
     return cut >= 64 ? ~0ull : ((1ull << cut) - 1ull);
   };
+  if (total <= NB_CHUNK && ni <= 32 &&
+      nbuild_cell_fast(X, in, i0, ni, rs, rc, my_lo, total, before_mask(0), before_mask(FIB_WAVE),
+                       rv2, rv2lj, Wsw, Wion, cnt_sw, nbr_sw, cnt_ion, nbr_ion, rk_sw, off_sw,
+                       s_x, s_j))
+    return;
   const bool masks = total <= NB_ACC && ni <= 32;
   if (masks)
     for (int g = lane; g < total; g += FIB_WAVE) s_acc[g] = 0;
@@ -897,7 +1097,7 @@ __device__ __forceinline__ int locate_cell(const DInst *__restrict__ I, int nins
   return lo;
 }
 
-// Each wavefront builds NBC consecutive cells (NB_CELLS by default); a workgroup holds
+// Each wavefront builds NBC consecutive cells; a workgroup holds
 // NB_WAVES independent wavefronts (their own LDS, wave-level sync only), so
 // that the workgroup-per-CU limit does not cap the resident waves.  The cells
 // to build are all real cells, or under a gate the cells of the gated
@@ -906,13 +1106,9 @@ __device__ __forceinline__ int locate_cell(const DInst *__restrict__ I, int nins
 // at once (gated-out instances cost a launch of empty workgroups, no more).
 // The busy workgroups are remapped so that each XCD builds a contiguous run
 // of cells, whose halos then stay in its L2.  A wave decodes its first cell
-// once and steps through the rest in x-fastest order.  The occupancy hint
-// asks for seven waves per SIMD; allocation still ends at six (73 VGPRs),
-// but the schedule built for seven runs 3-4 % faster than the one for six
-// (same-box timing of both builds).
+// once and steps through the rest in x-fastest order.
 template <int NBC>
-__global__ __launch_bounds__(NB_WAVES * FIB_WAVE) __attribute__((amdgpu_waves_per_eu(7)))
-void k_nbuild(
+__global__ __launch_bounds__(NB_WAVES * FIB_WAVE) void k_nbuild(
     const double4 *__restrict__ X, const DInst *__restrict__ I, int ninst, int total_cells,
     const int *__restrict__ cstart, const int *__restrict__ bcnt, double rv2, double rv2lj,
     int Wsw, int Wion, int *__restrict__ cnt_sw, int *__restrict__ nbr_sw,
@@ -2907,6 +3103,16 @@ static int xcd_shift(const DevBufs &d) {
   return s;
 }
 
+// Cells per wavefront of the list build: a wavefront builds its cells one
+// after the other, each with two or three dependent loads, so a small batch
+// takes few per wavefront (4 k atoms, whole build: 8 cells 46 us, 4 cells 28,
+// 1 cell 12; 101 k atoms: 55, 50 and 50) and a large one eight, which share
+// the decoding of their position (2.1 M atoms: 4 cells 682 us, 8 cells 651,
+// 16 cells 675).
+static int nb_cells_auto(int total_cells) {
+  return total_cells < 65536 ? 1 : total_cells < 131072 ? 2 : total_cells < 262144 ? 4 : 8;
+}
+
 // Times the launches issued in its scope under one key.
 struct KScope {
   const KTimer *t;
@@ -3039,16 +3245,19 @@ void launch_nbuild(const DevBufs &d, const FConst &fc, hipStream_t s) {
   }
   if (d.total_cells > 0) {
     KScope ks_(d, KT_NBUILD);
-    const int nbc = d.nb_cells ? d.nb_cells : NB_CELLS;
+    const int nbc = d.nb_cells ? d.nb_cells : nb_cells_auto(d.total_cells);
 #define NB_LAUNCH(C)                                                                          \
   hipLaunchKernelGGL(k_nbuild<C>, dim3(nblk(d.total_cells, C * NB_WAVES)),                    \
                      dim3(NB_WAVES * FIB_WAVE), 0, s, d.X[d.cur], d.I, d.ninst, d.total_cells, \
                      d.cstart, d.bcnt, fc.rv2, fc.rv2lj, d.Wsw, d.Wion, d.cnt_sw, d.nbr_sw,   \
                      d.cnt_ion, d.nbr_ion, d.rk_sw, d.off_sw, d.gate)
-    if (nbc == NB_CELLS) NB_LAUNCH(NB_CELLS);
-    else if (nbc == 4) NB_LAUNCH(4);
-    else if (nbc == 16) NB_LAUNCH(16);
-    else NB_LAUNCH(8);
+    switch (nbc) {
+      case 1: NB_LAUNCH(1); break;
+      case 2: NB_LAUNCH(2); break;
+      case 4: NB_LAUNCH(4); break;
+      case 16: NB_LAUNCH(16); break;
+      default: NB_LAUNCH(8); break;
+    }
 #undef NB_LAUNCH
   }
   {
