@@ -6,8 +6,8 @@
 #include "../../include/fibgpu.h"
 #include "fib_device.h"
 
-// Workgroup size of the per-instance reductions (k_finalize).
-#define FIB_FIN_T 1024
+#define FIB_FIN_CH 256    // blocks whose partials one wavefront reduces (k_finalize)
+#define FIB_SORT_N 8192   // most atoms and buckets of an instance sorted by one workgroup
 #define FIB_LEAVE_CAP 256  // atoms that may leave the simulation in one MD step
 
 // Per-step arguments of the integrate kernels (onestep, timeint.f90:158-242).
@@ -72,7 +72,6 @@ struct DevBufs {
   double4 *X[2];
   double *V[2], *F[2], *Xi[2];
   int *inv;                  // [NA] atom_off + orig -> sorted position
-  int *ibase;                // [ninst] scan offset of each instance's first bucket
   int *binst;                // [NA / FIB_BLOCK] instance of each block of FIB_BLOCK atoms
   int *bkey, *brank, *bcnt, *cstart, *perm, *bsum;
   int *cnt_sw, *nbr_sw, *cnt_ion, *nbr_ion;
@@ -93,8 +92,9 @@ struct DevBufs {
   double *Fout, *uout;       // force-only results [3*NA], [NA]
   double *partials;          // [2 * FIB_NRED * pstride], layout [region][slot][block]
   int max_pad;               // largest padded atom count of an instance
+  int max_bucket;            // most buckets of an instance
   double *fin_tmp;           // chunk results of big instances' reductions
-                             // [ninst * (max_pad / 64 / FIB_FIN_T + 1) * FIB_NRED]
+                             // [ninst * (max_pad / 256 / FIB_FIN_CH + 1) * FIB_NRED]
   int pstride;               // NA/64 + 1
   TabEntry *tab;             // [ntable + 3]
   double *xfer;              // staging [3*NA] for host transfers
@@ -106,16 +106,15 @@ struct DevBufs {
 };
 
 namespace fibk {
-void launch_bin(const DevBufs &d, hipStream_t s);
-void launch_scan(const DevBufs &d, hipStream_t s);
-// scatter + fixup + reorder: flips cur, or (inplace) copies back and keeps cur
-void launch_sort(const DevBufs &d, hipStream_t s, bool inplace = false);
-// list build + longest-list reduction (DCtl::maxcnt_*)
-void launch_nbuild(const DevBufs &d, const FConst &fc, hipStream_t s);
+// binning, sort and list build of every instance (or of the gated ones): the
+// arrays move to the other buffers (the caller flips cur), or (inplace) back
+// into the current ones
+void launch_build(const DevBufs &d, const FConst &fc, hipStream_t s, bool inplace);
+// the list build alone, of the positions X[from] (again, after the lists
+// grew); back: copies the reordered arrays into the current ones beside it.
+// A list longer than its width goes to DCtl::maxcnt_*.
+void launch_nbuild(const DevBufs &d, const FConst &fc, hipStream_t s, int from, bool back = false);
 void launch_cellid(const DevBufs &d, int inst, int32_t *dout, hipStream_t s);
-// positions of the new build (Xb), displacement bookkeeping reset; count =
-// false repeats a build after the lists grew (the build count stays)
-void launch_mark_build(const DevBufs &d, hipStream_t s, bool count = true);
 // ELL rows into a wider layout: dst[p * wnew + k] = src[p * wold + k]
 void launch_copy_rows(int NA, int wold, const int *src, int wnew, int *dst, hipStream_t s);
 void launch_copy_rows(int NA, int wold, const uint16_t *src, int wnew, uint16_t *dst,
@@ -127,7 +126,7 @@ void launch_fill_zero(void *p, size_t bytes, hipStream_t s);
 void launch_copy_utot(const DevBufs &d, double *out, hipStream_t s);
 // clears the leaving mark of every atom (after a removal-list overflow)
 void launch_clear_leaving(const DevBufs &d, hipStream_t s);
-// lists = true: clears the list-overflow flags and the halt flag; false: the
+// lists = true: clears the list-overflow flags, the longest lists and the halt flag; false: the
 // removal-list overflow flags
 void launch_clear_overflow(const DevBufs &d, hipStream_t s, bool lists = true);
 // passes 1-2 (k_legs, k_tri): own pair terms and legs, centre-term shares

@@ -81,6 +81,14 @@ __device__ __forceinline__ bool block_gated_out(const int *gate, const int *__re
 
 // ---------------------------------------------------------------------------
 // helpers
+#define OFF_W 32        // bytes per atom of the stencil-offset table (27 used)
+// states of an atom's near list (see near_mark_moved): its number of entries,
+// at most NEAR_CAP, or one of
+#define NEAR_CAP 16
+#define NEAR_J 0x7ffffffu
+#define NEAR_MOVED 253  // moved more than delta / 2 and told its partners
+#define NEAR_FULL 254   // no near list
+#define NEAR_FRESH 255  // just built: the next pass makes the near list
 __device__ __forceinline__ uint64_t wbits(const double4 &x) {
   return (uint64_t)__double_as_longlong(x.w);
 }
@@ -303,103 +311,131 @@ __device__ void block_partials(double (&v)[NV], const int (&op)[NV], int lblock,
   }
 }
 
-#define FIN_T FIB_FIN_T
-// Per instance, combine the partials of its blocks in a fixed order.  One
-// workgroup per instance when the instance has at most FIN_T blocks (thread t
-// takes block t, then a fixed tree); otherwise workgroup (inst, c) reduces
-// blocks [c*FIN_T, (c+1)*FIN_T) into tmp and k_finalize2 combines the
-// chunks in order -- a big instance then spreads over many CUs.  All NV
-// slots at once, so the loads of every slot are in flight together.
+// Per instance, combine the partials of its blocks in a fixed order that
+// depends on the instance alone: one wavefront per chunk of FIN_CH blocks
+// (lane l takes blocks l, l + 64, ..., then a butterfly), and, when the
+// instance has more than one, one wavefront over its chunks the same way.
+// All NV slots at once, so the loads of every slot are in flight together.
+// A wavefront per chunk instead of a workgroup of 1024 threads per 1024
+// blocks: 14 -> 5 us a reduction, at 4 k as at 2 M atoms.
+#define FIN_CH FIB_FIN_CH
+// red_merge with the operations of a RedSpec: k_md_pos' six slots start with a
+// top-two triple, every other reduction is sums and maxima.
 template <int NV>
-__device__ __forceinline__ void fin_block_tree(double (&x)[NV], const RedSpec &rs,
-                                               double (*red)[NV]) {
-  const int lane = threadIdx.x % FIB_WAVE, wid = threadIdx.x / FIB_WAVE;
+__device__ __forceinline__ void fin_merge(double (&x)[NV], const double (&y)[NV],
+                                          const RedSpec &rs) {
+  constexpr int K0 = NV == 6 ? 3 : 0;
+  if constexpr (NV == 6) top2_merge(x[0], x[1], x[2], y[0], y[1], y[2]);
+#pragma unroll
+  for (int k = K0; k < NV; ++k) x[k] = rs.op[k] == RED_MAX ? fmax(x[k], y[k]) : x[k] + y[k];
+}
+__device__ __forceinline__ int fin_chunks(const DInst &in, int bs) {
+  return (in.natm_pad / bs + FIN_CH - 1) / FIN_CH;
+}
+template <int NV>
+__device__ __forceinline__ void fin_wave(double (&x)[NV], const RedSpec &rs) {
   for (int o = FIB_WAVE / 2; o > 0; o >>= 1) {
     double y[NV];
 #pragma unroll
     for (int k = 0; k < NV; ++k) y[k] = __shfl_xor(x[k], o);
-    red_merge<NV>(x, y, rs.op);
+    fin_merge<NV>(x, y, rs);
   }
-  if (lane == 0) {
-#pragma unroll
-    for (int k = 0; k < NV; ++k) red[wid][k] = x[k];
-  }
-  __syncthreads();
 }
+// chunk c of instance `in` from the producers' partials
 template <int NV>
-__global__ __launch_bounds__(FIN_T) void k_finalize(const DInst *__restrict__ I,
-                                                    const double *__restrict__ partials,
-                                                    int pstride, RedSpec rs,
-                                                    DCtl *__restrict__ ctl,
-                                                    const int *__restrict__ gate,
-                                                    double *__restrict__ tmp,
-                                                    const int *__restrict__ halt) {
-  GATE_OR_RETURN(gate);
-  HALT_OR_RETURN(halt);
-  __shared__ double red[FIN_T / FIB_WAVE][NV];
-  const int inst = blockIdx.x, ch = blockIdx.y, nch = gridDim.y;
-  if (gated_out(gate, inst)) return;  // its producer skipped its blocks
-  const int blk0 = I[inst].atom_off / rs.bs, nblk = I[inst].natm_pad / rs.bs;
-  double x[NV];
+__device__ __forceinline__ void fin_chunk(double (&x)[NV], const DInst &in, int c,
+                                          const double *__restrict__ partials, int pstride,
+                                          const RedSpec &rs) {
+  const int blk0 = in.atom_off / rs.bs, nblk = in.natm_pad / rs.bs;
+  const int lane = threadIdx.x % FIB_WAVE;
 #pragma unroll
   for (int k = 0; k < NV; ++k) x[k] = red_identity(rs.op[k]);
-  const int b_lo = nch == 1 ? 0 : ch * FIN_T;
-  const int b_hi = nch == 1 ? nblk : min(nblk, b_lo + FIN_T);
-  for (int b = b_lo + (int)threadIdx.x; b < b_hi; b += FIN_T) {
+  constexpr int UN = NV < 10 ? FIN_CH / FIB_WAVE : 1;
+#pragma unroll UN
+  for (int m = 0; m < FIN_CH / FIB_WAVE; ++m) {
+    const int b = c * FIN_CH + m * FIB_WAVE + lane;
+    if (b < nblk)
+      for (int r = 0; r < (NV == 10 ? rs.nreg : 1); ++r) {
+        double y[NV];
+#pragma unroll
+        for (int k = 0; k < NV; ++k)
+          y[k] = partials[(size_t)(r * FIB_NRED + k) * pstride + blk0 + b];
+        fin_merge<NV>(x, y, rs);
+      }
+  }
+  fin_wave<NV>(x, rs);
+}
+// the chunks of an instance
+template <int NV>
+__device__ __forceinline__ void fin_combine(double (&x)[NV], int inst, int nci, int nch,
+                                            const double *__restrict__ tmp, const RedSpec &rs) {
+#pragma unroll
+  for (int k = 0; k < NV; ++k) x[k] = red_identity(rs.op[k]);
+  for (int c = threadIdx.x % FIB_WAVE; c < nci; c += FIB_WAVE) {
     double y[NV];
 #pragma unroll
-    for (int k = 0; k < NV; ++k) y[k] = partials[(size_t)k * pstride + blk0 + b];
-    for (int r = 1; r < rs.nreg; ++r) {
-      double y2[NV];
-#pragma unroll
-      for (int k = 0; k < NV; ++k) y2[k] = partials[(size_t)(r * FIB_NRED + k) * pstride + blk0 + b];
-      red_merge<NV>(y, y2, rs.op);
-    }
-    red_merge<NV>(x, y, rs.op);
+    for (int k = 0; k < NV; ++k) y[k] = tmp[((size_t)inst * nch + c) * NV + k];
+    fin_merge<NV>(x, y, rs);
   }
-  fin_block_tree<NV>(x, rs, red);
-  if (threadIdx.x == 0) {
-    double t[NV];
+  fin_wave<NV>(x, rs);
+}
+template <int NV>
+__device__ __forceinline__ void fin_store(const double (&x)[NV], const RedSpec &rs, DCtl &ctl) {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) t[k] = red[0][k];
-    for (int w = 1; w < FIN_T / FIB_WAVE; ++w) {
-      double y[NV];
+  for (int k = 0; k < NV; ++k)
+    if (rs.dst[k] >= 0) reinterpret_cast<double *>(&ctl)[rs.dst[k]] = x[k];
+}
+// one wavefront of any workgroup: the rest of the reduction of instance
+// `inst` into its control record, with how = FIN_ALL from the partials (the
+// instance has one chunk), FIN_COMBINE from the chunks k_finalize left in
+// tmp, FIN_DONE nothing
+enum { FIN_DONE = 0, FIN_COMBINE = 1, FIN_ALL = 2 };
+template <int NV>
+__device__ __forceinline__ void fin_finish(int how, int inst, const DInst &in,
+                                           const double *__restrict__ partials, int pstride,
+                                           const double *__restrict__ tmp, int nch,
+                                           const RedSpec &rs, DCtl &ctl) {
+  if (how == FIN_DONE) return;
+  double x[NV];
+  if (how == FIN_ALL) {
+    fin_chunk<NV>(x, in, 0, partials, pstride, rs);
+  } else {
+    const int nci = fin_chunks(in, rs.bs);
+    if (nci < 2) return;  // k_finalize stored it
+    fin_combine<NV>(x, inst, nci, nch, tmp, rs);
+  }
+  if (threadIdx.x % FIB_WAVE == 0) fin_store<NV>(x, rs, ctl);
+}
+template <int NV>
+__global__ __launch_bounds__(FIB_WAVE) void k_finalize(const DInst *__restrict__ I,
+                                                       const double *__restrict__ partials,
+                                                       int pstride, RedSpec rs,
+                                                       DCtl *__restrict__ ctl,
+                                                       double *__restrict__ tmp,
+                                                       const int *__restrict__ halt) {
+  HALT_OR_RETURN(halt);
+  const int inst = blockIdx.x, c = blockIdx.y, nch = gridDim.y;
+  const DInst &in = I[inst];
+  const int nci = fin_chunks(in, rs.bs);
+  if (c >= nci) return;
+  double x[NV];
+  fin_chunk<NV>(x, in, c, partials, pstride, rs);
+  if (threadIdx.x != 0) return;
+  if (nci == 1) {
+    fin_store<NV>(x, rs, ctl[inst]);
+  } else {
 #pragma unroll
-      for (int k = 0; k < NV; ++k) y[k] = red[w][k];
-      red_merge<NV>(t, y, rs.op);
-    }
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-      if (nch == 1) {
-        if (rs.dst[k] >= 0) reinterpret_cast<double *>(&ctl[inst])[rs.dst[k]] = t[k];
-      } else {
-        tmp[((size_t)inst * nch + ch) * NV + k] = t[k];
-      }
-    }
+    for (int k = 0; k < NV; ++k) tmp[((size_t)inst * nch + c) * NV + k] = x[k];
   }
 }
 template <int NV>
-__global__ void k_finalize2(const DInst *__restrict__ I, int nch, RedSpec rs,
-                            DCtl *__restrict__ ctl, const int *__restrict__ gate,
-                            const double *__restrict__ tmp, const int *__restrict__ halt) {
-  GATE_OR_RETURN(gate);
+__global__ __launch_bounds__(FIB_WAVE) void k_finalize2(const DInst *__restrict__ I, int nch,
+                                                        RedSpec rs, DCtl *__restrict__ ctl,
+                                                        const double *__restrict__ tmp,
+                                                        const int *__restrict__ halt) {
   HALT_OR_RETURN(halt);
   const int inst = blockIdx.x;
-  if (threadIdx.x != 0 || gated_out(gate, inst)) return;
-  const int nci = (I[inst].natm_pad / rs.bs + FIN_T - 1) / FIN_T;
-  const double *t0 = tmp + (size_t)inst * nch * NV;
-  double t[NV];
-#pragma unroll
-  for (int k = 0; k < NV; ++k) t[k] = red_identity(rs.op[k]);
-  for (int c = 0; c < nci; ++c) {
-    double y[NV];
-#pragma unroll
-    for (int k = 0; k < NV; ++k) y[k] = t0[(size_t)c * NV + k];
-    red_merge<NV>(t, y, rs.op);
-  }
-#pragma unroll
-  for (int k = 0; k < NV; ++k)
-    if (rs.dst[k] >= 0) reinterpret_cast<double *>(&ctl[inst])[rs.dst[k]] = t[k];
+  fin_finish<NV>(FIN_COMBINE, inst, I[inst], nullptr, 0, tmp, nch, rs, ctl[inst]);
 }
 
 // ---------------------------------------------------------------------------
@@ -407,6 +443,33 @@ __global__ void k_finalize2(const DInst *__restrict__ I, int nch, RedSpec rs,
 // lanes of a wavefront form runs of equal buckets: each run takes its ranks
 // with one atomic add of its length.  Ranks only need to be distinct; k_fixup
 // orders every bucket by previous position.
+// Bucket of an atom within its instance (not a padding slot): its cell, or the
+// last two buckets for atoms outside every list and removed ones.
+__device__ __forceinline__ int bucket_of(const double4 &x, const DInst &in, DCtl &ctl) {
+  if (meta_of(x) & META_DEAD) return in.nbucket - 1;
+  if (!(isfinite(x.x) && isfinite(x.y) && isfinite(x.z))) {
+    atomicOr(&ctl.nonfinite, 1);
+    return in.nbucket - 1;
+  }
+  const int c0 = ref_cell(x.x, in.ilb[0], in.lb[0], in.h[0]);
+  const int c1 = ref_cell(x.y, in.ilb[1], in.lb[1], in.h[1]);
+  const int c2 = ref_cell(x.z, in.ilb[2], in.lb[2], in.h[2]);
+  // Cell N+1 with N > 2 is overwritten by the periodic halo copy of
+  // chainlist (nlist.f90:53-64): such atoms drop out of every list.
+  const bool drop = (c0 == in.nc[0] + 1 && in.nc[0] > 2) ||
+                    (c1 == in.nc[1] + 1 && in.nc[1] > 2) ||
+                    (c2 == in.nc[2] + 1 && in.nc[2] > 2) || c0 < 1 || c1 < 1 || c2 < 1 ||
+                    c0 > in.nc[0] + 1 || c1 > in.nc[1] + 1 || c2 > in.nc[2] + 1;
+  if (drop) return in.nbucket - 2;
+  return ((c2 - 1) * in.next[1] + (c1 - 1)) * in.next[0] + (c0 - 1);
+}
+// whether that bucket is a cell of the grid, whose atoms k_nbuild gives a row
+__device__ __forceinline__ bool bucket_is_cell(int local, const DInst &in) {
+  if (local >= in.nbucket - 2) return false;
+  return local % in.next[0] < in.nc[0] && (local / in.next[0]) % in.next[1] < in.nc[1] &&
+         local / (in.next[0] * in.next[1]) < in.nc[2];
+}
+
 __global__ void k_bin(const double4 *__restrict__ X, int NA, const DInst *__restrict__ I,
                       int *__restrict__ bkey, int *__restrict__ brank, int *__restrict__ bcnt,
                       DCtl *__restrict__ ctl, const int *__restrict__ binst,
@@ -425,26 +488,7 @@ __global__ void k_bin(const double4 *__restrict__ X, int NA, const DInst *__rest
     int b = -1;
     if (!(m & META_PAD)) {
       const DInst &in = I[inst_of(m)];
-      int local;
-      if (m & META_DEAD) {
-        local = in.nbucket - 1;
-      } else if (!(isfinite(x.x) && isfinite(x.y) && isfinite(x.z))) {
-        local = in.nbucket - 1;
-        atomicOr(&ctl[inst_of(m)].nonfinite, 1);
-      } else {
-        int c0 = ref_cell(x.x, in.ilb[0], in.lb[0], in.h[0]);
-        int c1 = ref_cell(x.y, in.ilb[1], in.lb[1], in.h[1]);
-        int c2 = ref_cell(x.z, in.ilb[2], in.lb[2], in.h[2]);
-        // Cell N+1 with N > 2 is overwritten by the periodic halo copy of
-        // chainlist (nlist.f90:53-64): such atoms drop out of every list.
-        bool drop = (c0 == in.nc[0] + 1 && in.nc[0] > 2) ||
-                    (c1 == in.nc[1] + 1 && in.nc[1] > 2) ||
-                    (c2 == in.nc[2] + 1 && in.nc[2] > 2) || c0 < 1 || c1 < 1 || c2 < 1 ||
-                    c0 > in.nc[0] + 1 || c1 > in.nc[1] + 1 || c2 > in.nc[2] + 1;
-        if (drop) local = in.nbucket - 2;
-        else local = ((c2 - 1) * in.next[1] + (c1 - 1)) * in.next[0] + (c0 - 1);
-      }
-      b = in.bucket_off + local;
+      b = in.bucket_off + bucket_of(x, in, ctl[inst_of(m)]);
     }
     // runs of equal buckets among the lanes; skipped lanes (-1) join none
     const int prev = __shfl_up(b, 1);
@@ -463,12 +507,6 @@ __global__ void k_bin(const double4 *__restrict__ X, int NA, const DInst *__rest
   }
 }
 
-// Zero fill (used instead of a memset node so the step can be captured).
-__global__ void k_zero_i32(int *__restrict__ p, int n, const int *__restrict__ gate) {
-  GATE_OR_RETURN(gate);
-  GRID_STRIDE(k, n) p[k] = 0;
-}
-
 // Export of the reference cell ids in original atom order.
 __global__ void k_cellid(const double4 *__restrict__ X, int NA, const DInst *__restrict__ I,
                          int inst, int32_t *__restrict__ out) {
@@ -485,7 +523,7 @@ __global__ void k_cellid(const double4 *__restrict__ X, int NA, const DInst *__r
 }
 
 // ---------------------------------------------------------------------------
-// exclusive scan (3 phases), chunk = 256 threads x 8 elements
+// exclusive scan (2 phases), chunk = 256 threads x 8 elements
 #define SCAN_T 256
 #define SCAN_E 8
 #define SCAN_CH (SCAN_T * SCAN_E)
@@ -524,127 +562,230 @@ __global__ void k_scan_reduce(const int *__restrict__ in, int n, int *__restrict
   if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
 }
 
-__global__ void k_scan_top(int *__restrict__ bsum, int nb, const int *__restrict__ gate) {
-  GATE_OR_RETURN(gate);
-  int carry = 0;
-  for (int base = 0; base < nb; base += SCAN_T) {
-    int idx = base + threadIdx.x;
-    int v = idx < nb ? bsum[idx] : 0;
-    int tot;
-    int ex = block_scan_excl(v, tot);
-    if (idx < nb) bsum[idx] = ex + carry;
-    carry += tot;
-    __syncthreads();
-  }
-}
-
-// out[b] = exclusive prefix over all buckets (made instance-local by
-// k_scan_base / k_scan_fix)
+// out[b] = exclusive prefix over all buckets, out[n] = total: every block
+// adds up the totals of the blocks before it.  A bucket's atoms start at
+// out[b] - out[first bucket of its instance] + atom_off, whatever other
+// instances hold, so an instance can be sorted while the others stay in
+// place (bucket_base).
 __global__ void k_scan_down(const int *__restrict__ in, int n, const int *__restrict__ bsum,
-                            const DInst *__restrict__ I, int ninst, int *__restrict__ out,
-                            const int *__restrict__ gate) {
+                            int *__restrict__ out, const int *__restrict__ gate) {
   GATE_OR_RETURN(gate);
-  int base = blockIdx.x * SCAN_CH + threadIdx.x * SCAN_E;
+  int before = 0;
+  for (int k = threadIdx.x; k < (int)blockIdx.x; k += SCAN_T) before += bsum[k];
+  int carry;
+  block_scan_excl(before, carry);
+  const int base = blockIdx.x * SCAN_CH + threadIdx.x * SCAN_E;
   int vals[SCAN_E];
   int s = 0;
   for (int e = 0; e < SCAN_E; ++e) {
-    int idx = base + e;
+    const int idx = base + e;
     vals[e] = idx < n ? in[idx] : 0;
     s += vals[e];
   }
   int tot;
-  int ex = block_scan_excl(s, tot) + bsum[blockIdx.x];
+  int ex = block_scan_excl(s, tot) + carry;
   for (int e = 0; e < SCAN_E; ++e) {
-    int idx = base + e;
-    if (idx < n) out[idx] = ex;
+    const int idx = base + e;
+    if (idx <= n) out[idx] = ex;
     ex += vals[e];
   }
 }
-
-// Instance-local start positions: bucket b of instance k starts at
-// atom_off(k) + (atoms of k in buckets before b), whatever other instances
-// hold, so an instance can be sorted while the others stay in place.
-__global__ void k_scan_base(const int *__restrict__ out, const DInst *__restrict__ I, int ninst,
-                            int *__restrict__ ibase, const int *__restrict__ gate) {
-  GATE_OR_RETURN(gate);
-  for (int k = threadIdx.x; k < ninst; k += blockDim.x)
-    ibase[k] = out[I[k].bucket_off] - I[k].atom_off;
-}
-__global__ void k_scan_fix(int *__restrict__ out, int n, const DInst *__restrict__ I, int ninst,
-                           const int *__restrict__ ibase, const int *__restrict__ gate) {
-  GATE_OR_RETURN(gate);
-  GRID_STRIDE(b, n) out[b] -= ibase[find_inst_by_bucket(I, ninst, b)];
+// Sorted position = cstart[b] + bucket_base for the buckets b of `in`.
+__device__ __forceinline__ int bucket_base(const int *__restrict__ cstart, const DInst &in) {
+  return in.atom_off - cstart[in.bucket_off];
 }
 
+// (and the histogram cleared for the next build: its counts are the
+// differences of cstart from here on)
 __global__ void k_scatter(const int *__restrict__ bkey, const int *__restrict__ brank, int NA,
-                          const int *__restrict__ cstart, int *__restrict__ perm,
+                          const DInst *__restrict__ I, const int *__restrict__ cstart,
+                          int *__restrict__ perm, int *__restrict__ bcnt, int nb,
                           const int *__restrict__ binst, const int *__restrict__ gate) {
   GATE_OR_RETURN(gate);
+  GRID_STRIDE(b, nb) bcnt[b] = 0;
   GRID_STRIDE(p, NA) {
     if (block_gated_out(gate, binst, p)) continue;
+    const DInst &in = I[__builtin_amdgcn_readfirstlane(binst[p / FIB_BLOCK])];
     const int b = bkey[p];
-    if (b >= 0) perm[cstart[b] + brank[p]] = p;
+    if (b >= 0) perm[cstart[b] + bucket_base(cstart, in) + brank[p]] = p;
   }
 }
 
 // Deterministic order inside a bucket: ascending previous position.
-__global__ void k_fixup(const int *__restrict__ cstart, const int *__restrict__ bcnt, int nb,
-                        int *__restrict__ perm, const int *__restrict__ gate) {
+template <typename T>
+__device__ __forceinline__ void sort_ascending(T *a, int n) {
+  for (int i = 1; i < n; ++i) {
+    const T v = a[i];
+    int j = i - 1;
+    while (j >= 0 && a[j] > v) { a[j + 1] = a[j]; --j; }
+    a[j + 1] = v;
+  }
+}
+__global__ void k_fixup(const int *__restrict__ cstart, int nb, const DInst *__restrict__ I,
+                        int ninst, int *__restrict__ perm, const int *__restrict__ gate) {
   GATE_OR_RETURN(gate);
   GRID_STRIDE(b, nb) {
-    const int n = bcnt[b];
+    const int n = cstart[b + 1] - cstart[b];
     if (n < 2) continue;
-    int *a = perm + cstart[b];
-    for (int i = 1; i < n; ++i) {
-      int v = a[i], j = i - 1;
-      while (j >= 0 && a[j] > v) { a[j + 1] = a[j]; --j; }
-      a[j + 1] = v;
+    const DInst &in = I[find_inst_by_bucket(I, ninst, b)];
+    sort_ascending(perm + cstart[b] + bucket_base(cstart, in), n);
+  }
+}
+
+// The whole sort of a small instance (at most SORT_N atoms and buckets) by
+// one workgroup in LDS: binning, histogram, scan, scatter and the order
+// inside the buckets: one launch of 9 us (4 k atoms) for the general sort's
+// five of about 5 us, and one instead of five when the build is gated off.
+#define SORT_T 1024
+#define SORT_N FIB_SORT_N
+__global__ __launch_bounds__(SORT_T) void k_sort_small(
+    const double4 *__restrict__ X, const DInst *__restrict__ I, int *__restrict__ bkey,
+    int *__restrict__ cstart, int *__restrict__ perm, DCtl *__restrict__ ctl,
+    const int *__restrict__ gate) {
+  GATE_OR_RETURN(gate);
+  const int inst = blockIdx.x, t = threadIdx.x;
+  if (gated_out(gate, inst)) return;
+  constexpr int E = SORT_N / SORT_T;
+  __shared__ int cnt[SORT_N + 1];
+  __shared__ uint16_t lp[SORT_N];
+  __shared__ int ws[SORT_T / FIB_WAVE];
+  const DInst &in = I[inst];
+  const int n = in.natm_pad, nb = in.nbucket;
+  for (int b = t; b <= nb; b += SORT_T) cnt[b] = 0;
+  __syncthreads();
+  int key[E], rank[E];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int q = e * SORT_T + t;
+    key[e] = -1;
+    if (q < n) {
+      const double4 x = X[in.atom_off + q];
+      if (!(meta_of(x) & META_PAD)) {
+        key[e] = bucket_of(x, in, ctl[inst]);
+        rank[e] = atomicAdd(&cnt[key[e]], 1);
+      }
+      bkey[in.atom_off + q] = key[e] < 0 ? -1 : in.bucket_off + key[e];
+    }
+  }
+  __syncthreads();
+  // exclusive scan of the counts, E consecutive buckets per thread
+  int v[E], s = 0;
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int b = t * E + e;
+    v[e] = b < nb ? cnt[b] : 0;
+    s += v[e];
+  }
+  const int lane = t % FIB_WAVE, wid = t / FIB_WAVE;
+  int inc = s;
+  for (int o = 1; o < FIB_WAVE; o <<= 1) {
+    const int y = __shfl_up(inc, o);
+    if (lane >= o) inc += y;
+  }
+  if (lane == FIB_WAVE - 1) ws[wid] = inc;
+  __syncthreads();
+  int ex = inc - s;
+  for (int w = 0; w < wid; ++w) ex += ws[w];
+#pragma unroll
+  for (int e = 0; e < E; ++e) {
+    const int b = t * E + e;
+    if (b < nb) {
+      cnt[b] = ex;
+      cstart[in.bucket_off + b] = in.atom_off + ex;
+      ex += v[e];
+      if (b == nb - 1) cnt[nb] = ex;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int e = 0; e < E; ++e)
+    if (key[e] >= 0) lp[cnt[key[e]] + rank[e]] = (uint16_t)(e * SORT_T + t);
+  __syncthreads();
+  for (int b = t; b < nb; b += SORT_T) sort_ascending(lp + cnt[b], cnt[b + 1] - cnt[b]);
+  __syncthreads();
+  const int total = cnt[nb];
+  for (int q = t; q < total; q += SORT_T) perm[in.atom_off + q] = in.atom_off + (int)lp[q];
+}
+
+// Every per-atom array into the new order, and what a build resets: the
+// positions of the build (Xb), displacements, near lists, the lists of atoms
+// outside every cell (k_nbuild writes the others), and the instance's record.
+__global__ void k_reorder(int NA, const int *__restrict__ perm, const int *__restrict__ bkey,
+                          const DInst *__restrict__ I, const double4 *__restrict__ X0,
+                          double4 *__restrict__ X1, const double *__restrict__ V0,
+                          double *__restrict__ V1, const double *__restrict__ F0,
+                          double *__restrict__ F1, const double *__restrict__ Xi0,
+                          double *__restrict__ Xi1, int *__restrict__ inv,
+                          double4 *__restrict__ Xb, float *__restrict__ disp,
+                          uint8_t *__restrict__ nst, int *__restrict__ cnt_sw,
+                          int *__restrict__ cnt_ion, uint8_t *__restrict__ off_sw,
+                          DCtl *__restrict__ ctl, const int *__restrict__ binst,
+                          const int *__restrict__ gate) {
+  GATE_OR_RETURN(gate);
+  GRID_STRIDE(p, NA) {
+    if (block_gated_out(gate, binst, p)) continue;
+    const int inst = __builtin_amdgcn_readfirstlane(binst[p / FIB_BLOCK]);
+    const DInst &in = I[inst];
+    if (p == in.atom_off) {
+      DCtl &c = ctl[inst];
+      c.maxdisp = 0.0;
+      c.maxdisp2 = 0.0;
+      c.nmaxdisp = 0.0;
+      c.maxcnt_sw = 0.0;
+      c.maxcnt_ion = 0.0;
+      c.near_off = 0;
+      c.extra_any = 0;
+      c.builds += 1.0;
+    }
+    if (meta_of(X0[p]) & META_PAD) {
+      if (nst) nst[p] = 0;
+      continue;
+    }
+    const int s = perm[p];
+    const double4 x = X0[s];
+    X1[p] = x;
+    for (int c = 0; c < 3; ++c) {
+      const size_t a = (size_t)c * NA;
+      V1[a + p] = V0[a + s];
+      if (F0) F1[a + p] = F0[a + s];
+      Xi1[a + p] = Xi0[a + s];
+    }
+    inv[in.atom_off + orig_of(x)] = p;
+    Xb[p] = x;
+    disp[p] = 0.0f;
+    if (nst) nst[p] = NEAR_FRESH;
+    if (!bucket_is_cell(bkey[s] - in.bucket_off, in)) {
+      cnt_sw[p] = 0;
+      cnt_ion[p] = 0;
+      // no row: offsets past any row (see k_force3)
+      uint4 *o = reinterpret_cast<uint4 *>(off_sw + (size_t)p * OFF_W);
+      o[0] = make_uint4(~0u, ~0u, ~0u, ~0u);
+      o[1] = make_uint4(~0u, ~0u, ~0u, ~0u);
     }
   }
 }
 
-__global__ void k_reorder(int NA, const int *__restrict__ perm, const DInst *__restrict__ I,
-                          const double4 *__restrict__ X0, double4 *__restrict__ X1,
-                          const double *__restrict__ V0, double *__restrict__ V1,
-                          const double *__restrict__ F0, double *__restrict__ F1,
-                          const double *__restrict__ Xi0, double *__restrict__ Xi1,
-                          int *__restrict__ inv, const int *__restrict__ binst,
-                          const int *__restrict__ gate) {
-  GATE_OR_RETURN(gate);
-  GRID_STRIDE(p, NA) {
-  if (block_gated_out(gate, binst, p)) continue;
-  uint32_t mp = meta_of(X0[p]);
-  if (mp & META_PAD) continue;
-  int s = perm[p];
-  double4 x = X0[s];
-  X1[p] = x;
-  for (int c = 0; c < 3; ++c) {
-    size_t a = (size_t)c * NA;
-    V1[a + p] = V0[a + s];
-    if (F0) F1[a + p] = F0[a + s];
-    Xi1[a + p] = Xi0[a + s];
-  }
-  const DInst &in = I[inst_of(mp)];
-  inv[in.atom_off + orig_of(x)] = p;
-  }
-}
-
-// In-place variant of the sort: copy the reordered arrays back, so the
-// arrays stay where a captured step expects them.
-__global__ void k_copyback(int NA, const double4 *__restrict__ X1, double4 *__restrict__ X0,
-                           const double *__restrict__ V1, double *__restrict__ V0,
-                           const double *__restrict__ F1, double *__restrict__ F0,
-                           const double *__restrict__ Xi1, double *__restrict__ Xi0,
-                           const int *__restrict__ binst, const int *__restrict__ gate) {
-  GATE_OR_RETURN(gate);
-  GRID_STRIDE(p, NA) {
-    if (block_gated_out(gate, binst, p)) continue;
-    X0[p] = X1[p];
+// In-place variant of the sort: the reordered arrays copied back, so they
+// stay where a captured step expects them.  k_nbuild reads the reordered
+// positions, so extra workgroups of its launch do this beside the build.
+struct CopyBack {
+  int blocks;  // workgroups of FIB_BLOCK threads (0: none)
+  const double4 *X1;
+  double4 *X0;
+  const double *V1, *Xi1;
+  double *V0, *Xi0;
+  const int *binst;
+  int NA;
+};
+__device__ __forceinline__ void copy_back(const CopyBack &cb, int block,
+                                          const int *__restrict__ gate) {
+  for (int p = block * FIB_BLOCK + threadIdx.x; p < cb.NA; p += cb.blocks * FIB_BLOCK) {
+    if (block_gated_out(gate, cb.binst, p)) continue;
+    cb.X0[p] = cb.X1[p];
     for (int c = 0; c < 3; ++c) {
-      const size_t a = (size_t)c * NA + p;
-      V0[a] = V1[a];
-      if (F0) F0[a] = F1[a];
-      Xi0[a] = Xi1[a];
+      const size_t a = (size_t)c * cb.NA + p;
+      cb.V0[a] = cb.V1[a];
+      cb.Xi0[a] = cb.Xi1[a];
     }
   }
 }
@@ -656,7 +797,6 @@ __global__ void k_copyback(int NA, const double4 *__restrict__ X1, double4 *__re
 #ifndef NB_WAVES
 #define NB_WAVES 4  // independent wavefronts per k_nbuild workgroup
 #endif
-#define OFF_W 32    // bytes per atom of the stencil-offset table (27 used)
 // A row entry of rk_sw holds (stencil cell << 8 | rank) as the build wrote
 // it, or, once a force pass has worked it out, RK_SLOT | the slot of the
 // row's atom in the neighbour's row (values >= the list width, at most 127,
@@ -721,7 +861,7 @@ __device__ __forceinline__ int mbcnt(uint64_t m) {
 __device__ __forceinline__ bool nbuild_cell_fast(
     const double4 *__restrict__ X, const DInst &in, int i0, int ni, int rs, int rc, int my_lo,
     int total, uint64_t lm0, uint64_t lm1, double rv2, double rv2lj, int Wsw, int Wion,
-    int *__restrict__ cnt_sw, int *__restrict__ nbr_sw, int *__restrict__ cnt_ion,
+    int &most_sw, int &most_ion, int *__restrict__ cnt_sw, int *__restrict__ nbr_sw, int *__restrict__ cnt_ion,
     int *__restrict__ nbr_ion, uint16_t *__restrict__ rk_sw, uint8_t *__restrict__ off_sw,
     double4 *s_x, int *s_j) {
 #pragma clang fp contract(off)
@@ -880,6 +1020,8 @@ __device__ __forceinline__ bool nbuild_cell_fast(
         st_nt<NBNT>(cnt_sw + i, nsw);
         st_nt<NBNT>(cnt_ion + i, nion);
       }
+      most_sw = max(most_sw, nsw);
+      most_ion = max(most_ion, nion);
     }
   };
   if (nk <= FIB_WAVE) rows(std::integral_constant<int, 1>{});
@@ -890,8 +1032,8 @@ __device__ __forceinline__ bool nbuild_cell_fast(
 // One cell (cx, cy, cz) of instance `in`, built by one wave.
 __device__ __forceinline__ void nbuild_cell(
     const double4 *__restrict__ X, const DInst &in, int cx, int cy, int cz, int sd0, int sd1,
-    int sd2, const int *__restrict__ cstart, const int *__restrict__ bcnt, double rv2,
-    double rv2lj, int Wsw, int Wion, int *__restrict__ cnt_sw, int *__restrict__ nbr_sw,
+    int sd2, const int *__restrict__ cstart, int base, double rv2, double rv2lj, int Wsw, int Wion,
+    int &most_sw, int &most_ion, int *__restrict__ cnt_sw, int *__restrict__ nbr_sw,
     int *__restrict__ cnt_ion, int *__restrict__ nbr_ion, uint16_t *__restrict__ rk_sw,
     uint8_t *__restrict__ off_sw, double4 *s_x, int *s_j, uint8_t *s_st, int *s_rs, int *s_off,
     uint32_t *s_acc) {
@@ -900,7 +1042,7 @@ __device__ __forceinline__ void nbuild_cell(
   // the previous cell of this wave is done with the shared arrays
   wave_lds_sync();
   const int bi = in.bucket_off + (cz * in.next[1] + cy) * in.next[0] + cx;
-  const int i0 = cstart[bi], ni = bcnt[bi];
+  const int c0 = cstart[bi], ni = cstart[bi + 1] - c0, i0 = c0 + base;
   if (ni == 0) return;
 
   // lane s < 27 owns stencil cell s = (sd0, sd1, sd2) + 1 in base 3
@@ -913,7 +1055,8 @@ __device__ __forceinline__ void nbuild_cell(
     if (ok) {
       const int b = in.bucket_off + (e2 * in.next[1] + e1) * in.next[0] + e0;
       rs = cstart[b];
-      rc = bcnt[b];
+      rc = cstart[b + 1] - rs;
+      rs += base;
     }
   }
   // inclusive scan of rc over lanes 0..31 (the stencil lanes)
@@ -933,8 +1076,8 @@ __device__ __forceinline__ void nbuild_cell(
   };
   if (total <= NB_CHUNK && ni <= 32 &&
       nbuild_cell_fast(X, in, i0, ni, rs, rc, my_lo, total, before_mask(0), before_mask(FIB_WAVE),
-                       rv2, rv2lj, Wsw, Wion, cnt_sw, nbr_sw, cnt_ion, nbr_ion, rk_sw, off_sw,
-                       s_x, s_j))
+                       rv2, rv2lj, Wsw, Wion, most_sw, most_ion, cnt_sw, nbr_sw, cnt_ion, nbr_ion,
+                       rk_sw, off_sw, s_x, s_j))
     return;
   const bool masks = total <= NB_ACC && ni <= 32;
   if (masks)
@@ -1072,6 +1215,8 @@ __device__ __forceinline__ void nbuild_cell(
       st_nt<NBNT>(cnt_sw + i, nsw);
       st_nt<NBNT>(cnt_ion + i, nion);
     }
+    most_sw = max(most_sw, nsw);
+    most_ion = max(most_ion, nion);
   }
 }
 
@@ -1106,31 +1251,42 @@ __device__ __forceinline__ int locate_cell(const DInst *__restrict__ I, int nins
 // at once (gated-out instances cost a launch of empty workgroups, no more).
 // The busy workgroups are remapped so that each XCD builds a contiguous run
 // of cells, whose halos then stay in its L2.  A wave decodes its first cell
-// once and steps through the rest in x-fastest order.
+// once and steps through the rest in x-fastest order.  A list longer than
+// its width is cut; the longest goes to the instance's record, and in MD-step
+// mode (under a gate) the rest of the step halts until the host has grown
+// the lists and rebuilt them.
 template <int NBC>
-__global__ __launch_bounds__(NB_WAVES * FIB_WAVE) void k_nbuild(
+__global__ __launch_bounds__(NB_WAVES * FIB_WAVE) __attribute__((amdgpu_waves_per_eu(4)))
+void k_nbuild(
     const double4 *__restrict__ X, const DInst *__restrict__ I, int ninst, int total_cells,
-    const int *__restrict__ cstart, const int *__restrict__ bcnt, double rv2, double rv2lj,
-    int Wsw, int Wion, int *__restrict__ cnt_sw, int *__restrict__ nbr_sw,
-    int *__restrict__ cnt_ion, int *__restrict__ nbr_ion, uint16_t *__restrict__ rk_sw,
-    uint8_t *__restrict__ off_sw, const int *__restrict__ gate) {
+    const int *__restrict__ cstart, double rv2, double rv2lj, int Wsw, int Wion,
+    int *__restrict__ cnt_sw, int *__restrict__ nbr_sw, int *__restrict__ cnt_ion,
+    int *__restrict__ nbr_ion, uint16_t *__restrict__ rk_sw, uint8_t *__restrict__ off_sw,
+    DCtl *__restrict__ ctl, const int *__restrict__ gate, int *__restrict__ halt,
+    const CopyBack cb) {
   GATE_OR_RETURN(gate);
+  static_assert(NB_WAVES * FIB_WAVE == FIB_BLOCK, "copy_back's blocks");
   __shared__ double4 s_x[NB_WAVES][NB_CHUNK];
   __shared__ int s_j[NB_WAVES][NB_CHUNK];
   __shared__ uint8_t s_st[NB_WAVES][NB_CHUNK];
   __shared__ int s_rs[NB_WAVES][27], s_off[NB_WAVES][28];
   __shared__ uint32_t s_acc[NB_WAVES][NB_ACC];
+  if ((int)blockIdx.x < cb.blocks) {
+    copy_back(cb, blockIdx.x, gate);
+    return;
+  }
+  const int block = blockIdx.x - cb.blocks;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / FIB_WAVE);  // wave-uniform
   const int *cplan = gate ? gate + 1 + ninst : nullptr;
   const int ncell = gate ? cplan[ninst] : total_cells;
   constexpr int CPB = NB_WAVES * NBC;  // cells per workgroup
   const int nbusy = (ncell + CPB - 1) / CPB;
-  if ((int)blockIdx.x >= nbusy) return;
-  const int c0 = xcd_remap(blockIdx.x, nbusy) * CPB + w * NBC;
+  if (block >= nbusy) return;
+  const int c0 = xcd_remap(block, nbusy) * CPB + w * NBC;
   const int c1 = min(ncell, c0 + NBC);
   const int lane = threadIdx.x % FIB_WAVE;
   const int sd0 = lane % 3 - 1, sd1 = (lane / 3) % 3 - 1, sd2 = lane / 9 - 1;
-  int cend = c0, k = 0, cx = 0, cy = 0, cz = 0;
+  int cend = c0, k = 0, cx = 0, cy = 0, cz = 0, base = 0;
   for (int c = c0; c < c1; ++c) {
     if (c >= cend) {
       // first cell, or the first of the next instance
@@ -1142,49 +1298,29 @@ __global__ __launch_bounds__(NB_WAVES * FIB_WAVE) void k_nbuild(
       cy = (loc / in.nc[0]) % in.nc[1];
       cz = loc / (in.nc[0] * in.nc[1]);
       cend = first + in.nc[0] * in.nc[1] * in.nc[2];
+      base = bucket_base(cstart, in);
     }
     const DInst &in = I[k];
-    nbuild_cell(X, in, cx, cy, cz, sd0, sd1, sd2, cstart, bcnt, rv2, rv2lj, Wsw, Wion, cnt_sw,
-                nbr_sw, cnt_ion, nbr_ion, rk_sw, off_sw, s_x[w], s_j[w], s_st[w], s_rs[w],
-                s_off[w], s_acc[w]);
+    int most_sw = 0, most_ion = 0;
+    nbuild_cell(X, in, cx, cy, cz, sd0, sd1, sd2, cstart, base, rv2, rv2lj, Wsw, Wion, most_sw,
+                most_ion, cnt_sw, nbr_sw, cnt_ion, nbr_ion, rk_sw, off_sw, s_x[w], s_j[w],
+                s_st[w], s_rs[w], s_off[w], s_acc[w]);
+    if ((most_sw > Wsw || most_ion > Wion) && lane == 0) {
+      // (positive doubles order as their bits)
+      atomicMax(reinterpret_cast<unsigned long long *>(&ctl[k].maxcnt_sw),
+                (unsigned long long)__double_as_longlong((double)most_sw));
+      atomicMax(reinterpret_cast<unsigned long long *>(&ctl[k].maxcnt_ion),
+                (unsigned long long)__double_as_longlong((double)most_ion));
+      if (gate) {
+        ctl[k].overflow = 1;
+        if (halt) *halt = 1;
+      }
+    }
     if (++cx == in.nc[0]) {
       cx = 0;
       if (++cy == in.nc[1]) { cy = 0; ++cz; }
     }
   }
-}
-
-// Atoms outside every scanned cell (dropped, dead, or phantom i-atoms) get
-// empty lists; k_nbuild only writes the atoms of real cells.
-__global__ void k_clear_counts(int NA, int *__restrict__ cnt_sw, int *__restrict__ cnt_ion,
-                               uint8_t *__restrict__ off_sw, const int *__restrict__ binst,
-                               const int *__restrict__ gate) {
-  GATE_OR_RETURN(gate);
-  GRID_STRIDE(p, NA) {
-    if (block_gated_out(gate, binst, p)) continue;
-    cnt_sw[p] = 0;
-    cnt_ion[p] = 0;
-    // no row until k_nbuild writes one: offsets past any row (see k_force3)
-    uint4 *o = reinterpret_cast<uint4 *>(off_sw + (size_t)p * OFF_W);
-    o[0] = make_uint4(~0u, ~0u, ~0u, ~0u);
-    o[1] = make_uint4(~0u, ~0u, ~0u, ~0u);
-  }
-}
-
-// Longest SW / ion lists of the build (overflow check).
-// Under a gate only the rebuilt instances' blocks take part (their finalize
-// skips the others, whose maxima stay those of their own last build).
-__global__ __launch_bounds__(FIB_BLOCK) void k_maxcnt(const int *__restrict__ cnt_sw,
-                                                      const int *__restrict__ cnt_ion,
-                                                      int pstride, double *__restrict__ partials,
-                                                      const int *__restrict__ binst,
-                                                      const int *__restrict__ gate) {
-  GATE_OR_RETURN(gate);
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (block_gated_out(gate, binst, i)) return;
-  double v[2] = {(double)cnt_sw[i], (double)cnt_ion[i]};
-  const int op[2] = {1, 1};
-  block_partials<2, FIB_BLOCK>(v, op, blockIdx.x, pstride, partials);
 }
 
 // Slot of the n-th set bit of m (n is small).
@@ -1448,11 +1584,6 @@ struct FAcc<true> {
 // mixed, per step: 181 us over whole rows before, 122 us over the near lists
 // and 207 us in the pass that makes them; 194 -> 144 us over 40 steps with 16
 // replica rebuilds (FP64, 2 x 512 k: 138 -> 111 us).
-#define NEAR_CAP 16
-#define NEAR_J 0x7ffffffu
-#define NEAR_MOVED 253  // moved more than delta / 2 and told its partners
-#define NEAR_FULL 254   // no near list
-#define NEAR_FRESH 255  // just built: the next pass makes the near list
 __device__ __forceinline__ void near_mark_moved(int i, int Wsw, const int *__restrict__ cnt_sw,
                                                 const int *__restrict__ nbr_sw,
                                                 uint8_t *__restrict__ nst) {
@@ -2247,39 +2378,6 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
   }
 }
 
-// After a list build: positions of the build, displacement bookkeeping reset.
-__global__ void k_mark_build(int NA, int ninst, int Wsw, int Wion, const double4 *__restrict__ X,
-                             double4 *__restrict__ Xb, float *__restrict__ disp,
-                             uint8_t *__restrict__ nst, DCtl *__restrict__ ctl,
-                             const int *__restrict__ binst,
-                             const int *__restrict__ gate, int *__restrict__ halt, double inc) {
-  GATE_OR_RETURN(gate);
-  GRID_STRIDE(i, max(NA, ninst)) {
-  // NA is a multiple of FIB_BLOCK: the lanes of a block are all below it or all above
-  if (i < NA && !block_gated_out(gate, binst, i)) {
-    Xb[i] = X[i];
-    disp[i] = 0.0f;
-    nst[i] = NEAR_FRESH;
-  }
-  if (i < ninst && !gated_out(gate, i)) {
-    ctl[i].near_off = 0;
-    ctl[i].maxdisp = 0.0;
-    ctl[i].maxdisp2 = 0.0;
-    ctl[i].nmaxdisp = 0.0;
-    ctl[i].extra_any = 0;
-    // a list longer than its width was cut: sticky, checked by the host;
-    // in MD-step mode the rest of the step halts until the host has grown
-    // the lists and rebuilt them (inc = 0 then: the same build once more)
-    if (ctl[i].maxcnt_sw > Wsw || ctl[i].maxcnt_ion > Wion) {
-      ctl[i].overflow = 1;
-      if (halt) *halt = 1;
-    }
-    ctl[i].builds += inc;
-  }
-  }
-}
-
-
 // ---------------------------------------------------------------------------
 // MD-step mode: velocity Verlet with a per-instance adaptive timestep
 // dt = min(dt_max, dx_max / |v|max), all step control on the device, so one
@@ -2515,7 +2613,8 @@ __global__ __launch_bounds__(DECIDE_T) void k_md_decide(
     int ninst, const DInst *__restrict__ I, DCtl *__restrict__ ctl, double skin,
     int *__restrict__ gate, int *__restrict__ leave, double4 *__restrict__ X, const FConst fc,
     int Wsw, int Wion, const int *__restrict__ cnt_sw, const int *__restrict__ nbr_sw,
-    const int *__restrict__ cnt_ion, const int *__restrict__ nbr_ion,
+    const int *__restrict__ cnt_ion, const int *__restrict__ nbr_ion, int how, const RedSpec rs,
+    const double *__restrict__ partials, int pstride, const double *__restrict__ tmp, int nch,
     const int *__restrict__ halt) {
   // halted: no build in this step either (the host restores the flag)
   if (halt && *halt) {
@@ -2526,7 +2625,14 @@ __global__ __launch_bounds__(DECIDE_T) void k_md_decide(
   __shared__ int s_any;
   __shared__ int s_list[FIB_LEAVE_CAP];
   __shared__ double s_e[FIB_LEAVE_CAP];
-  const int t = threadIdx.x, lane = t % FIB_WAVE, wv = t / FIB_WAVE;
+  const int t = threadIdx.x, lane = t % FIB_WAVE;
+  const int wv = __builtin_amdgcn_readfirstlane(t / FIB_WAVE);
+  // the rest of k_md_pos' reductions, an instance per wavefront
+  if (how != FIN_DONE) {
+    for (int k = wv; k < ninst; k += DECIDE_T / FIB_WAVE)
+      fin_finish<6>(how, k, I[k], partials, pstride, tmp, nch, rs, ctl[k]);
+    __syncthreads();
+  }
   // atoms removed in this step: their interaction energy with the atoms that
   // stay goes to the energy carried out, summed in atom order (the list is
   // filled in arbitrary order and sorted here), so the ledger is the same
@@ -2617,12 +2723,18 @@ __global__ void k_fire_energy(int q, const int *__restrict__ inv, const double4 
 
 // After the step's second half kick: advance time, choose the next dt and
 // the next Berendsen factor of the shells.
-__global__ void k_md_ctl(int ninst, DCtl *__restrict__ ctl, StepArgs sa,
-                         const int *__restrict__ halt) {
+// One wavefront per instance, which first finishes k_force3's reductions.
+__global__ __launch_bounds__(FIB_WAVE) void k_md_ctl(const DInst *__restrict__ I,
+                                                     DCtl *__restrict__ ctl, StepArgs sa, int how,
+                                                     const RedSpec rs,
+                                                     const double *__restrict__ partials,
+                                                     int pstride, const double *__restrict__ tmp,
+                                                     int nch, const int *__restrict__ halt) {
   HALT_OR_RETURN(halt);
-  const int k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= ninst) return;
+  const int k = blockIdx.x;
   DCtl &c = ctl[k];
+  fin_finish<4>(how, k, I[k], partials, pstride, tmp, nch, rs, c);
+  if (threadIdx.x != 0) return;
   c.cfg_time += c.cfg_dt;
   c.cfg_steps += 1.0;
   c.cfg_dt_min = fmin(c.cfg_dt_min, c.cfg_dt);
@@ -3125,18 +3237,10 @@ struct KScope {
   }
 };
 
-template <int NV>
-static void fin_launch(const DevBufs &d, const RedSpec &rs, int nch, const int *gate,
-                       hipStream_t s) {
-  hipLaunchKernelGGL(k_finalize<NV>, dim3(d.ninst, nch), dim3(FIN_T), 0, s, d.I, d.partials,
-                     d.pstride, rs, d.ctl, gate, d.fin_tmp, d.halt);
-  if (nch > 1)
-    hipLaunchKernelGGL(k_finalize2<NV>, dim3(d.ninst), dim3(FIB_WAVE), 0, s, d.I, nch, rs, d.ctl,
-                       gate, d.fin_tmp, d.halt);
-}
+// chunks of the largest instance
+static int fin_nch(const DevBufs &d, int bs) { return (d.max_pad / bs + FIN_CH - 1) / FIN_CH; }
 
-static void finalize(const DevBufs &d, int nv, int bs, const int *op, const int *dst,
-                     hipStream_t s, int nreg = 1, const int *gate = nullptr) {
+static RedSpec red_spec(int nv, int bs, const int *op, const int *dst, int nreg = 1) {
   RedSpec rs;
   rs.nv = nv;
   rs.bs = bs;
@@ -3145,18 +3249,33 @@ static void finalize(const DevBufs &d, int nv, int bs, const int *op, const int 
     rs.op[k] = k < nv ? op[k] : 0;
     rs.dst[k] = k < nv ? dst[k] : -1;
   }
-  // chunks per instance: one workgroup up to FIN_T blocks of the producer
-  const int nch = (d.max_pad / bs + FIN_T - 1) / FIN_T;
+  return rs;
+}
+
+template <int NV>
+static void fin_launch(const DevBufs &d, const RedSpec &rs, hipStream_t s) {
+  hipLaunchKernelGGL(k_finalize<NV>, dim3(d.ninst, fin_nch(d, rs.bs)), dim3(FIB_WAVE), 0, s, d.I,
+                     d.partials, d.pstride, rs, d.ctl, d.fin_tmp, d.halt);
+}
+
+static void finalize(const DevBufs &d, int nv, int bs, const int *op, const int *dst,
+                     hipStream_t s, int nreg = 1) {
+  const RedSpec rs = red_spec(nv, bs, op, dst, nreg);
+  const int nch = fin_nch(d, bs);
   KScope ks_(d, KT_REDUCE);
+#define FIN_CASE(N)                                                                          \
+  case N:                                                                                    \
+    fin_launch<N>(d, rs, s);                                                                 \
+    if (nch > 1)                                                                             \
+      hipLaunchKernelGGL(k_finalize2<N>, dim3(d.ninst), dim3(FIB_WAVE), 0, s, d.I, nch, rs,  \
+                         d.ctl, d.fin_tmp, d.halt);                                          \
+    break;
   switch (nv) {
-    case 1: fin_launch<1>(d, rs, nch, gate, s); break;
-    case 2: fin_launch<2>(d, rs, nch, gate, s); break;
-    case 3: fin_launch<3>(d, rs, nch, gate, s); break;
-    case 4: fin_launch<4>(d, rs, nch, gate, s); break;
-    case 5: fin_launch<5>(d, rs, nch, gate, s); break;
-    case 6: fin_launch<6>(d, rs, nch, gate, s); break;
-    default: fin_launch<10>(d, rs, nch, gate, s); break;
+    FIN_CASE(4)
+    FIN_CASE(5)
+    FIN_CASE(10)
   }
+#undef FIN_CASE
 }
 
 static void finalize_thermo(const DevBufs &d, hipStream_t s) {
@@ -3166,108 +3285,69 @@ static void finalize_thermo(const DevBufs &d, hipStream_t s) {
   finalize(d, 5, FIB_BLOCK, op, dst, s);
 }
 
-void launch_bin(const DevBufs &d, hipStream_t s) {
-  {
-    KScope ks_(d, KT_BIN);
-    hipLaunchKernelGGL(k_zero_i32, dim3(gcap(d.nbucket)), dim3(FIB_BLOCK), 0, s, d.bcnt,
-                       d.nbucket, d.gate);
-  }
-  {
-    KScope ks_(d, KT_BIN);
-    hipLaunchKernelGGL(k_bin, dim3(gcap(d.NA)), dim3(FIB_BLOCK), 0, s, d.X[d.cur], d.NA,
-                       d.I, d.bkey, d.brank, d.bcnt, d.ctl, d.binst, d.gate);
-  }
+// Sort of every instance small enough for one workgroup (k_sort_small).
+static bool small_sort(const DevBufs &d) {
+  return d.max_pad <= SORT_N && d.max_bucket <= SORT_N;
 }
 
-void launch_scan(const DevBufs &d, hipStream_t s) {
-  const int nb = nblk(d.nbucket, SCAN_CH);
-  {
+void launch_build(const DevBufs &d, const FConst &fc, hipStream_t s, bool inplace) {
+  const int c = d.cur, n = 1 - d.cur;
+  if (small_sort(d)) {
     KScope ks_(d, KT_SORT);
+    hipLaunchKernelGGL(k_sort_small, dim3(d.ninst), dim3(SORT_T), 0, s, d.X[c], d.I, d.bkey,
+                       d.cstart, d.perm, d.ctl, d.gate);
+  } else {
+    {
+      KScope ks_(d, KT_BIN);
+      hipLaunchKernelGGL(k_bin, dim3(gcap(d.NA)), dim3(FIB_BLOCK), 0, s, d.X[c], d.NA, d.I,
+                         d.bkey, d.brank, d.bcnt, d.ctl, d.binst, d.gate);
+    }
+    KScope ks_(d, KT_SORT);
+    // (the scan writes one entry past the buckets)
+    const int nb = nblk(d.nbucket + 1, SCAN_CH);
     hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(SCAN_T), 0, s, d.bcnt, d.nbucket, d.bsum,
                        d.gate);
+    hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(SCAN_T), 0, s, d.bcnt, d.nbucket, d.bsum,
+                       d.cstart, d.gate);
+    hipLaunchKernelGGL(k_scatter, dim3(gcap(d.NA)), dim3(FIB_BLOCK), 0, s, d.bkey, d.brank, d.NA,
+                       d.I, d.cstart, d.perm, d.bcnt, d.nbucket, d.binst, d.gate);
+    hipLaunchKernelGGL(k_fixup, dim3(gcap(d.nbucket)), dim3(FIB_BLOCK), 0, s, d.cstart, d.nbucket,
+                       d.I, d.ninst, d.perm, d.gate);
   }
-  {
-    KScope ks_(d, KT_SORT);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(SCAN_T), 0, s, d.bsum, nb, d.gate);
-  }
-  {
-    KScope ks_(d, KT_SORT);
-    hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(SCAN_T), 0, s, d.bcnt, d.nbucket, d.bsum, d.I,
-                       d.ninst, d.cstart, d.gate);
-  }
-  {
-    KScope ks_(d, KT_SORT);
-    hipLaunchKernelGGL(k_scan_base, dim3(1), dim3(SCAN_T), 0, s, d.cstart, d.I, d.ninst, d.ibase,
-                       d.gate);
-  }
-  {
-    KScope ks_(d, KT_SORT);
-    hipLaunchKernelGGL(k_scan_fix, dim3(gcap(d.nbucket)), dim3(FIB_BLOCK), 0, s,
-                       d.cstart, d.nbucket, d.I, d.ninst, d.ibase, d.gate);
-  }
-}
-
-void launch_sort(const DevBufs &d, hipStream_t s, bool inplace) {
-  {
-    KScope ks_(d, KT_SORT);
-    hipLaunchKernelGGL(k_scatter, dim3(gcap(d.NA)), dim3(FIB_BLOCK), 0, s, d.bkey,
-                       d.brank, d.NA, d.cstart, d.perm, d.binst, d.gate);
-  }
-  {
-    KScope ks_(d, KT_SORT);
-    hipLaunchKernelGGL(k_fixup, dim3(gcap(d.nbucket)), dim3(FIB_BLOCK), 0, s, d.cstart,
-                       d.bcnt, d.nbucket, d.perm, d.gate);
-  }
-  const int c = d.cur, n = 1 - d.cur;
   // the in-place sort of MD-step mode leaves the forces behind: every caller
   // (an MD step's build, the fire-time build) computes them anew before
   // anything reads them
   double *const F0 = inplace ? nullptr : d.F[c];
   {
     KScope ks_(d, KT_SORT);
-    hipLaunchKernelGGL(k_reorder, dim3(gcap(d.NA)), dim3(FIB_BLOCK), 0, s, d.NA, d.perm,
-                       d.I, d.X[c], d.X[n], d.V[c], d.V[n], F0, d.F[n], d.Xi[c], d.Xi[n],
-                       d.inv, d.binst, d.gate);
+    hipLaunchKernelGGL(k_reorder, dim3(gcap(d.NA)), dim3(FIB_BLOCK), 0, s, d.NA, d.perm, d.bkey,
+                       d.I, d.X[c], d.X[n], d.V[c], d.V[n], F0, d.F[n], d.Xi[c], d.Xi[n], d.inv,
+                       d.Xb, d.disp, d.nst, d.cnt_sw, d.cnt_ion, d.off_sw, d.ctl, d.binst, d.gate);
   }
-  if (inplace) {
-    KScope ks_(d, KT_SORT);
-    hipLaunchKernelGGL(k_copyback, dim3(gcap(d.NA)), dim3(FIB_BLOCK), 0, s, d.NA, d.X[n],
-                       d.X[c], d.V[n], d.V[c], (const double *)nullptr, (double *)nullptr,
-                       d.Xi[n], d.Xi[c], d.binst, d.gate);
-  }
+  launch_nbuild(d, fc, s, n, inplace);
 }
 
-void launch_nbuild(const DevBufs &d, const FConst &fc, hipStream_t s) {
-  {
-    KScope ks_(d, KT_LISTAUX);
-    hipLaunchKernelGGL(k_clear_counts, dim3(gcap(d.NA)), dim3(FIB_BLOCK), 0, s, d.NA,
-                       d.cnt_sw, d.cnt_ion, d.off_sw, d.binst, d.gate);
+void launch_nbuild(const DevBufs &d, const FConst &fc, hipStream_t s, int from, bool back) {
+  CopyBack cb{};
+  if (back) {
+    const int c = d.cur, n = 1 - d.cur;
+    cb = CopyBack{gcap(d.NA), d.X[n], d.X[c], d.V[n], d.Xi[n], d.V[c], d.Xi[c], d.binst, d.NA};
   }
-  if (d.total_cells > 0) {
-    KScope ks_(d, KT_NBUILD);
-    const int nbc = d.nb_cells ? d.nb_cells : nb_cells_auto(d.total_cells);
-#define NB_LAUNCH(C)                                                                          \
-  hipLaunchKernelGGL(k_nbuild<C>, dim3(nblk(d.total_cells, C * NB_WAVES)),                    \
-                     dim3(NB_WAVES * FIB_WAVE), 0, s, d.X[d.cur], d.I, d.ninst, d.total_cells, \
-                     d.cstart, d.bcnt, fc.rv2, fc.rv2lj, d.Wsw, d.Wion, d.cnt_sw, d.nbr_sw,   \
-                     d.cnt_ion, d.nbr_ion, d.rk_sw, d.off_sw, d.gate)
-    switch (nbc) {
-      case 1: NB_LAUNCH(1); break;
-      case 2: NB_LAUNCH(2); break;
-      case 4: NB_LAUNCH(4); break;
-      case 16: NB_LAUNCH(16); break;
-      default: NB_LAUNCH(8); break;
-    }
+  KScope ks_(d, KT_NBUILD);
+  const int nbc = d.nb_cells ? d.nb_cells : nb_cells_auto(d.total_cells);
+#define NB_LAUNCH(C)                                                                           \
+  hipLaunchKernelGGL(k_nbuild<C>, dim3(cb.blocks + nblk(d.total_cells, C * NB_WAVES)),         \
+                     dim3(NB_WAVES * FIB_WAVE), 0, s, d.X[from], d.I, d.ninst, d.total_cells,  \
+                     d.cstart, fc.rv2, fc.rv2lj, d.Wsw, d.Wion, d.cnt_sw, d.nbr_sw, d.cnt_ion, \
+                     d.nbr_ion, d.rk_sw, d.off_sw, d.ctl, d.gate, d.halt, cb)
+  switch (nbc) {
+    case 1: NB_LAUNCH(1); break;
+    case 2: NB_LAUNCH(2); break;
+    case 4: NB_LAUNCH(4); break;
+    case 16: NB_LAUNCH(16); break;
+    default: NB_LAUNCH(8); break;
+  }
 #undef NB_LAUNCH
-  }
-  {
-    KScope ks_(d, KT_LISTAUX);
-    hipLaunchKernelGGL(k_maxcnt, dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), 0, s, d.cnt_sw,
-                       d.cnt_ion, d.pstride, d.partials, d.binst, d.gate);
-  }
-  const int op[2] = {1, 1};
-  const int dst[2] = {DCTL_IDX(maxcnt_sw), DCTL_IDX(maxcnt_ion)};
-  finalize(d, 2, FIB_BLOCK, op, dst, s, 1, d.gate);
 }
 
 void launch_cellid(const DevBufs &d, int inst, int32_t *dout, hipStream_t s) {
@@ -3343,11 +3423,7 @@ static void force_c(const DevBufs &d, const FConst &fc, const StepArgs &sa, doub
                        (const T4 *)d.EXself, d.exmask, d.halt, xcd_shift(d));
   }
   if (MODE == 1) finalize_thermo(d, s);
-  if (MODE == 2) {
-    const int op[4] = {1, 0, 0, 0};
-    const int dst[4] = {DCTL_IDX(vmax), DCTL_IDX(ke_sum), DCTL_IDX(ke_shell), DCTL_IDX(n_shell)};
-    finalize(d, 4, FIB_BLOCK, op, dst, s);
-  }
+  // (MODE 2: launch_md_ctl reduces)
 }
 
 void launch_force_a(const DevBufs &d, const FConst &fc, bool mixed, bool energy, bool virial,
@@ -3401,10 +3477,16 @@ void launch_md_pos(const DevBufs &d, const FConst &fc, const StepArgs &sa, int *
   const int op[6] = {RED_TOP2, RED_TOP2_CNT, RED_TOP2_SND, RED_SUM, RED_SUM, RED_SUM};
   const int dst[6] = {DCTL_IDX(maxdisp), DCTL_IDX(nmaxdisp), DCTL_IDX(maxdisp2),
                       DCTL_IDX(e_bath_step), DCTL_IDX(e_out_step), DCTL_IDX(movers)};
-  finalize(d, 6, FIB_BLOCK, op, dst, s);
+  const RedSpec rs = red_spec(6, FIB_BLOCK, op, dst);
+  const int nch = fin_nch(d, FIB_BLOCK);
+  // a few small instances: k_md_decide's four wavefronts reduce them, two
+  // each; otherwise a wavefront per chunk does, and k_md_decide combines
+  const int how = nch == 1 ? (d.ninst <= 8 ? FIN_ALL : FIN_DONE) : FIN_COMBINE;
+  KScope ks_(d, KT_REDUCE);
+  if (how != FIN_ALL) fin_launch<6>(d, rs, s);
   hipLaunchKernelGGL(k_md_decide, dim3(1), dim3(DECIDE_T), 0, s, d.ninst, d.I, d.ctl, sa.skin,
                      gate, leave, d.X[d.cur], fc, d.Wsw, d.Wion, d.cnt_sw, d.nbr_sw, d.cnt_ion,
-                     d.nbr_ion, d.halt);
+                     d.nbr_ion, how, rs, d.partials, d.pstride, d.fin_tmp, nch, d.halt);
 }
 
 void launch_fire_energy(const DevBufs &d, const FConst &fc, int q, hipStream_t s) {
@@ -3413,8 +3495,15 @@ void launch_fire_energy(const DevBufs &d, const FConst &fc, int q, hipStream_t s
 }
 
 void launch_md_ctl(const DevBufs &d, const StepArgs &sa, hipStream_t s) {
-  hipLaunchKernelGGL(k_md_ctl, dim3(nblk(d.ninst, FIB_BLOCK)), dim3(FIB_BLOCK), 0, s, d.ninst,
-                     d.ctl, sa, d.halt);
+  const int op[4] = {RED_MAX, RED_SUM, RED_SUM, RED_SUM};
+  const int dst[4] = {DCTL_IDX(vmax), DCTL_IDX(ke_sum), DCTL_IDX(ke_shell), DCTL_IDX(n_shell)};
+  const RedSpec rs = red_spec(4, FIB_BLOCK, op, dst);
+  const int nch = fin_nch(d, FIB_BLOCK);
+  KScope ks_(d, KT_REDUCE);
+  if (nch > 1) fin_launch<4>(d, rs, s);
+  hipLaunchKernelGGL(k_md_ctl, dim3(d.ninst), dim3(FIB_WAVE), 0, s, d.I, d.ctl, sa,
+                     nch > 1 ? FIN_COMBINE : FIN_ALL, rs, d.partials, d.pstride, d.fin_tmp, nch,
+                     d.halt);
 }
 
 void launch_md_init(const DevBufs &d, const StepArgs &sa, bool reset, hipStream_t s) {
@@ -3432,13 +3521,6 @@ void launch_md_report(const DevBufs &d, const StepArgs &sa, hipStream_t s) {
   const int dst[4] = {DCTL_IDX(n_removed), DCTL_IDX(n_ga_removed), DCTL_IDX(n_displaced),
                       DCTL_IDX(ion_z)};
   finalize(d, 4, FIB_BLOCK, op, dst, s);
-}
-
-void launch_mark_build(const DevBufs &d, hipStream_t s, bool count) {
-  KScope ks_(d, KT_LISTAUX);
-  hipLaunchKernelGGL(k_mark_build, dim3(gcap(std::max(d.NA, d.ninst))), dim3(FIB_BLOCK), 0,
-                     s, d.NA, d.ninst, d.Wsw, d.Wion, d.X[d.cur], d.Xb, d.disp, d.nst, d.ctl, d.binst,
-                     d.gate, d.halt, count ? 1.0 : 0.0);
 }
 
 // Rows of an ELL list copied into a wider layout (the list grew).
@@ -3478,7 +3560,12 @@ __global__ void k_clear_overflow(int ninst, DCtl *__restrict__ ctl, int *__restr
                                  int lists) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k < ninst) {
-    if (lists) ctl[k].overflow = 0; else ctl[k].leave_overflow = 0;
+    if (lists) {
+      ctl[k].overflow = 0;
+      ctl[k].maxcnt_sw = ctl[k].maxcnt_ion = 0.0;
+    } else {
+      ctl[k].leave_overflow = 0;
+    }
   }
   if (k == 0 && lists && halt) *halt = 0;
 }

@@ -281,7 +281,7 @@ static void derive_constants(fib_handle *h) {
 
 static int32_t free_bufs(fib_handle *h) {
   DevBufs &d = h->d;
-  void *ptrs[] = {d.I, d.ctl, d.ibase, d.binst, d.X[0], d.X[1], d.V[0], d.V[1], d.F[0], d.F[1], d.Xi[0], d.Xi[1],
+  void *ptrs[] = {d.I, d.ctl, d.binst, d.X[0], d.X[1], d.V[0], d.V[1], d.F[0], d.F[1], d.Xi[0], d.Xi[1],
                   d.inv, d.bkey, d.brank, d.bcnt, d.cstart, d.perm, d.bsum, d.cnt_sw, d.nbr_sw,
                   d.cnt_ion, d.nbr_ion, d.rk_sw, d.off_sw, d.near, d.nst, d.G, d.RA, d.amask, d.Xb, d.disp, d.EX, d.EXself, d.exmask, d.Fpart, d.upart, d.Fout, d.uout,
                   d.partials, d.fin_tmp, d.tab, d.xfer};
@@ -448,7 +448,6 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
     ALLOC(d.Xi[c], 3 * NA);
   }
   ALLOC(d.inv, NA);
-  ALLOC(d.ibase, (size_t)ninst);
   ALLOC(d.binst, (size_t)NA / FIB_BLOCK);
   ALLOC(d.bkey, NA);
   ALLOC(d.brank, NA);
@@ -478,8 +477,12 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
   d.pstride = d.NA / FIB_WAVE + 1;
   ALLOC(d.partials, (size_t)d.pstride * FIB_NRED * 3);
   d.max_pad = 0;
-  for (const DInst &in : h->inst) d.max_pad = std::max(d.max_pad, in.natm_pad);
-  ALLOC(d.fin_tmp, (size_t)ninst * (d.max_pad / FIB_WAVE / FIB_FIN_T + 1) * FIB_NRED);
+  d.max_bucket = 0;
+  for (const DInst &in : h->inst) {
+    d.max_pad = std::max(d.max_pad, in.natm_pad);
+    d.max_bucket = std::max(d.max_bucket, in.nbucket);
+  }
+  ALLOC(d.fin_tmp, (size_t)ninst * (d.max_pad / FIB_BLOCK / FIB_FIN_CH + 1) * FIB_NRED);
   ALLOC(d.tab, h->tab.size());
   ALLOC(d.xfer, 3 * NA);
 #undef ALLOC
@@ -498,6 +501,7 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
     e = hipMemcpy(d.binst, binst.data(), sizeof(int) * binst.size(), hipMemcpyHostToDevice);
   }
   if (e == hipSuccess) e = hipMemset(d.ctl, 0, sizeof(DCtl) * ninst);
+  if (e == hipSuccess) e = hipMemset(d.bcnt, 0, sizeof(int) * (size_t)d.nbucket);
   if (e == hipSuccess) e = hipMemset(d.cnt_sw, 0, sizeof(int) * NA);
   if (e == hipSuccess) e = hipMemset(d.cnt_ion, 0, sizeof(int) * NA);
   if (e == hipSuccess) e = hipMemset(d.nst, 254, NA);
@@ -675,13 +679,14 @@ extern "C" int32_t fib_bin_cells(fib_handle *h, int32_t inst, int32_t *icell) {
 // overflowed (the reference only prints, si.f90:264-272).
 static int32_t build_lists(fib_handle *h) {
   DevBufs &d = h->d;
-  fibk::launch_bin(d, h->stream);
-  fibk::launch_scan(d, h->stream);
-  fibk::launch_sort(d, h->stream);
+  fibk::launch_build(d, h->fc, h->stream, false);
   d.cur = 1 - d.cur;
   for (int attempt = 0; attempt < 4; ++attempt) {
-    // k_nbuild reports max list lengths into DCtl::maxcnt_*
-    fibk::launch_nbuild(d, h->fc, h->stream);
+    // k_nbuild reports lists longer than their width into DCtl::maxcnt_*
+    if (attempt > 0) {
+      fibk::launch_clear_overflow(d, h->stream);
+      fibk::launch_nbuild(d, h->fc, h->stream, d.cur);
+    }
     std::vector<DCtl> c(d.ninst);
     HIPCHK(h, hipMemcpyAsync(c.data(), d.ctl, sizeof(DCtl) * d.ninst, hipMemcpyDeviceToHost,
                              h->stream));
@@ -700,7 +705,6 @@ static int32_t build_lists(fib_handle *h) {
     }
     if (nonfin) return fail(h, FIB_ERR_NONFINITE, "non-finite position detected while binning");
     if (msw <= d.Wsw && mion <= d.Wion) {
-      fibk::launch_mark_build(d, h->stream);
       h->graph_valid = false;  // the sort moved the arrays a graph refers to
       h->have_lists = true;
       h->have_force = false;
@@ -1068,11 +1072,7 @@ static void enqueue_md_step(fib_handle *h) {
   // list rebuild, skipped on the device unless the gate is set; the sort is
   // in place so every array stays where the step (or its graph) expects it
   d.gate = h->md_gate;
-  fibk::launch_bin(d, h->stream);
-  fibk::launch_scan(d, h->stream);
-  fibk::launch_sort(d, h->stream, true);
-  fibk::launch_nbuild(d, h->fc, h->stream);
-  fibk::launch_mark_build(d, h->stream);
+  fibk::launch_build(d, h->fc, h->stream, true);
   d.gate = nullptr;
   const bool mixed = h->prec == FIB_PREC_MIXED;
   // no stale-list pass: a step either rebuilt an instance's lists or left
@@ -1142,8 +1142,7 @@ static int32_t md_recover(fib_handle *h, bool finish_step) {
     const int one = 1;
     HIPCHK(h, hipMemcpyAsync(h->md_gate, &one, sizeof(int), hipMemcpyHostToDevice, h->stream));
     d.gate = h->md_gate;
-    fibk::launch_nbuild(d, h->fc, h->stream);
-    fibk::launch_mark_build(d, h->stream, false);
+    fibk::launch_nbuild(d, h->fc, h->stream, d.cur);
     d.gate = nullptr;
     HIPCHK(h, hipStreamSynchronize(h->stream));
     bool halted = false;
@@ -1249,11 +1248,7 @@ extern "C" int32_t fib_md_fire_many(fib_handle *h, int32_t count, const int32_t 
   HIPCHK(h, hipMemcpyAsync(h->md_gate, g.data(), sizeof(int) * g.size(), hipMemcpyHostToDevice,
                            h->stream));
   d.gate = h->md_gate;
-  fibk::launch_bin(d, h->stream);
-  fibk::launch_scan(d, h->stream);
-  fibk::launch_sort(d, h->stream, true);
-  fibk::launch_nbuild(d, h->fc, h->stream);
-  fibk::launch_mark_build(d, h->stream);
+  fibk::launch_build(d, h->fc, h->stream, true);
   d.gate = nullptr;
   HIPCHK(h, hipStreamSynchronize(h->stream));
   bool halted = false;
@@ -1654,12 +1649,20 @@ int32_t fib_arena_force(const fib_params *p, int32_t precision, int32_t natm, in
   d.Wion = 64;
   d.pstride = d.NA / FIB_WAVE + 1;
   d.max_pad = in.natm_pad;
+  d.max_bucket = in.nbucket;
   const size_t NA = (size_t)d.NA;
   const bool mixed = precision == FIB_PREC_MIXED;
   const size_t g4 = mixed ? sizeof(float4) : sizeof(double4);
   Arena A{static_cast<char *>(arena), arena_bytes};
-  d.I = A.take<DInst>(1);
+  // the arrays that start from zero, in a row: one fill
+  char *zero = A.take<char>(1);
+  const size_t zero_off = (size_t)(zero - A.base);
   d.ctl = A.take<DCtl>(1);
+  d.binst = A.take<int>(NA / FIB_BLOCK);
+  d.bcnt = A.take<int>((size_t)d.nbucket);
+  A.used = (A.used + 3) & ~(size_t)3;
+  const size_t zero_bytes = A.used - zero_off;
+  d.I = A.take<DInst>(1);
   for (int c = 0; c < 2; ++c) {
     d.X[c] = A.take<double4>(NA);
     d.V[c] = A.take<double>(3 * NA);
@@ -1667,11 +1670,8 @@ int32_t fib_arena_force(const fib_params *p, int32_t precision, int32_t natm, in
     d.Xi[c] = A.take<double>(3 * NA);
   }
   d.inv = A.take<int>(NA);
-  d.ibase = A.take<int>(1);
-  d.binst = A.take<int>(NA / FIB_BLOCK);
   d.bkey = A.take<int>(NA);
   d.brank = A.take<int>(NA);
-  d.bcnt = A.take<int>((size_t)d.nbucket);
   d.cstart = A.take<int>((size_t)d.nbucket + 1);
   d.perm = A.take<int>(NA);
   d.bsum = A.take<int>((size_t)d.nbucket / 2048 + 2);
@@ -1688,7 +1688,7 @@ int32_t fib_arena_force(const fib_params *p, int32_t precision, int32_t natm, in
   d.Fout = A.take<double>(3 * NA);
   d.uout = A.take<double>(NA);
   d.partials = A.take<double>((size_t)d.pstride * FIB_NRED * 3);
-  d.fin_tmp = A.take<double>((d.max_pad / FIB_WAVE / FIB_FIN_T + 1) * FIB_NRED);
+  d.fin_tmp = A.take<double>((d.max_pad / FIB_BLOCK / FIB_FIN_CH + 1) * FIB_NRED);
   d.tab = A.take<TabEntry>(g_tab.tab.size());
   d.nbr_sw = A.take<int>((size_t)d.Wsw * NA);
   d.nbr_ion = A.take<int>((size_t)d.Wion * NA);
@@ -1701,27 +1701,18 @@ int32_t fib_arena_force(const fib_params *p, int32_t precision, int32_t natm, in
                                 std::to_string(arena_bytes >> 20) + " MiB arena (" +
                                 std::to_string(d.nbucket) + " cell buckets)");
   // start state: instance record and zeroed bookkeeping, written by kernels
-  // (no memset or host copy of the arrays)
+  // (no memset or host copy of the arrays; the build and the force passes
+  // write the rest before they read it)
   fibk::launch_put_inst(d, in, s);
-  fibk::launch_fill_zero(d.binst, NA / FIB_BLOCK * sizeof(int), s);
-  fibk::launch_fill_zero(d.ctl, sizeof(DCtl), s);
-  fibk::launch_fill_zero(d.cnt_sw, NA * sizeof(int), s);
-  fibk::launch_fill_zero(d.cnt_ion, NA * sizeof(int), s);
-  fibk::launch_fill_zero(d.amask, NA * sizeof(uint64_t), s);
-  fibk::launch_fill_zero(d.exmask, NA * sizeof(uint64_t), s);
-  fibk::launch_fill_zero(d.off_sw, 32 * NA, s);
-  fibk::launch_fill_zero(d.disp, NA * sizeof(float), s);
+  fibk::launch_fill_zero(zero, zero_bytes, s);
   if (!mixed) {
     hipError_t e = hipMemcpyAsync(d.tab, g_tab.tab.data(), sizeof(TabEntry) * g_tab.tab.size(),
                                   hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return bad(FIB_ERR_HIP, std::string("hipMemcpyAsync: ") + hipGetErrorString(e));
   }
   fibk::launch_import(d, 0, in, X, nullptr, atype, nullptr, nullptr, s);
-  fibk::launch_bin(d, s);
-  fibk::launch_scan(d, s);
-  fibk::launch_sort(d, s);
+  fibk::launch_build(d, g_tab.fc, s, false);
   d.cur = 1 - d.cur;
-  fibk::launch_nbuild(d, g_tab.fc, s);
   // the widths cannot grow here: a longer list is an error
   DCtl c;
   hipError_t e = hipMemcpyAsync(&c, d.ctl, sizeof(DCtl), hipMemcpyDeviceToHost, s);
