@@ -1630,17 +1630,26 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
     const int *__restrict__ nbr_sw, const int *__restrict__ cnt_ion,
     const int *__restrict__ nbr_ion, uint64_t *__restrict__ amask,
     double *__restrict__ Fpart, double *__restrict__ upart, uint32_t *__restrict__ near,
-    uint8_t *__restrict__ nst, const DCtl *__restrict__ ctl, int pstride,
-    double *__restrict__ partials, const int *__restrict__ halt, int xs) {
-  HALT_OR_RETURN(halt);
+    uint8_t *__restrict__ nst, const DCtl *__restrict__ ctl, const int *__restrict__ binst,
+    int pstride, double *__restrict__ partials, const int *__restrict__ halt, int xs) {
   typedef typename Prec<MIXED>::T T;
   constexpr bool NT = (FIB_NT_LD & 1) != 0, NTS = (FIB_NT_ST & 1) != 0;
   const int lb = xcd_remap(blockIdx.x, gridDim.x, xs);
   const int i = lb * FIB_BLOCK + threadIdx.x;
+  // what the pass needs first, asked for at once (a load takes about a
+  // microsecond in a small batch, whose data other XCDs have just written);
+  // near entries past the list's end are not used
+  const int kin = binst[lb];
   const double4 xi = X[i];
+  const uint32_t st = near ? nst[i] : NEAR_FULL;
+  uint32_t en[NEAR_BATCH];
+#pragma unroll
+  for (int v = 0; v < NEAR_BATCH; ++v)
+    en[v] = near ? ld_nt<NT>(near + (size_t)v * NA + i) : 0u;
+  const int nion = cnt_ion[i];
+  HALT_OR_RETURN(halt);
   const uint32_t mi = meta_of(xi);
   // every block lies inside one instance: scalar loads of the instance record
-  const int kin = __builtin_amdgcn_readfirstlane(inst_of(mi));
   const DInst &in = I[kin];
   const bool live = !(mi & (META_PAD | META_DEAD));
   const int ti = type_of(mi);
@@ -1740,15 +1749,12 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
   // A pair below gate2 is in range; one below leg2 is a leg (beyond, E =
   // exp(gamma/(r-a)) is zero in FP64 and below e^-30 in the mixed mode: each
   // of its terms is below 1e-9 eps/sigma).
-  const uint32_t st = near ? nst[i] : NEAR_FULL;
   if (near && !ctl[kin].near_off && __ballot(st > NEAR_CAP) == 0ull) {
     const int n = sw_atom ? (int)st : 0;
     // NEAR_BATCH entries at a time: their positions load together, and the
     // next entries while these arrive
-    uint32_t en[NEAR_BATCH];
 #pragma unroll
-    for (int v = 0; v < NEAR_BATCH; ++v)
-      en[v] = v < n ? ld_nt<NT>(near + (size_t)v * NA + i) : (uint32_t)i;
+    for (int v = 0; v < NEAR_BATCH; ++v) en[v] = v < n ? en[v] : (uint32_t)i;
     for (int q = 0; q < n; q += NEAR_BATCH) {
       double4 xq[NEAR_BATCH];
       uint32_t slot[NEAR_BATCH];
@@ -1843,7 +1849,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
 
   // ---- Moliere pairs (si.f90:426-446): both atoms must be fired ----------
   if (live) {
-    const int ci = min(cnt_ion[i], Wion);
+    const int ci = min(nion, Wion);
     const bool ifired = !(ti == 3 && orig_of(xi) >= in.nsg + in.impact);
     const int *ri = nbr_ion + (size_t)i * Wion;
     for (int k = 0; ifired && k < ci; ++k) {
@@ -1948,18 +1954,24 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
 #define TRI_QROWS 8   // most legs of an atom whose pairs share cos + 1/3 (mixed)
 #define TRI_TAB 384   // legs whose owner and list slot are tabled at once
 #define TRI_TAB_VIR 256
+// Batches of up to TRI_SMALL atoms have 16 atoms per wavefront instead of 64:
+// 4 k atoms are 64 wavefronts of 64 for 1,024 SIMDs, and the passes of one
+// wavefront follow each other (24.4 -> 12.3 us).  A large batch fills the
+// chip either way and pays for 16 with emptier last passes (262 k atoms 39.7
+// -> 48.4 us, 811 k 90 -> 126).
+#define TRI_SMALL 131072
 template <bool MIXED>
 struct TriStage {
   static constexpr int N = MIXED ? TRI_NS_MIXED : TRI_NS_FP64;
 };
-template <bool MIXED, bool EN, bool VIR, int NS, int TB>
+template <bool MIXED, bool EN, bool VIR, int NS, int TB, int APW>
 __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
     const double4 *__restrict__ X, const DInst *__restrict__ I, const FConst fc, int NA,
     int Wsw, const int *__restrict__ nbr_sw, uint16_t *__restrict__ rk_sw,
     const uint8_t *__restrict__ off_sw, const uint64_t *__restrict__ amask,
     typename Prec<MIXED>::T4 *__restrict__ G, uint32_t *__restrict__ RA, int pstride,
-    double *__restrict__ partials, const int *__restrict__ halt, int xs) {
-  HALT_OR_RETURN(halt);
+    double *__restrict__ partials, const int *__restrict__ binst, const int *__restrict__ halt,
+    int xs) {
   typedef typename Prec<MIXED>::T T;
   typedef typename Prec<MIXED>::T4 T4;
   constexpr int NW = FIB_BLOCK / FIB_WAVE, QR = TRI_QROWS, FL = NS / 2;
@@ -1978,7 +1990,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
   const int lb = xcd_remap(blockIdx.x, gridDim.x, xs);
   const int lane = threadIdx.x % FIB_WAVE;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / FIB_WAVE);
-  const int i0 = lb * FIB_BLOCK + wid * FIB_WAVE;
+  const int i0 = (lb * NW + wid) * APW;
   const double escale = MIXED ? fc.eps[0][0] : 1.0;
   const double fscale = MIXED ? fc.eps[0][0] * fc.isig[0][0] : 1.0;
   const double lscale = MIXED ? 1.0 / fc.isig[0][0] : 1.0;
@@ -1988,12 +2000,16 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
   const T lp[4] = {(T)(fc.leps[0][0][0] * lu), (T)(fc.leps[0][0][1] * lu),
                    (T)(fc.leps[0][1][1] * lu), (T)(fc.leps[1][1][1] * lu)};
 
-  // this lane's atom as a centre; every block lies inside one instance
-  const int ic = i0 + lane;
+  // this lane's atom as a centre; every block lies inside one instance (what
+  // is needed first is asked for at once, see k_legs)
+  const int kin = binst[i0 / FIB_BLOCK];
+  const int ic = i0 + (APW < FIB_WAVE ? min(lane, APW - 1) : lane);
   const double4 xc = X[ic];
+  const uint64_t amv = amask[ic];
+  HALT_OR_RETURN(halt);
+  const uint64_t amc = lane < APW ? amv : 0ull;
   const int tci = type_of(meta_of(xc));
-  const uint64_t amc = amask[ic];
-  const DInst &in = I[__builtin_amdgcn_readfirstlane(inst_of(meta_of(xc)))];
+  const DInst &in = I[kin];
   // legs of the wave's atoms: this atom's are [exc, inc)
   const int nl = __popcll(amc);
   int inc = nl;
@@ -2024,11 +2040,11 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
     wave_lds_sync();
   };
 
-  for (int r0 = 0; r0 < FIB_WAVE;) {
+  for (int r0 = 0; r0 < APW;) {
     // atoms [r0, r1) whose legs fit the table (an atom has at most Wsw <= 64
     // legs, so every run takes at least one atom, as does every pass)
     const int rs = __builtin_amdgcn_readlane(exc, r0);
-    const int r1 = r0 + __popcll(__ballot(lane >= r0 && inc - rs <= TAB));
+    const int r1 = r0 + __popcll(__ballot(lane >= r0 && lane < APW && inc - rs <= TAB));
     wave_lds_sync();
     if (lane >= r0 && lane < r1) {
       uint64_t m = amc;
@@ -2207,7 +2223,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
     }
     r0 = r1;
   }
-  write_out(FIB_WAVE);
+  write_out(APW);
   if (EN || VIR) {
     double v[10];
     // every unordered term was summed twice, as (a, b) and (b, a)
@@ -2242,7 +2258,8 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
     const uint64_t *__restrict__ amask,
     const float *__restrict__ disp, DCtl *__restrict__ ctl, typename Prec<MIXED>::T4 *__restrict__ EX,
     typename Prec<MIXED>::T4 *__restrict__ EXself, uint64_t *__restrict__ exmask, int pstride,
-    double *__restrict__ partials, const int *__restrict__ halt) {
+    double *__restrict__ partials, const uint8_t *__restrict__ nst,
+    const int *__restrict__ halt) {
   HALT_OR_RETURN(halt);
   typedef typename Prec<MIXED>::T T;
   typedef typename Prec<MIXED>::T4 T4;
@@ -2278,15 +2295,33 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
   T W[9];
 #pragma unroll
   for (int w = 0; w < 9; ++w) W[w] = 0;
-  if (live && tb < 3) {
+  // An atom with a near list has no partner that moved more than delta / 2
+  // (see near_mark_moved), so no two of its partners moved by the skin.  The
+  // others look at their partners' displacements first: in most wavefronts
+  // no atom has one of more than half the skin.  (Without the two checks the
+  // pass took 37 to 49 us for 5.8 k atoms of a fib_step call, a serial chain
+  // of gathers per pair.)
+  const bool moved = !nst || ctl[kin].near_off || nst[b] > NEAR_CAP;
+  if (live && tb < 3 && moved) {
     const int cs = min(cnt_sw[b], Wsw);
     const int *rowb = nbr_sw + (size_t)b * Wsw;
     const uint64_t amb = amask[b];
-    const int na = __popcll(amb);
+    // of the two, one moved more than half the skin
+    uint64_t far = 0;
+    for (int k0 = 0; k0 < cs; k0 += 4) {
+      float dk[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) dk[v] = k0 + v < cs ? disp[rowb[k0 + v]] : 0.0f;
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (dk[v] > 0.4999f * skin) far |= 1ull << (k0 + v);
+    }
+    const int na = far ? __popcll(amb) : 0;
     for (int n = 0; n < na; ++n) {
       const int kc = nth_bit(amb, n);  // b's list slot of c
       const int c = rowb[kc];
       const float dc = disp[c];
+      const bool cfar = (far >> kc) & 1ull;
       const double4 xc = X[c];
       const int tc = type_of(meta_of(xc));
       Leg<T> Lbc;  // b's leg to c: unit vector from c to b
@@ -2294,6 +2329,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
       const int *rowc = nbr_sw + (size_t)c * Wsw;
       const int cc = min(cnt_sw[c], Wsw);
       for (int k = 0; k < cs; ++k) {
+        if (!cfar && !((far >> k) & 1ull)) continue;
         const int a = rowb[k];
         if (a == c || !(disp[a] + dc > skin)) continue;
         const double4 xa = X[a];
@@ -2409,14 +2445,22 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_md_pos(double4 *__restrict__ X,
                                                       const int *__restrict__ nbr_sw,
                                                       uint8_t *__restrict__ nst,
                                                       int *__restrict__ leave,
+                                                      const int *__restrict__ binst,
                                                       const int *__restrict__ halt, int xs) {
-  HALT_OR_RETURN(halt);
   constexpr bool NT = (FIB_NT_LD & 8) != 0, NTS = (FIB_NT_ST & 8) != 0;
   const int lb = xcd_remap(blockIdx.x, gridDim.x, xs);
   const int i = lb * FIB_BLOCK + threadIdx.x;
+  // every load asked for at once (see k_legs)
+  const int kin = binst[lb];
   double4 x = X[i];
+  const double4 xb = ld_nt<NT>(Xb + i);
+  double v[3], f[3];
+  for (int c = 0; c < 3; ++c) {
+    v[c] = ld_nt<NT>(V + (size_t)c * NA + i);
+    f[c] = ld_nt<NT>(F + (size_t)c * NA + i);
+  }
+  HALT_OR_RETURN(halt);
   uint32_t mi = meta_of(x);
-  const int kin = __builtin_amdgcn_readfirstlane(inst_of(mi));
   const DInst &in = I[kin];
   const bool live = !(mi & (META_PAD | META_DEAD));
   const double dt = ctl[kin].cfg_dt, lam = ctl[kin].cfg_lambda;
@@ -2428,15 +2472,14 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_md_pos(double4 *__restrict__ X,
   if (live) {
     const int t = type_of(mi);
     const double m = sa.mass[t - 1];
-    double v[3], xx[3] = {x.x, x.y, x.z};
-    for (int c = 0; c < 3; ++c) v[c] = ld_nt<NT>(V + (size_t)c * NA + i);
+    double xx[3] = {x.x, x.y, x.z};
     if (sa.shell_w > 0.0 && t < 3 && !(mi & META_FROZEN) &&
         in_shell(xx[0], xx[1], xx[2], in, sa.shell_w)) {
       red[3] = 0.5 * m * (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]) * (1.0 - lam * lam);
       for (int c = 0; c < 3; ++c) v[c] *= lam;
     }
     for (int c = 0; c < 3; ++c) {
-      v[c] += 0.5 * ld_nt<NT>(F + (size_t)c * NA + i) * dt / m;
+      v[c] += 0.5 * f[c] * dt / m;
       xx[c] += v[c] * dt;
     }
     if (mi & META_FROZEN) {
@@ -2462,7 +2505,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_md_pos(double4 *__restrict__ X,
     X[i] = x;
     for (int c = 0; c < 3; ++c) st_nt<NTS>(V + (size_t)c * NA + i, v[c]);
     double e0, e1, e2;
-    min_image_fast(x, ld_nt<NT>(Xb + i), in, e0, e1, e2);
+    min_image_fast(x, xb, in, e0, e1, e2);
     const float dd = (float)sqrt(e0 * e0 + e1 * e1 + e2 * e2);
     st_nt<NTS>(disp + i, dd);
     red[0] = (double)dd;
@@ -2803,15 +2846,12 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_md_report(const double4 *__restri
 // force pass 3: own terms + the G entries neighbours wrote for this atom;
 // MODE 0 = store forces, MODE 1 = reference velocity update
 // (timeint.f90:231-236) + thermostat sums; MODE 2 = MD-step mode.
-// partner lookups in flight per atom in k_force3: FP64 8 (most atoms have at
-// most 8 legs; 6 % faster on the dose batch than 4), mixed 4 (8 was 4 %
-// slower: the registers cost occupancy)
-#ifndef F3_BATCH_FP64
-#define F3_BATCH_FP64 8
-#endif
-#ifndef F3_BATCH_MIXED
-#define F3_BATCH_MIXED 4
-#endif
+// Bound by the gather of the partners' entries (and, in small batches, by
+// the chain of dependent loads): two batches of F3_BATCH legs, their own
+// entries and the partners' places first, then the partners' entries, all of
+// a batch in flight at once.  FP64, 2 x 512 k atoms: 119 us leg by leg, 109
+// so; the mixed mode's 4 x 512 k did not change (131).
+#define F3_BATCH 4
 template <bool MIXED, bool EN, int MODE>
 __global__ __launch_bounds__(FIB_BLOCK) void k_force3(
     const double4 *__restrict__ X, const DInst *__restrict__ I, int NA, int Wsw,
@@ -2824,55 +2864,92 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_force3(
     StepArgs sa, int pstride, double *__restrict__ partials, const DCtl *__restrict__ ctl,
     const typename Prec<MIXED>::T4 *__restrict__ EX,
     const typename Prec<MIXED>::T4 *__restrict__ EXself, const uint64_t *__restrict__ exmask,
-    const int *__restrict__ halt, int xs) {
-  HALT_OR_RETURN(halt);
+    const int *__restrict__ binst, const int *__restrict__ halt, int xs) {
   typedef typename Prec<MIXED>::T4 T4;
   constexpr bool NT = (FIB_NT_LD & 4) != 0, NTS = (FIB_NT_ST & 4) != 0;
   const int lb = xcd_remap(blockIdx.x, gridDim.x, xs);
   const int i = lb * FIB_BLOCK + threadIdx.x;
+  // what the pass needs first, asked for at once (see k_legs); entries of
+  // legs the atom does not have are not used
+  const int kin = binst[lb];
   const double4 xi = X[i];
+  const uint64_t am = ld_nt<NT>(amask + i);
+  const double fp[3] = {ld_nt<NT>(Fpart + i), ld_nt<NT>(Fpart + (size_t)NA + i),
+                        ld_nt<NT>(Fpart + 2 * (size_t)NA + i)};
+  T4 own[F3_BATCH];
+  uint32_t ra[F3_BATCH];
+#pragma unroll
+  for (int u = 0; u < F3_BATCH; ++u) {
+    ra[u] = ld_nt<NT>(RA + (size_t)u * NA + i);
+    own[u] = G[(size_t)u * NA + i];
+  }
+  double vold[3] = {0, 0, 0};
+  if (MODE == 2)
+    for (int c = 0; c < 3; ++c) vold[c] = ld_nt<NT>(V + (size_t)c * NA + i);
+  HALT_OR_RETURN(halt);
   const uint32_t mi = meta_of(xi);
-  const int kin = __builtin_amdgcn_readfirstlane(inst_of(mi));
   const DInst &in = I[kin];
   const bool live = !(mi & (META_PAD | META_DEAD));
   double f0 = 0, f1 = 0, f2 = 0, u = 0;
   if (live) {
-    f0 = ld_nt<NT>(Fpart + i);
-    f1 = ld_nt<NT>(Fpart + (size_t)NA + i);
-    f2 = ld_nt<NT>(Fpart + 2 * (size_t)NA + i);
+    f0 = fp[0];
+    f1 = fp[1];
+    f2 = fp[2];
     if (EN) u = upart[i];
     const size_t row = (size_t)i * Wsw;
     double g0 = 0, g1 = 0, g2 = 0, gu = 0;
+    const int na = __popcll(am);
+    // the partners' entries (at the places k_tri noted for the legs) of the
+    // first legs, and what the next legs need
+    auto partner = [&](uint32_t at, T4 &g) {
+      if (at != ~0u) {
+        g = G[at];
+      } else {
+        g.x = g.y = g.z = g.w = 0;
+      }
+    };
+    T4 theirs[F3_BATCH], own2[F3_BATCH];
+    uint32_t ra2[F3_BATCH];
+#pragma unroll
+    for (int u = 0; u < F3_BATCH; ++u) {
+      partner(u < na ? ra[u] : ~0u, theirs[u]);
+      ra2[u] = ~0u;
+      own2[u].x = own2[u].y = own2[u].z = own2[u].w = 0;
+      if (F3_BATCH + u < na) {
+        ra2[u] = ld_nt<NT>(RA + (size_t)(F3_BATCH + u) * NA + i);
+        own2[u] = G[(size_t)(F3_BATCH + u) * NA + i];
+      }
+    }
     // reaction on the centre: minus the forces its own terms put on its legs
-    const int na = __popcll(ld_nt<NT>(amask + i));
-    for (int n = 0; n < na; ++n) {
-      const T4 g = G[(size_t)n * NA + i];
+    auto minus = [&](const T4 &g) {
       g0 -= (double)g.x; g1 -= (double)g.y; g2 -= (double)g.z;
       if (EN) gu += 0.5 * (double)g.w;
-    }
-    // forces the partners' terms put on this atom, at the places k_tri
-    // noted for its legs: one lookup per leg, F3_BATCH in flight
-    constexpr int F3_BATCH = MIXED ? F3_BATCH_MIXED : F3_BATCH_FP64;
-    for (int n0 = 0; n0 < na; n0 += F3_BATCH) {
-      uint32_t ra[F3_BATCH];
-      T4 g4[F3_BATCH];
+    };
+    // forces the partners' terms put on this atom
+    auto plus = [&](const T4 &g) {
+      g0 += (double)g.x; g1 += (double)g.y; g2 += (double)g.z;
+      if (EN) gu += (double)g.w;
+    };
 #pragma unroll
-      for (int u = 0; u < F3_BATCH; ++u)
-        ra[u] = (n0 + u < na) ? ld_nt<NT>(RA + (size_t)(n0 + u) * NA + i) : ~0u;
+    for (int u = 0; u < F3_BATCH; ++u)
+      if (u < na) minus(own[u]);
 #pragma unroll
-      for (int u = 0; u < F3_BATCH; ++u) {
-        if (ra[u] != ~0u) {
-          g4[u] = G[ra[u]];
-        } else {
-          g4[u].x = g4[u].y = g4[u].z = g4[u].w = 0;
-        }
-      }
+    for (int u = 0; u < F3_BATCH; ++u)
+      if (F3_BATCH + u < na) minus(own2[u]);
+    for (int n = 2 * F3_BATCH; n < na; ++n) minus(G[(size_t)n * NA + i]);
+    T4 theirs2[F3_BATCH];
 #pragma unroll
-      for (int u = 0; u < F3_BATCH; ++u)
-        if (n0 + u < na) {
-          g0 += (double)g4[u].x; g1 += (double)g4[u].y; g2 += (double)g4[u].z;
-          if (EN) gu += (double)g4[u].w;
-        }
+    for (int u = 0; u < F3_BATCH; ++u) partner(ra2[u], theirs2[u]);
+#pragma unroll
+    for (int u = 0; u < F3_BATCH; ++u)
+      if (u < na) plus(theirs[u]);
+#pragma unroll
+    for (int u = 0; u < F3_BATCH; ++u)
+      if (F3_BATCH + u < na) plus(theirs2[u]);
+    for (int n = 2 * F3_BATCH; n < na; ++n) {
+      T4 g;
+      partner(ld_nt<NT>(RA + (size_t)n * NA + i), g);
+      plus(g);
     }
     // vertex terms outside the centre's list (k_extra), when there are any
     if (ctl[kin].extra_any) {
@@ -2917,7 +2994,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_force3(
       double vv[3];
       for (int c = 0; c < 3; ++c) {
         const size_t a = (size_t)c * NA + i;
-        vv[c] = pinned ? 0.0 : ld_nt<NT>(V + a) + 0.5 * fn[c] * dt / m;
+        vv[c] = pinned ? 0.0 : vold[c] + 0.5 * fn[c] * dt / m;
         st_nt<NTS>(V + a, vv[c]);
         st_nt<NTS>(Fout + a, fn[c]);
       }
@@ -3366,7 +3443,7 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
     hipLaunchKernelGGL((k_legs<MIXED, EN, VIR>), dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), 0, s,
                        d.X[d.cur], d.I, fc, d.tab, d.NA, d.Wsw, d.Wion, d.cnt_sw, d.nbr_sw,
                        d.cnt_ion, d.nbr_ion, d.amask, d.Fpart, d.upart, d.near,
-                       d.nst, d.ctl, d.pstride, d.partials, d.halt, xcd_shift(d));
+                       d.nst, d.ctl, d.binst, d.pstride, d.partials, d.halt, xcd_shift(d));
   }
   {
     KScope ks_(d, KT_TRI);
@@ -3374,19 +3451,24 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
     // in the default tile
     const int ns = (EN || VIR || !d.tri_ns) ? TriStage<MIXED>::N : d.tri_ns;
     const int tb = (EN || VIR || !d.tri_tb) ? TRI_BATCH : d.tri_tb;
-#define TRI_LAUNCH(NS_, TB_)                                                                  \
-  hipLaunchKernelGGL((k_tri<MIXED, EN, VIR, NS_, TB_>), dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), \
-                     0, s, d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.nbr_sw, d.rk_sw,              \
-                     d.off_sw, d.amask, (T4 *)d.G, d.RA, d.pstride,                          \
-                     d.partials + (size_t)FIB_NRED * d.pstride, d.halt, xcd_shift(d))
+#define TRI_LAUNCH(NS_, TB_, APW_)                                                            \
+  hipLaunchKernelGGL((k_tri<MIXED, EN, VIR, NS_, TB_, APW_>),                                 \
+                     dim3(d.NA / (FIB_BLOCK / FIB_WAVE * APW_)), dim3(FIB_BLOCK), 0, s,       \
+                     d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.nbr_sw, d.rk_sw, d.off_sw, d.amask,  \
+                     (T4 *)d.G, d.RA, d.pstride, d.partials + (size_t)FIB_NRED * d.pstride,   \
+                     d.binst, d.halt, xcd_shift(d) + (APW_ == 16 ? 2 : 0))
     if constexpr (EN || VIR) {
-      TRI_LAUNCH(TriStage<MIXED>::N, TRI_BATCH);
+      // (one partial per 256 atoms: 64 atoms per wavefront)
+      TRI_LAUNCH(TriStage<MIXED>::N, TRI_BATCH, FIB_WAVE);
+    } else if (d.NA <= TRI_SMALL && !d.tri_ns && !d.tri_tb) {
+      TRI_LAUNCH(128, TRI_BATCH, 16);
     } else {
-      if (ns == TriStage<MIXED>::N && tb == TRI_BATCH) TRI_LAUNCH(TriStage<MIXED>::N, TRI_BATCH);
-      else if (ns == 128 && tb == 2) TRI_LAUNCH(128, 2);
-      else if (ns == 128 && tb == 4) TRI_LAUNCH(128, 4);
-      else if (ns == 256 && tb == 2) TRI_LAUNCH(256, 2);
-      else TRI_LAUNCH(256, 4);
+      if (ns == TriStage<MIXED>::N && tb == TRI_BATCH)
+        TRI_LAUNCH(TriStage<MIXED>::N, TRI_BATCH, FIB_WAVE);
+      else if (ns == 128 && tb == 2) TRI_LAUNCH(128, 2, FIB_WAVE);
+      else if (ns == 128 && tb == 4) TRI_LAUNCH(128, 4, FIB_WAVE);
+      else if (ns == 256 && tb == 2) TRI_LAUNCH(256, 2, FIB_WAVE);
+      else TRI_LAUNCH(256, 4, FIB_WAVE);
     }
 #undef TRI_LAUNCH
   }
@@ -3398,7 +3480,7 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
                        d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.cnt_sw, d.nbr_sw, d.amask,
                        d.disp, d.ctl, (T4 *)d.EX,
                        (T4 *)d.EXself, d.exmask, d.pstride,
-                       d.partials + (size_t)2 * FIB_NRED * d.pstride, d.halt);
+                       d.partials + (size_t)2 * FIB_NRED * d.pstride, d.nst, d.halt);
   }
   if (EN || VIR) {
     int op[10], dst[10];
@@ -3420,7 +3502,7 @@ static void force_c(const DevBufs &d, const FConst &fc, const StepArgs &sa, doub
                        (const T4 *)d.G, d.RA, d.amask, d.cnt_sw, d.Fpart,
                        d.upart, fscale, escale, Fo,
                        d.uout, d.V[d.cur], sa, d.pstride, d.partials, d.ctl, (const T4 *)d.EX,
-                       (const T4 *)d.EXself, d.exmask, d.halt, xcd_shift(d));
+                       (const T4 *)d.EXself, d.exmask, d.binst, d.halt, xcd_shift(d));
   }
   if (MODE == 1) finalize_thermo(d, s);
   // (MODE 2: launch_md_ctl reduces)
@@ -3471,8 +3553,8 @@ void launch_md_pos(const DevBufs &d, const FConst &fc, const StepArgs &sa, int *
     KScope ks_(d, KT_POS);
     hipLaunchKernelGGL(k_md_pos, dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), 0, s, d.X[d.cur], d.I,
                        d.NA, d.V[d.cur], d.F[d.cur], d.Xi[d.cur], sa, d.pstride, d.partials,
-                       d.ctl, d.Xb, d.disp, d.Wsw, d.cnt_sw, d.nbr_sw, d.nst, leave, d.halt,
-                       xcd_shift(d));
+                       d.ctl, d.Xb, d.disp, d.Wsw, d.cnt_sw, d.nbr_sw, d.nst, leave,
+                       d.binst, d.halt, xcd_shift(d));
   }
   const int op[6] = {RED_TOP2, RED_TOP2_CNT, RED_TOP2_SND, RED_SUM, RED_SUM, RED_SUM};
   const int dst[6] = {DCTL_IDX(maxdisp), DCTL_IDX(nmaxdisp), DCTL_IDX(maxdisp2),
