@@ -1669,7 +1669,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
   const double leg2 = MIXED ? fc.mixed_xleg * fc.mixed_xleg : fc.cut_sw * fc.cut_sw;
   const double iumax = MIXED ? 0.0 : 1.0 / fc.umax;
   const size_t row = (size_t)i * Wsw;
-  __shared__ uint32_t hold[FIB_BLOCK / FIB_WAVE][NEAR_CAP][FIB_WAVE];
+  __shared__ __attribute__((aligned(16))) uint32_t hold[FIB_BLOCK / FIB_WAVE][NEAR_CAP][FIB_WAVE];
   const int lane = threadIdx.x % FIB_WAVE;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / FIB_WAVE);
 
@@ -1848,58 +1848,122 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
   st_nt<NTS>(amask + i, am);
 
   // ---- Moliere pairs (si.f90:426-446): both atoms must be fired ----------
-  if (live) {
-    const int ci = min(nion, Wion);
-    const bool ifired = !(ti == 3 && orig_of(xi) >= in.nsg + in.impact);
-    const int *ri = nbr_ion + (size_t)i * Wion;
-    for (int k = 0; ifired && k < ci; ++k) {
-      const int j = ri[k];
-      const double4 xj = X[j];
-      const uint32_t mj = meta_of(xj);
-      const int tj = type_of(mj);
-      if (tj == 3 && orig_of(xj) >= in.nsg + in.impact) continue;
-      if (mj & META_DEAD) continue;
-      double d0, d1, d2;
-      min_image_fast(xi, xj, in, d0, d1, d2);
-      const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
-      if (!(r2 < fc.rlj2)) continue;
-      const double r = sqrt(r2);
-      const double aa = fc.aamol[ti - 1][tj - 1];
-      const double zz = fc.ie0 * fc.zmol[ti - 1] * fc.zmol[tj - 1] * fc.ec * fc.ec;
-      if (!MIXED || r < fc.mixed_r64) {
-        const double x = r / aa;
-        const double e1 = exp(-fc.molb[0] * x), e2 = exp(-fc.molb[1] * x),
-                     e3 = exp(-fc.molb[2] * x);
-        const double sa = fc.molc[0] * e1 + fc.molc[1] * e2 + fc.molc[2] * e3;
-        const double sb = (fc.molc[0] * fc.molb[0] * e1 + fc.molc[1] * fc.molb[1] * e2 +
-                           fc.molc[2] * fc.molb[2] * e3) / aa;
-        const double fcm = zz / r * (sa / r + sb);
-        const double rinv = 1.0 / r;
-        const double h0 = fcm * d0 * rinv, h1 = fcm * d1 * rinv, h2 = fcm * d2 * rinv;
-        f.add((T)1, (T)(h0 / fscale), (T)(h1 / fscale), (T)(h2 / fscale));
-        if (VIR) addW((T)(d0 / lscale), (T)(d1 / lscale), (T)(d2 / lscale),
-                      (T)(0.5 * h0 / fscale), (T)(0.5 * h1 / fscale), (T)(0.5 * h2 / fscale));
-        if (EN) { const double ul = 0.5 * zz / r * sa; ui += ul; etot += ul; }
-      } else {
-        // FP32 with lengths in units of aa; F = (zz/aa^2) (1/x)(sa/x + sb) d/(aa x)
-        const float x = (float)(r / aa);
-        const float e1 = __expf(-(float)fc.molb[0] * x), e2 = __expf(-(float)fc.molb[1] * x),
-                    e3 = __expf(-(float)fc.molb[2] * x);
-        const float c0 = (float)fc.molc[0], c1 = (float)fc.molc[1], c2 = (float)fc.molc[2];
-        const float sa = c0 * e1 + c1 * e2 + c2 * e3;
-        const float sb = c0 * (float)fc.molb[0] * e1 + c1 * (float)fc.molb[1] * e2 +
-                         c2 * (float)fc.molb[2] * e3;
-        const float ix = __builtin_amdgcn_rcpf(x);
-        const float fr = ix * (sa * ix + sb) * ix;
-        const float scl = (float)(zz / (aa * aa) / fscale);
-        const float g0 = fr * (float)(d0 / aa), g1 = fr * (float)(d1 / aa),
-                    g2 = fr * (float)(d2 / aa);
-        const float h0 = g0 * scl, h1 = g1 * scl, h2 = g2 * scl;
-        f.add((T)scl, (T)g0, (T)g1, (T)g2);
-        if (VIR) addW((T)(d0 / lscale), (T)(d1 / lscale), (T)(d2 / lscale), (T)(0.5f * h0),
-                      (T)(0.5f * h1), (T)(0.5f * h2));
-        if (EN) { const double ul = 0.5 * zz / aa * (double)(sa * ix); ui += ul; etot += ul; }
+  // One pair of atom a (species ta) with list entry j, where it is in range:
+  // the force as v[0] (v[1], v[2], v[3]), the difference v[4..6] in the
+  // virial's length unit, and the atom's half of the energy.
+  auto moliere = [&](const double4 &xa, int ta, int j, T (&v)[7], double &ul) -> bool {
+    const double4 xj = X[j];
+    const uint32_t mj = meta_of(xj);
+    const int tj = type_of(mj);
+    if (tj == 3 && orig_of(xj) >= in.nsg + in.impact) return false;
+    if (mj & META_DEAD) return false;
+    double d0, d1, d2;
+    min_image_fast(xa, xj, in, d0, d1, d2);
+    const double r2 = d0 * d0 + d1 * d1 + d2 * d2;
+    if (!(r2 < fc.rlj2)) return false;
+    const double r = sqrt(r2);
+    const double aa = fc.aamol[ta - 1][tj - 1];
+    const double zz = fc.ie0 * fc.zmol[ta - 1] * fc.zmol[tj - 1] * fc.ec * fc.ec;
+    if (!MIXED || r < fc.mixed_r64) {
+      const double x = r / aa;
+      const double e1 = exp(-fc.molb[0] * x), e2 = exp(-fc.molb[1] * x),
+                   e3 = exp(-fc.molb[2] * x);
+      const double sa = fc.molc[0] * e1 + fc.molc[1] * e2 + fc.molc[2] * e3;
+      const double sb = (fc.molc[0] * fc.molb[0] * e1 + fc.molc[1] * fc.molb[1] * e2 +
+                         fc.molc[2] * fc.molb[2] * e3) / aa;
+      const double fcm = zz / r * (sa / r + sb);
+      const double rinv = 1.0 / r;
+      v[0] = T(1);
+      v[1] = (T)(fcm * d0 * rinv / fscale);
+      v[2] = (T)(fcm * d1 * rinv / fscale);
+      v[3] = (T)(fcm * d2 * rinv / fscale);
+      if (EN) ul = 0.5 * zz / r * sa;
+    } else {
+      // FP32 with lengths in units of aa; F = (zz/aa^2) (1/x)(sa/x + sb) d/(aa x)
+      const float x = (float)(r / aa);
+      const float e1 = __expf(-(float)fc.molb[0] * x), e2 = __expf(-(float)fc.molb[1] * x),
+                  e3 = __expf(-(float)fc.molb[2] * x);
+      const float c0 = (float)fc.molc[0], c1 = (float)fc.molc[1], c2 = (float)fc.molc[2];
+      const float sa = c0 * e1 + c1 * e2 + c2 * e3;
+      const float sb = c0 * (float)fc.molb[0] * e1 + c1 * (float)fc.molb[1] * e2 +
+                       c2 * (float)fc.molb[2] * e3;
+      const float ix = __builtin_amdgcn_rcpf(x);
+      const float fr = ix * (sa * ix + sb) * ix;
+      v[0] = (T)(float)(zz / (aa * aa) / fscale);
+      v[1] = (T)(fr * (float)(d0 / aa));
+      v[2] = (T)(fr * (float)(d1 / aa));
+      v[3] = (T)(fr * (float)(d2 / aa));
+      if (EN) ul = 0.5 * zz / aa * (double)(sa * ix);
+    }
+    if (VIR) {
+      v[4] = (T)(d0 / lscale);
+      v[5] = (T)(d1 / lscale);
+      v[6] = (T)(d2 / lscale);
+    }
+    return true;
+  };
+  // The wavefront's pairs stand in a row, atom by atom, and its lanes take one
+  // each; their results wait in LDS and every atom adds its own in list order.
+  // (A Ga atom lists some forty partners, and its lane used to work them off
+  // alone, two dependent loads and a few hundred instructions each, while the
+  // rest of the pass had long ended: k_legs of 64 x 4 k atoms, mixed, 59.3 ->
+  // 34.4 us; of one 4 k slab, FP64, 37.8 -> 20.7.)
+  const bool fired = !(ti == 3 && orig_of(xi) >= in.nsg + in.impact);
+  const int ci = live && fired ? min(nion, Wion) : 0;
+  const uint64_t rows = __ballot(ci > 0);
+  if (rows != 0ull) {
+    T *const sv = reinterpret_cast<T *>(&hold[wid][0][0]);  // [7][64], then the energies
+    double *const su = reinterpret_cast<double *>(sv + 7 * FIB_WAVE);
+    static_assert(sizeof(hold[0]) >= FIB_WAVE * (7 * sizeof(T) + sizeof(double)), "hold");
+    int np = 1;  // pairs in the row
+    for (int p0 = 0; p0 < np; p0 += FIB_WAVE) {
+      const int p = p0 + lane;
+      // whose pair p is, which of its list, and where this atom's pairs start
+      int own = lane, k = 0, first = 0;
+      np = 0;
+      for (uint64_t m = rows; m != 0ull; m &= m - 1) {
+        const int o = __ffsll((unsigned long long)m) - 1;
+        if (p >= np) {
+          own = o;
+          k = p - np;
+        }
+        if (lane == o) first = np;
+        np += __builtin_amdgcn_readlane(ci, o);
       }
+      double4 xo;
+      xo.x = __shfl(xi.x, own);
+      xo.y = __shfl(xi.y, own);
+      xo.z = __shfl(xi.z, own);
+      xo.w = 0.0;
+      const int to = __shfl(ti, own);
+      T v[7];
+      double ul = 0;
+      const bool hit =
+          p < np &&
+          moliere(xo, to, nbr_ion[(size_t)(i - lane + own) * Wion + k], v, ul);
+      const uint64_t hits = __ballot(hit);
+      wave_lds_sync();
+      if (hit) {
+#pragma unroll
+        for (int c = 0; c < (VIR ? 7 : 4); ++c) sv[c * FIB_WAVE + lane] = v[c];
+        if (EN) su[lane] = ul;
+      }
+      wave_lds_sync();
+      const int q1 = min(first + ci - p0, FIB_WAVE);
+      for (int q = max(first - p0, 0); q < q1; ++q) {
+        if (!((hits >> q) & 1ull)) continue;
+#pragma unroll
+        for (int c = 0; c < (VIR ? 7 : 4); ++c) v[c] = sv[c * FIB_WAVE + q];
+        f.add(v[0], v[1], v[2], v[3]);
+        if (VIR)
+          addW(v[4], v[5], v[6], T(0.5) * (v[0] * v[1]), T(0.5) * (v[0] * v[2]),
+               T(0.5) * (v[0] * v[3]));
+        if (EN) {
+          ui += su[q];
+          etot += su[q];
+        }
+      }
+      wave_lds_sync();
     }
   }
 
