@@ -97,7 +97,6 @@ struct DevBufs {
                              // [ninst * (max_pad / 256 / FIB_FIN_CH + 1) * FIB_NRED]
   int pstride;               // NA/64 + 1
   TabEntry *tab;             // [ntable + 3]
-  double *xfer;              // staging [3*NA] for host transfers
   const KTimer *kt;          // timing hook (may be null)
   const int *gate;           // non-null: [2 + 2*ninst] build gates and the cell prefix of
                              // the gated instances, see k_md_decide
@@ -123,7 +122,6 @@ void launch_copy_rows(int NA, int wold, const uint16_t *src, int wnew, uint16_t 
 // 4), energy total of instance 0 into a device double
 void launch_put_inst(const DevBufs &d, const DInst &in, hipStream_t s);
 void launch_fill_zero(void *p, size_t bytes, hipStream_t s);
-void launch_copy_utot(const DevBufs &d, double *out, hipStream_t s);
 // clears the leaving mark of every atom (after a removal-list overflow)
 void launch_clear_leaving(const DevBufs &d, hipStream_t s);
 // lists = true: clears the list-overflow flags, the longest lists and the halt flag; false: the
@@ -159,11 +157,18 @@ void launch_sums(const DevBufs &d, const StepArgs &sa, hipStream_t s);
 void launch_import(const DevBufs &d, int inst, const DInst &in, const double *X,
                    const double *V, const int32_t *atype, const int32_t *xsides,
                    const double *Xi, hipStream_t s);
-void launch_export_x(const DevBufs &d, int inst, const DInst &in, double *out, hipStream_t s);
-void launch_export_vec(const DevBufs &d, int inst, const DInst &in, const double *src,
-                       double *out, hipStream_t s);
-void launch_export_scalar(const DevBufs &d, int inst, const DInst &in, const double *src,
-                          double *out, hipStream_t s);
+// What launch_export writes, in the caller's atom order; null: left out.
+struct ExportArgs {
+  double *x;              // positions (natm,3)
+  const double *src[2];   // planes [3][NA] of the sorted atoms ...
+  double *vec[2];         // ... to (natm,3) each
+  const double *scal_src; // [NA] ...
+  double *scal;           // ... to (natm)
+  const DCtl *ctl;        // the instance's control record ...
+  DCtl *ctl_out;          // ... whole, and
+  double *utot;           // its energy
+};
+void launch_export(const DevBufs &d, const DInst &in, const ExportArgs &ex, hipStream_t s);
 // sa supplies the masses for the ledger's e_in
 void launch_set_atom(const DevBufs &d, int p, const double x[3], const double v[3],
                      const StepArgs &sa, hipStream_t s);

@@ -3294,34 +3294,33 @@ __global__ void k_import(int inst, DInst in, int NA, const double *__restrict__ 
   inv[p] = p;
 }
 
-__global__ void k_export_x(DInst in, const double4 *__restrict__ X, double *__restrict__ out) {
+// One launch for all that a call hands back (three to five kernels of 3 us
+// and their gaps before, for 4 k atoms).
+__global__ void k_export(DInst in, int NA, const double4 *__restrict__ X, const ExportArgs ex) {
   const int o = blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= in.natm_pad) return;
-  const double4 x = X[in.atom_off + o];
-  if (meta_of(x) & META_PAD) return;
-  const int g = orig_of(x);
-  out[g] = x.x; out[in.natm + g] = x.y; out[2 * in.natm + g] = x.z;
-}
-
-__global__ void k_export_vec(DInst in, int NA, const double4 *__restrict__ X,
-                             const double *__restrict__ src, double *__restrict__ out) {
-  const int o = blockIdx.x * blockDim.x + threadIdx.x;
-  if (o >= in.natm_pad) return;
-  const int p = in.atom_off + o;
-  const double4 x = X[p];
-  if (meta_of(x) & META_PAD) return;
-  const int g = orig_of(x);
-  for (int c = 0; c < 3; ++c) out[(size_t)c * in.natm + g] = src[(size_t)c * NA + p];
-}
-
-__global__ void k_export_scalar(DInst in, const double4 *__restrict__ X,
-                                const double *__restrict__ src, double *__restrict__ out) {
-  const int o = blockIdx.x * blockDim.x + threadIdx.x;
+  if (blockIdx.x == 0) {
+    constexpr int NWORD = sizeof(DCtl) / sizeof(uint32_t);
+    if (ex.ctl_out)
+      for (int k = threadIdx.x; k < NWORD; k += blockDim.x)
+        reinterpret_cast<uint32_t *>(ex.ctl_out)[k] =
+            reinterpret_cast<const uint32_t *>(ex.ctl)[k];
+    if (ex.utot && threadIdx.x == 0) *ex.utot = ex.ctl->utot;
+  }
   if (o >= in.natm_pad) return;
   const int p = in.atom_off + o;
   const double4 x = X[p];
   if (meta_of(x) & META_PAD) return;
-  out[orig_of(x)] = src[p];
+  const size_t g = orig_of(x), n = in.natm;
+  if (ex.x) {
+    ex.x[g] = x.x;
+    ex.x[n + g] = x.y;
+    ex.x[2 * n + g] = x.z;
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+    if (ex.vec[q])
+      for (int c = 0; c < 3; ++c) ex.vec[q][c * n + g] = ex.src[q][(size_t)c * NA + p];
+  if (ex.scal) ex.scal[g] = ex.scal_src[p];
 }
 
 // Places atom p (a fired ion) and books its change of kinetic energy as
@@ -3722,7 +3721,7 @@ void launch_clear_overflow(const DevBufs &d, hipStream_t s, bool lists) {
 }
 
 // Start state of a handle-free evaluation, written by kernels: the instance
-// record (by value), zeroed bookkeeping, the energy total out.
+// record (by value) and zeroed bookkeeping.
 __global__ void k_put_inst(DInst in, DInst *__restrict__ I) {
   if (blockIdx.x == 0 && threadIdx.x == 0) I[0] = in;
 }
@@ -3730,9 +3729,6 @@ __global__ void k_fill_zero(uint32_t *__restrict__ p, size_t nwords) {
   for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < nwords;
        k += (size_t)gridDim.x * blockDim.x)
     p[k] = 0u;
-}
-__global__ void k_copy_utot(const DCtl *__restrict__ ctl, double *__restrict__ out) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) out[0] = ctl[0].utot;
 }
 
 void launch_put_inst(const DevBufs &d, const DInst &in, hipStream_t s) {
@@ -3742,9 +3738,6 @@ void launch_fill_zero(void *p, size_t bytes, hipStream_t s) {
   const size_t nw = bytes / 4;  // every array of the arena is a multiple of 4 bytes
   hipLaunchKernelGGL(k_fill_zero, dim3(gcap((long)std::min<size_t>(nw, 1u << 30))),
                      dim3(FIB_BLOCK), 0, s, static_cast<uint32_t *>(p), nw);
-}
-void launch_copy_utot(const DevBufs &d, double *out, hipStream_t s) {
-  hipLaunchKernelGGL(k_copy_utot, dim3(1), dim3(FIB_WAVE), 0, s, d.ctl, out);
 }
 
 void launch_clear_leaving(const DevBufs &d, hipStream_t s) {
@@ -3771,32 +3764,11 @@ void launch_import(const DevBufs &d, int inst, const DInst &in, const double *X,
   }
 }
 
-void launch_export_x(const DevBufs &d, int inst, const DInst &in, double *out, hipStream_t s) {
-  (void)inst;
+void launch_export(const DevBufs &d, const DInst &in, const ExportArgs &ex, hipStream_t s) {
   {
     KScope ks_(d, KT_IO);
-    hipLaunchKernelGGL(k_export_x, dim3(nblk(in.natm_pad, FIB_BLOCK)), dim3(FIB_BLOCK), 0, s, in,
-                       d.X[d.cur], out);
-  }
-}
-
-void launch_export_vec(const DevBufs &d, int inst, const DInst &in, const double *src,
-                       double *out, hipStream_t s) {
-  (void)inst;
-  {
-    KScope ks_(d, KT_IO);
-    hipLaunchKernelGGL(k_export_vec, dim3(nblk(in.natm_pad, FIB_BLOCK)), dim3(FIB_BLOCK), 0, s, in,
-                       d.NA, d.X[d.cur], src, out);
-  }
-}
-
-void launch_export_scalar(const DevBufs &d, int inst, const DInst &in, const double *src,
-                          double *out, hipStream_t s) {
-  (void)inst;
-  {
-    KScope ks_(d, KT_IO);
-    hipLaunchKernelGGL(k_export_scalar, dim3(nblk(in.natm_pad, FIB_BLOCK)), dim3(FIB_BLOCK), 0, s,
-                       in, d.X[d.cur], src, out);
+    hipLaunchKernelGGL(k_export, dim3(nblk(in.natm_pad, FIB_BLOCK)), dim3(FIB_BLOCK), 0, s, in,
+                       d.NA, d.X[d.cur], ex);
   }
 }
 
