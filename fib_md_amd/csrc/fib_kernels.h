@@ -70,6 +70,9 @@ struct DevBufs {
   DInst *I;                  // [ninst]
   DCtl *ctl;                 // [ninst]
   double4 *X[2];
+  // [cur] holds the state, the others take a build's reordered atoms.  Between
+  // builds F[1 - cur] (and V[1 - cur]) hold k_tri's sums of each centre's own
+  // terms, forces (and energies), for k_force3.
   double *V[2], *F[2], *Xi[2];
   int *inv;                  // [NA] atom_off + orig -> sorted position
   int *binst;                // [NA / FIB_BLOCK] instance of each block of FIB_BLOCK atoms
@@ -79,7 +82,8 @@ struct DevBufs {
   uint8_t *off_sw;           // [NA * 32]: row start of each stencil cell, [27] = has a row
   uint32_t *near;            // near lists [16 * NA] (null: none are kept)
   uint8_t *nst;              // state of each atom's near list [NA], see k_legs
-  void *G;                   // centre-term force on each leg, T4 [NA * Wsw]
+  void *G;                   // centre-term force on each leg [NA * Wsw]: three components,
+                             // or four (T4) where energies are wanted
   uint32_t *RA;              // per leg [NA * Wsw]: index into G of the partner's force
                              // on the atom (~0: none); needs NA * Wsw < 2^32
   uint64_t *amask;           // legs of the last evaluation, by list slot [NA]

@@ -1368,6 +1368,21 @@ struct Prec<true> {
   typedef float4 T4;
 };
 
+// Entry of G: the force a centre's terms put on one of its legs and, where
+// energies are wanted, a share of them.
+template <typename T>
+struct Vec3 {
+  T x, y, z;
+};
+template <bool MIXED, bool EN>
+struct GRec {
+  typedef Vec3<typename Prec<MIXED>::T> type;
+};
+template <bool MIXED>
+struct GRec<MIXED, true> {
+  typedef typename Prec<MIXED>::T4 type;
+};
+
 template <typename T>
 struct Leg {
   T e0, e1, e2;  // unit vector from the neighbour to the centre
@@ -2033,11 +2048,13 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
     const double4 *__restrict__ X, const DInst *__restrict__ I, const FConst fc, int NA,
     int Wsw, const int *__restrict__ nbr_sw, uint16_t *__restrict__ rk_sw,
     const uint8_t *__restrict__ off_sw, const uint64_t *__restrict__ amask,
-    typename Prec<MIXED>::T4 *__restrict__ G, uint32_t *__restrict__ RA, int pstride,
+    typename GRec<MIXED, EN>::type *__restrict__ G, uint32_t *__restrict__ RA,
+    double *__restrict__ Gown, double *__restrict__ Gown_u, int pstride,
     double *__restrict__ partials, const int *__restrict__ binst, const int *__restrict__ halt,
     int xs) {
   typedef typename Prec<MIXED>::T T;
   typedef typename Prec<MIXED>::T4 T4;
+  typedef typename GRec<MIXED, EN>::type GV;
   constexpr int NW = FIB_BLOCK / FIB_WAVE, QR = TRI_QROWS, FL = NS / 2;
   constexpr bool NT = (FIB_NT_LD & 2) != 0, NTS = (FIB_NT_ST & 2) != 0;
   constexpr bool U = EN || VIR;  // the terms' energies are wanted
@@ -2088,18 +2105,32 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
 #pragma unroll
   for (int w = 0; w < 9; ++w) W[w] = 0;
 
-  // results of the legs [fs, ...) of the atoms [f0, f1) wait in sG and sR
+  // results of the legs [fs, ...) of the atoms [f0, f1) wait in sG and sR;
+  // each atom's own sum of them, the reaction on the centre, goes with them
   int f0 = 0, fs = 0;
   auto write_out = [&](int f1) {
     wave_lds_sync();
     const bool mine = lane >= f0 && lane < f1;
+    double g0 = 0, g1 = 0, g2 = 0, gu = 0;
     for (int a = 0; __ballot(mine && a < nl) != 0ull; ++a) {
       if (mine && a < nl) {
         const size_t at = (size_t)a * NA + ic;
         const int q = exc + a - fs;
-        st_nt<NTS>(G + at, sG[wid][q]);
+        const T4 g = sG[wid][q];
+        GV gv;
+        gv.x = g.x; gv.y = g.y; gv.z = g.z;
+        if constexpr (EN) gv.w = g.w;
+        G[at] = gv;
         st_nt<NTS>(RA + at, sR[wid][q]);
+        g0 -= (double)g.x; g1 -= (double)g.y; g2 -= (double)g.z;
+        if (EN) gu += 0.5 * (double)g.w;
       }
+    }
+    if (mine) {
+      st_nt<NTS>(Gown + ic, g0);
+      st_nt<NTS>(Gown + (size_t)NA + ic, g1);
+      st_nt<NTS>(Gown + 2 * (size_t)NA + ic, g2);
+      if (EN) st_nt<NTS>(Gown_u + ic, gu);
     }
     wave_lds_sync();
   };
@@ -2911,17 +2942,23 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_md_report(const double4 *__restri
 // MODE 0 = store forces, MODE 1 = reference velocity update
 // (timeint.f90:231-236) + thermostat sums; MODE 2 = MD-step mode.
 // Bound by the gather of the partners' entries (and, in small batches, by
-// the chain of dependent loads): two batches of F3_BATCH legs, their own
-// entries and the partners' places first, then the partners' entries, all of
-// a batch in flight at once.  FP64, 2 x 512 k atoms: 119 us leg by leg, 109
-// so; the mixed mode's 4 x 512 k did not change (131).
+// the chain of dependent loads): two batches of F3_BATCH legs, the partners'
+// places first, then their entries, all of a batch in flight at once.  The
+// reaction on the centre comes summed from k_tri, which holds the terms in
+// LDS, instead of from its own G entries read again, and G has three
+// components where no energies are wanted: 24 B per atom and 4.2 entries of
+// 12 B (mixed) or 24 B for 8.4 of 16 or 32.  k_force3 and, for the sums,
+// k_tri: 4 x 512 k atoms, mixed, 118 -> 102 us and 206 -> 211; 2 x 512 k,
+// FP64, 109 -> 86 and 174 -> 180; 64 x 4 k, mixed, 24 -> 21.5 and 39.5 ->
+// 41.4.
 #define F3_BATCH 4
 template <bool MIXED, bool EN, int MODE>
 __global__ __launch_bounds__(FIB_BLOCK) void k_force3(
     const double4 *__restrict__ X, const DInst *__restrict__ I, int NA, int Wsw,
     const int *__restrict__ nbr_sw, const uint16_t *__restrict__ rk_sw,
-    const uint8_t *__restrict__ off_sw, const typename Prec<MIXED>::T4 *__restrict__ G,
-    const uint32_t *__restrict__ RA,
+    const uint8_t *__restrict__ off_sw, const typename GRec<MIXED, EN>::type *__restrict__ G,
+    const uint32_t *__restrict__ RA, const double *__restrict__ Gown,
+    const double *__restrict__ Gown_u,
     const uint64_t *__restrict__ amask, const int *__restrict__ cnt_sw,
     const double *__restrict__ Fpart, const double *__restrict__ upart, double fscale,
     double escale, double *__restrict__ Fout, double *__restrict__ uout, double *__restrict__ V,
@@ -2930,6 +2967,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_force3(
     const typename Prec<MIXED>::T4 *__restrict__ EXself, const uint64_t *__restrict__ exmask,
     const int *__restrict__ binst, const int *__restrict__ halt, int xs) {
   typedef typename Prec<MIXED>::T4 T4;
+  typedef typename GRec<MIXED, EN>::type GV;
   constexpr bool NT = (FIB_NT_LD & 4) != 0, NTS = (FIB_NT_ST & 4) != 0;
   const int lb = xcd_remap(blockIdx.x, gridDim.x, xs);
   const int i = lb * FIB_BLOCK + threadIdx.x;
@@ -2940,13 +2978,11 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_force3(
   const uint64_t am = ld_nt<NT>(amask + i);
   const double fp[3] = {ld_nt<NT>(Fpart + i), ld_nt<NT>(Fpart + (size_t)NA + i),
                         ld_nt<NT>(Fpart + 2 * (size_t)NA + i)};
-  T4 own[F3_BATCH];
+  const double go[3] = {ld_nt<NT>(Gown + i), ld_nt<NT>(Gown + (size_t)NA + i),
+                        ld_nt<NT>(Gown + 2 * (size_t)NA + i)};
   uint32_t ra[F3_BATCH];
 #pragma unroll
-  for (int u = 0; u < F3_BATCH; ++u) {
-    ra[u] = ld_nt<NT>(RA + (size_t)u * NA + i);
-    own[u] = G[(size_t)u * NA + i];
-  }
+  for (int u = 0; u < F3_BATCH; ++u) ra[u] = ld_nt<NT>(RA + (size_t)u * NA + i);
   double vold[3] = {0, 0, 0};
   if (MODE == 2)
     for (int c = 0; c < 3; ++c) vold[c] = ld_nt<NT>(V + (size_t)c * NA + i);
@@ -2961,47 +2997,29 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_force3(
     f2 = fp[2];
     if (EN) u = upart[i];
     const size_t row = (size_t)i * Wsw;
-    double g0 = 0, g1 = 0, g2 = 0, gu = 0;
+    // the reaction on the centre, and the forces that the partners' terms put
+    // on this atom, from the places k_tri noted for its legs
+    double g0 = go[0], g1 = go[1], g2 = go[2], gu = EN ? Gown_u[i] : 0.0;
     const int na = __popcll(am);
-    // the partners' entries (at the places k_tri noted for the legs) of the
-    // first legs, and what the next legs need
-    auto partner = [&](uint32_t at, T4 &g) {
+    auto partner = [&](uint32_t at, GV &g) {
       if (at != ~0u) {
         g = G[at];
       } else {
-        g.x = g.y = g.z = g.w = 0;
+        g.x = g.y = g.z = 0;
+        if constexpr (EN) g.w = 0;
       }
     };
-    T4 theirs[F3_BATCH], own2[F3_BATCH];
+    auto plus = [&](const GV &g) {
+      g0 += (double)g.x; g1 += (double)g.y; g2 += (double)g.z;
+      if constexpr (EN) gu += (double)g.w;
+    };
+    GV theirs[F3_BATCH], theirs2[F3_BATCH];
     uint32_t ra2[F3_BATCH];
 #pragma unroll
     for (int u = 0; u < F3_BATCH; ++u) {
       partner(u < na ? ra[u] : ~0u, theirs[u]);
-      ra2[u] = ~0u;
-      own2[u].x = own2[u].y = own2[u].z = own2[u].w = 0;
-      if (F3_BATCH + u < na) {
-        ra2[u] = ld_nt<NT>(RA + (size_t)(F3_BATCH + u) * NA + i);
-        own2[u] = G[(size_t)(F3_BATCH + u) * NA + i];
-      }
+      ra2[u] = F3_BATCH + u < na ? ld_nt<NT>(RA + (size_t)(F3_BATCH + u) * NA + i) : ~0u;
     }
-    // reaction on the centre: minus the forces its own terms put on its legs
-    auto minus = [&](const T4 &g) {
-      g0 -= (double)g.x; g1 -= (double)g.y; g2 -= (double)g.z;
-      if (EN) gu += 0.5 * (double)g.w;
-    };
-    // forces the partners' terms put on this atom
-    auto plus = [&](const T4 &g) {
-      g0 += (double)g.x; g1 += (double)g.y; g2 += (double)g.z;
-      if (EN) gu += (double)g.w;
-    };
-#pragma unroll
-    for (int u = 0; u < F3_BATCH; ++u)
-      if (u < na) minus(own[u]);
-#pragma unroll
-    for (int u = 0; u < F3_BATCH; ++u)
-      if (F3_BATCH + u < na) minus(own2[u]);
-    for (int n = 2 * F3_BATCH; n < na; ++n) minus(G[(size_t)n * NA + i]);
-    T4 theirs2[F3_BATCH];
 #pragma unroll
     for (int u = 0; u < F3_BATCH; ++u) partner(ra2[u], theirs2[u]);
 #pragma unroll
@@ -3011,7 +3029,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_force3(
     for (int u = 0; u < F3_BATCH; ++u)
       if (F3_BATCH + u < na) plus(theirs2[u]);
     for (int n = 2 * F3_BATCH; n < na; ++n) {
-      T4 g;
+      GV g;
       partner(ld_nt<NT>(RA + (size_t)n * NA + i), g);
       plus(g);
     }
@@ -3518,7 +3536,8 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
   hipLaunchKernelGGL((k_tri<MIXED, EN, VIR, NS_, TB_, APW_>),                                 \
                      dim3(d.NA / (FIB_BLOCK / FIB_WAVE * APW_)), dim3(FIB_BLOCK), 0, s,       \
                      d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.nbr_sw, d.rk_sw, d.off_sw, d.amask,  \
-                     (T4 *)d.G, d.RA, d.pstride, d.partials + (size_t)FIB_NRED * d.pstride,   \
+                     (typename GRec<MIXED, EN>::type *)d.G, d.RA, d.F[1 - d.cur],             \
+                     d.V[1 - d.cur], d.pstride, d.partials + (size_t)FIB_NRED * d.pstride,    \
                      d.binst, d.halt, xcd_shift(d) + (APW_ == 16 ? 2 : 0))
     if constexpr (EN || VIR) {
       // (one partial per 256 atoms: 64 atoms per wavefront)
@@ -3562,7 +3581,8 @@ static void force_c(const DevBufs &d, const FConst &fc, const StepArgs &sa, doub
     KScope ks_(d, KT_GATHER);
     hipLaunchKernelGGL((k_force3<MIXED, EN, MODE>), dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK),
                        0, s, d.X[d.cur], d.I, d.NA, d.Wsw, d.nbr_sw, d.rk_sw, d.off_sw,
-                       (const T4 *)d.G, d.RA, d.amask, d.cnt_sw, d.Fpart,
+                       (const typename GRec<MIXED, EN>::type *)d.G, d.RA, d.F[1 - d.cur],
+                       d.V[1 - d.cur], d.amask, d.cnt_sw, d.Fpart,
                        d.upart, fscale, escale, Fo,
                        d.uout, d.V[d.cur], sa, d.pstride, d.partials, d.ctl, (const T4 *)d.EX,
                        (const T4 *)d.EXself, d.exmask, d.binst, d.halt, xcd_shift(d));

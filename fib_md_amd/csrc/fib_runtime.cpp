@@ -945,12 +945,13 @@ extern "C" int32_t fib_get_nlist(fib_handle *h, int32_t inst, int32_t *nss, int3
 // mode 0: forces into dst (default d.Fout); mode 1: MD velocity update.
 static int32_t run_force(fib_handle *h, int flags, int mode, const StepArgs &sa,
                          double *dst = nullptr) {
-  const bool en = (flags & FIB_EVAL_ENERGY) != 0, vir = (flags & FIB_EVAL_VIRIAL) != 0;
+  const bool en = mode == 0 && (flags & FIB_EVAL_ENERGY) != 0;
+  const bool vir = (flags & FIB_EVAL_VIRIAL) != 0;
   const bool mixed = h->prec == FIB_PREC_MIXED;
   DevBufs &d = h->d;
   double *Fo = mode == 0 ? (dst ? dst : d.Fout) : d.F[d.cur];
   fibk::launch_force_a(d, h->fc, mixed, en, vir, h->stream);
-  fibk::launch_force_b(d, h->fc, mixed, en && mode == 0, mode, sa, Fo, h->stream);
+  fibk::launch_force_b(d, h->fc, mixed, en, mode, sa, Fo, h->stream);
   return FIB_OK;
 }
 
@@ -1885,7 +1886,7 @@ int32_t fib_arena_force(const fib_params *p, int32_t precision, int32_t natm, in
     return bad(FIB_ERR_OVERFLOW, "fib_force_noalloc: a neighbour list is longer than its "
                                  "fixed width (SW 32, ion 64)");
   fibk::launch_force_a(d, g_tab.fc, mixed, utot != nullptr, false, s);
-  fibk::launch_force_b(d, g_tab.fc, mixed, false, 0, StepArgs{}, d.Fout, s);
+  fibk::launch_force_b(d, g_tab.fc, mixed, utot != nullptr, 0, StepArgs{}, d.Fout, s);
   fibk::ExportArgs ex{};
   ex.src[0] = d.Fout;
   ex.vec[0] = F;
