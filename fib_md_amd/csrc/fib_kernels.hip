@@ -2020,7 +2020,10 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
 // so that the stores coalesce.
 // 4 x 512 k thermal Si atoms, per step: mixed 4,903 vector instructions per
 // wavefront and 300 us with one term per (leg, partner), 3,090 and 213 us
-// so; FP64 245 -> 173 us (2 x 512 k).
+// so; FP64 245 -> 173 us (2 x 512 k).  With the virial, its terms of a run
+// of 256 legs used to wait in 24 (FP64: 48) KiB of LDS, which left two blocks
+// to a CU; they now turn to their lanes through shuffles, and three fit:
+// 2.1 M atoms, mixed, with energies, just built: 588 -> 477 us.
 #ifndef TRI_BATCH
 #define TRI_BATCH 4  // 4: the next pass's positions load during this one; 2: only its row entries
 #endif
@@ -2065,9 +2068,6 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
   __shared__ uint32_t sR[NW][FL];
   constexpr int TAB = VIR ? TRI_TAB_VIR : TRI_TAB;
   __shared__ uint16_t tab[NW][TAB];  // owner lane | list slot << 6
-  // the virial's terms of a run, which lane q % 64 sums for leg q (the FP32
-  // sums of the mixed mode then do not depend on how a run is cut into passes)
-  __shared__ T sW[NW][VIR ? 6 : 1][VIR ? TAB : 1];
   const int lb = xcd_remap(blockIdx.x, gridDim.x, xs);
   const int lane = threadIdx.x % FIB_WAVE;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / FIB_WAVE);
@@ -2293,28 +2293,25 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
         sG[wid][P.ps - fs + lane] = gv;
         sR[wid][P.ps - fs + lane] = ra;
         if (U) uc += (double)Gu;
-        if (VIR) {
-          // r_a = x_a - x_i = -e_a / rinv_a
-          const T rl = -T(1) / La.rinv;
-          const T v[6] = {rl * La.e0, rl * La.e1, rl * La.e2, Ga0, Ga1, Ga2};
+      }
+      if (VIR) {
+        // r_a = x_a - x_i = -e_a / rinv_a.  Lane q % 64 sums for leg q of a
+        // run (the FP32 sums of the mixed mode then do not depend on how a
+        // run is cut into passes): the pass's values turn by its start.
+        const T rl = -T(1) / La.rinv;
+        T v[6] = {rl * La.e0, rl * La.e1, rl * La.e2, Ga0, Ga1, Ga2};
+        const int src = (lane - (P.ps - rs)) & (FIB_WAVE - 1);
 #pragma unroll
-          for (int c = 0; c < 6; ++c) sW[wid][c][P.ps - rs + lane] = v[c];
+        for (int c = 0; c < 6; ++c) v[c] = __shfl(v[c], src);
+        if (src < P.n) {
+#pragma unroll
+          for (int c = 0; c < 9; ++c) W[c] = fma_t(v[c / 3], v[3 + c % 3], W[c]);
         }
       }
       wave_lds_sync();
       if (!more) break;
       P = Q;
       if (TB < 4) partners(P);
-    }
-    if (VIR) {
-      const int nq = __builtin_amdgcn_readlane(inc, r1 - 1) - rs;
-      for (int q = lane; q < nq; q += FIB_WAVE) {
-        T v[6];
-#pragma unroll
-        for (int c = 0; c < 6; ++c) v[c] = sW[wid][c][q];
-#pragma unroll
-        for (int c = 0; c < 9; ++c) W[c] = fma_t(v[c / 3], v[3 + c % 3], W[c]);
-      }
     }
     r0 = r1;
   }
