@@ -97,6 +97,7 @@ struct DevBufs {
   double *partials;          // [2 * FIB_NRED * pstride], layout [region][slot][block]
   int max_pad;               // largest padded atom count of an instance
   int max_bucket;            // most buckets of an instance
+  double max_cell;           // largest cell volume
   double *fin_tmp;           // chunk results of big instances' reductions
                              // [ninst * (max_pad / 256 / FIB_FIN_CH + 1) * FIB_NRED]
   int pstride;               // NA/64 + 1

@@ -793,6 +793,7 @@ __device__ __forceinline__ void copy_back(const CopyBack &cb, int block,
 // ---------------------------------------------------------------------------
 // neighbour build: one 64-lane block per real cell
 #define NB_CHUNK 128
+#define NB_CAND 192   // candidates that a cell's fast build takes
 #define NB_ACC 384  // candidates whose acceptance masks are kept for the ranks
 #ifndef NB_WAVES
 #define NB_WAVES 4  // independent wavefronts per k_nbuild workgroup
@@ -858,9 +859,10 @@ __device__ __forceinline__ int mbcnt(uint64_t m) {
 // 2.1 M atoms (whole build): 720 -> 523 vector instructions a cell, 871 ->
 // 651 us (four waves per SIMD; asked for five or six it spills and takes
 // longer than before).
+template <int NT>
 __device__ __forceinline__ bool nbuild_cell_fast(
     const double4 *__restrict__ X, const DInst &in, int i0, int ni, int rs, int rc, int my_lo,
-    int total, uint64_t lm0, uint64_t lm1, double rv2, double rv2lj, int Wsw, int Wion,
+    int total, const uint64_t (&lm)[NT], double rv2, double rv2lj, int Wsw, int Wion,
     int &most_sw, int &most_ion, int *__restrict__ cnt_sw, int *__restrict__ nbr_sw, int *__restrict__ cnt_ion,
     int *__restrict__ nbr_ion, uint16_t *__restrict__ rk_sw, uint8_t *__restrict__ off_sw,
     double4 *s_x, int *s_j) {
@@ -885,79 +887,150 @@ __device__ __forceinline__ bool nbuild_cell_fast(
       hi[a] = fmaxf(hi[a], r);
     }
   }
-  // differences to the cell's first atom
-  const bool two = total > FIB_WAVE;
-  uint32_t up[2];
-  double4 x[2];
-  double e0[2][3];
-  bool have[2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    have[t] = t * FIB_WAVE + lane < total;
-    up[t] = have[t] ? (uint32_t)s_j[t * FIB_WAVE + lane] : ~0u;
-    if (t == 0 || two) x[t] = X[have[t] ? (int)(up[t] & JM) : i0];
-  }
-  int far[3] = {0, 0, 0};
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    if (t == 1 && !two) x[1] = x[0];
-    e0[t][0] = c[0] - x[t].x;
-    e0[t][1] = c[1] - x[t].y;
-    e0[t][2] = c[2] - x[t].z;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) far[a] = max(far[a], __double2hiint(e0[t][a]) & 0x7fffffff);
-  }
-  // all of them below 0.12 of the box (by the upper words): then every
-  // difference from an atom of the cell is below 0.24 and no shift is wanted
-  bool any = false;
-#pragma unroll
-  for (int a = 0; a < 3; ++a) any = any || far[a] >= __double2hiint(0.12 * in.lb[a]);
-  const bool wraps = __ballot(any) != 0ull;
-  uint32_t code[2] = {0x150u, 0x150u};
-  if (wraps) {
-    bool bad = false;
+  // candidates kept, and (lane s) those of them before stencil cell s
+  int nk = 0, klo = 0;
+  bool ions = false, wraps = false;
+  if constexpr (NT == 2) {
+    // differences to the cell's first atom
+    const bool two = total > FIB_WAVE;
+    uint32_t up[2];
+    double4 x[2];
+    double e0[2][3];
+    bool have[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      const bool mine = (up[t] >> NB_JBITS) == 13u;
-      code[t] = 0;
+      have[t] = t * FIB_WAVE + lane < total;
+      up[t] = have[t] ? (uint32_t)s_j[t * FIB_WAVE + lane] : ~0u;
+      if (t == 0 || two) x[t] = X[have[t] ? (int)(up[t] & JM) : i0];
+    }
+    int far[3] = {0, 0, 0};
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      if (t == 1 && !two) x[1] = x[0];
+      e0[t][0] = c[0] - x[t].x;
+      e0[t][1] = c[1] - x[t].y;
+      e0[t][2] = c[2] - x[t].z;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) far[a] = max(far[a], __double2hiint(e0[t][a]) & 0x7fffffff);
+    }
+    // all of them below 0.12 of the box (by the upper words): then every
+    // difference from an atom of the cell is below 0.24 and no shift is wanted
+    bool any = false;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) any = any || far[a] >= __double2hiint(0.12 * in.lb[a]);
+    wraps = __ballot(any) != 0ull;
+    uint32_t code[2] = {0x150u, 0x150u};
+    if (wraps) {
+      bool bad = false;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const bool mine = (up[t] >> NB_JBITS) == 13u;
+        code[t] = 0;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const double k = rint(e0[t][a] * in.ilb[a]);
+          const double e = e0[t][a] - k * in.lb[a];
+          e0[t][a] = e;
+          // shifts 0 and +-1 are coded 1, 2, 0
+          code[t] |= (uint32_t)((int)k + 1) << (4 + 2 * a);
+          bad = bad || (have[t] && (fabs(k) > 1.0 || fabs(e) > 0.49 * in.lb[a] - 1.001 * in.h[a] ||
+                                    (mine && (k != 0.0 || fabs(e) > 1.001 * in.h[a]))));
+        }
+      }
+      if (__ballot(bad) != 0ull) return false;
+    }
+    float d2[2];
+    bool ion = town == 3;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      float sum = 0.0f;
 #pragma unroll
       for (int a = 0; a < 3; ++a) {
-        const double k = rint(e0[t][a] * in.ilb[a]);
-        const double e = e0[t][a] - k * in.lb[a];
-        e0[t][a] = e;
-        // shifts 0 and +-1 are coded 1, 2, 0
-        code[t] |= (uint32_t)((int)k + 1) << (4 + 2 * a);
-        bad = bad || (have[t] && (fabs(k) > 1.0 || fabs(e) > 0.49 * in.lb[a] - 1.001 * in.h[a] ||
-                                  (mine && (k != 0.0 || fabs(e) > 1.001 * in.h[a]))));
+        const float r = (float)-e0[t][a];
+        const float d = fmaxf(fmaxf(lo[a] - r, r - hi[a]), 0.0f);
+        sum += d * d;
       }
+      const uint32_t ty = meta_of(x[t]) & META_TYPE_MASK;
+      ion = ion || ty == 3u;
+      x[t].w = __longlong_as_double((long long)((uint64_t)up[t] << 32 | (uint64_t)(code[t] | ty)));
+      d2[t] = have[t] ? sum : 3.0e38f;
     }
-    if (__ballot(bad) != 0ull) return false;
-  }
-  float d2[2];
-  bool ion = town == 3;
+    // without a Ga atom around, only pairs within the SW list radius are wanted
+    ions = __ballot(ion) != 0ull;
+    const float r2max = (float)(ions ? fmax(rv2, rv2lj) : rv2) * 1.0001f;
+    const uint64_t k0 = __ballot(d2[0] <= r2max), k1 = __ballot(d2[1] <= r2max);
+    const int n0 = __popcll(k0);
+    nk = n0 + __popcll(k1);
+    if (d2[0] <= r2max) s_x[mbcnt(k0)] = x[0];
+    if (d2[1] <= r2max) s_x[n0 + mbcnt(k1)] = x[1];
+    klo = __popcll(k0 & lm[0]) + __popcll(k1 & lm[1]);
+  } else {
+    // a batch at a time: the registers do not hold three at once
+    const bool last = total > (NT - 1) * FIB_WAVE;  // the last NT-th is wanted
+    uint32_t up[NT];
+    double4 x[NT];
+    bool ion = town == 3;
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    float sum = 0.0f;
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      const float r = (float)-e0[t][a];
-      const float d = fmaxf(fmaxf(lo[a] - r, r - hi[a]), 0.0f);
-      sum += d * d;
+    for (int t = 0; t < NT; ++t) {
+      const bool have = t * FIB_WAVE + lane < total;
+      up[t] = have ? (uint32_t)s_j[t * FIB_WAVE + lane] : ~0u;
+      if (t < NT - 1 || last) x[t] = X[have ? (int)(up[t] & JM) : i0];
     }
-    const uint32_t ty = meta_of(x[t]) & META_TYPE_MASK;
-    ion = ion || ty == 3u;
-    x[t].w = __longlong_as_double((long long)((uint64_t)up[t] << 32 | (uint64_t)(code[t] | ty)));
-    d2[t] = have[t] ? sum : 3.0e38f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      if (t == NT - 1 && !last) x[t] = x[0];
+      ion = ion || type_of(meta_of(x[t])) == 3;
+    }
+    // without a Ga atom around, only pairs within the SW list radius are wanted
+    ions = __ballot(ion) != 0ull;
+    const float r2max = (float)(ions ? fmax(rv2, rv2lj) : rv2) * 1.0001f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const bool have = t * FIB_WAVE + lane < total;
+      // differences to the cell's first atom
+      double e0[3] = {c[0] - x[t].x, c[1] - x[t].y, c[2] - x[t].z};
+      // all of them below 0.12 of the box (by the upper words): then every
+      // difference from an atom of the cell is below 0.24 and no shift is wanted
+      bool any = false;
+#pragma unroll
+      for (int a = 0; a < 3; ++a)
+        any = any || (__double2hiint(e0[a]) & 0x7fffffff) >= __double2hiint(0.12 * in.lb[a]);
+      uint32_t code = 0x150u;
+      if (__ballot(any) != 0ull) {
+        wraps = true;
+        const bool mine = (up[t] >> NB_JBITS) == 13u;
+        bool bad = false;
+        code = 0;
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+          const double k = rint(e0[a] * in.ilb[a]);
+          const double e = e0[a] - k * in.lb[a];
+          e0[a] = e;
+          // shifts 0 and +-1 are coded 1, 2, 0
+          code |= (uint32_t)((int)k + 1) << (4 + 2 * a);
+          bad = bad || (have && (fabs(k) > 1.0 || fabs(e) > 0.49 * in.lb[a] - 1.001 * in.h[a] ||
+                                 (mine && (k != 0.0 || fabs(e) > 1.001 * in.h[a]))));
+        }
+        if (__ballot(bad) != 0ull) return false;
+      }
+      float d2 = 0.0f;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const float r = (float)-e0[a];
+        const float d = fmaxf(fmaxf(lo[a] - r, r - hi[a]), 0.0f);
+        d2 += d * d;
+      }
+      const bool keep = have && d2 <= r2max;
+      const uint64_t km = __ballot(keep);
+      const int n = __popcll(km);
+      if (NT > 2 && nk + n > NB_CHUNK) return false;
+      x[t].w = __longlong_as_double(
+          (long long)((uint64_t)up[t] << 32 | (uint64_t)(code | (meta_of(x[t]) & META_TYPE_MASK))));
+      if (keep) s_x[nk + mbcnt(km)] = x[t];
+      nk += n;
+      klo += __popcll(km & lm[t]);
+    }
   }
-  // without a Ga atom around, only pairs within the SW list radius are wanted
-  const bool ions = __ballot(ion) != 0ull;
-  const float r2max = (float)(ions ? fmax(rv2, rv2lj) : rv2) * 1.0001f;
-  const uint64_t k0 = __ballot(d2[0] <= r2max), k1 = __ballot(d2[1] <= r2max);
-  const int n0 = __popcll(k0), nk = n0 + __popcll(k1);
-  if (d2[0] <= r2max) s_x[mbcnt(k0)] = x[0];
-  if (d2[1] <= r2max) s_x[n0 + mbcnt(k1)] = x[1];
-  // kept candidates before stencil cell s (lane s)
-  const int klo = __popcll(k0 & lm0) + __popcll(k1 & lm1);
   wave_lds_sync();
   auto rows = [&](auto sets) {
     constexpr int NS = decltype(sets)::value;
@@ -1030,6 +1103,7 @@ __device__ __forceinline__ bool nbuild_cell_fast(
 }
 
 // One cell (cx, cy, cz) of instance `in`, built by one wave.
+template <bool WIDE>
 __device__ __forceinline__ void nbuild_cell(
     const double4 *__restrict__ X, const DInst &in, int cx, int cy, int cz, int sd0, int sd1,
     int sd2, const int *__restrict__ cstart, int base, double rv2, double rv2lj, int Wsw, int Wion,
@@ -1074,11 +1148,19 @@ __device__ __forceinline__ void nbuild_cell(
     const int cut = min(max(my_lo - b, 0), 64);
     return cut >= 64 ? ~0ull : ((1ull << cut) - 1ull);
   };
-  if (total <= NB_CHUNK && ni <= 32 &&
-      nbuild_cell_fast(X, in, i0, ni, rs, rc, my_lo, total, before_mask(0), before_mask(FIB_WAVE),
-                       rv2, rv2lj, Wsw, Wion, most_sw, most_ion, cnt_sw, nbr_sw, cnt_ion, nbr_ion,
-                       rk_sw, off_sw, s_x, s_j))
-    return;
+  if (total <= NB_CHUNK && ni <= 32) {
+    const uint64_t lm[2] = {before_mask(0), before_mask(FIB_WAVE)};
+    if (nbuild_cell_fast<2>(X, in, i0, ni, rs, rc, my_lo, total, lm, rv2, rv2lj, Wsw, Wion,
+                            most_sw, most_ion, cnt_sw, nbr_sw, cnt_ion, nbr_ion, rk_sw, off_sw,
+                            s_x, s_j))
+      return;
+  } else if (WIDE && total <= NB_CAND && ni <= 32) {
+    const uint64_t lm[3] = {before_mask(0), before_mask(FIB_WAVE), before_mask(2 * FIB_WAVE)};
+    if (nbuild_cell_fast<3>(X, in, i0, ni, rs, rc, my_lo, total, lm, rv2, rv2lj, Wsw, Wion,
+                            most_sw, most_ion, cnt_sw, nbr_sw, cnt_ion, nbr_ion, rk_sw, off_sw,
+                            s_x, s_j))
+      return;
+  }
   const bool masks = total <= NB_ACC && ni <= 32;
   if (masks)
     for (int g = lane; g < total; g += FIB_WAVE) s_acc[g] = 0;
@@ -1255,7 +1337,7 @@ __device__ __forceinline__ int locate_cell(const DInst *__restrict__ I, int nins
 // its width is cut; the longest goes to the instance's record, and in MD-step
 // mode (under a gate) the rest of the step halts until the host has grown
 // the lists and rebuilt them.
-template <int NBC>
+template <int NBC, bool WIDE>
 __global__ __launch_bounds__(NB_WAVES * FIB_WAVE) __attribute__((amdgpu_waves_per_eu(4)))
 void k_nbuild(
     const double4 *__restrict__ X, const DInst *__restrict__ I, int ninst, int total_cells,
@@ -1267,7 +1349,7 @@ void k_nbuild(
   GATE_OR_RETURN(gate);
   static_assert(NB_WAVES * FIB_WAVE == FIB_BLOCK, "copy_back's blocks");
   __shared__ double4 s_x[NB_WAVES][NB_CHUNK];
-  __shared__ int s_j[NB_WAVES][NB_CHUNK];
+  __shared__ int s_j[NB_WAVES][WIDE ? NB_CAND : NB_CHUNK];
   __shared__ uint8_t s_st[NB_WAVES][NB_CHUNK];
   __shared__ int s_rs[NB_WAVES][27], s_off[NB_WAVES][28];
   __shared__ uint32_t s_acc[NB_WAVES][NB_ACC];
@@ -1302,7 +1384,7 @@ void k_nbuild(
     }
     const DInst &in = I[k];
     int most_sw = 0, most_ion = 0;
-    nbuild_cell(X, in, cx, cy, cz, sd0, sd1, sd2, cstart, base, rv2, rv2lj, Wsw, Wion, most_sw,
+    nbuild_cell<WIDE>(X, in, cx, cy, cz, sd0, sd1, sd2, cstart, base, rv2, rv2lj, Wsw, Wion, most_sw,
                 most_ion, cnt_sw, nbr_sw, cnt_ion, nbr_ion, rk_sw, off_sw, s_x[w], s_j[w],
                 s_st[w], s_rs[w], s_off[w], s_acc[w]);
     if ((most_sw > Wsw || most_ion > Wion) && lane == 0) {
@@ -3380,6 +3462,19 @@ static int nb_cells_auto(int total_cells) {
   return total_cells < 65536 ? 1 : total_cells < 131072 ? 2 : total_cells < 262144 ? 4 : 8;
 }
 
+// Whether the list build expects cells with 129 to 192 candidates, which its
+// WIDE variant takes on the fast path too: those of boxes whose sides are not
+// close to a multiple of the cutoff, or of long lists.  Silicon has 0.46 atoms
+// per sigma^3 (27 cells of rc^3 hold 96 candidates for lists of 1.1 cutoffs,
+// 110 for 1.15), and the counts vary by about a tenth.  5 and 5.04 atoms per
+// cell (1,000 and 1,728 atoms): 29 -> 14 us; 4.1 and 4.4 (4,096 and 5,832):
+// 13.3 -> 13.7 and 13.9 -> 14.4; 2.1 M atoms, 3.6 per cell: 730 -> 780, so
+// the variant is left out where it is not wanted.
+static bool wide_cells(const DevBufs &d, const FConst &fc) {
+  const double is = std::min(fc.isig[0][0], fc.isig[1][1]);
+  return 27.0 * 0.46 * d.max_cell * is * is * is > 120.0;
+}
+
 // Times the launches issued in its scope under one key.
 struct KScope {
   const KTimer *t;
@@ -3490,17 +3585,19 @@ void launch_nbuild(const DevBufs &d, const FConst &fc, hipStream_t s, int from, 
   }
   KScope ks_(d, KT_NBUILD);
   const int nbc = d.nb_cells ? d.nb_cells : nb_cells_auto(d.total_cells);
+  const bool wide = wide_cells(d, fc);
 #define NB_LAUNCH(C)                                                                           \
-  hipLaunchKernelGGL(k_nbuild<C>, dim3(cb.blocks + nblk(d.total_cells, C * NB_WAVES)),         \
+  auto *const f = wide ? k_nbuild<C, true> : k_nbuild<C, false>;                               \
+  hipLaunchKernelGGL(f, dim3(cb.blocks + nblk(d.total_cells, C * NB_WAVES)),                   \
                      dim3(NB_WAVES * FIB_WAVE), 0, s, d.X[from], d.I, d.ninst, d.total_cells,  \
                      d.cstart, fc.rv2, fc.rv2lj, d.Wsw, d.Wion, d.cnt_sw, d.nbr_sw, d.cnt_ion, \
                      d.nbr_ion, d.rk_sw, d.off_sw, d.ctl, d.gate, d.halt, cb)
   switch (nbc) {
-    case 1: NB_LAUNCH(1); break;
-    case 2: NB_LAUNCH(2); break;
-    case 4: NB_LAUNCH(4); break;
-    case 16: NB_LAUNCH(16); break;
-    default: NB_LAUNCH(8); break;
+    case 1: { NB_LAUNCH(1); break; }
+    case 2: { NB_LAUNCH(2); break; }
+    case 4: { NB_LAUNCH(4); break; }
+    case 16: { NB_LAUNCH(16); break; }
+    default: { NB_LAUNCH(8); break; }
   }
 #undef NB_LAUNCH
 }

@@ -649,9 +649,11 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
   ALLOC(d.partials, (size_t)d.pstride * FIB_NRED * 3);
   d.max_pad = 0;
   d.max_bucket = 0;
+  d.max_cell = 0;
   for (const DInst &in : h->inst) {
     d.max_pad = std::max(d.max_pad, in.natm_pad);
     d.max_bucket = std::max(d.max_bucket, in.nbucket);
+    d.max_cell = std::max(d.max_cell, in.h[0] * in.h[1] * in.h[2]);
   }
   ALLOC(d.fin_tmp, (size_t)ninst * (d.max_pad / FIB_BLOCK / FIB_FIN_CH + 1) * FIB_NRED);
   ALLOC(d.tab, h->tab.size());
@@ -1813,6 +1815,7 @@ int32_t fib_arena_force(const fib_params *p, int32_t precision, int32_t natm, in
   d.pstride = d.NA / FIB_WAVE + 1;
   d.max_pad = in.natm_pad;
   d.max_bucket = in.nbucket;
+  d.max_cell = in.h[0] * in.h[1] * in.h[2];
   const size_t NA = (size_t)d.NA;
   const bool mixed = precision == FIB_PREC_MIXED;
   const size_t g4 = mixed ? sizeof(float4) : sizeof(double4);

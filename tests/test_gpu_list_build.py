@@ -1,7 +1,8 @@
 """The list build (k_nbuild) in every path of a cell: halos that fit two
 candidates per lane with one or two registers of them left after the box
 filter, denser ones, boxes of few cells (no unique periodic shift), cells at
-the faces of larger ones (shifts of +-L), positions outside the box, Ga ions
+the faces of larger ones (shifts of +-L), wide cells (three candidates per
+lane, or more than are kept), positions outside the box, Ga ions
 among the candidates, empty cells; and 1 to 16 cells per wavefront.
 
 Neighbour sets equal the oracle's; FP64 forces agree with it within 1e-10 of
@@ -22,6 +23,9 @@ CASES = {
     "flat": ((14, 3, 4), 5.431, 0.1, 1.0, 0, False),
     "dense": ((6, 6, 6), 4.95, 0.05, 1.0, 3, False),
     "very_dense": ((7, 6, 6), 4.5, 0.02, 1.0, 2, False),
+    "wide_cells": ((7, 6, 6), 5.431, 0.1, 1.0, 3, False),
+    "wide_cells_outside": ((6, 5, 7), 5.431, 0.05, 1.0, 2, True),
+    "wide_cells_dense": ((6, 6, 6), 5.1, 0.02, 1.0, 0, False),
     "sparse": ((8, 8, 8), 5.431, 0.2, 0.25, 6, False),
     "outside_the_box": ((18, 5, 5), 5.431, 0.1, 1.0, 3, True),
 }
