@@ -138,8 +138,8 @@ struct DCtl {
 struct RedSpec {
   int32_t nv;
   int32_t bs;            // block size of the producing kernel
-  int32_t nreg;          // 1, or 2: two producers wrote partials of the same
-                         // blocks at partials and partials + FIB_NRED * pstride
+  int32_t sub;           // nv == 10: partials of the second of the three producers
+                         // (at partials, + FIB_NRED * pstride, + twice that) per block
   int32_t op[FIB_NRED];
   int32_t dst[FIB_NRED];
 };

@@ -315,9 +315,12 @@ __device__ void block_partials(double (&v)[NV], const int (&op)[NV], int lblock,
 // depends on the instance alone: one wavefront per chunk of FIN_CH blocks
 // (lane l takes blocks l, l + 64, ..., then a butterfly), and, when the
 // instance has more than one, one wavefront over its chunks the same way.
-// All NV slots at once, so the loads of every slot are in flight together.
-// A wavefront per chunk instead of a workgroup of 1024 threads per 1024
-// blocks: 14 -> 5 us a reduction, at 4 k as at 2 M atoms.
+// All NV slots at once, so the loads of every slot are in flight together,
+// except the ten of the energies and the virial, of three producers: a
+// wavefront per slot.  A wavefront per chunk instead of a workgroup of 1024
+// threads per 1024 blocks: 14 -> 5 us a reduction, at 4 k as at 2 M atoms; up
+// to FIN_ONE chunks combined where they are reduced, and the ten slots side by
+// side: 101 k atoms (two chunks, ten slots) 18.7 -> 12.8 us.
 #define FIN_CH FIB_FIN_CH
 // red_merge with the operations of a RedSpec: k_md_pos' six slots start with a
 // top-two triple, every other reduction is sums and maxima.
@@ -350,20 +353,39 @@ __device__ __forceinline__ void fin_chunk(double (&x)[NV], const DInst &in, int 
   const int lane = threadIdx.x % FIB_WAVE;
 #pragma unroll
   for (int k = 0; k < NV; ++k) x[k] = red_identity(rs.op[k]);
-  constexpr int UN = NV < 10 ? FIN_CH / FIB_WAVE : 1;
-#pragma unroll UN
+#pragma unroll
   for (int m = 0; m < FIN_CH / FIB_WAVE; ++m) {
     const int b = c * FIN_CH + m * FIB_WAVE + lane;
-    if (b < nblk)
-      for (int r = 0; r < (NV == 10 ? rs.nreg : 1); ++r) {
-        double y[NV];
+    if (b < nblk) {
+      double y[NV];
 #pragma unroll
-        for (int k = 0; k < NV; ++k)
-          y[k] = partials[(size_t)(r * FIB_NRED + k) * pstride + blk0 + b];
-        fin_merge<NV>(x, y, rs);
-      }
+      for (int k = 0; k < NV; ++k) y[k] = partials[(size_t)k * pstride + blk0 + b];
+      fin_merge<NV>(x, y, rs);
+    }
   }
   fin_wave<NV>(x, rs);
+}
+// slot k of it, a sum over the regions of k_legs, k_tri (rs.sub blocks for one
+// of the others') and k_extra
+__device__ __forceinline__ double fin_chunk_slot(int k, const DInst &in, int c,
+                                                 const double *__restrict__ partials, int pstride,
+                                                 const RedSpec &rs) {
+  const int blk0 = in.atom_off / rs.bs, nblk = in.natm_pad / rs.bs;
+  const double *const p = partials + (size_t)k * pstride;
+  const size_t reg = (size_t)FIB_NRED * pstride;
+  double x = 0;
+#pragma unroll
+  for (int m = 0; m < FIN_CH / FIB_WAVE; ++m) {
+    const int b = c * FIN_CH + m * FIB_WAVE + (int)(threadIdx.x % FIB_WAVE);
+    if (b < nblk) {
+      const size_t at = (size_t)(blk0 + b);
+      x += p[at];
+      for (int u = 0; u < rs.sub; ++u) x += p[reg + at * rs.sub + u];
+      x += p[2 * reg + at];
+    }
+  }
+  for (int o = FIB_WAVE / 2; o > 0; o >>= 1) x += __shfl_xor(x, o);
+  return x;
 }
 // the chunks of an instance
 template <int NV>
@@ -401,31 +423,52 @@ __device__ __forceinline__ void fin_finish(int how, int inst, const DInst &in,
     fin_chunk<NV>(x, in, 0, partials, pstride, rs);
   } else {
     const int nci = fin_chunks(in, rs.bs);
-    if (nci < 2) return;  // k_finalize stored it
+    if (nci <= 1) return;  // k_finalize stored it
     fin_combine<NV>(x, inst, nci, nch, tmp, rs);
   }
   if (threadIdx.x % FIB_WAVE == 0) fin_store<NV>(x, rs, ctl);
 }
+// Workgroup (k, y): chunks [y * per, (y + 1) * per) of instance k, a wavefront
+// each (NV == 10: one per slot of each).  Instances of up to FIN_ONE chunks are
+// reduced by one workgroup, which also combines them; of larger ones
+// k_finalize2, or the next kernel, combines the chunks.
+#define FIN_ONE 8
+#define FIN_WAVES 16
 template <int NV>
-__global__ __launch_bounds__(FIB_WAVE) void k_finalize(const DInst *__restrict__ I,
-                                                       const double *__restrict__ partials,
-                                                       int pstride, RedSpec rs,
-                                                       DCtl *__restrict__ ctl,
-                                                       double *__restrict__ tmp,
-                                                       const int *__restrict__ halt) {
+__global__ __launch_bounds__(FIN_WAVES *FIB_WAVE) void k_finalize(
+    const DInst *__restrict__ I, const double *__restrict__ partials, int pstride, RedSpec rs,
+    int per, DCtl *__restrict__ ctl, double *__restrict__ tmp, const int *__restrict__ halt) {
   HALT_OR_RETURN(halt);
-  const int inst = blockIdx.x, c = blockIdx.y, nch = gridDim.y;
+  constexpr int SL = NV == 10 ? NV : 1;  // wavefronts per chunk
+  __shared__ double s_x[FIN_ONE * NV];
+  const int inst = blockIdx.x, c0 = blockIdx.y * per, nch = gridDim.y * per;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / FIB_WAVE);
   const DInst &in = I[inst];
-  const int nci = fin_chunks(in, rs.bs);
-  if (c >= nci) return;
-  double x[NV];
-  fin_chunk<NV>(x, in, c, partials, pstride, rs);
-  if (threadIdx.x != 0) return;
-  if (nci == 1) {
-    fin_store<NV>(x, rs, ctl[inst]);
-  } else {
+  const int nci = fin_chunks(in, rs.bs), n = min(nci - c0, per);
+  for (int q = wid; q < n * SL; q += blockDim.x / FIB_WAVE) {
+    if constexpr (NV == 10) {
+      const double x = fin_chunk_slot(q % SL, in, c0 + q / SL, partials, pstride, rs);
+      if (threadIdx.x % FIB_WAVE == 0) s_x[q] = x;
+    } else {
+      double x[NV];
+      fin_chunk<NV>(x, in, c0 + q, partials, pstride, rs);
+      if (threadIdx.x % FIB_WAVE == 0) {
+        if (nci == 1) fin_store<NV>(x, rs, ctl[inst]);  // nothing to combine
 #pragma unroll
-    for (int k = 0; k < NV; ++k) tmp[((size_t)inst * nch + c) * NV + k] = x[k];
+        for (int k = 0; k < NV; ++k) s_x[q * NV + k] = x[k];
+      }
+    }
+  }
+  if (SL == 1 && nci == 1) return;
+  __syncthreads();
+  if (nci <= per) {
+    if (wid != 0) return;
+    double x[NV];
+    fin_combine<NV>(x, 0, nci, 0, s_x, rs);
+    if (threadIdx.x == 0) fin_store<NV>(x, rs, ctl[inst]);
+  } else {
+    for (int q = threadIdx.x; q < n * NV; q += blockDim.x)
+      tmp[((size_t)inst * nch + c0) * NV + q] = s_x[q];
   }
 }
 template <int NV>
@@ -2122,7 +2165,8 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
 // 4 k atoms are 64 wavefronts of 64 for 1,024 SIMDs, and the passes of one
 // wavefront follow each other (24.4 -> 12.3 us).  A large batch fills the
 // chip either way and pays for 16 with emptier last passes (262 k atoms 39.7
-// -> 48.4 us, 811 k 90 -> 126).
+// -> 48.4 us, 811 k 90 -> 126).  With energies and the virial, just built:
+// 4 k atoms, FP64, 32.8 -> 17.5 us; 2 k, mixed, without the virial, 26 -> 13.
 #define TRI_SMALL 131072
 template <bool MIXED>
 struct TriStage {
@@ -3490,11 +3534,11 @@ struct KScope {
 // chunks of the largest instance
 static int fin_nch(const DevBufs &d, int bs) { return (d.max_pad / bs + FIN_CH - 1) / FIN_CH; }
 
-static RedSpec red_spec(int nv, int bs, const int *op, const int *dst, int nreg = 1) {
+static RedSpec red_spec(int nv, int bs, const int *op, const int *dst, int sub = 1) {
   RedSpec rs;
   rs.nv = nv;
   rs.bs = bs;
-  rs.nreg = nreg;
+  rs.sub = sub;
   for (int k = 0; k < FIB_NRED; ++k) {
     rs.op[k] = k < nv ? op[k] : 0;
     rs.dst[k] = k < nv ? dst[k] : -1;
@@ -3502,23 +3546,29 @@ static RedSpec red_spec(int nv, int bs, const int *op, const int *dst, int nreg 
   return rs;
 }
 
+// Chunks per workgroup of k_finalize: all of an instance, or one.
+static int fin_per(const DevBufs &d, int bs) { return fin_nch(d, bs) <= FIN_ONE ? FIN_ONE : 1; }
+
+// Reduces every instance, or the chunks of instances of more than FIN_ONE
+// (fin_per is 1: tmp is left to combine).
 template <int NV>
 static void fin_launch(const DevBufs &d, const RedSpec &rs, hipStream_t s) {
-  hipLaunchKernelGGL(k_finalize<NV>, dim3(d.ninst, fin_nch(d, rs.bs)), dim3(FIB_WAVE), 0, s, d.I,
-                     d.partials, d.pstride, rs, d.ctl, d.fin_tmp, d.halt);
+  const int nch = fin_nch(d, rs.bs), per = fin_per(d, rs.bs);
+  const int waves = std::min(FIN_WAVES, std::min(nch, per) * (NV == 10 ? NV : 1));
+  hipLaunchKernelGGL(k_finalize<NV>, dim3(d.ninst, per == 1 ? nch : 1), dim3(waves * FIB_WAVE), 0,
+                     s, d.I, d.partials, d.pstride, rs, per, d.ctl, d.fin_tmp, d.halt);
 }
 
 static void finalize(const DevBufs &d, int nv, int bs, const int *op, const int *dst,
-                     hipStream_t s, int nreg = 1) {
-  const RedSpec rs = red_spec(nv, bs, op, dst, nreg);
-  const int nch = fin_nch(d, bs);
+                     hipStream_t s, int sub = 1) {
+  const RedSpec rs = red_spec(nv, bs, op, dst, sub);
   KScope ks_(d, KT_REDUCE);
 #define FIN_CASE(N)                                                                          \
   case N:                                                                                    \
     fin_launch<N>(d, rs, s);                                                                 \
-    if (nch > 1)                                                                             \
-      hipLaunchKernelGGL(k_finalize2<N>, dim3(d.ninst), dim3(FIB_WAVE), 0, s, d.I, nch, rs,  \
-                         d.ctl, d.fin_tmp, d.halt);                                          \
+    if (fin_per(d, bs) == 1)                                                                 \
+      hipLaunchKernelGGL(k_finalize2<N>, dim3(d.ninst), dim3(FIB_WAVE), 0, s, d.I,           \
+                         fin_nch(d, bs), rs, d.ctl, d.fin_tmp, d.halt);                      \
     break;
   switch (nv) {
     FIN_CASE(4)
@@ -3620,12 +3670,15 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
                        d.cnt_ion, d.nbr_ion, d.amask, d.Fpart, d.upart, d.near,
                        d.nst, d.ctl, d.binst, d.pstride, d.partials, d.halt, xcd_shift(d));
   }
+  int tri_bs = FIB_BLOCK;  // atoms per workgroup, and partial sum, of k_tri
   {
     KScope ks_(d, KT_TRI);
     // the MD step's variant (no energy, no virial) in every tile; the others
     // in the default tile
     const int ns = (EN || VIR || !d.tri_ns) ? TriStage<MIXED>::N : d.tri_ns;
     const int tb = (EN || VIR || !d.tri_tb) ? TRI_BATCH : d.tri_tb;
+    const bool small = !(MIXED && VIR) && d.NA <= TRI_SMALL && !d.tri_ns && !d.tri_tb;
+    if (small) tri_bs = 4 * 16;
 #define TRI_LAUNCH(NS_, TB_, APW_)                                                            \
   hipLaunchKernelGGL((k_tri<MIXED, EN, VIR, NS_, TB_, APW_>),                                 \
                      dim3(d.NA / (FIB_BLOCK / FIB_WAVE * APW_)), dim3(FIB_BLOCK), 0, s,       \
@@ -3633,11 +3686,12 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
                      (typename GRec<MIXED, EN>::type *)d.G, d.RA, d.F[1 - d.cur],             \
                      d.V[1 - d.cur], d.pstride, d.partials + (size_t)FIB_NRED * d.pstride,    \
                      d.binst, d.halt, xcd_shift(d) + (APW_ == 16 ? 2 : 0))
-    if constexpr (EN || VIR) {
-      // (one partial per 256 atoms: 64 atoms per wavefront)
-      TRI_LAUNCH(TriStage<MIXED>::N, TRI_BATCH, FIB_WAVE);
-    } else if (d.NA <= TRI_SMALL && !d.tri_ns && !d.tri_tb) {
+    // (the mixed mode's virial is summed in FP32 over runs of a wavefront's
+    // legs, which have to stay those of 64 atoms)
+    if (small) {
       TRI_LAUNCH(128, TRI_BATCH, 16);
+    } else if constexpr (EN || VIR) {
+      TRI_LAUNCH(TriStage<MIXED>::N, TRI_BATCH, FIB_WAVE);
     } else {
       if (ns == TriStage<MIXED>::N && tb == TRI_BATCH)
         TRI_LAUNCH(TriStage<MIXED>::N, TRI_BATCH, FIB_WAVE);
@@ -3661,7 +3715,7 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
   if (EN || VIR) {
     int op[10], dst[10];
     for (int k = 0; k < 10; ++k) { op[k] = 0; dst[k] = DCTL_IDX(utot) + k; }
-    finalize(d, 10, FIB_BLOCK, op, dst, s, 3);
+    finalize(d, 10, FIB_BLOCK, op, dst, s, FIB_BLOCK / tri_bs);
   }
 }
 
@@ -3740,7 +3794,9 @@ void launch_md_pos(const DevBufs &d, const FConst &fc, const StepArgs &sa, int *
   const int nch = fin_nch(d, FIB_BLOCK);
   // a few small instances: k_md_decide's four wavefronts reduce them, two
   // each; otherwise a wavefront per chunk does, and k_md_decide combines
-  const int how = nch == 1 ? (d.ninst <= 8 ? FIN_ALL : FIN_DONE) : FIN_COMBINE;
+  const int how = nch == 1 && d.ninst <= 8 ? FIN_ALL
+                  : fin_per(d, FIB_BLOCK) > 1 ? FIN_DONE
+                                              : FIN_COMBINE;
   KScope ks_(d, KT_REDUCE);
   if (how != FIN_ALL) fin_launch<6>(d, rs, s);
   hipLaunchKernelGGL(k_md_decide, dim3(1), dim3(DECIDE_T), 0, s, d.ninst, d.I, d.ctl, sa.skin,
@@ -3761,7 +3817,7 @@ void launch_md_ctl(const DevBufs &d, const StepArgs &sa, hipStream_t s) {
   KScope ks_(d, KT_REDUCE);
   if (nch > 1) fin_launch<4>(d, rs, s);
   hipLaunchKernelGGL(k_md_ctl, dim3(d.ninst), dim3(FIB_WAVE), 0, s, d.I, d.ctl, sa,
-                     nch > 1 ? FIN_COMBINE : FIN_ALL, rs, d.partials, d.pstride, d.fin_tmp, nch,
+                     nch == 1 ? FIN_ALL : fin_per(d, FIB_BLOCK) > 1 ? FIN_DONE : FIN_COMBINE, rs, d.partials, d.pstride, d.fin_tmp, nch,
                      d.halt);
 }
 

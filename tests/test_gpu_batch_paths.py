@@ -39,10 +39,11 @@ def _run(slabs, precision):
                   np.array([0.0, 1.0e4, -5.0e4]))
     g.md_run(STEPS)
     out = []
+    epot = g.md_energy()
     for k in range(len(slabs)):
         r = g.md_report(k)
         X, V = g.state(k)[:2]
-        out.append((np.asarray(X), np.asarray(V), r))
+        out.append((np.asarray(X), np.asarray(V), r, epot[k]))
     g.close()
     return out
 
@@ -71,11 +72,15 @@ def test_alone_and_in_a_batch(name, precision):
     np.testing.assert_array_equal(batch[0][0], alone[0])
     np.testing.assert_array_equal(batch[0][1], alone[1])
     assert batch[0][2] == alone[2]
+    # (the vertex pass's workgroups, and with them the order of the sum of up
+    # to 1.4e5 terms, depend on the batch: sqrt(1.4e5) 2^-53 = 4e-14 of it)
+    assert abs(batch[0][3] - alone[3]) <= 1e-12 * abs(alone[3])
     if len(rest) == 1:  # and the other one
         other = _run(rest, precision)[0]
         np.testing.assert_array_equal(batch[1][0], other[0])
         np.testing.assert_array_equal(batch[1][1], other[1])
         assert batch[1][2] == other[2]
+        assert abs(batch[1][3] - other[3]) <= 1e-12 * abs(other[3])
 
 
 @pytest.mark.parametrize("n", [(3, 11, 31), (8, 8, 16), (5, 5, 41)])
