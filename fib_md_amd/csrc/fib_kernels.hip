@@ -836,6 +836,7 @@ __device__ __forceinline__ void copy_back(const CopyBack &cb, int block,
 // ---------------------------------------------------------------------------
 // neighbour build: one 64-lane block per real cell
 #define NB_CHUNK 128
+#define NB_XS 4      // log2 of the workgroups that an XCD takes in a row
 #define NB_CAND 192   // candidates that a cell's fast build takes
 #define NB_ACC 384  // candidates whose acceptance masks are kept for the ranks
 #ifndef NB_WAVES
@@ -1374,8 +1375,12 @@ __device__ __forceinline__ int locate_cell(const DInst *__restrict__ I, int nins
 // instances, numbered by the prefix that k_md_decide writes after the gates;
 // the grid covers all real cells and the workgroups past the gated ones leave
 // at once (gated-out instances cost a launch of empty workgroups, no more).
-// The busy workgroups are remapped so that each XCD builds a contiguous run
-// of cells, whose halos then stay in its L2.  A wave decodes its first cell
+// The busy workgroups are remapped so that each XCD builds runs of consecutive
+// cells, whose halos then stay in its L2; short ones (2^NB_XS workgroups),
+// because a slab's vacuum is empty cells: with an eighth of the box for each
+// XCD, one of them builds a 40 x 40 x 12 slab under 540 A of vacuum alone
+// (398 us, in runs of 16 workgroups 109; 2.1 M atoms without vacuum 728 and
+// 742).  A wave decodes its first cell
 // once and steps through the rest in x-fastest order.  A list longer than
 // its width is cut; the longest goes to the instance's record, and in MD-step
 // mode (under a gate) the rest of the step halts until the host has grown
@@ -1407,7 +1412,7 @@ void k_nbuild(
   constexpr int CPB = NB_WAVES * NBC;  // cells per workgroup
   const int nbusy = (ncell + CPB - 1) / CPB;
   if (block >= nbusy) return;
-  const int c0 = xcd_remap(block, nbusy) * CPB + w * NBC;
+  const int c0 = xcd_remap(block, nbusy, NB_XS) * CPB + w * NBC;
   const int c1 = min(ncell, c0 + NBC);
   const int lane = threadIdx.x % FIB_WAVE;
   const int sd0 = lane % 3 - 1, sd1 = (lane / 3) % 3 - 1, sd2 = lane / 9 - 1;
