@@ -120,14 +120,24 @@ struct HostPart {
 // 2.1 M atoms: set_state 3.4 -> 1.9 ms (and no allocations), forces 7.0 ->
 // 3.3 ms, state 14.6 -> 5.3 ms; 4 k atoms: set_state 88 -> 43 us.
 struct Stage {
-  static constexpr size_t SMALL = 256u << 10, CHUNK = 2u << 20;
+  static constexpr size_t SMALL = 256u << 10, CHUNK_MAX = 2u << 20;
   static constexpr int LANES = 4;
+  size_t chunk = CHUNK_MAX, least = SMALL;  // see fit()
   int device = 0;
   char *dev = nullptr, *pin = nullptr;
   size_t dev_cap = 0;
   std::vector<char> row;           // of a small call
   hipEvent_t ev[LANES] = {};       // the lane's copy has ended
 
+  // Sizes for a handle whose largest instance has n atoms: forces and energies
+  // fill the lanes' chunks once (pinned memory is slow to come by, 0.3 ms per
+  // MiB on its first use), and the first buffer holds them, so that calls for
+  // them after a smaller first call do not allocate again.
+  void fit(size_t n) {
+    const size_t set = n * 4 * sizeof(double);
+    chunk = std::min(std::max((set / LANES + 0xffff) & ~(size_t)0xffff, SMALL), CHUNK_MAX);
+    least = set + 4096;
+  }
   // Room for a call of `bytes`; without pinned memory (pin == nullptr) the
   // copies take the caller's pages.
   hipError_t reserve(size_t bytes) {
@@ -135,14 +145,14 @@ struct Stage {
       if (dev) (void)hipFree(dev);
       dev = nullptr;
       dev_cap = 0;
-      bytes = std::max(bytes, SMALL);
-      hipError_t e = hipMalloc((void **)&dev, bytes);
+      const size_t cap = std::max(bytes, std::max(SMALL, least));
+      hipError_t e = hipMalloc((void **)&dev, cap);
       if (e != hipSuccess) return e;
-      dev_cap = bytes;
+      dev_cap = cap;
     }
     if (bytes <= SMALL) return hipSuccess;
     if (!pin &&
-        hipHostMalloc((void **)&pin, LANES * CHUNK, hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void **)&pin, LANES * chunk, hipHostMallocDefault) != hipSuccess) {
       pin = nullptr;
       (void)hipGetLastError();
     }
@@ -178,8 +188,8 @@ struct Stage {
     if (total <= SMALL) return copy_row(up, parts, total, s);
     std::vector<HostPart> ch;
     for (const HostPart &q : parts)
-      for (size_t o = 0; o < q.bytes; o += CHUNK)
-        ch.push_back({q.off + o, std::min(CHUNK, q.bytes - o), (char *)q.host + o});
+      for (size_t o = 0; o < q.bytes; o += chunk)
+        ch.push_back({q.off + o, std::min(chunk, q.bytes - o), (char *)q.host + o});
     std::atomic<int> bad{(int)hipSuccess};
     auto lane = [&](int w) {
       hipError_t e = hipSetDevice(device);
@@ -225,7 +235,7 @@ struct Stage {
   }
   // lane w takes chunks w, w + LANES, ..., through its pinned one
   hipError_t lane_up(int w, const std::vector<HostPart> &ch, hipStream_t s) {
-    char *const slot = pin + (size_t)w * CHUNK;
+    char *const slot = pin + (size_t)w * chunk;
     hipError_t e = hipSuccess;
     for (size_t c = w; e == hipSuccess && c < ch.size(); c += LANES) {
       if (c >= LANES) e = hipEventSynchronize(ev[w]);
@@ -237,7 +247,7 @@ struct Stage {
     return e;
   }
   hipError_t lane_back(int w, const std::vector<HostPart> &ch, hipStream_t s) {
-    char *const slot = pin + (size_t)w * CHUNK;
+    char *const slot = pin + (size_t)w * chunk;
     hipError_t e = hipSuccess;
     for (size_t c = w; e == hipSuccess && c < ch.size(); c += LANES) {
       e = hipMemcpyAsync(slot, dev + ch[c].off, ch[c].bytes, hipMemcpyDeviceToHost, s);
@@ -653,6 +663,7 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
   for (const DInst &in : h->inst) {
     d.max_pad = std::max(d.max_pad, in.natm_pad);
     d.max_bucket = std::max(d.max_bucket, in.nbucket);
+    h->stage.fit((size_t)d.max_pad);
     d.max_cell = std::max(d.max_cell, in.h[0] * in.h[1] * in.h[2]);
   }
   ALLOC(d.fin_tmp, (size_t)ninst * (d.max_pad / FIB_BLOCK / FIB_FIN_CH + 1) * FIB_NRED);
