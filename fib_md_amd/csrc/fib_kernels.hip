@@ -2052,7 +2052,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
   // (A Ga atom lists some forty partners, and its lane used to work them off
   // alone, two dependent loads and a few hundred instructions each, while the
   // rest of the pass had long ended: k_legs of 64 x 4 k atoms, mixed, 59.3 ->
-  // 34.4 us; of one 4 k slab, FP64, 37.8 -> 20.7.)
+  // 32.6 us; of one 4 k slab, FP64, 37.8 -> 18.)
   const bool fired = !(ti == 3 && orig_of(xi) >= in.nsg + in.impact);
   const int ci = live && fired ? min(nion, Wion) : 0;
   const uint64_t rows = __ballot(ci > 0);
@@ -2086,17 +2086,18 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
       const bool hit =
           p < np &&
           moliere(xo, to, nbr_ion[(size_t)(i - lane + own) * Wion + k], v, ul);
-      const uint64_t hits = __ballot(hit);
+      // (a pair out of range adds zeros: the sums are the same, and their
+      // values come from LDS several at a time)
       wave_lds_sync();
-      if (hit) {
+      if (p < np) {
 #pragma unroll
-        for (int c = 0; c < (VIR ? 7 : 4); ++c) sv[c * FIB_WAVE + lane] = v[c];
-        if (EN) su[lane] = ul;
+        for (int c = 0; c < (VIR ? 7 : 4); ++c) sv[c * FIB_WAVE + lane] = hit ? v[c] : T(0);
+        if (EN) su[lane] = hit ? ul : 0.0;
       }
       wave_lds_sync();
       const int q1 = min(first + ci - p0, FIB_WAVE);
+#pragma unroll 4
       for (int q = max(first - p0, 0); q < q1; ++q) {
-        if (!((hits >> q) & 1ull)) continue;
 #pragma unroll
         for (int c = 0; c < (VIR ? 7 : 4); ++c) v[c] = sv[c * FIB_WAVE + q];
         f.add(v[0], v[1], v[2], v[3]);
@@ -2173,6 +2174,8 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
 // -> 48.4 us, 811 k 90 -> 126).  With energies and the virial, just built:
 // 4 k atoms, FP64, 32.8 -> 17.5 us; 2 k, mixed, without the virial, 26 -> 13.
 #define TRI_SMALL 131072
+// and of up to TRI_TINY eight, about 34 legs, one pass: 4 k atoms 12.7 -> 10.5.
+#define TRI_TINY 16384
 template <bool MIXED>
 struct TriStage {
   static constexpr int N = MIXED ? TRI_NS_MIXED : TRI_NS_FP64;
@@ -3690,11 +3693,17 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
                      d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.nbr_sw, d.rk_sw, d.off_sw, d.amask,  \
                      (typename GRec<MIXED, EN>::type *)d.G, d.RA, d.F[1 - d.cur],             \
                      d.V[1 - d.cur], d.pstride, d.partials + (size_t)FIB_NRED * d.pstride,    \
-                     d.binst, d.halt, xcd_shift(d) + (APW_ == 16 ? 2 : 0))
+                     d.binst, d.halt, xcd_shift(d) + (APW_ == 8 ? 3 : APW_ == 16 ? 2 : 0))
     // (the mixed mode's virial is summed in FP32 over runs of a wavefront's
     // legs, which have to stay those of 64 atoms)
     if (small) {
-      TRI_LAUNCH(128, TRI_BATCH, 16);
+      // (energies: a partial sum per 64 atoms at most)
+      if constexpr (!EN && !VIR) {
+        if (d.NA <= TRI_TINY) TRI_LAUNCH(128, TRI_BATCH, 8);
+        else TRI_LAUNCH(128, TRI_BATCH, 16);
+      } else {
+        TRI_LAUNCH(128, TRI_BATCH, 16);
+      }
     } else if constexpr (EN || VIR) {
       TRI_LAUNCH(TriStage<MIXED>::N, TRI_BATCH, FIB_WAVE);
     } else {

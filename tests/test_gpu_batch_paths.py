@@ -3,7 +3,7 @@ whatever reductions the batch takes: one workgroup per instance sorts up to
 8,192 atoms and cells (k_sort_small), the scans and scatters sort more; up to
 eight instances of at most 65,536 atoms are reduced where the next kernel
 decides, more of them by a launch of their own, larger ones in chunks; small
-batches have 16 atoms per wavefront in the vertex pass, large ones 64."""
+batches have eight or 16 atoms per wavefront in the vertex pass, large ones 64."""
 import numpy as np
 import pytest
 
