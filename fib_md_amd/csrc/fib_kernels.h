@@ -34,7 +34,7 @@ enum KKey {
   KT_BIN = 0,   // k_bin
   KT_SORT,      // scan, scatter, fixup, reorder
   KT_NBUILD,    // k_nbuild
-  KT_LISTAUX,   // k_clear_counts, k_maxcnt
+  KT_LISTAUX,   // (no kernel left)
   KT_LEGS,      // k_legs
   KT_TRI,       // k_tri
   KT_GATHER,    // k_force3

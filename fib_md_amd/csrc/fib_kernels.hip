@@ -1,33 +1,42 @@
 // fib_kernels.hip -- gfx950 kernels of the FIB_MD force-and-integrate path.
 //
-// Pipeline per neighbor rebuild (replaces si_nlist, si.f90:87-276):
-//   k_bin       cell of every atom with the reference's FP64 arithmetic
-//               (nlist.f90:29), atomic histogram per cell bucket
-//   k_scan_*    exclusive scan of the bucket histogram
-//   k_scatter   counting-sort scatter; k_fixup restores a deterministic
-//               order inside each bucket (old sorted position)
-//   k_reorder   gathers every per-atom array into cell order
-//   k_nbuild    one wavefront per cell: the 27-cell halo is staged in LDS,
-//               the reference pair predicate (si.f90:156-170) is evaluated
-//               lane-parallel and survivors are compacted with ballots
+// Pipeline per neighbor rebuild (replaces si_nlist, si.f90:87-276), three to
+// seven launches:
+//   k_sort_small  the sort of instances of up to 8,192 atoms and cells, each by
+//                 one workgroup; of larger ones:
+//   k_bin         cell of every atom with the reference's FP64 arithmetic
+//                 (nlist.f90:29), atomic histogram per cell bucket
+//   k_scan_*      exclusive scan of the bucket histogram in two passes
+//   k_scatter     counting-sort scatter; k_fixup restores a deterministic
+//                 order inside each bucket (old sorted position)
+//   k_reorder     gathers every per-atom array into cell order and resets
+//                 what a build resets
+//   k_nbuild      one wavefront per cell: the 27-cell halo filtered by the box
+//                 around the cell's atoms, the reference pair predicate
+//                 (si.f90:156-170) lane-parallel, survivors compacted with
+//                 ballots; beside it the copy back of the in-place sort
 // Per force evaluation (replaces si_force, si.f90:384-552):
-//   k_legs      one thread per atom: SW pair and Moliere forces in registers,
-//               the atom's three-body legs to the leg arrays
-//   k_tri       one lane per leg, legs staged in LDS: the vertex terms
-//               centred on the leg's atom, force on the leg's neighbour into
-//               G, and where the neighbour keeps its force on the atom (RA)
-//   k_extra     vertex terms of the stale build-time triplet graph
-//   k_force3    one thread per atom: own terms + the G entries its neighbours
-//               wrote for it; the velocity update of either integrator
+//   k_legs        one thread per atom: SW pair and Moliere forces in registers
+//                 and which pairs are three-body legs; from the rows right
+//                 after a build, from the near lists it then keeps later on
+//   k_tri         one lane per leg, legs staged in LDS: the vertex terms
+//                 centred on the leg's atom, force on the leg's neighbour into
+//                 G, where the neighbour keeps its force on the atom (RA), and
+//                 the reaction on the centre
+//   k_extra       vertex terms of the stale build-time triplet graph
+//   k_force3      one thread per atom: own terms + the G entries its neighbours
+//                 wrote for it; the velocity update of either integrator
 // Per step (replaces the inline Verlet of onestep, timeint.f90:165-236):
-//   k_pos       thermostat scaling, position update, side freeze, rebox and
-//               the sputter-layer rules in one pass
-//   k_md_pos    the benchmark configurations' integrator (MD-step mode):
-//               shells, half kick, drift, pins, removal, displacements
+//   k_pos         thermostat scaling, position update, side freeze, rebox and
+//                 the sputter-layer rules in one pass
+//   k_md_pos      the MD-step mode's integrator: shells, half kick, drift,
+//                 pins, removal, displacements
+//   k_md_decide   which instances rebuild, and what removed atoms carry out
+//   k_md_ctl      the next dt
 //
-// Reductions (energy, virial, thermostat sums, max KE) use per-block
-// partials; the last block of an instance sums them in block order, so every
-// result is deterministic.
+// Reductions (energy, virial, thermostat sums, max KE) use per-block partials,
+// which a wavefront per 256 blocks sums in a fixed order, so every result is
+// deterministic.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -1462,23 +1471,23 @@ __device__ __forceinline__ int nth_bit(uint64_t m, int n) {
 // ---------------------------------------------------------------------------
 // Force evaluation in three passes, no atomics.
 //
-// k_legs (one thread per atom): the atom's buffered SW list is scanned once.
-// Pairs inside the pair-force range add the SW pair force (and the ion list
-// the Moliere pairs) to the atom in registers.  Pairs inside the three-body
-// range are the atom's "legs": unit vector, E = exp(gamma/(r/sigma - a)),
-// d ln E/dr, 1/r and the neighbour's index go to the leg arrays, slot-major
-// by compact leg index n ([n * NA + i]), legs in list-slot order.
+// k_legs (one thread per atom): the atom's buffered SW list, or its near list,
+// is scanned once.  Pairs inside the pair-force range add the SW pair force
+// (and the ion list the Moliere pairs) to the atom in registers.  Pairs inside
+// the three-body range are the atom's "legs": a bit each in its leg mask, by
+// list slot.  n counts an atom's legs in list-slot order; per-leg arrays are
+// slot-major by it ([n * NA + i]).
 //
 // k_tri (one lane per leg): every vertex term centred on atom i,
 // h(a, i, b) = leps E(r_a) E(r_b) (cos + 1/3)^2, is a pair of i's legs.  The
 // lane owning leg a sums the force on a's atom over all partners b into
-// G[n(a)][i] (w: a's third of the energy).  A wavefront takes the legs of 64
+// G[n(a)][i] (w, where energies are wanted: a's third of the energy), and the
+// legs of an atom sum to the reaction on it.  A wavefront takes the legs of 64
 // atoms in turn (a prefix sum over the atoms' leg counts in LDS maps lanes to
 // legs), so atoms with many legs do not stall the others.
 //
-// k_force3 (one thread per atom): F_i = own pair/Moliere force - sum of its
-// own G row (the reaction on the centre) + the G entries its neighbours wrote
-// for it.  Neighbour c's entry for i is the leg of c in the list slot r that
+// k_force3 (one thread per atom): F_i = own pair/Moliere force + the reaction
+// on the centre + the G entries its neighbours wrote for it.  Neighbour c's entry for i is the leg of c in the list slot r that
 // holds i; its compact index is the popcount of c's leg mask below r.  r
 // follows from the stencil offsets the list build stores (see k_nbuild); k_tri
 // works the index out per leg and leaves it in RA, so k_force3 makes one
@@ -3685,7 +3694,8 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
     // in the default tile
     const int ns = (EN || VIR || !d.tri_ns) ? TriStage<MIXED>::N : d.tri_ns;
     const int tb = (EN || VIR || !d.tri_tb) ? TRI_BATCH : d.tri_tb;
-    const bool small = !(MIXED && VIR) && d.NA <= TRI_SMALL && !d.tri_ns && !d.tri_tb;
+    const bool small = !(MIXED && VIR) && d.NA <= TRI_SMALL && ns == TriStage<MIXED>::N &&
+                       tb == TRI_BATCH;  // (another tile was asked for otherwise)
     if (small) tri_bs = 4 * 16;
 #define TRI_LAUNCH(NS_, TB_, APW_)                                                            \
   hipLaunchKernelGGL((k_tri<MIXED, EN, VIR, NS_, TB_, APW_>),                                 \
