@@ -109,20 +109,23 @@ struct HostPart {
 // than SMALL bytes, LANES pinned chunks.
 //
 // A small call's arrays go as one copy, from or to a row of host memory: a
-// copy costs 10 us whatever it moves, and pinned memory would gain 1 us in 11
-// for 64 KiB and cost 100 us on the first call.  A large call's arrays go in
-// chunks through LANES lanes, a host thread and a pinned chunk each, so that
-// the lanes empty or fill theirs while another's is on the bus.  One thread
-// moves 25 GB/s between warm pages and pinned memory and 12 into pages that
-// the caller has not touched yet, the bus 55, and every copy costs some 20 us
-// on its stream: chunks of 512 KiB take 3.2 ms for 56 MB, of 1 MiB 2.3, of
-// 2 MiB 1.9, of 4 MiB 1.8; six lanes or a stream per lane gain 2 to 7 %.
-// 2.1 M atoms: set_state 3.4 -> 1.9 ms (and no allocations), forces 7.0 ->
-// 3.3 ms, state 14.6 -> 5.3 ms; 4 k atoms: set_state 88 -> 43 us.
+// copy costs 10 us whatever it moves, pinned memory would gain 1 us in 11 for
+// 64 KiB and cost 100 us on the first call, and the lanes' threads cost 30 us
+// or more each (X, V, Xi and the types of 4 k, 12 k, 28 k and 100 k atoms: one
+// copy 53, 101, 201 and 595 us, lanes 117, 194, 240 and 640).  A large call's
+// arrays go in chunks through LANES lanes, a host thread and a pinned chunk
+// each, so that the lanes empty or fill theirs while another's is on the bus.
+// One thread moves 25 GB/s between warm pages and pinned memory and 12 into
+// pages that the caller has not touched yet, the bus 55, and every copy costs
+// some 20 us on its stream: chunks of 512 KiB take 3.2 ms for 56 MB, of 1 MiB
+// 2.3, of 2 MiB 1.9, of 4 MiB 1.8; six lanes or a stream per lane gain 2 to
+// 7 %.  2.1 M atoms: set_state 3.4 -> 1.9 ms (and no allocations), forces 7.0
+// -> 3.3 ms, state 14.6 -> 5.3 ms; 4 k atoms: set_state 88 -> 43 us.
 struct Stage {
-  static constexpr size_t SMALL = 256u << 10, CHUNK_MAX = 2u << 20;
+  static constexpr size_t SMALL = 2u << 20, CHUNK_MIN = 256u << 10,
+                          CHUNK_MAX = 2u << 20;
   static constexpr int LANES = 4;
-  size_t chunk = CHUNK_MAX, least = SMALL;  // see fit()
+  size_t chunk = CHUNK_MAX, least = 0;  // see fit()
   int device = 0;
   char *dev = nullptr, *pin = nullptr;
   size_t dev_cap = 0;
@@ -135,7 +138,7 @@ struct Stage {
   // them after a smaller first call do not allocate again.
   void fit(size_t n) {
     const size_t set = n * 4 * sizeof(double);
-    chunk = std::min(std::max((set / LANES + 0xffff) & ~(size_t)0xffff, SMALL), CHUNK_MAX);
+    chunk = std::min(std::max((set / LANES + 0xffff) & ~(size_t)0xffff, CHUNK_MIN), CHUNK_MAX);
     least = set + 4096;
   }
   // Room for a call of `bytes`; without pinned memory (pin == nullptr) the
@@ -145,7 +148,7 @@ struct Stage {
       if (dev) (void)hipFree(dev);
       dev = nullptr;
       dev_cap = 0;
-      const size_t cap = std::max(bytes, std::max(SMALL, least));
+      const size_t cap = std::max(bytes, std::max(CHUNK_MIN, least));
       hipError_t e = hipMalloc((void **)&dev, cap);
       if (e != hipSuccess) return e;
       dev_cap = cap;
@@ -223,7 +226,7 @@ struct Stage {
     return hipStreamSynchronize(s);
   }
   hipError_t copy_row(bool up, const std::vector<HostPart> &parts, size_t total, hipStream_t s) {
-    row.resize(SMALL);
+    row.resize(std::max(row.size(), total));
     if (up)
       for (const HostPart &q : parts) std::memcpy(row.data() + q.off, q.host, q.bytes);
     hipError_t e = up ? hipMemcpyAsync(dev, row.data(), total, hipMemcpyHostToDevice, s)

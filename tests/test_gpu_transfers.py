@@ -1,5 +1,5 @@
-"""Host transfers at the sizes where their path changes: one copy up to 256 KiB,
-then chunks of 2 MiB through up to four lanes; the arrays are given
+"""Host transfers at the sizes where their path changes: one copy up to 2 MiB,
+then chunks of 256 KiB to 2 MiB through up to four lanes; the arrays are given
 back bit for bit, on a handle used for the first time, reused, and from two
 threads with a handle each."""
 import threading
@@ -28,10 +28,10 @@ def _round_trip(g, n, seed, inst=0, with_v=True):
     np.testing.assert_array_equal(gF, np.zeros_like(V))
 
 
-# 3,638 and 3,641 atoms: 72 B each, either side of 256 KiB in state(); 3,276
-# and 3,277: 80 B in set_state; 87,382: X just over one chunk; 262,144: whole
-# chunks, more of them than lanes
-@pytest.mark.parametrize("n", [1, 3276, 3277, 3638, 3641, 87381, 87382, 262144, 300007])
+# 29,127 and 29,130 atoms: 72 B each, either side of 2 MiB in state(); 26,214
+# and 26,215: 80 B in set_state; 349,525 and 349,526: X of whole chunks and one
+# more atom; 262,144: more chunks than lanes
+@pytest.mark.parametrize("n", [1, 3277, 26214, 26215, 29127, 29130, 87382, 262144, 349525, 349526])
 def test_round_trip(n):
     from fib_md_amd import FibGPU
     print(n, flush=True)
