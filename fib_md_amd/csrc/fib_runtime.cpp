@@ -132,13 +132,13 @@ struct Stage {
   std::vector<char> row;           // of a small call
   hipEvent_t ev[LANES] = {};       // the lane's copy has ended
 
-  // Sizes for a handle whose largest instance has n atoms: forces and energies
-  // fill the lanes' chunks once (pinned memory is slow to come by, 0.3 ms per
-  // MiB on its first use), and the first buffer holds them, so that calls for
-  // them after a smaller first call do not allocate again.
+  // Sizes for a handle whose largest instance has n atoms.  Two chunks hold an
+  // (n,3) array: pinned memory is slow to come by, 0.3 ms per MiB on its first
+  // use.  The first buffer holds forces and energies, so that calls for them
+  // after a smaller first call do not allocate again.
   void fit(size_t n) {
     const size_t set = n * 4 * sizeof(double);
-    chunk = std::min(std::max((set / LANES + 0xffff) & ~(size_t)0xffff, CHUNK_MIN), CHUNK_MAX);
+    chunk = std::min(std::max((set * 3 / 8 + 0xffff) & ~(size_t)0xffff, CHUNK_MIN), CHUNK_MAX);
     least = set + 4096;
   }
   // Room for a call of `bytes`; without pinned memory (pin == nullptr) the
