@@ -119,7 +119,7 @@ struct DCtl {
   double e_bath_step;   // the bath and removal terms of the last step (k_md_ctl
   double e_out_step;    // adds them in)
   int32_t nonfinite;    // set by k_bin on a NaN/Inf position
-  int32_t extra_any;    // k_extra found vertex terms outside a centre's list
+  int32_t extra_any;    // extra_pass found vertex terms outside a centre's list
   int32_t overflow;     // a neighbour list exceeded its width (sticky)
   int32_t near_off;     // too many movers: no near lists until the next build
   int32_t reserved;

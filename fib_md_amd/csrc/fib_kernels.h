@@ -38,7 +38,7 @@ enum KKey {
   KT_LEGS,      // k_legs
   KT_TRI,       // k_tri
   KT_GATHER,    // k_force3
-  KT_EXTRA,     // k_extra
+  KT_EXTRA,     // (none: extra_pass runs in k_tri's launch)
   KT_POS,       // k_pos
   KT_REDUCE,    // k_finalize, k_sums
   KT_IO,        // import / export / set-atom / cell-id kernels

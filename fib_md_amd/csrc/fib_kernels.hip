@@ -23,7 +23,8 @@
 //                 centred on the leg's atom, force on the leg's neighbour into
 //                 G, where the neighbour keeps its force on the atom (RA), and
 //                 the reaction on the centre
-//   k_extra       vertex terms of the stale build-time triplet graph
+//     extra_pass  in the same launch: vertex terms of the stale build-time
+//                 triplet graph
 //   k_force3      one thread per atom: own terms + the G entries its neighbours
 //                 wrote for it; the velocity update of either integrator
 // Per step (replaces the inline Verlet of onestep, timeint.f90:165-236):
@@ -375,7 +376,7 @@ __device__ __forceinline__ void fin_chunk(double (&x)[NV], const DInst &in, int 
   fin_wave<NV>(x, rs);
 }
 // slot k of it, a sum over the regions of k_legs, k_tri (rs.sub blocks for one
-// of the others') and k_extra
+// of the others') and extra_pass
 __device__ __forceinline__ double fin_chunk_slot(int k, const DInst &in, int c,
                                                  const double *__restrict__ partials, int pstride,
                                                  const RedSpec &rs) {
@@ -2140,6 +2141,197 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
 }
 
 
+// ---------------------------------------------------------------------------
+// Vertex terms of the build-time graph that the centre's own list misses.
+//
+// The reference stores its triplets once per list build (si.f90:191-232):
+// every connected triple of the buffered graph.  Between builds the vertex
+// term centred on c with legs a and b is evaluated whenever both legs are in
+// range *now* (si.f90:491-509), so after atoms have moved more than the list
+// skin a term can exist whose leg c-a is not a listed pair, the triple being
+// connected through the pairs c-b and b-a instead.  k_legs/k_tri only pair
+// legs from c's own list; this pass adds the rest, exactly and without
+// atomics: the term (a, c, b) is found by the bridge atom b, which lists both
+// a and c.  b keeps its own share and writes the forces on a and c into
+// EX[slot][b] by its list slots of a and c; a and c gather them like G.
+// Nothing can be missing unless two atoms moved together by more than the
+// skin, so the pass exits at once while maxdisp + maxdisp2 <= skin.  Further
+// workgroups of k_tri's launch do it, whose results it does not need: a launch
+// of its own cost 4.7 us even with nothing to do (fib_step of 1.9 k atoms 47
+// -> 43 us a step, of 154 k 85 -> 82).
+template <bool MIXED, bool EN, bool VIR>
+__device__ __forceinline__ void extra_pass(
+    int lb,
+    const double4 *__restrict__ X, const DInst *__restrict__ I, const FConst fc, int NA, int Wsw,
+    const int *__restrict__ cnt_sw, const int *__restrict__ nbr_sw,
+    const uint64_t *__restrict__ amask,
+    const float *__restrict__ disp, DCtl *__restrict__ ctl, typename Prec<MIXED>::T4 *__restrict__ EX,
+    typename Prec<MIXED>::T4 *__restrict__ EXself, uint64_t *__restrict__ exmask, int pstride,
+    double *__restrict__ partials, const uint8_t *__restrict__ nst) {
+  typedef typename Prec<MIXED>::T T;
+  typedef typename Prec<MIXED>::T4 T4;
+  const int b = lb * FIB_BLOCK + threadIdx.x;
+  const double4 xb = X[b];
+  const uint32_t mb = meta_of(xb);
+  const int kin = __builtin_amdgcn_readfirstlane(inst_of(mb));
+  const DInst &in = I[kin];
+  const double isgS = fc.isig[0][0];
+  const double fscale = MIXED ? fc.eps[0][0] * isgS : 1.0;
+  const double escale = MIXED ? fc.eps[0][0] : 1.0;
+  const double lscale = MIXED ? 1.0 / isgS : 1.0;
+  double v[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  const int op[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+  // block-uniform: one instance per block
+  const bool active = ctl[kin].maxdisp + ctl[kin].maxdisp2 > fc.skin;
+  if (!active) {
+    // nothing to add: clear the instance's flag so the gather skips EX
+    if (threadIdx.x == 0 && lb * FIB_BLOCK == in.atom_off) ctl[kin].extra_any = 0;
+    if (EN || VIR) block_partials<10, FIB_BLOCK>(v, op, lb, pstride, partials);
+    return;
+  }
+  const bool live = !(mb & (META_PAD | META_DEAD));
+  const int tb = type_of(mb);
+  const double lu = MIXED ? 1.0 / fc.eps[0][0] : 1.0;
+  const T lp[4] = {(T)(fc.leps[0][0][0] * lu), (T)(fc.leps[0][0][1] * lu),
+                   (T)(fc.leps[0][1][1] * lu), (T)(fc.leps[1][1][1] * lu)};
+  const float skin = (float)fc.skin;
+  uint64_t em = 0;
+  double fb0 = 0, fb1 = 0, fb2 = 0;
+  T ub = 0, et = 0;
+  T W[9];
+#pragma unroll
+  for (int w = 0; w < 9; ++w) W[w] = 0;
+  // An atom with a near list has no partner that moved more than delta / 2
+  // (see near_mark_moved), so no two of its partners moved by the skin.  The
+  // others look at their partners' displacements first: in most wavefronts
+  // no atom has one of more than half the skin.  (Without the two checks the
+  // pass took 37 to 49 us for 5.8 k atoms of a fib_step call, a serial chain
+  // of gathers per pair.)
+  const bool moved = !nst || ctl[kin].near_off || nst[b] > NEAR_CAP;
+  if (live && tb < 3 && moved) {
+    const int cs = min(cnt_sw[b], Wsw);
+    const int *rowb = nbr_sw + (size_t)b * Wsw;
+    const uint64_t amb = amask[b];
+    // of the two, one moved more than half the skin
+    uint64_t far = 0;
+    for (int k0 = 0; k0 < cs; k0 += 4) {
+      float dk[4];
+#pragma unroll
+      for (int v = 0; v < 4; ++v) dk[v] = k0 + v < cs ? disp[rowb[k0 + v]] : 0.0f;
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (dk[v] > 0.4999f * skin) far |= 1ull << (k0 + v);
+    }
+    const int na = far ? __popcll(amb) : 0;
+    for (int n = 0; n < na; ++n) {
+      const int kc = nth_bit(amb, n);  // b's list slot of c
+      const int c = rowb[kc];
+      const float dc = disp[c];
+      const bool cfar = (far >> kc) & 1ull;
+      const double4 xc = X[c];
+      const int tc = type_of(meta_of(xc));
+      Leg<T> Lbc;  // b's leg to c: unit vector from c to b
+      make_leg<MIXED>(xb, xc, in, fc, tb, tc, Lbc);
+      const int *rowc = nbr_sw + (size_t)c * Wsw;
+      const int cc = min(cnt_sw[c], Wsw);
+      for (int k = 0; k < cs; ++k) {
+        if (!cfar && !((far >> k) & 1ull)) continue;
+        const int a = rowb[k];
+        if (a == c || !(disp[a] + dc > skin)) continue;
+        const double4 xa = X[a];
+        const int ta = type_of(meta_of(xa));
+        // leg c -> a: d = x_c - x_a (unit vector from a to the centre c)
+        double d0, d1, d2;
+        min_image_fast(xc, xa, in, d0, d1, d2);
+        const double isg = fc.isig[(tc == 2) ? 1 : 0][(ta == 2) ? 1 : 0];
+        const double s0 = MIXED ? d0 * isg : d0, s1 = MIXED ? d1 * isg : d1,
+                     s2 = MIXED ? d2 * isg : d2;
+        const double rr = s0 * s0 + s1 * s1 + s2 * s2;
+        if (MIXED && !(rr < fc.cut_sw2)) continue;
+        const double r = sqrt(rr);
+        if (!((MIXED ? r : r * isg) < (MIXED ? fc.mixed_xleg : fc.cut_sw))) continue;
+        bool listed = false;
+        for (int q = 0; q < cc; ++q) listed |= (rowc[q] == a);
+        if (listed) continue;
+        Leg<T> Lca;
+        leg_values<MIXED>(d0, d1, d2, isg, fc.rho[(tc == 2) ? 1 : 0][(ta == 2) ? 1 : 0], fc, Lca);
+        // leg c -> b is b's leg to c, reversed
+        Leg<T> Lcb = Lbc;
+        Lcb.e0 = -Lbc.e0; Lcb.e1 = -Lbc.e1; Lcb.e2 = -Lbc.e2;
+        Lcb.l0 = -Lbc.l0; Lcb.l1 = -Lbc.l1; Lcb.l2 = -Lbc.l2;
+        const int nge = (tc == 2) + (ta == 2) + (tb == 2);
+        T Fa[3], Fb[3], hh, cosv, D;
+        cos_d(Lca, Lcb, cosv, D);
+        // vterm gives the force on its first leg: once per end
+        vterm<T>(pick4(lp, nge), Lca, Lcb, cosv, D, Fa, hh);
+        vterm<T>(pick4(lp, nge), Lcb, Lca, cosv, D, Fb, hh);
+        const T Fc0 = -(Fa[0] + Fb[0]), Fc1 = -(Fa[1] + Fb[1]), Fc2 = -(Fa[2] + Fb[2]);
+        fb0 += (double)Fb[0]; fb1 += (double)Fb[1]; fb2 += (double)Fb[2];
+        const T third = hh * T(1.0 / 3.0);
+        // forces on a (slot k) and c (slot kc) for them to gather
+        const uint64_t bits[2] = {1ull << k, 1ull << kc};
+        const int slots[2] = {k, kc};
+        const T fx[2] = {Fa[0], Fc0}, fy[2] = {Fa[1], Fc1}, fz[2] = {Fa[2], Fc2};
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const size_t at = (size_t)slots[e] * NA + b;
+          T4 g;
+          if (em & bits[e]) {
+            g = EX[at];
+          } else {
+            g.x = g.y = g.z = g.w = T(0);
+          }
+          g.x += fx[e]; g.y += fy[e]; g.z += fz[e]; g.w += third;
+          EX[at] = g;
+          em |= bits[e];
+        }
+        ub += third;
+        et += hh;
+        if (VIR) {
+          // relative to the centre: r_a = x_a - x_c = -e_ca / rinv_ca, same for b
+          const T ra = -T(1) / Lca.rinv, rb = -T(1) / Lcb.rinv;
+          const T a0 = ra * Lca.e0, a1 = ra * Lca.e1, a2 = ra * Lca.e2;
+          const T b0 = rb * Lcb.e0, b1 = rb * Lcb.e1, b2 = rb * Lcb.e2;
+          W[0] += a0 * Fa[0] + b0 * Fb[0]; W[1] += a0 * Fa[1] + b0 * Fb[1];
+          W[2] += a0 * Fa[2] + b0 * Fb[2]; W[3] += a1 * Fa[0] + b1 * Fb[0];
+          W[4] += a1 * Fa[1] + b1 * Fb[1]; W[5] += a1 * Fa[2] + b1 * Fb[2];
+          W[6] += a2 * Fa[0] + b2 * Fb[0]; W[7] += a2 * Fa[1] + b2 * Fb[1];
+          W[8] += a2 * Fa[2] + b2 * Fb[2];
+        }
+      }
+    }
+  }
+  exmask[b] = em;
+  {
+    T4 g;
+    g.x = (T)fb0; g.y = (T)fb1; g.z = (T)fb2; g.w = ub;
+    EXself[b] = g;
+  }
+  if (em) {
+    // rare: only after atoms outran the list skin (global atomic, vector memory)
+    __hip_atomic_fetch_or(&ctl[kin].extra_any, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (EN || VIR) {
+    v[0] = (double)et * escale;
+    const double ws = MIXED ? fscale * lscale : 1.0;
+#pragma unroll
+    for (int w = 0; w < 9; ++w) v[1 + w] = (double)W[w] * ws;
+    block_partials<10, FIB_BLOCK>(v, op, lb, pstride, partials);
+  }
+}
+
+// What k_tri's further workgroups need for it (blocks of FIB_BLOCK atoms; 0:
+// none).
+struct ExtraArgs {
+  int blocks;
+  const int *cnt_sw;
+  const float *disp;
+  DCtl *ctl;
+  void *EX, *EXself;
+  uint64_t *exmask;
+  const uint8_t *nst;
+};
+
 // Lane-per-leg three-body pass.  Block = 4 independent wavefronts, each
 // owning 64 consecutive atoms, whose legs (the pairs of their leg masks) it
 // takes in passes of whole atoms with at most 64 legs: one lane computes one
@@ -2189,7 +2381,7 @@ template <bool MIXED>
 struct TriStage {
   static constexpr int N = MIXED ? TRI_NS_MIXED : TRI_NS_FP64;
 };
-template <bool MIXED, bool EN, bool VIR, int NS, int TB, int APW>
+template <bool MIXED, bool EN, bool VIR, int NS, int TB, int APW, bool XT>
 __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
     const double4 *__restrict__ X, const DInst *__restrict__ I, const FConst fc, int NA,
     int Wsw, const int *__restrict__ nbr_sw, uint16_t *__restrict__ rk_sw,
@@ -2197,7 +2389,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
     typename GRec<MIXED, EN>::type *__restrict__ G, uint32_t *__restrict__ RA,
     double *__restrict__ Gown, double *__restrict__ Gown_u, int pstride,
     double *__restrict__ partials, const int *__restrict__ binst, const int *__restrict__ halt,
-    int xs) {
+    int xs, const ExtraArgs xa) {
   typedef typename Prec<MIXED>::T T;
   typedef typename Prec<MIXED>::T4 T4;
   typedef typename GRec<MIXED, EN>::type GV;
@@ -2211,7 +2403,18 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
   __shared__ uint32_t sR[NW][FL];
   constexpr int TAB = VIR ? TRI_TAB_VIR : TRI_TAB;
   __shared__ uint16_t tab[NW][TAB];  // owner lane | list slot << 6
-  const int lb = xcd_remap(blockIdx.x, gridDim.x, xs);
+  const int nb = XT ? (int)gridDim.x - xa.blocks : (int)gridDim.x;
+  if constexpr (XT) {
+    if ((int)blockIdx.x >= nb) {
+      HALT_OR_RETURN(halt);
+      extra_pass<MIXED, EN, VIR>(xcd_remap(blockIdx.x - nb, xa.blocks), X, I, fc, NA, Wsw,
+                                 xa.cnt_sw, nbr_sw, amask, xa.disp, xa.ctl, (T4 *)xa.EX,
+                                 (T4 *)xa.EXself, xa.exmask, pstride,
+                                 partials + (size_t)FIB_NRED * pstride, xa.nst);
+      return;
+    }
+  }
+  const int lb = xcd_remap(blockIdx.x, nb, xs);
   const int lane = threadIdx.x % FIB_WAVE;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / FIB_WAVE);
   const int i0 = (lb * NW + wid) * APW;
@@ -2472,184 +2675,6 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
 }
 
 // ---------------------------------------------------------------------------
-// Vertex terms of the build-time graph that the centre's own list misses.
-//
-// The reference stores its triplets once per list build (si.f90:191-232):
-// every connected triple of the buffered graph.  Between builds the vertex
-// term centred on c with legs a and b is evaluated whenever both legs are in
-// range *now* (si.f90:491-509), so after atoms have moved more than the list
-// skin a term can exist whose leg c-a is not a listed pair, the triple being
-// connected through the pairs c-b and b-a instead.  k_legs/k_tri only pair
-// legs from c's own list; this pass adds the rest, exactly and without
-// atomics: the term (a, c, b) is found by the bridge atom b, which lists both
-// a and c.  b keeps its own share and writes the forces on a and c into
-// EX[slot][b] by its list slots of a and c; a and c gather them like G.
-// Nothing can be missing unless two atoms moved together by more than the
-// skin, so the pass exits at once while maxdisp + maxdisp2 <= skin.
-template <bool MIXED, bool EN, bool VIR>
-__global__ __launch_bounds__(FIB_BLOCK) void k_extra(
-    const double4 *__restrict__ X, const DInst *__restrict__ I, const FConst fc, int NA, int Wsw,
-    const int *__restrict__ cnt_sw, const int *__restrict__ nbr_sw,
-    const uint64_t *__restrict__ amask,
-    const float *__restrict__ disp, DCtl *__restrict__ ctl, typename Prec<MIXED>::T4 *__restrict__ EX,
-    typename Prec<MIXED>::T4 *__restrict__ EXself, uint64_t *__restrict__ exmask, int pstride,
-    double *__restrict__ partials, const uint8_t *__restrict__ nst,
-    const int *__restrict__ halt) {
-  HALT_OR_RETURN(halt);
-  typedef typename Prec<MIXED>::T T;
-  typedef typename Prec<MIXED>::T4 T4;
-  const int lb = xcd_remap(blockIdx.x, gridDim.x);
-  const int b = lb * FIB_BLOCK + threadIdx.x;
-  const double4 xb = X[b];
-  const uint32_t mb = meta_of(xb);
-  const int kin = __builtin_amdgcn_readfirstlane(inst_of(mb));
-  const DInst &in = I[kin];
-  const double isgS = fc.isig[0][0];
-  const double fscale = MIXED ? fc.eps[0][0] * isgS : 1.0;
-  const double escale = MIXED ? fc.eps[0][0] : 1.0;
-  const double lscale = MIXED ? 1.0 / isgS : 1.0;
-  double v[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  const int op[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-  // block-uniform: one instance per block
-  const bool active = ctl[kin].maxdisp + ctl[kin].maxdisp2 > fc.skin;
-  if (!active) {
-    // nothing to add: clear the instance's flag so the gather skips EX
-    if (threadIdx.x == 0 && lb * FIB_BLOCK == in.atom_off) ctl[kin].extra_any = 0;
-    if (EN || VIR) block_partials<10, FIB_BLOCK>(v, op, lb, pstride, partials);
-    return;
-  }
-  const bool live = !(mb & (META_PAD | META_DEAD));
-  const int tb = type_of(mb);
-  const double lu = MIXED ? 1.0 / fc.eps[0][0] : 1.0;
-  const T lp[4] = {(T)(fc.leps[0][0][0] * lu), (T)(fc.leps[0][0][1] * lu),
-                   (T)(fc.leps[0][1][1] * lu), (T)(fc.leps[1][1][1] * lu)};
-  const float skin = (float)fc.skin;
-  uint64_t em = 0;
-  double fb0 = 0, fb1 = 0, fb2 = 0;
-  T ub = 0, et = 0;
-  T W[9];
-#pragma unroll
-  for (int w = 0; w < 9; ++w) W[w] = 0;
-  // An atom with a near list has no partner that moved more than delta / 2
-  // (see near_mark_moved), so no two of its partners moved by the skin.  The
-  // others look at their partners' displacements first: in most wavefronts
-  // no atom has one of more than half the skin.  (Without the two checks the
-  // pass took 37 to 49 us for 5.8 k atoms of a fib_step call, a serial chain
-  // of gathers per pair.)
-  const bool moved = !nst || ctl[kin].near_off || nst[b] > NEAR_CAP;
-  if (live && tb < 3 && moved) {
-    const int cs = min(cnt_sw[b], Wsw);
-    const int *rowb = nbr_sw + (size_t)b * Wsw;
-    const uint64_t amb = amask[b];
-    // of the two, one moved more than half the skin
-    uint64_t far = 0;
-    for (int k0 = 0; k0 < cs; k0 += 4) {
-      float dk[4];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) dk[v] = k0 + v < cs ? disp[rowb[k0 + v]] : 0.0f;
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (dk[v] > 0.4999f * skin) far |= 1ull << (k0 + v);
-    }
-    const int na = far ? __popcll(amb) : 0;
-    for (int n = 0; n < na; ++n) {
-      const int kc = nth_bit(amb, n);  // b's list slot of c
-      const int c = rowb[kc];
-      const float dc = disp[c];
-      const bool cfar = (far >> kc) & 1ull;
-      const double4 xc = X[c];
-      const int tc = type_of(meta_of(xc));
-      Leg<T> Lbc;  // b's leg to c: unit vector from c to b
-      make_leg<MIXED>(xb, xc, in, fc, tb, tc, Lbc);
-      const int *rowc = nbr_sw + (size_t)c * Wsw;
-      const int cc = min(cnt_sw[c], Wsw);
-      for (int k = 0; k < cs; ++k) {
-        if (!cfar && !((far >> k) & 1ull)) continue;
-        const int a = rowb[k];
-        if (a == c || !(disp[a] + dc > skin)) continue;
-        const double4 xa = X[a];
-        const int ta = type_of(meta_of(xa));
-        // leg c -> a: d = x_c - x_a (unit vector from a to the centre c)
-        double d0, d1, d2;
-        min_image_fast(xc, xa, in, d0, d1, d2);
-        const double isg = fc.isig[(tc == 2) ? 1 : 0][(ta == 2) ? 1 : 0];
-        const double s0 = MIXED ? d0 * isg : d0, s1 = MIXED ? d1 * isg : d1,
-                     s2 = MIXED ? d2 * isg : d2;
-        const double rr = s0 * s0 + s1 * s1 + s2 * s2;
-        if (MIXED && !(rr < fc.cut_sw2)) continue;
-        const double r = sqrt(rr);
-        if (!((MIXED ? r : r * isg) < (MIXED ? fc.mixed_xleg : fc.cut_sw))) continue;
-        bool listed = false;
-        for (int q = 0; q < cc; ++q) listed |= (rowc[q] == a);
-        if (listed) continue;
-        Leg<T> Lca;
-        leg_values<MIXED>(d0, d1, d2, isg, fc.rho[(tc == 2) ? 1 : 0][(ta == 2) ? 1 : 0], fc, Lca);
-        // leg c -> b is b's leg to c, reversed
-        Leg<T> Lcb = Lbc;
-        Lcb.e0 = -Lbc.e0; Lcb.e1 = -Lbc.e1; Lcb.e2 = -Lbc.e2;
-        Lcb.l0 = -Lbc.l0; Lcb.l1 = -Lbc.l1; Lcb.l2 = -Lbc.l2;
-        const int nge = (tc == 2) + (ta == 2) + (tb == 2);
-        T Fa[3], Fb[3], hh, cosv, D;
-        cos_d(Lca, Lcb, cosv, D);
-        // vterm gives the force on its first leg: once per end
-        vterm<T>(pick4(lp, nge), Lca, Lcb, cosv, D, Fa, hh);
-        vterm<T>(pick4(lp, nge), Lcb, Lca, cosv, D, Fb, hh);
-        const T Fc0 = -(Fa[0] + Fb[0]), Fc1 = -(Fa[1] + Fb[1]), Fc2 = -(Fa[2] + Fb[2]);
-        fb0 += (double)Fb[0]; fb1 += (double)Fb[1]; fb2 += (double)Fb[2];
-        const T third = hh * T(1.0 / 3.0);
-        // forces on a (slot k) and c (slot kc) for them to gather
-        const uint64_t bits[2] = {1ull << k, 1ull << kc};
-        const int slots[2] = {k, kc};
-        const T fx[2] = {Fa[0], Fc0}, fy[2] = {Fa[1], Fc1}, fz[2] = {Fa[2], Fc2};
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          const size_t at = (size_t)slots[e] * NA + b;
-          T4 g;
-          if (em & bits[e]) {
-            g = EX[at];
-          } else {
-            g.x = g.y = g.z = g.w = T(0);
-          }
-          g.x += fx[e]; g.y += fy[e]; g.z += fz[e]; g.w += third;
-          EX[at] = g;
-          em |= bits[e];
-        }
-        ub += third;
-        et += hh;
-        if (VIR) {
-          // relative to the centre: r_a = x_a - x_c = -e_ca / rinv_ca, same for b
-          const T ra = -T(1) / Lca.rinv, rb = -T(1) / Lcb.rinv;
-          const T a0 = ra * Lca.e0, a1 = ra * Lca.e1, a2 = ra * Lca.e2;
-          const T b0 = rb * Lcb.e0, b1 = rb * Lcb.e1, b2 = rb * Lcb.e2;
-          W[0] += a0 * Fa[0] + b0 * Fb[0]; W[1] += a0 * Fa[1] + b0 * Fb[1];
-          W[2] += a0 * Fa[2] + b0 * Fb[2]; W[3] += a1 * Fa[0] + b1 * Fb[0];
-          W[4] += a1 * Fa[1] + b1 * Fb[1]; W[5] += a1 * Fa[2] + b1 * Fb[2];
-          W[6] += a2 * Fa[0] + b2 * Fb[0]; W[7] += a2 * Fa[1] + b2 * Fb[1];
-          W[8] += a2 * Fa[2] + b2 * Fb[2];
-        }
-      }
-    }
-  }
-  exmask[b] = em;
-  {
-    T4 g;
-    g.x = (T)fb0; g.y = (T)fb1; g.z = (T)fb2; g.w = ub;
-    EXself[b] = g;
-  }
-  if (em) {
-    // rare: only after atoms outran the list skin (global atomic, vector memory)
-    __hip_atomic_fetch_or(&ctl[kin].extra_any, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  }
-  if (EN || VIR) {
-    v[0] = (double)et * escale;
-    const double ws = MIXED ? fscale * lscale : 1.0;
-#pragma unroll
-    for (int w = 0; w < 9; ++w) v[1 + w] = (double)W[w] * ws;
-    block_partials<10, FIB_BLOCK>(v, op, lb, pstride, partials);
-  }
-}
-
-// ---------------------------------------------------------------------------
 // MD-step mode: velocity Verlet with a per-instance adaptive timestep
 // dt = min(dt_max, dx_max / |v|max), all step control on the device, so one
 // step is a fixed sequence of launches that can be captured in a graph:
@@ -2660,7 +2685,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_extra(
 //                add up to more than the skin)
 //   gated build  bin / sort in place / k_nbuild (skipped on the
 //                device when the gate is 0)
-//   forces       k_legs, k_tri, k_extra, k_force3 MODE 2 (second half kick,
+//   forces       k_legs, k_tri, extra_pass, k_force3 MODE 2 (second half kick,
 //                |v|max, shell sums)
 //   k_md_ctl     time += dt, next dt, next shell factor
 __device__ __forceinline__ bool in_shell(double x, double y, double z, const DInst &in, double w) {
@@ -2957,7 +2982,7 @@ __global__ __launch_bounds__(DECIDE_T) void k_md_decide(
       const DCtl &c = ctl[k];
       const double m2 = c.nmaxdisp >= 2.0 ? c.maxdisp : fmax(c.maxdisp2, 0.0);
       g = (c.maxdisp + m2 > skin) ? 1 : 0;
-      ctl[k].maxdisp2 = m2;  // the effective second maximum, for k_extra
+      ctl[k].maxdisp2 = m2;  // the effective second maximum, for extra_pass
       // with many atoms off their near lists, telling their partners costs
       // more than the lists that are left give
       if (c.movers * 16.0 > (double)I[k].natm) ctl[k].near_off = 1;
@@ -3173,7 +3198,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_force3(
       partner(ld_nt<NT>(RA + (size_t)n * NA + i), g);
       plus(g);
     }
-    // vertex terms outside the centre's list (k_extra), when there are any
+    // vertex terms outside the centre's list (extra_pass), when there are any
     if (ctl[kin].extra_any) {
       const T4 gs = EXself[i];
       g0 += (double)gs.x; g1 += (double)gs.y; g2 += (double)gs.z;
@@ -3292,7 +3317,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_pos(double4 *__restrict__ X,
   const DInst &in = I[kin];
   const bool live = !(mi & (META_PAD | META_DEAD));
   // slots: thermostat sum, max KE, max displacement, and the displacement
-  // again as the second maximum (k_extra tests maxdisp + maxdisp2)
+  // again as the second maximum (extra_pass tests maxdisp + maxdisp2)
   double red[4] = {0.0, -1.0, 0.0, 0.0};
   if (live) {
     const int t = type_of(mi);
@@ -3697,13 +3722,23 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
     const bool small = !(MIXED && VIR) && d.NA <= TRI_SMALL && ns == TriStage<MIXED>::N &&
                        tb == TRI_BATCH;  // (another tile was asked for otherwise)
     if (small) tri_bs = 4 * 16;
+    // extra_pass runs whenever its partials are reduced (energy, virial) or
+    // stale-list terms can exist; the MD step's gate rules the latter out
+    const bool xt = EN || VIR || extra;
+    const ExtraArgs xa{xt ? d.NA / FIB_BLOCK : 0, d.cnt_sw, d.disp, d.ctl, d.EX, d.EXself,
+                       d.exmask, d.nst};
 #define TRI_LAUNCH(NS_, TB_, APW_)                                                            \
-  hipLaunchKernelGGL((k_tri<MIXED, EN, VIR, NS_, TB_, APW_>),                                 \
-                     dim3(d.NA / (FIB_BLOCK / FIB_WAVE * APW_)), dim3(FIB_BLOCK), 0, s,       \
-                     d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.nbr_sw, d.rk_sw, d.off_sw, d.amask,  \
-                     (typename GRec<MIXED, EN>::type *)d.G, d.RA, d.F[1 - d.cur],             \
-                     d.V[1 - d.cur], d.pstride, d.partials + (size_t)FIB_NRED * d.pstride,    \
-                     d.binst, d.halt, xcd_shift(d) + (APW_ == 8 ? 3 : APW_ == 16 ? 2 : 0))
+  do {                                                                                        \
+    auto *f = k_tri<MIXED, EN, VIR, NS_, TB_, APW_, true>;                                    \
+    if constexpr (!EN && !VIR)                                                                \
+      if (!xt) f = k_tri<MIXED, EN, VIR, NS_, TB_, APW_, false>;                              \
+    hipLaunchKernelGGL(                                                                       \
+        f, dim3(d.NA / (FIB_BLOCK / FIB_WAVE * APW_) + xa.blocks), dim3(FIB_BLOCK), 0, s,     \
+        d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.nbr_sw, d.rk_sw, d.off_sw, d.amask,               \
+        (typename GRec<MIXED, EN>::type *)d.G, d.RA, d.F[1 - d.cur], d.V[1 - d.cur],          \
+        d.pstride, d.partials + (size_t)FIB_NRED * d.pstride, d.binst, d.halt,                \
+        xcd_shift(d) + (APW_ == 8 ? 3 : APW_ == 16 ? 2 : 0), xa);                             \
+  } while (0)
     // (the mixed mode's virial is summed in FP32 over runs of a wavefront's
     // legs, which have to stay those of 64 atoms)
     if (small) {
@@ -3725,16 +3760,6 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
       else TRI_LAUNCH(256, 4, FIB_WAVE);
     }
 #undef TRI_LAUNCH
-  }
-  // k_extra is launched whenever its partials are reduced (energy, virial)
-  // or stale-list terms can exist; the MD step's gate rules the latter out
-  if (extra || EN || VIR) {
-    KScope ks_(d, KT_EXTRA);
-    hipLaunchKernelGGL((k_extra<MIXED, EN, VIR>), dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), 0, s,
-                       d.X[d.cur], d.I, fc, d.NA, d.Wsw, d.cnt_sw, d.nbr_sw, d.amask,
-                       d.disp, d.ctl, (T4 *)d.EX,
-                       (T4 *)d.EXself, d.exmask, d.pstride,
-                       d.partials + (size_t)2 * FIB_NRED * d.pstride, d.nst, d.halt);
   }
   if (EN || VIR) {
     int op[10], dst[10];

@@ -1256,7 +1256,7 @@ static void enqueue_md_step(fib_handle *h) {
   const bool mixed = h->prec == FIB_PREC_MIXED;
   // no stale-list pass: a step either rebuilt an instance's lists or left
   // its two largest displacements within the skin, so every pair in range
-  // is listed and k_extra would find nothing
+  // is listed and extra_pass would find nothing
   fibk::launch_force_a(d, h->fc, mixed, false, false, h->stream, false);
   fibk::launch_force_b(d, h->fc, mixed, false, 2, sa, d.F[d.cur], h->stream);
   fibk::launch_md_ctl(d, sa, h->stream);
