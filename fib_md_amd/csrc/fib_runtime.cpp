@@ -627,8 +627,13 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
   std::vector<Place> places;
   size_t bytes = 0;
   auto take = [&](auto *&ptr, size_t n) {
+    // (large arrays at 2 MiB, as allocations of their own would be: k_force3 of
+    // 4 x 512 k atoms 102.8 us, packed 104.9)
+    const size_t b = std::max<size_t>(n, 1) * sizeof(*ptr);
+    const size_t al = b >= (1u << 20) ? 2u << 20 : 256;
+    bytes = (bytes + al - 1) & ~(al - 1);
     places.push_back({(void **)&ptr, bytes});
-    bytes += (std::max<size_t>(n, 1) * sizeof(*ptr) + 255) & ~(size_t)255;
+    bytes += b;
   };
   take(d.ctl, (size_t)ninst);
   take(d.bcnt, (size_t)d.nbucket);
