@@ -455,6 +455,9 @@ __global__ __launch_bounds__(FIN_WAVES *FIB_WAVE) void k_finalize(
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / FIB_WAVE);
   const DInst &in = I[inst];
   const int nci = fin_chunks(in, rs.bs), n = min(nci - c0, per);
+  // past the chunks of this instance (the grid has those of the largest):
+  // s_x stays unwritten, and the record is another workgroup's
+  if (n <= 0) return;
   for (int q = wid; q < n * SL; q += blockDim.x / FIB_WAVE) {
     if constexpr (NV == 10) {
       const double x = fin_chunk_slot(q % SL, in, c0 + q / SL, partials, pstride, rs);
