@@ -375,8 +375,8 @@ __device__ __forceinline__ void fin_chunk(double (&x)[NV], const DInst &in, int 
   }
   fin_wave<NV>(x, rs);
 }
-// slot k of it, a sum over the regions of k_legs, k_tri (rs.sub blocks for one
-// of the others') and extra_pass
+// slot k of it, a sum over the regions of k_legs, k_tri (rs.sub partials, one
+// or four, for one of the others': see tri_partials) and extra_pass
 __device__ __forceinline__ double fin_chunk_slot(int k, const DInst &in, int c,
                                                  const double *__restrict__ partials, int pstride,
                                                  const RedSpec &rs) {
@@ -390,7 +390,8 @@ __device__ __forceinline__ double fin_chunk_slot(int k, const DInst &in, int c,
     if (b < nblk) {
       const size_t at = (size_t)(blk0 + b);
       x += p[at];
-      for (int u = 0; u < rs.sub; ++u) x += p[reg + at * rs.sub + u];
+      const double *const t = p + reg + at * rs.sub;
+      x += rs.sub == 1 ? t[0] : (t[0] + t[1]) + (t[2] + t[3]);
       x += p[2 * reg + at];
     }
   }
@@ -2357,8 +2358,9 @@ struct ExtraArgs {
 // wavefront and 300 us with one term per (leg, partner), 3,090 and 213 us
 // so; FP64 245 -> 173 us (2 x 512 k).  With the virial, its terms of a run
 // of 256 legs used to wait in 24 (FP64: 48) KiB of LDS, which left two blocks
-// to a CU; they now turn to their lanes through shuffles, and three fit:
-// 2.1 M atoms, mixed, with energies, just built: 588 -> 477 us.
+// to a CU; they now turn to their lanes through shuffles (mixed) or are summed
+// by their centre's lane from the stage (FP64), and three fit: 2.1 M atoms,
+// mixed, with energies, just built: 588 -> 477 us.
 #ifndef TRI_BATCH
 #define TRI_BATCH 4  // 4: the next pass's positions load during this one; 2: only its row entries
 #endif
@@ -2384,6 +2386,31 @@ template <bool MIXED>
 struct TriStage {
   static constexpr int N = MIXED ? TRI_NS_MIXED : TRI_NS_FP64;
 };
+// The partial sums of k_tri, one per workgroup (of 256 or 64 atoms), from each
+// lane's sums (of its own atom; mixed virial: see there): neighbouring atoms
+// first, and pairs of wavefronts here as of workgroups in fin_chunk_slot, so
+// that an instance gives the same bits whether a wavefront has 64 atoms or 16.
+template <int APW>
+__device__ __forceinline__ void tri_partials(double (&v)[10], int lb, int pstride,
+                                             double *__restrict__ partials) {
+  constexpr int NW = FIB_BLOCK / FIB_WAVE;
+  static_assert(NW == 4, "two levels");
+  const int lane = threadIdx.x % FIB_WAVE, wid = threadIdx.x / FIB_WAVE;
+  for (int o = 1; o < APW; o <<= 1) {
+#pragma unroll
+    for (int k = 0; k < 10; ++k) v[k] += __shfl_xor(v[k], o);
+  }
+  __shared__ double red[NW][10];
+  if (lane == 0)
+#pragma unroll
+    for (int k = 0; k < 10; ++k) red[wid][k] = v[k];
+  __syncthreads();
+  if (threadIdx.x < 10) {
+    const int k = threadIdx.x;
+    partials[(size_t)k * pstride + lb] = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
+  }
+}
+
 template <bool MIXED, bool EN, bool VIR, int NS, int TB, int APW, bool XT>
 __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
     const double4 *__restrict__ X, const DInst *__restrict__ I, const FConst fc, int NA,
@@ -2468,11 +2495,14 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
         const T4 g = sG[wid][q];
         GV gv;
         gv.x = g.x; gv.y = g.y; gv.z = g.z;
-        if constexpr (EN) gv.w = g.w;
+        if constexpr (EN) {
+          gv.w = g.w * T(1.0 / 3.0);
+          gu += 0.5 * (double)gv.w;
+        }
+        if (U) uc += (double)g.w;
         G[at] = gv;
         st_nt<NTS>(RA + at, sR[wid][q]);
         g0 -= (double)g.x; g1 -= (double)g.y; g2 -= (double)g.z;
-        if (EN) gu += 0.5 * (double)g.w;
       }
     }
     if (mine) {
@@ -2638,15 +2668,41 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
       }
       if (act) {
         T4 gv;
-        gv.x = Ga0; gv.y = Ga1; gv.z = Ga2; gv.w = Gu * T(1.0 / 3.0);
+        gv.x = Ga0; gv.y = Ga1; gv.z = Ga2; gv.w = Gu;
         sG[wid][P.ps - fs + lane] = gv;
         sR[wid][P.ps - fs + lane] = ra;
-        if (U) uc += (double)Gu;
       }
-      if (VIR) {
-        // r_a = x_a - x_i = -e_a / rinv_a.  Lane q % 64 sums for leg q of a
-        // run (the FP32 sums of the mixed mode then do not depend on how a
-        // run is cut into passes): the pass's values turn by its start.
+      // r_a = x_a - x_i = -e_a / rinv_a
+      if constexpr (VIR && !MIXED) {
+        // each centre sums its own legs' terms, as its energy, in leg order:
+        // the sums do not depend on how many atoms a wavefront has
+        const T rl = -T(1) / La.rinv;
+        wave_lds_sync();
+        T4 r;
+        r.x = rl * La.e0; r.y = rl * La.e1; r.z = rl * La.e2; r.w = 0;
+        sE[wid][lane] = r;
+        wave_lds_sync();
+        const int nc = lane >= P.p0 && lane < P.p1 ? nl : 0;
+        constexpr int B = 4;  // legs whose values are read together
+        for (int l = 0; __ballot(l < nc) != 0ull; l += B) {
+          T v[B][6];
+#pragma unroll
+          for (int u = 0; u < B; ++u) {
+            const int q = l + u < nc ? exc - P.ps + l + u : 0;
+            const T4 x = sE[wid][q], g = sG[wid][P.ps - fs + q];
+            v[u][0] = x.x; v[u][1] = x.y; v[u][2] = x.z;
+            v[u][3] = g.x; v[u][4] = g.y; v[u][5] = g.z;
+          }
+#pragma unroll
+          for (int u = 0; u < B; ++u)
+            if (l + u < nc)
+#pragma unroll
+              for (int c = 0; c < 9; ++c) W[c] = fma_t(v[u][c / 3], v[u][3 + c % 3], W[c]);
+        }
+      } else if constexpr (VIR) {
+        // Lane q % 64 sums for leg q of a run (the FP32 sums then do not
+        // depend on how a run is cut into passes): the pass's values turn by
+        // its start.
         const T rl = -T(1) / La.rinv;
         T v[6] = {rl * La.e0, rl * La.e1, rl * La.e2, Ga0, Ga1, Ga2};
         const int src = (lane - (P.ps - rs)) & (FIB_WAVE - 1);
@@ -2665,15 +2721,14 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
     r0 = r1;
   }
   write_out(APW);
-  if (EN || VIR) {
+  if constexpr (EN || VIR) {
     double v[10];
     // every unordered term was summed twice, as (a, b) and (b, a)
     v[0] = uc * 0.5 * escale;
     const double ws = MIXED ? fscale * lscale : 1.0;
 #pragma unroll
     for (int w = 0; w < 9; ++w) v[1 + w] = (double)W[w] * ws;
-    const int op[10] = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    block_partials<10, FIB_BLOCK>(v, op, lb, pstride, partials);
+    tri_partials<APW>(v, lb, pstride, partials);
   }
 }
 
@@ -3707,7 +3762,6 @@ void launch_cellid(const DevBufs &d, int inst, int32_t *dout, hipStream_t s) {
 
 template <bool MIXED, bool EN, bool VIR>
 static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool extra) {
-  typedef typename Prec<MIXED>::T4 T4;
   {
     KScope ks_(d, KT_LEGS);
     hipLaunchKernelGGL((k_legs<MIXED, EN, VIR>), dim3(d.NA / FIB_BLOCK), dim3(FIB_BLOCK), 0, s,
@@ -3715,16 +3769,15 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
                        d.cnt_ion, d.nbr_ion, d.amask, d.Fpart, d.upart, d.near,
                        d.nst, d.ctl, d.binst, d.pstride, d.partials, d.halt, xcd_shift(d));
   }
-  int tri_bs = FIB_BLOCK;  // atoms per workgroup, and partial sum, of k_tri
+  const bool small = !(MIXED && VIR) && d.NA <= TRI_SMALL &&
+                     (EN || VIR || ((!d.tri_ns || d.tri_ns == TriStage<MIXED>::N) &&
+                                    (!d.tri_tb || d.tri_tb == TRI_BATCH)));
   {
     KScope ks_(d, KT_TRI);
     // the MD step's variant (no energy, no virial) in every tile; the others
     // in the default tile
     const int ns = (EN || VIR || !d.tri_ns) ? TriStage<MIXED>::N : d.tri_ns;
     const int tb = (EN || VIR || !d.tri_tb) ? TRI_BATCH : d.tri_tb;
-    const bool small = !(MIXED && VIR) && d.NA <= TRI_SMALL && ns == TriStage<MIXED>::N &&
-                       tb == TRI_BATCH;  // (another tile was asked for otherwise)
-    if (small) tri_bs = 4 * 16;
     // extra_pass runs whenever its partials are reduced (energy, virial) or
     // stale-list terms can exist; the MD step's gate rules the latter out
     const bool xt = EN || VIR || extra;
@@ -3745,7 +3798,7 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
     // (the mixed mode's virial is summed in FP32 over runs of a wavefront's
     // legs, which have to stay those of 64 atoms)
     if (small) {
-      // (energies: a partial sum per 64 atoms at most)
+      // (energies: 16 atoms per wavefront at least, see tri_partials)
       if constexpr (!EN && !VIR) {
         if (d.NA <= TRI_TINY) TRI_LAUNCH(128, TRI_BATCH, 8);
         else TRI_LAUNCH(128, TRI_BATCH, 16);
@@ -3767,7 +3820,7 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
   if (EN || VIR) {
     int op[10], dst[10];
     for (int k = 0; k < 10; ++k) { op[k] = 0; dst[k] = DCTL_IDX(utot) + k; }
-    finalize(d, 10, FIB_BLOCK, op, dst, s, FIB_BLOCK / tri_bs);
+    finalize(d, 10, FIB_BLOCK, op, dst, s, small ? 4 : 1);
   }
 }
 

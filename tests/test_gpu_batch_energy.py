@@ -55,3 +55,21 @@ def test_small_instances_beside_one_of_several_chunks(precision):
         assert abs(out[k]["utot"] - own["utot"]) <= 1e-12 * abs(own["utot"])
         assert abs(epot[k] - e) <= 1e-12 * abs(e)
         assert np.abs(out[k]["virial"] - own["virial"]).max() <= 1e-11 * np.abs(own["virial"]).max()
+
+
+# beside a 4 x 4 x 4 crystal (513 atoms): a batch of up to 131,072 atoms, one
+# of more (another split of the vertex pass), and instances just below and
+# above that size themselves
+@pytest.mark.parametrize("other", [(9, 8, 7), (25, 25, 26), (26, 25, 26), (5, 5, 41)])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_energies_and_virial_have_the_bits_of_the_instance_alone(other, precision):
+    """Sums within an instance have an order that depends on it alone."""
+    systems = [_crystal((4, 4, 4), 11), _crystal(other, 12), _crystal((26, 26, 25), 13)]
+    for batch in (systems[:2], systems):
+        out, epot = _evaluate(batch, precision)
+        for k, s in enumerate(batch):
+            (own,), (e,) = _evaluate([s], precision)
+            print(f"{precision} {len(s[0])} atoms: {out[k]['utot']!r} {own['utot']!r}", flush=True)
+            assert out[k]["utot"] == own["utot"] and epot[k] == e
+            np.testing.assert_array_equal(out[k]["u"], own["u"])
+            np.testing.assert_array_equal(out[k]["virial"], own["virial"])
