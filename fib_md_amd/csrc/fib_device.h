@@ -60,7 +60,9 @@ struct FConst {
   int32_t ntable;
   int32_t izero;      // first table index (1-based) whose T and successors are 0
   double mixed_r64;   // mixed precision: Moliere pairs below this use FP64
-  double near2;       // (cutoff + delta)^2 / sigma^2 of the near lists (k_legs)
+  double near2;       // (cutoff + delta)^2 / sigma^2 of the near lists (k_legs),
+  double near_c;      // its root, and
+  double near_isg;    // the largest 1 / sigma
   double skin;        // rc - (three-body range): pairs farther apart than rc at
                       // the build need a relative move above this to form a leg
   double mixed_xleg;  // mixed precision: three-body legs need r/sigma below

@@ -1731,10 +1731,12 @@ struct FAcc<true> {
 // Near lists.  Half of a row's entries lie so far beyond the cutoff that they
 // cannot come into range while no atom has moved much, and the pair pass is
 // bound by its gathers of the partners' positions (about 50 cycles for each
-// 16 bytes a lane).  The first pass after a build, at the positions of the
-// build, keeps the entries within cutoff + delta (FConst::near2, delta =
-// a tenth of the skin) in near[n * NA + i] = slot << 27 | partner, their
-// count in nst.  While neither the atom nor any partner of its row has moved
+// 16 bytes a lane).  The first pass after a build keeps the entries that were
+// within cutoff + delta at the build (FConst::near2, delta = a tenth of the
+// skin) in near[n * NA + i] = slot << 27 | partner, their count in nst.  It
+// runs at the positions of the build, or, when a program builds the lists and
+// then steps, after a move: the entries within cutoff + delta + twice the
+// largest displacement hold all of them.  While neither the atom nor any partner of its row has moved
 // more than delta / 2 since the build, a pair left out is out of range, and
 // the pass runs over the near list alone.  An atom that moves farther
 // (k_md_pos, k_pos) takes itself and its partners off their near lists until
@@ -1955,6 +1957,11 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
     constexpr int LB = LEGS_BATCH, NQ = LB / 4;
     int4 rn[NQ];
     int nn = 0;  // near entries, also those past the list's end
+    double near2 = fc.near2;
+    if (near && __ballot(st == NEAR_FRESH) != 0ull && ctl[kin].maxdisp > 0.0) {
+      const double c = fc.near_c + 2.0 * ctl[kin].maxdisp * fc.near_isg;
+      near2 = c * c;
+    }
 #pragma unroll
     for (int u = 0; u < NQ; ++u) rn[u] = (4 * u < cs) ? ld_nt<NT>(r4 + u) : make_int4(i, i, i, i);
     for (int k0 = 0; __ballot(k0 < cs) != 0ull; k0 += LB) {
@@ -1989,7 +1996,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
         const double rr = scaled_r2<MIXED>(d[0][v], d[1][v], d[2][v], jA ? isgA : isgB);
         // an atom removed since the build is out of the simulation (MD-step mode)
         const bool ok = k0 + v < cs && !(mj & META_DEAD);
-        if (ok && rr < fc.near2) {
+        if (ok && rr < near2) {
           if (nn < NEAR_CAP) hold[wid][nn][lane] = (uint32_t)(k0 + v) << 27 | (uint32_t)jq[v];
           nn += k0 + v < 32 ? 1 : NEAR_CAP + 1;
           if (rr < gate2) pair(d[0][v], d[1][v], d[2][v], jA);

@@ -448,7 +448,9 @@ static void derive_constants(fib_handle *h) {
   // in FP32, hence the margin)
   const double delta = std::max(0.0, 0.1 * c.skin);
   const double isgmax = std::max(c.isig[0][0], std::max(c.isig[0][1], c.isig[1][1]));
-  c.near2 = (gate + delta * isgmax * (1.0 + 1e-5)) * (gate + delta * isgmax * (1.0 + 1e-5));
+  c.near_isg = isgmax;
+  c.near_c = gate + delta * isgmax * (1.0 + 1e-5);
+  c.near2 = c.near_c * c.near_c;
   h->tab.assign(nt + 3, TabEntry{0, 0, 0, 0, 0, 0});
   for (int i = 1; i <= nt; ++i) {
     TabEntry &e = h->tab[i];
