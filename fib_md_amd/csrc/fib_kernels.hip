@@ -1540,7 +1540,7 @@ struct Leg {
 // ends of the exponent range): the hardware's estimate (24 bits), one
 // Goldschmidt step and two residual corrections of the root, one Newton step
 // of its reciprocal -- 13 operations instead of the 28 of sqrt() and a
-// division, each within 1 ulp.
+// division, each within 1 ulp.  (Both are NaN for a = 0.)
 __device__ __forceinline__ void sqrt_rsqrt(double a, double &s, double &si) {
   const double y = __builtin_amdgcn_rsq(a);
   double g = a * y, h = 0.5 * y;
@@ -1851,7 +1851,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
     if constexpr (!MIXED) {
       double r, rinv;
       sqrt_rsqrt(d0 * d0 + d1 * d1 + d2 * d2, r, rinv);
-      const double rs = r * isg;
+      const double rs = fmax(r * isg, 0.0);  // (coincident atoms: r and 1/r are NaN)
       // reference pair force: 3-point Lagrange on the derivative table
       // (si.f90:416-424, 554-573); rs / umax as its product with 1/umax,
       // corrected by the remainder
@@ -1883,7 +1883,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
       const double s0 = d0 * isg, s1 = d1 * isg, s2 = d2 * isg;
       double rs, rinv;
       sqrt_rsqrt(s0 * s0 + s1 * s1 + s2 * s2, rs, rinv);
-      if (!(rs < fc.cut_sw)) return;
+      if (rs >= fc.cut_sw) return;  // (coincident atoms: rs is NaN, and the force too)
       const double inv_ra = fast_rcp(rs - fc.al);
       const double ex = (double)expf((float)inv_ra);
       const double ir2 = rinv * rinv;
@@ -1899,7 +1899,9 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_legs(
         addW(r0 * q, r1 * q, r2 * q, 0.5f * h0, 0.5f * h1, 0.5f * h2);
       }
       if (EN) {
-        const double ul = 0.5 * (jA ? epsA : epsB) * (fc.A * (fc.B * ir4 - 1.0) * ex);
+        const double ul = rs == rs
+                              ? 0.5 * (jA ? epsA : epsB) * (fc.A * (fc.B * ir4 - 1.0) * ex)
+                              : (double)INFINITY;
         ui += ul;
         etot += ul;
       }
