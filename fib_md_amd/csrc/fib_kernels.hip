@@ -2384,12 +2384,19 @@ struct ExtraArgs {
 #define TRI_TAB_VIR 256
 // Batches of up to TRI_SMALL atoms have 16 atoms per wavefront instead of 64:
 // 4 k atoms are 64 wavefronts of 64 for 1,024 SIMDs, and the passes of one
-// wavefront follow each other (24.4 -> 12.3 us).  A large batch fills the
-// chip either way and pays for 16 with emptier last passes (262 k atoms 39.7
-// -> 48.4 us, 811 k 90 -> 126).  With energies and the virial, just built:
-// 4 k atoms, FP64, 32.8 -> 17.5 us; 2 k, mixed, without the virial, 26 -> 13.
-#define TRI_SMALL 131072
-// and of up to TRI_TINY eight, about 34 legs, one pass: 4 k atoms 12.7 -> 10.5.
+// wavefront follow each other.  A large batch fills the chip either way and
+// pays for 16 with emptier last passes.  us of an MD step's pass over a thermal
+// crystal, 64 and 16 atoms:
+//            4,096   64,000   130,000  238,080 atoms
+//   mixed  20, 12.5  22, 18   25, 30   34, 48
+//   FP64   25, 13    30, 25   35, 38   59, 61
+// and with energies 23, 14; 27, 21; 32, 35; 43, 58 (mixed) and 28, 14; 34, 29;
+// 42, 45; 70, 73 (FP64): the lines between cross at 98 k to 109 k atoms.
+#define TRI_SMALL 98304
+// and of up to TRI_TINY eight, about 34 legs, one pass.  16 and 8 atoms:
+//            4,096    16,128   32,768   64,000 atoms
+//   mixed  12.5, 9.9  13, 11   14, 13   18, 20
+//   FP64   13, 11     14, 13   16, 17   25, 25
 #define TRI_TINY 16384
 template <bool MIXED>
 struct TriStage {
