@@ -3614,12 +3614,18 @@ static int xcd_shift(const DevBufs &d) {
 
 // Cells per wavefront of the list build: a wavefront builds its cells one
 // after the other, each with two or three dependent loads, so a small batch
-// takes few per wavefront (4 k atoms, whole build: 8 cells 46 us, 4 cells 28,
-// 1 cell 12; 101 k atoms: 55, 50 and 50) and a large one eight, which share
-// the decoding of their position (2.1 M atoms: 4 cells 682 us, 8 cells 651,
-// 16 cells 675).
+// takes few per wavefront and a large one eight, which share the decoding of
+// their position.  us of a build of a crystal by 1, 2, 4 and 8 cells:
+//     1,000 cells  14   19   27   46      63,960 cells 109  103  102  108
+//     8,000        25   24   31   49     140,608       227  204  196  201
+//    17,576        39   40   46   54     257,920       392  352  335  335
+//    34,816        67   63   66   81     571,787       882  772  719  701
+// A gated build has the cells of a few of the batch's instances, hence the
+// line between 2 and 4 above that of whole builds: MD of 64 x 4 k atoms
+// (121,600 cells) 48 ms by 1 or 2 cells, 50 by 4, 53 by 8; of 12 uneven slabs
+// (254,772 cells) 61.5, 59.0, 59.0 and 60.5.
 static int nb_cells_auto(int total_cells) {
-  return total_cells < 65536 ? 1 : total_cells < 131072 ? 2 : total_cells < 262144 ? 4 : 8;
+  return total_cells < 32768 ? 1 : total_cells < 131072 ? 2 : total_cells < 262144 ? 4 : 8;
 }
 
 // Whether the list build expects cells with 129 to 192 candidates, which its
