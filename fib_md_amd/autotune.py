@@ -29,9 +29,9 @@ from .gpu import FibGPU, GPUError, default_params
 
 CANDIDATES = (1.10, 1.15, 1.20, 1.25, 1.30)
 # (legs per write-out, loads in flight) of the vertex pass; cells
-# per wavefront of the list build
+# per wavefront of the list build (0: the default of the handle's size)
 TRI_TILES = ((256, 4), (256, 2), (128, 4), (128, 2))
-NB_CELLS = (8, 4, 16)
+NB_CELLS = (0, 4, 16)
 
 
 def md_handle(instances, precision, params=None, use_graph=True):
@@ -87,15 +87,17 @@ def tune_tiles(g, steps=30, warmup=5, tri_tiles=TRI_TILES, nb_cells=NB_CELLS):
     first the vertex pass's (write-out size, loads in flight), then the list
     build's cells per wavefront with the best of those, each timed over
     `steps` MD steps after `warmup`.  Leaves the handle in the best tiles and
-    returns (best (tri_ns, tri_batch, nb_cells), [(tiles, ms per step)])."""
+    returns (best (tri_ns, tri_batch, nb_cells), [(tiles, ms per step)]), with
+    the number of cells that a 0 stands for."""
     table = []
     for ns, tb in tri_tiles:
         g.set_tiles(ns, tb, nb_cells[0])
-        table.append(((ns, tb, nb_cells[0]), _ms_per_step(g, steps, warmup)))
+        table.append((g.tiles(), _ms_per_step(g, steps, warmup)))
     ns, tb, _ = min(table, key=lambda r: r[1])[0]
     for nc in nb_cells[1:]:
         g.set_tiles(ns, tb, nc)
-        table.append(((ns, tb, nc), _ms_per_step(g, steps, warmup)))
+        if g.tiles() not in [t for t, _ in table]:
+            table.append((g.tiles(), _ms_per_step(g, steps, warmup)))
     best = min(table, key=lambda r: r[1])[0]
     g.set_tiles(*best)
     return best, table

@@ -3624,7 +3624,7 @@ static int xcd_shift(const DevBufs &d) {
 // line between 2 and 4 above that of whole builds: MD of 64 x 4 k atoms
 // (121,600 cells) 48 ms by 1 or 2 cells, 50 by 4, 53 by 8; of 12 uneven slabs
 // (254,772 cells) 61.5, 59.0, 59.0 and 60.5.
-static int nb_cells_auto(int total_cells) {
+int nb_cells_auto(int total_cells) {
   return total_cells < 32768 ? 1 : total_cells < 131072 ? 2 : total_cells < 262144 ? 4 : 8;
 }
 

@@ -1658,9 +1658,10 @@ extern "C" int32_t fib_set_tiles(fib_handle *h, int32_t tri_ns, int32_t tri_batc
   if (run_in_flight(h, "fib_set_tiles")) return FIB_ERR_STATE;
   if ((tri_ns != 0 && tri_ns != 128 && tri_ns != 256) ||
       (tri_batch != 0 && tri_batch != 2 && tri_batch != 4) ||
-      (nb_cells != 0 && nb_cells != 4 && nb_cells != 8 && nb_cells != 16))
-    return fail(h, FIB_ERR_ARG, "fib_set_tiles: tri_ns 128|256, tri_batch 2|4, nb_cells 4|8|16 "
-                                "(0: default)");
+      (nb_cells != 0 && nb_cells != 1 && nb_cells != 2 && nb_cells != 4 && nb_cells != 8 &&
+       nb_cells != 16))
+    return fail(h, FIB_ERR_ARG, "fib_set_tiles: tri_ns 128|256, tri_batch 2|4, nb_cells "
+                                "1|2|4|8|16 (0: default)");
   h->d.tri_ns = tri_ns;
   h->d.tri_tb = tri_batch;
   h->d.nb_cells = nb_cells;
@@ -1672,7 +1673,7 @@ extern "C" int32_t fib_get_tiles(const fib_handle *h, int32_t tiles[3]) {
   if (!h || !tiles) return FIB_ERR_ARG;
   tiles[0] = h->d.tri_ns ? h->d.tri_ns : 256;
   tiles[1] = h->d.tri_tb ? h->d.tri_tb : 4;
-  tiles[2] = h->d.nb_cells ? h->d.nb_cells : 8;
+  tiles[2] = h->d.nb_cells ? h->d.nb_cells : fibk::nb_cells_auto(h->d.total_cells);
   return FIB_OK;
 }
 

@@ -328,7 +328,8 @@ int32_t fib_get_list_width(const fib_handle *h, int32_t *wsw, int32_t *wion);
  * the results of up to tri_ns / 2 legs of a wavefront back and writes them
  * out together; tri_batch: 4 loads the next legs' positions during a pass
  * over up to 64 legs, 2 only their row entries; nb_cells cells per wavefront
- * of the list build (4, 8 or 16); 0 keeps a tile at its default (256, 4, 8).
+ * of the list build (1, 2, 4, 8 or 16); 0 keeps a tile at its default (256, 4,
+ * and 1, 2, 4 or 8 by the handle's number of cells).
  * Results are the same bit for bit in every tile, only the time changes.
  * The reference's only tuning knob of this kind is its cell count, rc and Nc
  * (si.f90:55-56). */
