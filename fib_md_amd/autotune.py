@@ -5,8 +5,14 @@ cell size of the list build and the skin rc - 0.999 a sigma that decides
 how often an instance rebuilds (when the two largest displacements since
 the build add up to more than the skin).  A larger factor means fewer
 rebuilds but more candidates per build and longer lists for the pair pass.  The best value depends on the workload (instance sizes,
-ion energies, precision), so it is measured: each candidate runs a short
-stretch of the actual batch on the GPU and the fastest steps win.  Lists
+ion energies, precision), so it is measured: each candidate runs two short
+stretches of the actual batch on the GPU, one after the ions are fired and one
+in their cascades, and the fastest steps win.  The first alone favours long
+lists: while few atoms move the pair pass reads near lists, whose length hardly
+depends on the factor, and builds are rare.  1,024 replicas of a 500 eV
+impact on 4 k atoms, ms per step by 1.10, 1.15, 1.20, 1.25: steps 20 to 80
+1.13, 1.08, 1.07, 1.05; steps 480 to 540 1.72, 1.59, 1.65, 1.67; all 2,000
+steps 1.65, 1.55, 1.63, 2.04.  Lists
 hold every pair within rc and rc lies beyond the SW cutoff, so the mixed
 path's forces (analytic pair term) are the same for every candidate up to
 the summation order; the FP64 path's tabulated pair derivative spans
@@ -47,10 +53,12 @@ def md_handle(instances, precision, params=None, use_graph=True):
     return g
 
 
-def tune_listfac(instances, precision="mixed", candidates=CANDIDATES, steps=60, warmup=20):
+def tune_listfac(instances, precision="mixed", candidates=CANDIDATES, steps=60, warmup=20,
+                 cascade=400):
     """Time `steps` MD steps (after `warmup`) of the batch for each candidate
-    listfac; returns (best listfac, [(listfac, ms per step or None, note)]).
-    A candidate whose lists outgrow their width is skipped."""
+    listfac, and as many again `cascade` steps later; returns (best listfac,
+    [(listfac, ms per step over both or None, note)]).  A candidate whose
+    lists outgrow their width is skipped."""
     table = []
     for lf in candidates:
         p = default_params()
@@ -58,11 +66,8 @@ def tune_listfac(instances, precision="mixed", candidates=CANDIDATES, steps=60, 
         g = None
         try:
             g = md_handle(instances, precision, params=p)
-            g.md_run(warmup)
-            t0 = time.perf_counter()
-            g.md_run(steps)  # returns after the stream has drained
-            t = time.perf_counter() - t0
-            table.append((float(lf), t * 1e3 / steps, ""))
+            first = _ms_per_step(g, steps, warmup)
+            table.append((float(lf), 0.5 * (first + _ms_per_step(g, steps, cascade)), ""))
         except GPUError as e:
             table.append((float(lf), None, str(e)))
         finally:
