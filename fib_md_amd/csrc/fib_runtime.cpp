@@ -108,6 +108,7 @@ struct fib_handle {
   std::vector<DInst> inst;
   DevBufs d{};
   bool have_state = false, have_lists = false, have_force = false;
+  bool inst_stale = false;  // a copy of instance records to the device has not ended well
   // MD-step mode
   bool md_on = false;
   fib_md_params md{};
@@ -654,11 +655,14 @@ extern "C" int32_t fib_get_state(fib_handle *h, int32_t inst, double *X, double 
 extern "C" int32_t fib_set_impact(fib_handle *h, int32_t inst, int32_t impact) {
   if (run_in_flight(h, "fib_set_impact")) return FIB_ERR_STATE;
   if (bad_inst(h, inst) || impact < 0) return fail(h, FIB_ERR_ARG, "fib_set_impact: bad argument");
-  if (h->inst[inst].impact == impact) return FIB_OK;  // the device's record agrees with the host's
+  if (h->inst[inst].impact == impact && !h->inst_stale) return FIB_OK;
   h->inst[inst].impact = impact;
-  HIPCHK(h, hipMemcpyAsync(&h->d.I[inst], &h->inst[inst], sizeof(DInst), hipMemcpyHostToDevice,
+  const size_t k0 = h->inst_stale ? 0 : (size_t)inst, n = h->inst_stale ? h->inst.size() : 1;
+  h->inst_stale = true;
+  HIPCHK(h, hipMemcpyAsync(&h->d.I[k0], &h->inst[k0], sizeof(DInst) * n, hipMemcpyHostToDevice,
                            h->stream));
   HIPCHK(h, hipStreamSynchronize(h->stream));
+  h->inst_stale = false;
   return FIB_OK;
 }
 
@@ -1184,8 +1188,10 @@ extern "C" int32_t fib_md_begin(fib_handle *h, const fib_md_params *p, const dou
     h->inst[k].surf_z = surface_z[k];
     h->inst[k].bot_z = bottom_z[k];
   }
+  h->inst_stale = true;
   HIPCHK(h, hipMemcpy(h->d.I, h->inst.data(), sizeof(DInst) * h->inst.size(),
                       hipMemcpyHostToDevice));
+  h->inst_stale = false;
   h->md = *p;
   StepArgs &sa = h->md_sa;
   sa = h->base;
@@ -1232,6 +1238,8 @@ extern "C" int32_t fib_md_fire_many(fib_handle *h, int32_t count, const int32_t 
     HIPCHK(h, hipMemcpy(&pos[q], d.inv + in.atom_off + in.nsg + ion[q] - 1, sizeof(int),
                         hipMemcpyDeviceToHost));
   }
+  const bool stale = h->inst_stale;
+  h->inst_stale = true;
   for (int q = 0; q < count; ++q) {
     fibk::launch_set_atom(d, pos[q], x + 3 * (size_t)q, v + 3 * (size_t)q, h->md_sa, h->stream);
     DInst &in = h->inst[inst[q]];
@@ -1256,6 +1264,7 @@ extern "C" int32_t fib_md_fire_many(fib_handle *h, int32_t count, const int32_t 
   fibk::launch_build(d, h->fc, h->stream, true);
   d.gate = nullptr;
   HIPCHK(h, hipStreamSynchronize(h->stream));
+  h->inst_stale = stale;
   bool halted = false;
   int32_t r = md_halted(h, halted);
   if (r != FIB_OK) return r;
