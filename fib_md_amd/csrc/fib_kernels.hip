@@ -3732,7 +3732,7 @@ void launch_build(const DevBufs &d, const FConst &fc, hipStream_t s, bool inplac
                        d.gate);
     hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(SCAN_T), 0, s, d.bcnt, d.nbucket, d.bsum,
                        d.cstart, d.gate);
-    hipLaunchKernelGGL(k_scatter, dim3(gcap(d.NA)), dim3(FIB_BLOCK), 0, s, d.bkey, d.brank, d.NA,
+    hipLaunchKernelGGL(k_scatter, dim3(gcap(std::max(d.NA, d.nbucket))), dim3(FIB_BLOCK), 0, s, d.bkey, d.brank, d.NA,
                        d.I, d.cstart, d.perm, d.bcnt, d.nbucket, d.binst, d.gate);
     hipLaunchKernelGGL(k_fixup, dim3(gcap(d.nbucket)), dim3(FIB_BLOCK), 0, s, d.cstart, d.nbucket,
                        d.I, d.ninst, d.perm, d.gate);
