@@ -114,6 +114,8 @@ namespace fibk {
 // arrays move to the other buffers (the caller flips cur), or (inplace) back
 // into the current ones
 void launch_build(const DevBufs &d, const FConst &fc, hipStream_t s, bool inplace);
+// length of DevBufs::bsum
+size_t bsum_len(int nbucket);
 // cells per wavefront of the list build where DevBufs::nb_cells is 0
 int nb_cells_auto(int total_cells);
 // the list build alone, of the positions X[from] (again, after the lists

@@ -620,17 +620,23 @@ __global__ void k_scan_reduce(const int *__restrict__ in, int n, int *__restrict
 }
 
 // out[b] = exclusive prefix over all buckets, out[n] = total: every block
-// adds up the totals of the blocks before it.  A bucket's atoms start at
+// adds up the totals of the blocks before it, or (SCANNED) finds them added
+// up, where there are too many (see scan_top).  A bucket's atoms start at
 // out[b] - out[first bucket of its instance] + atom_off, whatever other
 // instances hold, so an instance can be sorted while the others stay in
 // place (bucket_base).
+template <bool SCANNED>
 __global__ void k_scan_down(const int *__restrict__ in, int n, const int *__restrict__ bsum,
                             int *__restrict__ out, const int *__restrict__ gate) {
   GATE_OR_RETURN(gate);
-  int before = 0;
-  for (int k = threadIdx.x; k < (int)blockIdx.x; k += SCAN_T) before += bsum[k];
   int carry;
-  block_scan_excl(before, carry);
+  if (SCANNED) {
+    carry = bsum[blockIdx.x];
+  } else {
+    int before = 0;
+    for (int k = threadIdx.x; k < (int)blockIdx.x; k += SCAN_T) before += bsum[k];
+    block_scan_excl(before, carry);
+  }
   const int base = blockIdx.x * SCAN_CH + threadIdx.x * SCAN_E;
   int vals[SCAN_E];
   int s = 0;
@@ -3725,6 +3731,17 @@ static bool small_sort(const DevBufs &d) {
   return d.max_pad <= SORT_N && d.max_bucket <= SORT_N;
 }
 
+// Whether the totals of the scan's nb blocks are scanned by launches of their
+// own: the blocks' sums over the totals before them grow with nb squared.
+// k_scan_down of 2,747 blocks (5.6 million buckets) 27 us without them, about
+// what it takes to read and write the buckets; of 43,500 574 us, 324 (and two
+// launches of 5) with them; of 348,500 14.8 ms, 2.5.
+static bool scan_top(int nb) { return nb > 8192; }
+size_t bsum_len(int nbucket) {
+  const size_t nb = (size_t)nblk((long)nbucket + 1, SCAN_CH);
+  return nb + (scan_top((int)nb) ? nb + 1 + (size_t)nblk((long)nb + 1, SCAN_CH) : 0);
+}
+
 void launch_build(const DevBufs &d, const FConst &fc, hipStream_t s, bool inplace) {
   const int c = d.cur, n = 1 - d.cur;
   if (small_sort(d)) {
@@ -3742,8 +3759,18 @@ void launch_build(const DevBufs &d, const FConst &fc, hipStream_t s, bool inplac
     const int nb = nblk(d.nbucket + 1, SCAN_CH);
     hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(SCAN_T), 0, s, d.bcnt, d.nbucket, d.bsum,
                        d.gate);
-    hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(SCAN_T), 0, s, d.bcnt, d.nbucket, d.bsum,
-                       d.cstart, d.gate);
+    if (scan_top(nb)) {
+      int *const top = d.bsum + nb, *const sum = top + nb + 1;
+      const int nt = nblk(nb + 1, SCAN_CH);
+      hipLaunchKernelGGL(k_scan_reduce, dim3(nt), dim3(SCAN_T), 0, s, d.bsum, nb, sum, d.gate);
+      hipLaunchKernelGGL(k_scan_down<false>, dim3(nt), dim3(SCAN_T), 0, s, d.bsum, nb, sum, top,
+                         d.gate);
+      hipLaunchKernelGGL(k_scan_down<true>, dim3(nb), dim3(SCAN_T), 0, s, d.bcnt, d.nbucket, top,
+                         d.cstart, d.gate);
+    } else {
+      hipLaunchKernelGGL(k_scan_down<false>, dim3(nb), dim3(SCAN_T), 0, s, d.bcnt, d.nbucket,
+                         d.bsum, d.cstart, d.gate);
+    }
     hipLaunchKernelGGL(k_scatter, dim3(gcap(std::max(d.NA, d.nbucket))), dim3(FIB_BLOCK), 0, s, d.bkey, d.brank, d.NA,
                        d.I, d.cstart, d.perm, d.bcnt, d.nbucket, d.binst, d.gate);
     hipLaunchKernelGGL(k_fixup, dim3(gcap(d.nbucket)), dim3(FIB_BLOCK), 0, s, d.cstart, d.nbucket,

@@ -479,7 +479,7 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
   take(d.brank, NA);
   take(d.cstart, (size_t)d.nbucket + 1);
   take(d.perm, NA);
-  take(d.bsum, (size_t)d.nbucket / 2048 + 2);
+  take(d.bsum, fibk::bsum_len(d.nbucket));
   take(d.near, (size_t)16 * NA);
   take(d.nst, NA);
   take(d.Xb, NA);
@@ -1693,7 +1693,7 @@ int32_t fib_arena_force(const fib_params *p, int32_t precision, int32_t natm, in
   d.brank = A.take<int>(NA);
   d.cstart = A.take<int>((size_t)d.nbucket + 1);
   d.perm = A.take<int>(NA);
-  d.bsum = A.take<int>((size_t)d.nbucket / 2048 + 2);
+  d.bsum = A.take<int>(fibk::bsum_len(d.nbucket));
   d.cnt_sw = A.take<int>(NA);
   d.cnt_ion = A.take<int>(NA);
   d.amask = A.take<uint64_t>(NA);

@@ -36,9 +36,11 @@ def _listed(g):
 
 
 # cells: 3 x 3 x 20,000; 241 x 241 x 48 (2.8 million); 100 x 3 x 3; two atoms'
-# worth of buckets past a multiple of the scan's chunks; boxes of two cells a side
+# worth of buckets past a multiple of the scan's chunks; boxes of two cells a side; 17.2
+# million, more than 8,192 chunks
 @pytest.mark.parametrize("cells,n", [((3, 3, 20000), 40), ((241, 241, 48), 60), ((100, 3, 3), 30),
-                                     ((32, 16, 16), 20), ((2, 2, 5000), 30), ((2, 600, 600), 40)])
+                                     ((32, 16, 16), 20), ((2, 2, 5000), 30), ((2, 600, 600), 40),
+                                     ((262, 257, 256), 60)])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_lists_of_clusters_in_vacuum(cells, n, precision):
     pytest.importorskip("scipy")
