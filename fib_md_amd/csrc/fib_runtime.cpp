@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <limits>
 #include <string>
 #include <vector>
 
@@ -480,8 +481,6 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
   take(d.cstart, (size_t)d.nbucket + 1);
   take(d.perm, NA);
   take(d.bsum, fibk::bsum_len(d.nbucket));
-  take(d.near, (size_t)16 * NA);
-  take(d.nst, NA);
   take(d.Xb, NA);
   char *exself = nullptr;
   take(exself, (h->prec == FIB_PREC_MIXED ? sizeof(float4) : sizeof(double4)) * NA);
@@ -502,14 +501,32 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
   }
   take(d.fin_tmp, (size_t)ninst * (d.max_pad / FIB_BLOCK / FIB_FIN_CH + 1) * FIB_NRED);
   take(d.tab, h->tab.size());
-  if (hipMalloc((void **)&h->arrays, bytes) != hipSuccess) {
-    rc_ = FIB_ERR_HIP;
-    h->err = "hipMalloc failed for the arrays of the handle";
-  } else {
+  // the near lists last: a handle that fits only without them does without
+  const size_t least = bytes;
+  take(d.near, (size_t)16 * NA);
+  take(d.nst, NA);
+  const DevBufs none = d;
+  auto alloc = [&](bool near) -> int32_t {
+    if (hipMalloc((void **)&h->arrays, near ? bytes : least) != hipSuccess) {
+      h->err = "hipMalloc failed for the arrays of the handle";
+      return FIB_ERR_HIP;
+    }
     for (const Place &q : places) *q.p = h->arrays + q.off;
     d.EXself = exself;
+    if (!near) {
+      d.near = nullptr;
+      d.nst = nullptr;
+    }
+    return alloc_lists(h, 32, 64);
+  };
+  rc_ = alloc(true);
+  if (rc_ == FIB_ERR_HIP) {
+    (void)hipGetLastError();
+    free_bufs(h);
+    d = none;
+    h->base.near_d = std::numeric_limits<float>::infinity();
+    rc_ = alloc(false);
   }
-  if (rc_ == FIB_OK) rc_ = alloc_lists(h, 32, 64);
   if (rc_ != FIB_OK) {
     free_bufs(h);
     (void)hipStreamDestroy(h->stream);
@@ -524,7 +541,7 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
     e = hipMemcpy(d.binst, binst.data(), sizeof(int) * binst.size(), hipMemcpyHostToDevice);
   }
   if (e == hipSuccess) e = hipMemset(h->arrays, 0, zeroed);
-  if (e == hipSuccess) e = hipMemset(d.nst, 254, NA);
+  if (e == hipSuccess && d.nst) e = hipMemset(d.nst, 254, NA);
   if (e == hipSuccess)
     e = hipMemcpy(d.tab, h->tab.data(), sizeof(TabEntry) * h->tab.size(), hipMemcpyHostToDevice);
   if (e != hipSuccess) {

@@ -1,0 +1,84 @@
+"""A handle for which the device has room without the near lists only: it is
+made, and gives the same bits as one with them, force evaluations and MD steps
+alike (the forces do not depend on which list the pair pass reads)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from fib_md_amd import _lib, configs
+
+pytestmark = pytest.mark.gpu
+
+
+class _Hog:
+    """Device memory held back, by the HIP that the library is linked with."""
+
+    def __init__(self):
+        self.hip, self.held = _lib.lib(), []
+
+    def free(self):
+        a, b = C.c_size_t(), C.c_size_t()
+        assert self.hip.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    def take(self, n):
+        p = C.c_void_p()
+        assert self.hip.hipMalloc(C.byref(p), C.c_size_t(n)) == 0
+        self.held.append(p)
+
+    def give_back(self):
+        while self.held:
+            assert self.hip.hipFree(self.held.pop()) == 0
+
+
+def _run(X, V, at, L, precision, hog=None):
+    from fib_md_amd import FibGPU
+    g = FibGPU([(len(X), len(X) - 1, 1, L)], precision=precision)
+    if hog:  # (the device's memory is free again: staging, captured steps)
+        hog.give_back()
+    g.set_state(X, V=V, atype=at, Xi=X)
+    g.build_nlist()
+    r = g.force(impact=1, energy=True, virial=True)
+    g.md_begin([L[2]], [0.0])
+    g.md_fire(0, 1, X[-1], np.array([0.0, 1.0e4, -5.0e4]))
+    g.md_run(60)
+    X1, V1, F1 = g.state()
+    rep = g.md_report(0)
+    g.close()
+    return [r["F"], r["u"], r["utot"], r["virial"], X1, V1, F1], rep
+
+
+def test_handle_without_room_for_near_lists():
+    from fib_md_amd import FibGPU
+    precision = "mixed"
+    n = (60, 60, 40)
+    rng = np.random.default_rng(4)
+    L = tuple(configs.A_SI * c for c in n)
+    X = configs.diamond(*n)
+    X = np.mod(X + rng.normal(0.0, 0.05e-10, X.shape), L)
+    X = np.asfortranarray(np.vstack([X, [[1.625 * configs.A_SI] * 3]]))
+    V = np.asfortranarray(np.vstack([rng.normal(0.0, 420.0, (len(X) - 1, 3)), np.zeros((1, 3))]))
+    at = np.concatenate([np.ones(len(X) - 1, np.int32), [3]]).astype(np.int32)
+    want, rep = _run(X, V, at, L, precision)
+    # the device's memory less what such a handle takes, plus half of its near lists
+    hog = _Hog()
+    before = hog.free()
+    g = FibGPU([(len(X), len(X) - 1, 1, L)], precision=precision)
+    took = before - hog.free()
+    g.close()
+    near = 65 * len(X)
+    assert took > 20 * near
+    for _ in range(4):
+        if hog.free() > took - 0.4 * near:
+            hog.take(int(hog.free() - (took - 0.5 * near)))
+    left = hog.free()
+    print(f"{precision}: a handle takes {took >> 20} MiB, its near lists {near >> 20}, left {left >> 20}",
+          flush=True)
+    if not took - 0.7 * near < left < took - 0.3 * near:
+        hog.give_back()
+        pytest.skip("the allocator left another size than asked for")
+    got, rep2 = _run(X, V, at, L, precision, hog)
+    for a, b in zip(got, want):
+        np.testing.assert_array_equal(a, b)
+    assert rep2 == rep
