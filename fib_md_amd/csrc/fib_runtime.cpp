@@ -658,7 +658,16 @@ extern "C" int32_t fib_get_state(fib_handle *h, int32_t inst, double *X, double 
   const size_t b3 = 3 * n * sizeof(double);
   const size_t ox = P.add(b3, X), ov = P.add(b3, V), of = P.add(b3, F);
   if (P.n == 0) return FIB_OK;
-  HIPCHK(h, h->stage.reserve(P.used));
+  hipError_t e = h->stage.reserve(P.used);
+  if (e == hipErrorOutOfMemory && P.n > 1) {
+    // the device has no room for all of them beside each other
+    (void)hipGetLastError();
+    int32_t r = X ? fib_get_state(h, inst, X, nullptr, nullptr) : FIB_OK;
+    if (r == FIB_OK && V) r = fib_get_state(h, inst, nullptr, V, nullptr);
+    if (r == FIB_OK && F) r = fib_get_state(h, inst, nullptr, nullptr, F);
+    return r;
+  }
+  HIPCHK(h, e);
   char *const dv = h->stage.dev;
   fibk::ExportArgs ex{};
   if (X) ex.x = (double *)(dv + ox);

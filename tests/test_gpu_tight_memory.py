@@ -82,3 +82,36 @@ def test_handle_without_room_for_near_lists():
     for a, b in zip(got, want):
         np.testing.assert_array_equal(a, b)
     assert rep2 == rep
+
+
+def test_state_without_room_for_all_its_arrays():
+    """fib_get_state with room on the device for one of X, V and F at a time
+    only, as fib_set_state of positions and species leaves it."""
+    from fib_md_amd import FibGPU
+    from fib_md_amd.gpu import GPUError
+    n = 600000
+    rng = np.random.default_rng(6)
+    L = (400e-10,) * 3
+    X = np.asfortranarray(rng.random((n, 3)) * np.array(L))
+    at = np.ones(n, np.int32)
+    g = FibGPU([(n, n, 0, L)], precision="mixed")
+    g.set_state(X, atype=at)
+    hog = _Hog()
+    try:
+        for size in (1 << 34, 1 << 31, 1 << 28, 1 << 25, 1 << 23):
+            while hog.free() > size + (4 << 20) and len(hog.held) < 300:
+                try:
+                    hog.take(size)
+                except AssertionError:
+                    break
+        print(f"free {hog.free() >> 20} MiB", flush=True)
+        try:
+            Xg, Vg, Fg = g.state()
+        except GPUError as e:
+            pytest.fail(f"state refused: {e}")
+    finally:
+        hog.give_back()
+    np.testing.assert_array_equal(Xg, X)
+    assert not Vg.any() and not Fg.any()
+    np.testing.assert_array_equal(g.state()[0], X)
+    g.close()
