@@ -303,6 +303,7 @@ static hipError_t dalloc(T **p, size_t n) {
 
 static int32_t alloc_lists(fib_handle *h, int Wsw, int Wion) {
   DevBufs &d = h->d;
+  h->stage.release();  // (the next transfer makes it anew: room for the lists now)
   if (d.nbr_sw) (void)hipFree(d.nbr_sw);
   if (d.nbr_ion) (void)hipFree(d.nbr_ion);
   void *old[] = {d.rk_sw, d.G, d.RA, d.EX};
@@ -336,6 +337,7 @@ static int32_t regrow_lists(fib_handle *h, int Wsw, int Wion) {
   const size_t NA = (size_t)d.NA;
   if ((uint64_t)Wsw * NA >= (1ull << 32))
     return fail(h, FIB_ERR_ARG, "too many atoms for one handle: atoms x list width >= 2^32");
+  h->stage.release();  // as in alloc_lists
   int *nsw = nullptr, *nion = nullptr;
   uint16_t *rk = nullptr;
   HIPCHK(h, dalloc(&nsw, (size_t)Wsw * NA));
@@ -1451,7 +1453,13 @@ extern "C" int32_t fib_snapshot_begin(fib_handle *h, int32_t inst, int32_t slot)
     if (sn.dev) { (void)hipFree(sn.dev); sn.dev = nullptr; }
     if (sn.host) { (void)hipHostFree(sn.host); sn.host = nullptr; }
     sn.cap = 0;
-    HIPCHK(h, hipMalloc((void **)&sn.dev, need * sizeof(double)));
+    hipError_t e = hipMalloc((void **)&sn.dev, need * sizeof(double));
+    if (e == hipErrorOutOfMemory) {  // (with what the transfers hold, perhaps)
+      (void)hipGetLastError();
+      h->stage.release();
+      e = hipMalloc((void **)&sn.dev, need * sizeof(double));
+    }
+    HIPCHK(h, e);
     HIPCHK(h, hipHostMalloc((void **)&sn.host, need * sizeof(double), hipHostMallocDefault));
     sn.cap = need;
   }

@@ -27,6 +27,16 @@ class _Hog:
         assert self.hip.hipMalloc(C.byref(p), C.c_size_t(n)) == 0
         self.held.append(p)
 
+    def fill(self, rest):
+        """Holds the memory back but for some `rest` bytes."""
+        for size in (1 << 34, 1 << 31, 1 << 28, 1 << 25, 1 << 23):
+            while self.free() > size + rest and len(self.held) < 300:
+                try:
+                    self.take(size)
+                except AssertionError:
+                    break
+        print(f"free {self.free() >> 20} MiB", flush=True)
+
     def give_back(self):
         while self.held:
             assert self.hip.hipFree(self.held.pop()) == 0
@@ -98,13 +108,7 @@ def test_state_without_room_for_all_its_arrays():
     g.set_state(X, atype=at)
     hog = _Hog()
     try:
-        for size in (1 << 34, 1 << 31, 1 << 28, 1 << 25, 1 << 23):
-            while hog.free() > size + (4 << 20) and len(hog.held) < 300:
-                try:
-                    hog.take(size)
-                except AssertionError:
-                    break
-        print(f"free {hog.free() >> 20} MiB", flush=True)
+        hog.fill(4 << 20)
         try:
             Xg, Vg, Fg = g.state()
         except GPUError as e:
@@ -114,4 +118,30 @@ def test_state_without_room_for_all_its_arrays():
     np.testing.assert_array_equal(Xg, X)
     assert not Vg.any() and not Fg.any()
     np.testing.assert_array_equal(g.state()[0], X)
+    g.close()
+
+
+def test_snapshot_in_the_room_of_the_transfers():
+    """A snapshot where the device has room for its copy only once what the
+    handle keeps for its transfers (80 bytes per atom) is given back."""
+    from fib_md_amd import FibGPU
+    n = 600000
+    rng = np.random.default_rng(7)
+    L = (400e-10,) * 3
+    X = np.asfortranarray(rng.random((n, 3)) * np.array(L))
+    V = np.asfortranarray(rng.normal(0.0, 400.0, (n, 3)))
+    g = FibGPU([(n, n, 0, L)], precision="mixed")
+    g.set_state(X, V=V, atype=np.ones(n, np.int32), xsides=np.zeros(n, np.int32), Xi=X)
+    hog = _Hog()
+    try:
+        hog.fill(4 << 20)
+        g.snapshot_begin()
+        Xs, Vs = g.snapshot_wait()
+    finally:
+        hog.give_back()
+    np.testing.assert_array_equal(Xs, X)
+    np.testing.assert_array_equal(Vs, V)
+    Xg, Vg, _ = g.state()
+    np.testing.assert_array_equal(Xg, X)
+    np.testing.assert_array_equal(Vg, V)
     g.close()
