@@ -323,8 +323,7 @@ def run_gpu(X, at, L, precision, steps, warmup):
 
 
 STEPS_PER_IMPACT = 2000  # the single-impact configuration's step count
-STEP_KERNELS = ("k_pos", "k_bin", "sort", "k_nbuild", "list_aux", "k_legs", "k_tri",
-                "k_extra", "k_force3", "reduce")
+STEP_KERNELS = ("k_pos", "k_bin", "sort", "k_nbuild", "k_legs", "k_tri", "k_force3", "reduce")
 
 
 def _md_handle(instances, precision, use_graph=True, params=None):

@@ -34,11 +34,9 @@ enum KKey {
   KT_BIN = 0,   // k_bin
   KT_SORT,      // scan, scatter, fixup, reorder
   KT_NBUILD,    // k_nbuild
-  KT_LISTAUX,   // (no kernel left)
   KT_LEGS,      // k_legs
-  KT_TRI,       // k_tri
+  KT_TRI,       // k_tri (and extra_pass in its launch)
   KT_GATHER,    // k_force3
-  KT_EXTRA,     // (none: extra_pass runs in k_tri's launch)
   KT_POS,       // k_pos
   KT_REDUCE,    // k_finalize, k_sums
   KT_IO,        // import / export / set-atom / cell-id kernels
@@ -94,7 +92,8 @@ struct DevBufs {
   void *EXself;              // stale-graph terms: force on the bridge atom, T4 [NA]
   uint64_t *exmask;          // slots of EX written in the last evaluation [NA]
   double *Fout, *uout;       // force-only results [3*NA], [NA]
-  double *partials;          // [2 * FIB_NRED * pstride], layout [region][slot][block]
+  double *partials;          // [3 * FIB_NRED * pstride], layout [region][slot][block]: the
+                             // regions of k_legs (and every other reduction), k_tri, extra_pass
   int max_pad;               // largest padded atom count of an instance
   int max_bucket;            // most buckets of an instance
   double max_cell;           // largest cell volume
@@ -127,8 +126,7 @@ void launch_cellid(const DevBufs &d, int inst, int32_t *dout, hipStream_t s);
 void launch_copy_rows(int NA, int wold, const int *src, int wnew, int *dst, hipStream_t s);
 void launch_copy_rows(int NA, int wold, const uint16_t *src, int wnew, uint16_t *dst,
                       hipStream_t s);
-// handle-free evaluations: instance record, zero fill (bytes a multiple of
-// 4), energy total of instance 0 into a device double
+// handle-free evaluations: instance record, zero fill (bytes a multiple of 4)
 void launch_put_inst(const DevBufs &d, const DInst &in, hipStream_t s);
 void launch_fill_zero(void *p, size_t bytes, hipStream_t s);
 // clears the leaving mark of every atom (after a removal-list overflow)

@@ -2873,9 +2873,6 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_md_pos(double4 *__restrict__ X,
   block_partials<6, FIB_BLOCK>(red, op, lb, pstride, partials);
 }
 
-// Rebuild gates of the step: each instance whose two largest displacements
-// since the build add up to more than the skin (only then can a pair the
-// build left out have come within the cutoff), and whether there is any.
 // Interaction energy (FP64, J) of atom i with the atoms that stay in the
 // simulation: every SW pair and three-body term and every Moliere pair it
 // takes part in (si.f90:278-368 forms), each term divided by the number of
@@ -3003,6 +3000,9 @@ __device__ double interaction_energy(int i, const double4 *__restrict__ X,
   return e;
 }
 
+// Rebuild gates of the step: each instance whose two largest displacements
+// since the build add up to more than the skin (only then can a pair the
+// build left out have come within the cutoff), and whether there is any.
 #define DECIDE_T 256  // threads of k_md_decide (a small block keeps the removal path in registers)
 static_assert(FIB_LEAVE_CAP == DECIDE_T, "one thread per listed removal");
 __global__ __launch_bounds__(DECIDE_T) void k_md_decide(

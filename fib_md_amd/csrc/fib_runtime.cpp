@@ -79,8 +79,7 @@ struct Timer {
 };
 
 static const char *const kTimerNames[KT_N] = {
-    "k_bin", "sort", "k_nbuild", "list_aux", "k_legs",
-    "k_tri", "k_force3", "k_extra", "k_pos", "reduce", "io", "md_step"};
+    "k_bin", "sort", "k_nbuild", "k_legs", "k_tri", "k_force3", "k_pos", "reduce", "io", "md_step"};
 static_assert(KT_N <= FIB_NTIMERS, "timer table");
 
 struct RefCtl {
