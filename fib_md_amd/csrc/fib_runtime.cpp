@@ -1645,11 +1645,13 @@ thread_local TableCache g_tab;
 struct Arena {
   char *base;
   size_t size, used = 0;
+  bool full = false;  // an array did not fit (smaller ones after it may)
   template <typename T>
   T *take(size_t n) {
     const size_t b = (used + 255) & ~(size_t)255;
     const size_t e = b + std::max<size_t>(n, 1) * sizeof(T);
-    if (e > size) return nullptr;
+    full = full || e > size;
+    if (full) return nullptr;
     used = e;
     return reinterpret_cast<T *>(base + b);
   }
@@ -1748,7 +1750,7 @@ int32_t fib_arena_force(const fib_params *p, int32_t precision, int32_t natm, in
   d.G = A.take<char>(g4 * d.Wsw * NA);
   d.RA = A.take<uint32_t>((size_t)d.Wsw * NA);
   d.EX = A.take<char>(g4 * d.Wsw * NA);
-  if (!d.EX)
+  if (A.full)
     return bad(FIB_ERR_ARG, "fib_force_noalloc: the configuration needs more than the " +
                                 std::to_string(arena_bytes >> 20) + " MiB arena (" +
                                 std::to_string(d.nbucket) + " cell buckets)");
