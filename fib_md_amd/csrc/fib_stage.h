@@ -40,8 +40,9 @@ struct Parts {
 // A small call's arrays go as one copy, from or to a row of host memory: a
 // copy costs 10 us whatever it moves, pinned memory would gain 1 us in 11 for
 // 64 KiB and cost 100 us on the first call, and the lanes' threads cost 30 us
-// or more each (X, V, Xi and the types of 4 k, 12 k, 28 k and 100 k atoms: one
-// copy 53, 101, 201 and 595 us, lanes 117, 194, 240 and 640).  A large call's
+// or more each.  By one copy and by lanes: set_state of 2.2 MB 165 and 213 us,
+// of 4.0 MB 268 and 250, of 8.1 MB 490 and 355; state of 2.0 MB 194 and 206, of
+// 3.6 MB 410 and 233, of 7.3 MB 800 and 400.  A large call's
 // arrays go in chunks through LANES lanes, a host thread and a pinned chunk
 // each, so that the lanes empty or fill theirs while another's is on the bus.
 // One thread moves 25 GB/s between warm pages and pinned memory and 12 into
