@@ -142,6 +142,7 @@ struct RedSpec {
   int32_t bs;            // block size of the producing kernel
   int32_t sub;           // nv == 10: partials of the second of the three producers
                          // (at partials, + FIB_NRED * pstride, + twice that) per block
+                         // (0: by the instance's size, see k_tri)
   int32_t op[FIB_NRED];
   int32_t dst[FIB_NRED];
 };

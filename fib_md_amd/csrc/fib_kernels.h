@@ -7,6 +7,7 @@
 #include "fib_device.h"
 
 #define FIB_FIN_CH 256    // blocks whose partials one wavefront reduces (k_finalize)
+#define FIB_TRI_SMALL 98304  // most atoms of which 16 go to a wavefront of k_tri
 #define FIB_SORT_N 8192   // most atoms and buckets of an instance sorted by one workgroup
 #define FIB_LEAVE_CAP 256  // atoms that may leave the simulation in one MD step
 
@@ -94,7 +95,7 @@ struct DevBufs {
   double *Fout, *uout;       // force-only results [3*NA], [NA]
   double *partials;          // [3 * FIB_NRED * pstride], layout [region][slot][block]: the
                              // regions of k_legs (and every other reduction), k_tri, extra_pass
-  int max_pad;               // largest padded atom count of an instance
+  int max_pad, min_pad;      // largest and smallest padded atom count of an instance
   int max_bucket;            // most buckets of an instance
   double max_cell;           // largest cell volume
   double *fin_tmp;           // chunk results of big instances' reductions

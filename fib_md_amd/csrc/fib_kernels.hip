@@ -376,13 +376,15 @@ __device__ __forceinline__ void fin_chunk(double (&x)[NV], const DInst &in, int 
   fin_wave<NV>(x, rs);
 }
 // slot k of it, a sum over the regions of k_legs, k_tri (rs.sub partials, one
-// or four, for one of the others': see tri_partials) and extra_pass
+// or four, for one of the others', see tri_partials, or 0: one or four of four
+// places, by the instance) and extra_pass
 __device__ __forceinline__ double fin_chunk_slot(int k, const DInst &in, int c,
                                                  const double *__restrict__ partials, int pstride,
                                                  const RedSpec &rs) {
   const int blk0 = in.atom_off / rs.bs, nblk = in.natm_pad / rs.bs;
   const double *const p = partials + (size_t)k * pstride;
   const size_t reg = (size_t)FIB_NRED * pstride;
+  const bool four = rs.sub == 4 || (rs.sub == 0 && in.natm_pad <= FIB_TRI_SMALL);
   double x = 0;
 #pragma unroll
   for (int m = 0; m < FIN_CH / FIB_WAVE; ++m) {
@@ -390,8 +392,8 @@ __device__ __forceinline__ double fin_chunk_slot(int k, const DInst &in, int c,
     if (b < nblk) {
       const size_t at = (size_t)(blk0 + b);
       x += p[at];
-      const double *const t = p + reg + at * rs.sub;
-      x += rs.sub == 1 ? t[0] : (t[0] + t[1]) + (t[2] + t[3]);
+      const double *const t = p + reg + at * (rs.sub == 1 ? 1 : 4);
+      x += four ? (t[0] + t[1]) + (t[2] + t[3]) : t[0];
       x += p[2 * reg + at];
     }
   }
@@ -2386,9 +2388,10 @@ struct ExtraArgs {
 // wavefront and 300 us with one term per (leg, partner), 3,090 and 213 us
 // so; FP64 245 -> 173 us (2 x 512 k).  With the virial, its terms of a run
 // of 256 legs used to wait in 24 (FP64: 48) KiB of LDS, which left two blocks
-// to a CU; they now turn to their lanes through shuffles (mixed) or are summed
-// by their centre's lane from the stage (FP64), and three fit: 2.1 M atoms,
-// mixed, with energies, just built: 588 -> 477 us.
+// to a CU; they now turn to their lanes through shuffles, and three fit: 2.1 M
+// atoms, mixed, with energies, just built: 588 -> 477 us.  (Each centre summing
+// its own legs' terms would not depend on the split; in FP64 it took 570 to 640
+// us for the shuffles' 480 there, and 18 for 15.5 of 4 k atoms.)
 #ifndef TRI_BATCH
 #define TRI_BATCH 4  // 4: the next pass's positions load during this one; 2: only its row entries
 #endif
@@ -2411,7 +2414,7 @@ struct ExtraArgs {
 //   FP64   25, 13    30, 25   35, 38   59, 61
 // and with energies 23, 14; 27, 21; 32, 35; 43, 58 (mixed) and 28, 14; 34, 29;
 // 42, 45; 70, 73 (FP64): the lines between cross at 98 k to 109 k atoms.
-#define TRI_SMALL 98304
+#define TRI_SMALL FIB_TRI_SMALL
 // and of up to TRI_TINY eight, about 34 legs, one pass.  16 and 8 atoms:
 //            4,096    16,128   32,768   64,000 atoms
 //   mixed  12.5, 9.9  13, 11   14, 13   18, 20
@@ -2422,16 +2425,17 @@ struct TriStage {
   static constexpr int N = MIXED ? TRI_NS_MIXED : TRI_NS_FP64;
 };
 // The partial sums of k_tri, one per workgroup (of 256 or 64 atoms), from each
-// lane's sums (of its own atom; mixed virial: see there): neighbouring atoms
-// first, and pairs of wavefronts here as of workgroups in fin_chunk_slot, so
-// that an instance gives the same bits whether a wavefront has 64 atoms or 16.
-template <int APW>
-__device__ __forceinline__ void tri_partials(double (&v)[10], int lb, int pstride,
+// lane's sums (the energy, of its own atom; the virial, see there): neighbouring
+// atoms first, and pairs of wavefronts here as of workgroups in fin_chunk_slot,
+// so that an instance gives the energy's bits whether a wavefront has 64 atoms
+// or 16.
+template <int LANES>  // that hold sums: the atoms', or all where the virial's are
+__device__ __forceinline__ void tri_partials(double (&v)[10], int at, int pstride,
                                              double *__restrict__ partials) {
   constexpr int NW = FIB_BLOCK / FIB_WAVE;
   static_assert(NW == 4, "two levels");
   const int lane = threadIdx.x % FIB_WAVE, wid = threadIdx.x / FIB_WAVE;
-  for (int o = 1; o < APW; o <<= 1) {
+  for (int o = 1; o < LANES; o <<= 1) {
 #pragma unroll
     for (int k = 0; k < 10; ++k) v[k] += __shfl_xor(v[k], o);
   }
@@ -2442,7 +2446,7 @@ __device__ __forceinline__ void tri_partials(double (&v)[10], int lb, int pstrid
   __syncthreads();
   if (threadIdx.x < 10) {
     const int k = threadIdx.x;
-    partials[(size_t)k * pstride + lb] = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
+    partials[(size_t)k * pstride + at] = (red[0][k] + red[1][k]) + (red[2][k] + red[3][k]);
   }
 }
 
@@ -2502,6 +2506,8 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
   const uint64_t amc = lane < APW ? amv : 0ull;
   const int tci = type_of(meta_of(xc));
   const DInst &in = I[kin];
+  if constexpr (VIR && !MIXED)  // (the other launch has this instance: see force_ab)
+    if ((in.natm_pad <= TRI_SMALL) != (APW < FIB_WAVE)) return;
   // legs of the wave's atoms: this atom's are [exc, inc)
   const int nl = __popcll(amc);
   int inc = nl;
@@ -2707,37 +2713,10 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
         sG[wid][P.ps - fs + lane] = gv;
         sR[wid][P.ps - fs + lane] = ra;
       }
-      // r_a = x_a - x_i = -e_a / rinv_a
-      if constexpr (VIR && !MIXED) {
-        // each centre sums its own legs' terms, as its energy, in leg order:
-        // the sums do not depend on how many atoms a wavefront has
-        const T rl = -T(1) / La.rinv;
-        wave_lds_sync();
-        T4 r;
-        r.x = rl * La.e0; r.y = rl * La.e1; r.z = rl * La.e2; r.w = 0;
-        sE[wid][lane] = r;
-        wave_lds_sync();
-        const int nc = lane >= P.p0 && lane < P.p1 ? nl : 0;
-        constexpr int B = 4;  // legs whose values are read together
-        for (int l = 0; __ballot(l < nc) != 0ull; l += B) {
-          T v[B][6];
-#pragma unroll
-          for (int u = 0; u < B; ++u) {
-            const int q = l + u < nc ? exc - P.ps + l + u : 0;
-            const T4 x = sE[wid][q], g = sG[wid][P.ps - fs + q];
-            v[u][0] = x.x; v[u][1] = x.y; v[u][2] = x.z;
-            v[u][3] = g.x; v[u][4] = g.y; v[u][5] = g.z;
-          }
-#pragma unroll
-          for (int u = 0; u < B; ++u)
-            if (l + u < nc)
-#pragma unroll
-              for (int c = 0; c < 9; ++c) W[c] = fma_t(v[u][c / 3], v[u][3 + c % 3], W[c]);
-        }
-      } else if constexpr (VIR) {
-        // Lane q % 64 sums for leg q of a run (the FP32 sums then do not
-        // depend on how a run is cut into passes): the pass's values turn by
-        // its start.
+      if (VIR) {
+        // r_a = x_a - x_i = -e_a / rinv_a.  Lane q % 64 sums for leg q of a
+        // run (the FP32 sums of the mixed mode then do not depend on how a
+        // run is cut into passes): the pass's values turn by its start.
         const T rl = -T(1) / La.rinv;
         T v[6] = {rl * La.e0, rl * La.e1, rl * La.e2, Ga0, Ga1, Ga2};
         const int src = (lane - (P.ps - rs)) & (FIB_WAVE - 1);
@@ -2763,7 +2742,7 @@ __global__ __launch_bounds__(FIB_BLOCK) void k_tri(
     const double ws = MIXED ? fscale * lscale : 1.0;
 #pragma unroll
     for (int w = 0; w < 9; ++w) v[1 + w] = (double)W[w] * ws;
-    tri_partials<APW>(v, lb, pstride, partials);
+    tri_partials<VIR ? FIB_WAVE : APW>(v, VIR && !MIXED && APW == FIB_WAVE ? lb * NW : lb, pstride, partials);
   }
 }
 
@@ -3833,9 +3812,9 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
                        d.cnt_ion, d.nbr_ion, d.amask, d.Fpart, d.upart, d.near,
                        d.nst, d.ctl, d.binst, d.pstride, d.partials, d.halt, xcd_shift(d));
   }
-  const bool small = !(MIXED && VIR) && d.NA <= TRI_SMALL &&
-                     (EN || VIR || ((!d.tri_ns || d.tri_ns == TriStage<MIXED>::N) &&
-                                    (!d.tri_tb || d.tri_tb == TRI_BATCH)));
+  const bool small = !VIR && d.NA <= TRI_SMALL &&
+                     (EN || ((!d.tri_ns || d.tri_ns == TriStage<MIXED>::N) &&
+                             (!d.tri_tb || d.tri_tb == TRI_BATCH)));
   {
     KScope ks_(d, KT_TRI);
     // the MD step's variant (no energy, no virial) in every tile; the others
@@ -3845,7 +3824,7 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
     // extra_pass runs whenever its partials are reduced (energy, virial) or
     // stale-list terms can exist; the MD step's gate rules the latter out
     const bool xt = EN || VIR || extra;
-    const ExtraArgs xa{xt ? d.NA / FIB_BLOCK : 0, d.cnt_sw, d.disp, d.ctl, d.EX, d.EXself,
+    ExtraArgs xa{xt ? d.NA / FIB_BLOCK : 0, d.cnt_sw, d.disp, d.ctl, d.EX, d.EXself,
                        d.exmask, d.nst};
 #define TRI_LAUNCH(NS_, TB_, APW_)                                                            \
   do {                                                                                        \
@@ -3859,9 +3838,16 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
         d.pstride, d.partials + (size_t)FIB_NRED * d.pstride, d.binst, d.halt,                \
         xcd_shift(d) + (APW_ == 8 ? 3 : APW_ == 16 ? 2 : 0), xa);                             \
   } while (0)
-    // (the mixed mode's virial is summed in FP32 over runs of a wavefront's
-    // legs, which have to stay those of 64 atoms)
-    if (small) {
+    // (the virial is summed over runs of a wavefront's legs, so its bits depend
+    // on the split: in the mixed mode, FP32 sums, the runs stay those of 64
+    // atoms; in FP64 each instance has the split of its own size, whatever the
+    // batch's is, in one launch for each of the two that the batch holds)
+    if constexpr (VIR && !MIXED) {
+      const bool both = d.min_pad <= TRI_SMALL && d.max_pad > TRI_SMALL;
+      if (d.max_pad > TRI_SMALL) TRI_LAUNCH(TriStage<MIXED>::N, TRI_BATCH, FIB_WAVE);
+      if (both) xa.blocks = 0;
+      if (d.min_pad <= TRI_SMALL) TRI_LAUNCH(128, TRI_BATCH, 16);
+    } else if (small) {
       // (energies: 16 atoms per wavefront at least, see tri_partials)
       if constexpr (!EN && !VIR) {
         if (d.NA <= TRI_TINY) TRI_LAUNCH(128, TRI_BATCH, 8);
@@ -3884,7 +3870,7 @@ static void force_ab(const DevBufs &d, const FConst &fc, hipStream_t s, bool ext
   if (EN || VIR) {
     int op[10], dst[10];
     for (int k = 0; k < 10; ++k) { op[k] = 0; dst[k] = DCTL_IDX(utot) + k; }
-    finalize(d, 10, FIB_BLOCK, op, dst, s, small ? 4 : 1);
+    finalize(d, 10, FIB_BLOCK, op, dst, s, VIR && !MIXED ? 0 : small ? 4 : 1);
   }
 }
 

@@ -492,10 +492,12 @@ extern "C" int32_t fib_create(const fib_params *p, int32_t ninst, const fib_inst
   d.pstride = d.NA / FIB_WAVE + 1;
   take(d.partials, (size_t)d.pstride * FIB_NRED * 3);
   d.max_pad = 0;
+  d.min_pad = std::numeric_limits<int>::max();
   d.max_bucket = 0;
   d.max_cell = 0;
   for (const DInst &in : h->inst) {
     d.max_pad = std::max(d.max_pad, in.natm_pad);
+    d.min_pad = std::min(d.min_pad, in.natm_pad);
     d.max_bucket = std::max(d.max_bucket, in.nbucket);
     h->stage.fit((size_t)d.max_pad);
     d.max_cell = std::max(d.max_cell, in.h[0] * in.h[1] * in.h[2]);
@@ -1701,7 +1703,7 @@ int32_t fib_arena_force(const fib_params *p, int32_t precision, int32_t natm, in
   d.Wsw = 32;
   d.Wion = 64;
   d.pstride = d.NA / FIB_WAVE + 1;
-  d.max_pad = in.natm_pad;
+  d.max_pad = d.min_pad = in.natm_pad;
   d.max_bucket = in.nbucket;
   d.max_cell = in.h[0] * in.h[1] * in.h[2];
   const size_t NA = (size_t)d.NA;

@@ -57,10 +57,10 @@ def test_small_instances_beside_one_of_several_chunks(precision):
         assert np.abs(out[k]["virial"] - own["virial"]).max() <= 1e-11 * np.abs(own["virial"]).max()
 
 
-# beside a 4 x 4 x 4 crystal (513 atoms): a batch of up to 131,072 atoms, one
+# beside a 4 x 4 x 4 crystal (513 atoms): a batch of up to 98,304 atoms, one
 # of more (another split of the vertex pass), and instances just below and
 # above that size themselves
-@pytest.mark.parametrize("other", [(9, 8, 7), (25, 25, 26), (26, 25, 26), (5, 5, 41)])
+@pytest.mark.parametrize("other", [(9, 8, 7), (24, 23, 22), (32, 24, 16), (25, 25, 26), (5, 5, 41)])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_energies_and_virial_have_the_bits_of_the_instance_alone(other, precision):
     """Sums within an instance have an order that depends on it alone."""
